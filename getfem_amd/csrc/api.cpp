@@ -375,20 +375,43 @@ int gfx_mesh_im_destroy(gfx_mesh_im *mim) {
 }
 
 // ---------------------------------------------------------------- plans
+// The smallest value of a coefficient: the matrix-core forms ask for it at
+// every assembly, so it is known whenever one of them is the plan's form.
+static int coef_minimum(gfx_plan *p, int slot) {
+  if (p->min_known[slot]) return GFX_OK;
+  gfx_ctx *c = p->ctx;
+  const size_t n = (size_t)p->mf->mesh->n_cv;
+  p->coef_min[slot] = p->coef[slot].value;
+  if (p->coef[slot].kind == GFX_COEF_PER_ELEMENT) {
+    std::vector<double> h(n);
+    HIPCHK(c, hipMemcpyAsync(h.data(), p->d_coef[slot], 8 * n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    p->coef_min[slot] = n ? *std::min_element(h.begin(), h.end()) : 0.0;
+  }
+  p->min_known[slot] = true;
+  return GFX_OK;
+}
+
 static int plan_upload_coef(gfx_plan *p, int slot, const gfx_coef *cf) {
   gfx_ctx *c = p->ctx;
   if (cf->kind != GFX_COEF_CONST && cf->kind != GFX_COEF_PER_ELEMENT)
     return fail(c, GFX_E_INVALID, "unknown coefficient kind");
+  if (cf->kind == GFX_COEF_PER_ELEMENT && !cf->h_values)
+    return fail(c, GFX_E_INVALID, "per-element coefficient without values");
   p->coef[slot] = *cf;
   p->coef[slot].h_values = nullptr;
-  p->coef_min[slot] = cf->value;
-  dfree(p->d_coef[slot]);
   if (cf->kind == GFX_COEF_PER_ELEMENT) {
-    if (!cf->h_values) return fail(c, GFX_E_INVALID, "per-element coefficient without values");
-    const int64_t n = p->mf->mesh->n_cv;
-    p->coef_min[slot] = n ? *std::min_element(cf->h_values, cf->h_values + n) : 0.0;
-    HIPCHK(c, dalloc(&p->d_coef[slot], (size_t)n));
-    HIPCHK(c, hipMemcpy(p->d_coef[slot], cf->h_values, 8 * (size_t)n, hipMemcpyHostToDevice));
+    // into the buffer that the slot has (an allocation and a free each time
+    // would wait for the device twice), after the assemblies that read it
+    const size_t n = (size_t)p->mf->mesh->n_cv;
+    if (!p->d_coef[slot]) HIPCHK(c, dalloc(&p->d_coef[slot], n));
+    HIPCHK(c, hipMemcpyAsync(p->d_coef[slot], cf->h_values, 8 * n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
+  p->min_known[slot] = false;
+  if (p->precision >= GFX_PREC_BF16X2) {
+    int r = coef_minimum(p, slot);
+    if (r) return r;
   }
   p->values_changed = true;  // thresholds and pattern are re-derived at the next assembly
   return GFX_OK;
@@ -408,7 +431,7 @@ int gfx_plan_destroy(gfx_plan *p) {
   if (p->fork) (void)hipEventDestroy(p->fork);
   dfree(p->d_coef[0]); dfree(p->d_coef[1]); dfree(p->d_coef[2]);
   dfree(p->d_gref); dfree(p->d_qw); dfree(p->d_R);
-  dfree(p->d_rec); dfree(p->d_thr); dfree(p->d_keep);
+  dfree(p->d_rec); dfree(p->d_thr); dfree(p->d_keep); dfree(p->d_sig); dfree(p->d_Rp);
   dfree(p->d_gref32); dfree(p->d_qw32); dfree(p->d_R32); dfree(p->d_rec32); dfree(p->d_Rq); dfree(p->d_E32);
   dfree(p->d_E64);
   dfree(p->d_inc_ptr); dfree(p->d_inc); dfree(p->d_slot); dfree(p->d_nslots); dfree(p->d_order); dfree(p->d_desc);
@@ -552,6 +575,16 @@ int gfx_plan_create(gfx_mesh_fem *mf, gfx_mesh_im *mim, int term, const gfx_coef
     detect_int_reference(R, nd * nd, p->rk, p->r_L, rq);
     if (p->rk && e == hipSuccess) e = dalloc(&p->d_Rq, rq.size());
     if (p->rk && e == hipSuccess) e = hipMemcpy(p->d_Rq, rq.data(), rq.size(), hipMemcpyHostToDevice);
+    // upper pairs for the threshold pass (the integers N where R has that form)
+    std::vector<double> Rp;
+    for (int i = 0; i < nd; ++i)
+      for (int j = i; j < nd; ++j)
+        for (int t = 0; t < 9; ++t) {
+          const double r = R[((size_t)i * nd + j) * 9 + t];
+          Rp.push_back(p->rk ? std::nearbyint(r * p->r_L) : r);
+        }
+    if (e == hipSuccess) e = dalloc(&p->d_Rp, Rp.size());
+    if (e == hipSuccess) e = hipMemcpy(p->d_Rp, Rp.data(), 8 * Rp.size(), hipMemcpyHostToDevice);
   }
   if (!eb) {  // FP32 copies of the tables for the FP32 contraction form
     std::vector<float> gref32(gref.begin(), gref.end()), R32(R.begin(), R.end());
@@ -584,28 +617,61 @@ int gfx_plan_set_form(gfx_plan *p, int form, int precision) {
     return fail(p->ctx, GFX_E_UNSUPPORTED,
                 "the element-batched matrix-core forms need isotropic elasticity on a P2 or P3 vector field "
                 "of an affine tet mesh");
+  if (precision >= GFX_PREC_BF16X2) {
+    if (set_device(p->ctx)) return GFX_E_HIP;
+    int r;
+    if ((r = coef_minimum(p, 0)) || (r = coef_minimum(p, 1))) return r;
+  }
   p->form = form;
   p->precision = precision;
   return GFX_OK;
 }
 
-// Element records for the pattern build (FP64, no thresholds yet) or for an
-// assembly (with thresholds; FP32 records for the FP32 contraction form).
-static int plan_records(gfx_plan *p, bool with_thr) {
+static RecordArgs record_args(gfx_plan *p) {
   const gfx_mesh *m = p->mf->mesh;
-  gfx_ctx *c = p->ctx;
-  const bool fp32 = with_thr && p->precision == GFX_PREC_FP32;
-  if (fp32 && !p->d_rec32) HIPCHK(c, dalloc(&p->d_rec32, (size_t)kRecStride * m->n_cv));
   // coefficient c of the record: mu for elasticity (its Laplacian part), the
   // third coefficient of the isotropic term, none for the Laplacian
   const int sc = p->term == GFX_TERM_ISOTROPIC ? 2 : (p->term == GFX_TERM_ISO_ELAST ? 1 : -1);
   auto dptr = [&](int k) -> const double * {
     return k >= 0 && p->coef[k].kind == GFX_COEF_PER_ELEMENT ? p->d_coef[k] : nullptr;
   };
-  HIPCHK(c, launch_records_tet(c->stream, m->n_cv, m->d_pts, m->d_cvx, dptr(0), p->coef[0].value,
-                               dptr(1), p->coef[1].value, dptr(sc), sc >= 0 ? p->coef[sc].value : 0.0,
-                               with_thr ? p->d_thr : nullptr, p->rk ? 1.0 / p->r_L : 1.0, p->d_rec,
-                               fp32 ? p->d_rec32 : nullptr, p->d_err));
+  RecordArgs a{};
+  a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx;
+  a.ca = dptr(0); a.cb = dptr(1); a.cc = dptr(sc);
+  a.ca_c = p->coef[0].value; a.cb_c = p->coef[1].value; a.cc_c = sc >= 0 ? p->coef[sc].value : 0.0;
+  a.r_scale = p->rk ? 1.0 / p->r_L : 1.0;
+  a.rec = p->d_rec; a.err = p->d_err;
+  return a;
+}
+
+// the FP32 contraction form's records, allocated on its first use
+static int records32(gfx_plan *p, RecordArgs &a) {
+  if (p->precision != GFX_PREC_FP32) return GFX_OK;
+  if (!p->d_rec32) HIPCHK(p->ctx, dalloc(&p->d_rec32, (size_t)kRecStride * p->mf->mesh->n_cv));
+  a.rec32 = p->d_rec32;
+  return GFX_OK;
+}
+
+// Element records of an assembly at unchanged values (the thresholds stand).
+static int plan_records(gfx_plan *p) {
+  RecordArgs a = record_args(p);
+  int r;
+  if ((r = records32(p, a))) return r;
+  HIPCHK(p->ctx, launch_records_tet(p->ctx->stream, a, p->d_thr));
+  return GFX_OK;
+}
+
+// Records, thresholds and keep bits at the current values; check: the keep
+// signature is compared with the stored one, not written.
+static int plan_keep(gfx_plan *p, bool check) {
+  gfx_ctx *c = p->ctx;
+  const int64_t n_cv = p->mf->mesh->n_cv;
+  RecordArgs a = record_args(p);
+  int r;
+  if ((r = records32(p, a))) return r;
+  if (!p->d_sig) HIPCHK(c, dalloc(&p->d_sig, (size_t)keep_sig_words(p->term, p->nd, p->qdim, n_cv)));
+  HIPCHK(c, launch_keep(c->stream, p->term, p->nd, p->qdim, a, p->d_Rp, p->d_sig, check, p->d_thr, p->d_keep,
+                        p->kwords));
   return GFX_OK;
 }
 
@@ -803,12 +869,12 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   hipStream_t s = c->stream;
   int r;
   HIPCHK(c, hipMemsetAsync(p->d_err, 0, 4, s));
-  if (!p->eb && (r = plan_records(p, false))) return r;  // element-batched: with the keep bits below
   // incidences
   dfree(p->d_inc_ptr); dfree(p->d_inc); dfree(p->d_slot); dfree(p->d_nslots); dfree(p->d_order); dfree(p->d_desc);
   dfree(p->d_node_ok);
   dfree(p->d_nbr); dfree(p->d_mask); dfree(p->d_indptr); dfree(p->d_indices); dfree(p->d_vals);
-  dfree(p->d_keep);
+  dfree(p->d_keep); dfree(p->d_sig);
+  p->keep_ok = false;
   p->nnz = -1;
   p->bins.clear();
   p->n_inc = n_cv * nd;
@@ -849,13 +915,12 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   HIPCHK(c, dalloc(&p->d_keep, (size_t)n_cv * p->kwords));
   PatternArgs a{};
   a.n_cv = n_cv; a.n_nodes = nn; a.nd = nd; a.qdim = Q; a.nloc = p->nloc;
-  a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.rec = p->d_rec;
-  a.gref = p->d_gref; a.qw = p->d_qw; a.nq = p->nq; a.thr = p->d_thr; a.keep = p->d_keep;
+  a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.keep = p->d_keep;
   a.inc_ptr = p->d_inc_ptr; a.inc = p->d_inc; a.err = p->d_err;
   if (p->eb) {
     if ((r = plan_eb_elements(p, GFX_PREC_FP64, true))) return r;
   } else {
-    HIPCHK(c, launch_keep(s, p->term, a));
+    if ((r = plan_keep(p, false))) return r;
   }
   // patches (the patch kernel addresses presence words and slot pairs with
   // 32-bit word offsets)
@@ -901,6 +966,7 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   // the keep bits stay: re-validation after a change of values compares
   // the pattern they give with this one
   p->nnz = nnz;
+  p->keep_ok = true;
   p->pts_version = m->version;
   p->values_changed = false;
   p->pattern_id++;
@@ -910,49 +976,59 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
 
 // The values behind the stored pattern changed (coefficients, node positions
 // or state): re-derive the per-element thresholds and keep bits at the new
-// values, as GetFEM's per-assembly threshold does, and compare the presence
-// bits they give with the stored ones.  Equal: the pattern stands and the
-// new thresholds are used.  Different: the pattern is rebuilt (refused while
-// pinned).  A degenerate element is reported here, like GetFEM's "Non
-// invertible matrix" at every assembly.  For element-batched plans the FP64
-// element matrices computed here serve the assembly that follows (*eb_fresh).
-static int plan_validate(gfx_plan *p, bool *eb_fresh) {
+// values, as GetFEM's per-assembly threshold does, and see whether the
+// pattern they give is the stored one.  The keep bits of the affine terms are
+// compared with the stored ones first: the same bits give the same pattern.
+// Where they differ the presence bits they give are compared with the stored
+// ones.  Equal: the pattern stands and the new thresholds are used.
+// Different: the pattern is rebuilt (refused while pinned).  A degenerate
+// element is reported here, like GetFEM's "Non invertible matrix" at every
+// assembly.  The records (affine terms) or FP64 element matrices computed here
+// serve the assembly that follows (*fresh).
+static int plan_validate(gfx_plan *p, bool *fresh) {
   gfx_ctx *c = p->ctx;
   const gfx_mesh *m = p->mf->mesh;
   hipStream_t s = c->stream;
-  *eb_fresh = false;
+  *fresh = false;
   if (p->nnz == 0) {  // no element: nothing to re-derive
     p->pts_version = m->version;
     p->values_changed = false;
     return GFX_OK;
   }
-  int r;
+  int r, flag = 0;
+  auto read_flag = [&]() -> int {
+    HIPCHK(c, hipMemcpyAsync(&flag, p->d_err, 4, hipMemcpyDeviceToHost, s));
+    HIPCHK(c, hipStreamSynchronize(s));
+    return GFX_OK;
+  };
   HIPCHK(c, hipMemsetAsync(p->d_err, 0, 4, s));
+  if (!p->eb && p->keep_ok) {
+    if ((r = plan_keep(p, true)) || (r = read_flag())) return r;
+    if (flag & 1) return fail(c, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
+    if (!(flag & 32)) {
+      p->pts_version = m->version;
+      p->values_changed = false;
+      *fresh = true;
+      return GFX_OK;
+    }
+  }
+  p->keep_ok = false;  // until the new bits' pattern is confirmed or built
   if (!p->d_keep) HIPCHK(c, dalloc(&p->d_keep, (size_t)m->n_cv * p->kwords));
   PatternArgs a{};
   a.n_cv = m->n_cv; a.n_nodes = p->n_nodes; a.nd = p->nd; a.qdim = p->qdim; a.nloc = p->nloc;
-  a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.rec = p->d_rec;
-  a.gref = p->d_gref; a.qw = p->d_qw; a.nq = p->nq; a.thr = p->d_thr; a.keep = p->d_keep;
+  a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.keep = p->d_keep;
   a.inc_ptr = p->d_inc_ptr; a.inc = p->d_inc; a.slot = p->d_slot; a.nslots = p->d_nslots;
   a.mask = p->d_mask; a.err = p->d_err;
   if (!p->d_node_ok) HIPCHK(c, dalloc(&p->d_node_ok, (size_t)std::max<int64_t>(p->n_nodes, 1)));
   a.node_ok = p->d_node_ok;
-  if (p->eb) {
-    if ((r = plan_eb_elements(p, GFX_PREC_FP64, true))) return r;
-  } else {
-    if ((r = plan_records(p, false))) return r;
-    HIPCHK(c, launch_keep(s, p->term, a));
-  }
+  if ((r = p->eb ? plan_eb_elements(p, GFX_PREC_FP64, true) : plan_keep(p, false))) return r;
   // nodes whose rows keep every entry are confirmed by one pass; the exact
   // check runs only when some node is not
   HIPCHK(c, launch_mask_fast(s, a));
-  int flag = 0;
-  HIPCHK(c, hipMemcpyAsync(&flag, p->d_err, 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(c, hipStreamSynchronize(s));
+  if ((r = read_flag())) return r;
   if (flag & 16) {
     HIPCHK(c, launch_mask_exact(s, a, p->max_nslots));
-    HIPCHK(c, hipMemcpyAsync(&flag, p->d_err, 4, hipMemcpyDeviceToHost, s));
-    HIPCHK(c, hipStreamSynchronize(s));
+    if ((r = read_flag())) return r;
   }
   if (flag & 1) return fail(c, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
   if (flag & 4) {
@@ -961,12 +1037,13 @@ static int plan_validate(gfx_plan *p, bool *eb_fresh) {
                                   "(callers hold its CSR arrays): unpin it and assemble again");
     int64_t nnz = 0;
     if ((r = gfx_plan_build_pattern(p, &nnz))) return r;
-    *eb_fresh = p->eb;  // the rebuild ran the FP64 element kernel at the current values
+    *fresh = true;  // the rebuild ran at the current values
     return GFX_OK;
   }
+  p->keep_ok = true;
   p->pts_version = m->version;
   p->values_changed = false;
-  *eb_fresh = p->eb;
+  *fresh = true;
   return GFX_OK;
 }
 
@@ -976,9 +1053,9 @@ int gfx_plan_assemble(gfx_plan *p) {
   if (p->nnz < 0) return fail(c, GFX_E_STATE, "build the pattern first");
   if (set_device(c)) return GFX_E_HIP;
   int r;
-  bool eb_fresh = false;  // element-batched: E and thresholds already computed in FP64
+  bool fresh = false;  // element-batched: E and thresholds already computed in FP64; else the records
   if (p->values_changed || p->pts_version != p->mf->mesh->version)
-    if ((r = plan_validate(p, &eb_fresh))) return r;
+    if ((r = plan_validate(p, &fresh))) return r;
   hipEvent_t *ev = nullptr;
   if (p->timing) {
     const size_t need = 3 * (size_t)(p->n_timed + 1);
@@ -991,8 +1068,8 @@ int gfx_plan_assemble(gfx_plan *p) {
     p->n_timed++;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
   }
-  if (!(eb_fresh && p->precision == GFX_PREC_FP64))
-    if ((r = p->eb ? plan_eb_elements(p, p->precision) : plan_records(p, true))) return r;
+  if (!fresh || (p->eb && p->precision != GFX_PREC_FP64))
+    if ((r = p->eb ? plan_eb_elements(p, p->precision) : plan_records(p))) return r;
   const bool bdb = !p->eb && p->precision >= GFX_PREC_BF16X2;
   const bool bdb64 = bdb && p->precision == GFX_PREC_FP64_MFMA;
   if (bdb) {  // element matrices on the matrix cores, then the node-patch gather below

@@ -105,16 +105,24 @@ struct PatchArgs {
   int lds_flat;
 };
 
+// What the element records are formed from, and where they go.
+struct RecordArgs {
+  int64_t n_cv;
+  const double *pts;
+  const int32_t *cvx;
+  const double *ca, *cb, *cc;  // per-element coefficients or null (then ca_c, ...)
+  double ca_c, cb_c, cc_c;
+  double r_scale;              // scale of the reference tensor
+  double *rec;                 // kRecStride doubles per element
+  float *rec32;                // the FP32 form's records, or null
+  int *err;                    // bit 1: det K = 0
+};
+
 struct PatternArgs {
   int64_t n_cv, n_nodes;
   int nd, qdim, nloc, kwords, mwpi;
   const int32_t *dofs;
-  const double *rec;
-  const double *gref;
-  const double *qw;
-  int nq;
-  double *thr;              // out: per element threshold
-  uint32_t *keep;           // out: per element keep bits (row-major nloc x nloc)
+  uint32_t *keep;           // per element keep bits (row-major nloc x nloc)
   int32_t *inc_ptr;
   uint32_t *inc;
   uint16_t *slot;
@@ -274,15 +282,17 @@ void ref(gfx_mesh_im *mim);
 void unref(gfx_mesh_im *mim);
 
 // kernel launch wrappers (kernels.hip)
-hipError_t launch_records_tet(hipStream_t s, int64_t n_cv, const double *pts,
-                              const int32_t *cvx, const double *ca, double ca_c,
-                              const double *cb, double cb_c, const double *cc, double cc_c,
-                              const double *thr, double r_scale, double *rec, float *rec32,
-                              int *err);
+hipError_t launch_records_tet(hipStream_t s, const RecordArgs &a, const double *thr);
 hipError_t launch_incidences(hipStream_t s, int64_t n_cv, int nd, int qdim,
                              const int32_t *dofs, int64_t n_nodes,
                              int32_t *inc_ptr, uint32_t *inc, int32_t *tmp);
-hipError_t launch_keep(hipStream_t s, int term, const PatternArgs &a);
+// Records with thresholds and the keep signature (keep_sig_words u64) of
+// every element; Rp: the upper pairs' reference blocks in the records' scale.
+// check: the signature is compared with sig (bit 32 of the error flag when it
+// differs), else it is written, and the keep words formed from it.
+int64_t keep_sig_words(int term, int nd, int qdim, int64_t n_cv);
+hipError_t launch_keep(hipStream_t s, int term, int nd, int qdim, const RecordArgs &a, const double *Rp,
+                       uint64_t *sig, bool check, double *thr, uint32_t *keep, int kwords);
 hipError_t launch_patch_build(hipStream_t s, const PatternArgs &a, int max_cand);
 hipError_t launch_fill_columns(hipStream_t s, const PatternArgs &a);
 // the pattern check against new keep bits: the thread-per-node pass (sets bit
@@ -423,7 +433,8 @@ struct gfx_plan {
   int nd = 0, qdim = 1, nloc = 0, nq = 0, nv = 4;
   int kwords = 0, mwpi = 0;
   gfx_coef coef[3];
-  double coef_min[3] = {0.0, 0.0, 0.0};  // smallest value of each coefficient (host copy)
+  double coef_min[3] = {0.0, 0.0, 0.0};  // smallest value of each coefficient, where min_known
+  bool min_known[3] = {false, false, false};
   double *d_coef[3] = {nullptr, nullptr, nullptr};
   // The stored pattern is GetFEM's for the values it was built from.  After
   // the coefficients, the node positions (mesh version) or the state change,
@@ -445,7 +456,14 @@ struct gfx_plan {
   int rk = 0;
   double r_L = 1.0;
   uint8_t *d_Rq = nullptr;
+  // Keep bits of every element: as words (what the presence bits are made
+  // of) and, for the affine terms, as the signature that a check compares.
+  // keep_ok: they are those that the stored pattern was built from or
+  // confirmed with (false while a refused change of pattern is pending).
   uint32_t *d_keep = nullptr;
+  uint64_t *d_sig = nullptr;
+  double *d_Rp = nullptr;        // upper pairs' reference blocks, nd (nd + 1) / 2 x 9, in the records' scale
+  bool keep_ok = false;
   int64_t n_nodes = 0, n_inc = 0;
   int32_t *d_inc_ptr = nullptr;
   uint32_t *d_inc = nullptr;

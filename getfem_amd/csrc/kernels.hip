@@ -5,7 +5,8 @@
 // for the GPU):
 //   k_records_tet    per element, FP64: K = G grad(N), det K, B = K^{-T}
 //                    (bgeot_geometric_trans.cc:270-413) and the element's
-//                    coefficients -> one 128-byte record per element.
+//                    coefficients -> one 128-byte record per element (after
+//                    a change of values k_keep, with the new thresholds).
 //   k_assemble_patch one wavefront per group of up to 4 mesh nodes
 //                    ("patches"): for every element incident to a node,
 //                    computes the rows of the element matrix that belong to
@@ -34,59 +35,57 @@ __device__ __forceinline__ int64_t gtid() {
   return (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
 }
 
-__device__ __forceinline__ double wave_max(double v) {
-  for (int o = kWave / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kWave));
-  return v;
-}
-
 // ------------------------------------------------------------------------
 // geometry
 // ------------------------------------------------------------------------
+// One element's record: B = K^{-T} from cofactors, row-major B(r,c) = o[3r+c];
+// then the factorized form's scales |J| a s and |J| b s (s: the scale of the
+// stored reference tensor, 1/L for an integer table R = N/L), the insertion
+// threshold (0 here), the per-point form's |J| a, |J| b, |J| c, and |J| c s.
+// False where det K = 0.
+__device__ __forceinline__ bool tet_record(int64_t e, const RecordArgs &a, double (&o)[16]) {
+  const int4 v = *reinterpret_cast<const int4 *>(a.cvx + 4 * e);
+  const double *p0 = a.pts + 3 * (int64_t)v.x, *p1 = a.pts + 3 * (int64_t)v.y;
+  const double *p2 = a.pts + 3 * (int64_t)v.z, *p3 = a.pts + 3 * (int64_t)v.w;
+  // column-major K(r,c) = k[r + 3c] = x_{c+1}[r] - x_0[r]  (G . grad N for
+  // the P1 transformation)
+  double k[9];
+  for (int r = 0; r < 3; ++r) {
+    const double x0 = p0[r];
+    k[r] = p1[r] - x0;
+    k[r + 3] = p2[r] - x0;
+    k[r + 6] = p3[r] - x0;
+  }
+  const double a0 = k[4] * k[8] - k[5] * k[7];
+  const double a1 = k[5] * k[6] - k[3] * k[8];
+  const double a2 = k[3] * k[7] - k[4] * k[6];
+  const double J = k[0] * a0 + k[1] * a1 + k[2] * a2;
+  o[0] = a0 / J; o[1] = (k[2] * k[7] - k[1] * k[8]) / J;
+  o[2] = (k[1] * k[5] - k[2] * k[4]) / J; o[3] = a1 / J;
+  o[4] = (k[0] * k[8] - k[2] * k[6]) / J; o[5] = (k[2] * k[3] - k[0] * k[5]) / J;
+  o[6] = a2 / J; o[7] = (k[1] * k[6] - k[0] * k[7]) / J;
+  o[8] = (k[0] * k[4] - k[1] * k[3]) / J;
+  const double aJ = fabs(J), va = a.ca ? a.ca[e] : a.ca_c, vb = a.cb ? a.cb[e] : a.cb_c;
+  const double vc = a.cc ? a.cc[e] : a.cc_c;
+  o[9] = aJ * va * a.r_scale; o[10] = aJ * vb * a.r_scale;
+  o[11] = 0.0;
+  o[12] = aJ * va; o[13] = aJ * vb; o[14] = aJ * vc; o[15] = aJ * vc * a.r_scale;
+  return J != 0.0;
+}
+
 // rec (FP64) or rec32 (FP32 contraction form, 64 bytes per element) is written
-__global__ __launch_bounds__(256) void k_records_tet(
-    int64_t n_cv, const double *__restrict__ pts, const int32_t *__restrict__ cvx,
-    const double *__restrict__ ca, double ca_c, const double *__restrict__ cb,
-    double cb_c, const double *__restrict__ cc, double cc_c, const double *__restrict__ thr,
-    double r_scale, double *__restrict__ rec, float *__restrict__ rec32, int *__restrict__ err) {
+__global__ __launch_bounds__(256) void k_records_tet(RecordArgs a, const double *__restrict__ thr) {
   // The block's records are staged in LDS (rows padded by one 16-byte piece
   // against bank conflicts) and written back as one contiguous run: 16-byte
   // pieces of consecutive records from consecutive threads.
   __shared__ double2 stage[256 * 9];
   const int64_t e0 = (int64_t)blockIdx.x * 256, e = e0 + threadIdx.x;
-  const int nblk = (int)min<int64_t>(256, n_cv - e0);
-  if (e < n_cv) {
-    const int4 v = *reinterpret_cast<const int4 *>(cvx + 4 * e);
-    const double *p0 = pts + 3 * (int64_t)v.x, *p1 = pts + 3 * (int64_t)v.y;
-    const double *p2 = pts + 3 * (int64_t)v.z, *p3 = pts + 3 * (int64_t)v.w;
-    // column-major K(r,c) = k[r + 3c] = x_{c+1}[r] - x_0[r]  (G . grad N for
-    // the P1 transformation)
-    double k[9];
-    for (int r = 0; r < 3; ++r) {
-      const double x0 = p0[r];
-      k[r] = p1[r] - x0;
-      k[r + 3] = p2[r] - x0;
-      k[r + 6] = p3[r] - x0;
-    }
-    const double a0 = k[4] * k[8] - k[5] * k[7];
-    const double a1 = k[5] * k[6] - k[3] * k[8];
-    const double a2 = k[3] * k[7] - k[4] * k[6];
-    const double J = k[0] * a0 + k[1] * a1 + k[2] * a2;
-    if (J == 0.0) { atomicOr(err, 1); }
-    // Record: B = K^{-T} from cofactors, row-major B(r,c) = o[3r+c]; then the
-    // factorized form's scales |J| a s and |J| b s (s: the scale of the stored
-    // reference tensor, 1/L for an integer table R = N/L), the insertion
-    // threshold, the per-point form's |J| a, |J| b, |J| c, and |J| c s
+  const int nblk = (int)min<int64_t>(256, a.n_cv - e0);
+  float *rec32 = a.rec32;
+  if (e < a.n_cv) {
     double o[16];
-    o[0] = a0 / J; o[1] = (k[2] * k[7] - k[1] * k[8]) / J;
-    o[2] = (k[1] * k[5] - k[2] * k[4]) / J; o[3] = a1 / J;
-    o[4] = (k[0] * k[8] - k[2] * k[6]) / J; o[5] = (k[2] * k[3] - k[0] * k[5]) / J;
-    o[6] = a2 / J; o[7] = (k[1] * k[6] - k[0] * k[7]) / J;
-    o[8] = (k[0] * k[4] - k[1] * k[3]) / J;
-    const double aJ = fabs(J), va = ca ? ca[e] : ca_c, vb = cb ? cb[e] : cb_c;
-    const double vc = cc ? cc[e] : cc_c;
-    o[9] = aJ * va * r_scale; o[10] = aJ * vb * r_scale;
-    o[11] = thr ? thr[e] : 0.0;
-    o[12] = aJ * va; o[13] = aJ * vb; o[14] = aJ * vc; o[15] = aJ * vc * r_scale;
+    if (!tet_record(e, a, o)) atomicOr(a.err, 1);
+    if (thr) o[11] = thr[e];
     if (rec32) {
       float4 *st4 = reinterpret_cast<float4 *>(stage + 9 * threadIdx.x);
       for (int t = 0; t < 4; ++t)
@@ -99,7 +98,7 @@ __global__ __launch_bounds__(256) void k_records_tet(
   // 16-byte pieces: 8 per FP64 record, 4 per FP32 record
   const int per = rec32 ? 4 : 8;
   double2 *dst = rec32 ? reinterpret_cast<double2 *>(rec32 + (int64_t)kRecStride * e0)
-                       : reinterpret_cast<double2 *>(rec + (int64_t)kRecStride * e0);
+                       : reinterpret_cast<double2 *>(a.rec + (int64_t)kRecStride * e0);
   for (int x = threadIdx.x; x < nblk * per; x += 256) {
     const int r = x / per, piece = x - r * per;
     dst[x] = stage[9 * r + piece];
@@ -236,48 +235,151 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 }
 
 // ------------------------------------------------------------------------
-// per-element threshold and keep bits (one wavefront per element)
+// per-element threshold and keep signature
 // ------------------------------------------------------------------------
+// One lane per element, 64 elements per workgroup; the element's pair blocks
+// (i <= j: the matrix is symmetric) are shared out between the workgroup's
+// kKeepWaves wavefronts.  Pass 1 takes the largest entry (threshold 1e-14
+// max|elem|, an all-zero element gets infinity: GetFEM skips it,
+// compile_and_exec.cc:5441-5442), pass 2 forms the blocks again and compares.
+// The blocks are those of the factorized form, G = B R_ij B^T: an integral
+// instead of a sum over the points (P2: 63 products a block instead of 600),
+// and the reference blocks are the same for every lane, so they come through
+// the scalar cache as one operand of each product.  A comparison's result is
+// a 64-bit scalar, one bit per element; those scalars are the keep
+// signature, sig[group of 64 elements][pair][value] (value: (a, b) row-major,
+// or the one trace of a Laplacian).  Checking a pattern compares them with
+// the stored ones (CHECK: bit 32 of the error flag when any differs), on the
+// scalar unit.  The element records, needed with the threshold by the
+// assembly that follows, are formed here too (they would cost a launch and a
+// pass over the elements before and after).
+// Bound by FP64 issue: 8,000 products and sums a lane, 0.57 of the rate.
+// Measured at P2 elasticity, 40^3 x 6 = 384,000 elements: 146 us, and no
+// pattern pass where the bits stay, against 3,553 us of per-point blocks (a
+// wavefront per element, all pairs, twice) with 394 us of presence-bit passes
+// after them and 15 us of records before and after; an assembly with new
+// coefficients 4.91 -> 0.59 ms.
+constexpr int kKeepWaves = 4;
+
 template <int Q, int TERM>
-__global__ __launch_bounds__(256) void k_keep(PatternArgs a) {
-  extern __shared__ uint32_t kbits[];  // 4 waves x kwords
-  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  const int64_t e = (int64_t)blockIdx.x * 4 + w;
-  const bool live = e < a.n_cv;
-  const int nd = a.nd, nl = a.nloc, npair = nd * nd;
-  uint32_t *my = kbits + w * a.kwords;
-  for (int t = lane; t < a.kwords; t += kWave) my[t] = 0u;
+__device__ __forceinline__ void keep_block(const double *__restrict__ r, const double (&B)[9], double sa, double sb,
+                                           double sc, double (&v)[TERM == GFX_TERM_LAPLACE ? 1 : Q * Q]) {
+  double T[3][3], G[3][3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) T[c][b] = r[3 * c] * B[3 * b] + r[3 * c + 1] * B[3 * b + 1] + r[3 * c + 2] * B[3 * b + 2];
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) G[a][b] = B[3 * a] * T[0][b] + B[3 * a + 1] * T[1][b] + B[3 * a + 2] * T[2][b];
+  const double tr = G[0][0] + G[1][1] + G[2][2];
+  if constexpr (TERM == GFX_TERM_LAPLACE) {
+    v[0] = sa * tr;
+  } else {
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) {
+        if constexpr (TERM == GFX_TERM_ISO_ELAST) v[3 * a + b] = sa * G[a][b] + sb * (G[b][a] + (a == b ? tr : 0.0));
+        else v[3 * a + b] = sa * G[a][b] + sb * G[b][a] + (a == b ? sc * tr : 0.0);
+      }
+  }
+}
+
+template <int ND, int Q, int TERM, bool CHECK>
+__global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const double *__restrict__ Rp,
+                                                          const uint64_t *__restrict__ sig, uint64_t *sig_out,
+                                                          double *__restrict__ thr_out) {
+  constexpr int NP = ND * (ND + 1) / 2, NV = TERM == GFX_TERM_LAPLACE ? 1 : Q * Q;
+  __shared__ double2 stage[kWave * 9];  // records, rows padded as in k_records_tet
+  __shared__ double red[kKeepWaves][kWave];
+  const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t g = blockIdx.x, e0 = g * kWave;
+  const int nblk = (int)min<int64_t>(kWave, a.n_cv - e0);
+  if (w == 0 && lane < nblk) {
+    double o[16];
+    if (!tet_record(e0 + lane, a, o)) atomicOr(a.err, 1);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) stage[9 * lane + t] = make_double2(o[2 * t], o[2 * t + 1]);
+  }
+  __syncthreads();
+  double B[9], sa = 0.0, sb = 0.0, sc = 0.0;
+  {
+    const double *o = reinterpret_cast<const double *>(stage + 9 * lane);
+    const bool live = lane < nblk;  // a lane past the last element keeps nothing
+#pragma unroll
+    for (int t = 0; t < 9; ++t) B[t] = live ? o[t] : 0.0;
+    if (live) { sa = o[9]; sb = o[10]; sc = o[15]; }
+  }
   double mx = 0.0;
-  const double *rec = a.rec + (int64_t)kRecStride * (live ? e : 0);
-  if (live) {
-    for (int p = lane; p < npair; p += kWave) {
-      double v[Q][Q];
-      pair_block<Q, TERM, GFX_FORM_PERQP, double>(rec, p / nd, p % nd, nd, a.nq, a.gref, a.qw,
-                                                  nullptr, v);
-      for (int x = 0; x < Q; ++x)
-        for (int y = 0; y < Q; ++y) mx = fmax(mx, fabs(v[x][y]));
+  for (int p = w; p < NP; p += kKeepWaves) {
+    double v[NV];
+    keep_block<Q, TERM>(Rp + 9 * p, B, sa, sb, sc, v);
+#pragma unroll
+    for (int x = 0; x < NV; ++x) mx = fmax(mx, fabs(v[x]));
+  }
+  red[w][lane] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < kKeepWaves; ++x) mx = fmax(mx, red[x][lane]);
+  const double thr = mx > 0.0 ? mx * 1e-14 : INFINITY;
+  if (w == 0 && lane < nblk) {
+    thr_out[e0 + lane] = thr;
+    reinterpret_cast<double *>(stage + 9 * lane)[11] = thr;
+  }
+  const uint64_t *sg = sig + g * (NP * NV);
+  uint64_t diff = 0;
+  for (int p = w; p < NP; p += kKeepWaves) {
+    double v[NV];
+    keep_block<Q, TERM>(Rp + 9 * p, B, sa, sb, sc, v);
+#pragma unroll
+    for (int x = 0; x < NV; ++x) {
+      const uint64_t k = __ballot(fabs(v[x]) > thr);
+      if constexpr (CHECK) diff |= k ^ sg[p * NV + x];
+      else if (lane == x) sig_out[(g * NP + p) * NV + x] = k;
     }
   }
-  mx = wave_max(mx);
-  const double thr = mx * 1e-14;
+  if (CHECK && diff && lane == 0) atomicOr(a.err, 32);
   __syncthreads();
-  if (live && mx > 0.0) {  // an all-zero element is skipped (:5441-5442)
-    for (int p = lane; p < npair; p += kWave) {
-      const int i = p / nd, j = p % nd;
-      double v[Q][Q];
-      pair_block<Q, TERM, GFX_FORM_PERQP, double>(rec, i, j, nd, a.nq, a.gref, a.qw, nullptr, v);
-      for (int x = 0; x < Q; ++x)
-        for (int y = 0; y < Q; ++y)
-          if (fabs(v[x][y]) > thr) {
-            const int bit = (i * Q + x) * nl + (j * Q + y);
-            atomicOr(&my[bit >> 5], 1u << (bit & 31));
-          }
+  // the records, 16-byte pieces of consecutive records from consecutive threads
+  if (a.rec32) {
+    float4 *dst = reinterpret_cast<float4 *>(a.rec32 + (int64_t)kRecStride * e0);
+    for (int x = threadIdx.x; x < nblk * 4; x += kWave * kKeepWaves) {
+      const double2 u = stage[9 * (x / 4) + 2 * (x % 4)], v = stage[9 * (x / 4) + 2 * (x % 4) + 1];
+      dst[x] = make_float4((float)u.x, (float)u.y, (float)v.x, (float)v.y);
     }
   }
-  __syncthreads();
-  if (live) {
-    if (lane == 0) a.thr[e] = (mx > 0.0) ? thr : INFINITY;
-    for (int t = lane; t < a.kwords; t += kWave) a.keep[e * a.kwords + t] = my[t];
+  double2 *dst = reinterpret_cast<double2 *>(a.rec + (int64_t)kRecStride * e0);
+  for (int x = threadIdx.x; x < nblk * 8; x += kWave * kKeepWaves) dst[x] = stage[9 * (x / 8) + x % 8];
+}
+
+// the signature as keep bits per element, row-major nloc x nloc, for the
+// pattern build and its exact check: one lane per element, the words in order
+template <int ND, int Q, int TERM>
+__global__ __launch_bounds__(256) void k_keep_words(int64_t n_cv, int kwords, const uint64_t *__restrict__ sig,
+                                                    uint32_t *__restrict__ keep) {
+  constexpr int NP = ND * (ND + 1) / 2, NV = TERM == GFX_TERM_LAPLACE ? 1 : Q * Q, NL = ND * Q;
+  const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int64_t g = blockIdx.x, e = g * kWave + lane;
+  const uint64_t *sg = sig + g * (NP * NV);
+  for (int wd = w; wd < kwords; wd += 4) {
+    uint32_t bits = 0;
+    for (int b = 0; b < 32; ++b) {
+      const int bit = 32 * wd + b;
+      if (bit >= NL * NL) break;
+      const int r = bit / NL, c = bit - r * NL;
+      int i = r / Q, x = r - i * Q, j = c / Q, y = c - j * Q;
+      if (i > j) {  // the transposed block
+        int t = i; i = j; j = t;
+        t = x; x = y; y = t;
+      }
+      if (TERM == GFX_TERM_LAPLACE && x != y) continue;
+      const int p = i * ND - i * (i - 1) / 2 + (j - i);
+      const uint64_t k = sg[p * NV + (TERM == GFX_TERM_LAPLACE ? 0 : x * Q + y)];
+      bits |= (uint32_t)((k >> lane) & 1u) << b;
+    }
+    if (e < n_cv) keep[e * kwords + wd] = bits;
   }
 }
 
@@ -832,14 +934,9 @@ hipError_t scan_exclusive_i32(hipStream_t s, const int32_t *in, int32_t *out, in
 
 static unsigned nblocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-hipError_t launch_records_tet(hipStream_t s, int64_t n_cv, const double *pts,
-                              const int32_t *cvx, const double *ca, double ca_c,
-                              const double *cb, double cb_c, const double *cc, double cc_c,
-                              const double *thr, double r_scale, double *rec, float *rec32,
-                              int *err) {
-  if (n_cv == 0) return hipSuccess;
-  k_records_tet<<<nblocks(n_cv, 256), 256, 0, s>>>(n_cv, pts, cvx, ca, ca_c, cb, cb_c, cc, cc_c,
-                                                    thr, r_scale, rec, rec32, err);
+hipError_t launch_records_tet(hipStream_t s, const RecordArgs &a, const double *thr) {
+  if (a.n_cv == 0) return hipSuccess;
+  k_records_tet<<<nblocks(a.n_cv, 256), 256, 0, s>>>(a, thr);
   return hipGetLastError();
 }
 
@@ -865,20 +962,43 @@ hipError_t launch_incidences(hipStream_t s, int64_t n_cv, int nd, int qdim,
   return hipGetLastError();
 }
 
-hipError_t launch_keep(hipStream_t s, int term, const PatternArgs &a) {
-  const unsigned nb = nblocks(a.n_cv, 4);
-  const size_t lds = 4 * (size_t)a.kwords * sizeof(uint32_t);
-  if (a.qdim == 1 && term == GFX_TERM_LAPLACE)
-    k_keep<1, GFX_TERM_LAPLACE><<<nb, 256, lds, s>>>(a);
-  else if (a.qdim == 3 && term == GFX_TERM_LAPLACE)
-    k_keep<3, GFX_TERM_LAPLACE><<<nb, 256, lds, s>>>(a);
-  else if (a.qdim == 3 && term == GFX_TERM_ISO_ELAST)
-    k_keep<3, GFX_TERM_ISO_ELAST><<<nb, 256, lds, s>>>(a);
-  else if (a.qdim == 3 && term == GFX_TERM_ISOTROPIC)
-    k_keep<3, GFX_TERM_ISOTROPIC><<<nb, 256, lds, s>>>(a);
-  else
-    return hipErrorInvalidValue;
+int64_t keep_sig_words(int term, int nd, int qdim, int64_t n_cv) {
+  const int nv = term == GFX_TERM_LAPLACE ? 1 : qdim * qdim;
+  return (n_cv + kWave - 1) / kWave * (nd * (nd + 1) / 2) * nv;
+}
+
+template <int ND, int Q, int TERM>
+static hipError_t launch_keep3(hipStream_t s, const RecordArgs &a, const double *Rp, uint64_t *sig, bool check,
+                               double *thr, uint32_t *keep, int kwords) {
+  const unsigned grid = nblocks(a.n_cv, kWave);
+  if (check) {
+    k_keep<ND, Q, TERM, true><<<grid, kWave * kKeepWaves, 0, s>>>(a, Rp, sig, nullptr, thr);
+  } else {
+    k_keep<ND, Q, TERM, false><<<grid, kWave * kKeepWaves, 0, s>>>(a, Rp, sig, sig, thr);
+    k_keep_words<ND, Q, TERM><<<grid, 256, 0, s>>>(a.n_cv, kwords, sig, keep);
+  }
   return hipGetLastError();
+}
+
+hipError_t launch_keep(hipStream_t s, int term, int nd, int qdim, const RecordArgs &a, const double *Rp,
+                       uint64_t *sig, bool check, double *thr, uint32_t *keep, int kwords) {
+  if (a.n_cv == 0) return hipSuccess;
+  constexpr int L = GFX_TERM_LAPLACE, E = GFX_TERM_ISO_ELAST, I = GFX_TERM_ISOTROPIC;
+#define GFX_KEEP(ND, Q, T) \
+  if (nd == ND && qdim == Q && term == T) return launch_keep3<ND, Q, T>(s, a, Rp, sig, check, thr, keep, kwords)
+  GFX_KEEP(4, 1, L);
+  GFX_KEEP(10, 1, L);
+  GFX_KEEP(20, 1, L);
+  GFX_KEEP(4, 3, L);
+  GFX_KEEP(10, 3, L);
+  GFX_KEEP(4, 3, E);
+  GFX_KEEP(10, 3, E);
+  GFX_KEEP(20, 3, E);
+  GFX_KEEP(4, 3, I);
+  GFX_KEEP(10, 3, I);
+  GFX_KEEP(20, 3, I);
+#undef GFX_KEEP
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_patch_build(hipStream_t s, const PatternArgs &a, int max_cand) {

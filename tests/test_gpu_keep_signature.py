@@ -1,0 +1,86 @@
+"""The keep signature (one bit per element, pair and component, 64 elements to
+a word) behind the pattern build and its re-validation, at element counts that
+do not fill the last group: after new coefficients the plan's CSR equals the
+oracle's at those values, whether the bits stay (the pattern is kept) or
+change (it is rebuilt), and a change refused because the pattern is pinned
+stays refused until the values that the pattern was built from return."""
+import numpy as np
+import pytest
+
+import getfem_amd as ga
+import oracle
+from tests import problems
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "p1_laplace": (1, 1, oracle.TERM_LAPLACE), "p2_laplace": (2, 1, oracle.TERM_LAPLACE),
+    "p3_laplace": (3, 1, oracle.TERM_LAPLACE), "p1_elast": (1, 3, oracle.TERM_ISO_ELAST),
+    "p2_elast": (2, 3, oracle.TERM_ISO_ELAST), "p3_elast": (3, 3, oracle.TERM_ISO_ELAST),
+}
+IM = {1: "IM_TETRAHEDRON(1)", 2: "IM_TETRAHEDRON(5)", 3: "IM_TETRAHEDRON(8)"}
+
+
+def coefs(n_cv, q, seed):
+    rng = np.random.default_rng(seed)
+    return [rng.lognormal(0.0, 0.5, n_cv) for _ in range(2 if q == 3 else 1)]
+
+
+def at(case, c):
+    if case.term == oracle.TERM_LAPLACE:
+        case.a = c[0]
+    else:
+        case.lam, case.mu = c
+    return case.oracle_csr()
+
+
+def equal(plan, ref):
+    ip, ix, v = plan.csr()
+    assert np.array_equal(ip, ref[0]) and np.array_equal(ix, ref[1])
+    assert np.linalg.norm(v - ref[2]) <= 1e-12 * np.linalg.norm(ref[2])
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+@pytest.mark.parametrize("n", [1, 2, 3])
+def test_new_coefficients(ctx, name, n):
+    print("case: keep signature", name, n, flush=True)
+    k, q, term = CASES[name]
+    case = problems.Case(n, k, q, IM[k], term)
+    n_cv = case.cvx.shape[0]
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", case.pts, case.cvx)
+    mf = ga.MeshFem(mesh, case.fem, q)
+    c0 = coefs(n_cv, q, 1)
+    plan = ga.Plan(mf, ga.MeshIm(mesh, IM[k]), ga.TERM_ISO_ELAST if q == 3 else ga.TERM_LAPLACE, c0)
+    plan.build_pattern()
+    pid = plan.pattern_id()
+    plan.assemble()
+    equal(plan, at(case, c0))
+
+    def assemble(c):
+        for s, v in enumerate(c):
+            plan.set_coef(s, v)
+        plan.assemble()
+
+    c1 = coefs(n_cv, q, 2)  # the same bits
+    assemble(c1)
+    equal(plan, at(case, c1))
+    assert plan.pattern_id() == pid
+    c2 = [v.copy() for v in c1]  # no entry of the first and last elements
+    for v in c2:
+        v[0] = v[-1] = 0.0
+    refused = [v.copy() for v in c1]
+    for v in refused:
+        v[:] = 0.0
+    assemble(c2)
+    equal(plan, at(case, c2))
+    pid = plan.pattern_id()
+    views = plan.torch_csr_view()
+    for _ in range(2):  # the second time the signature is already that of the refused values
+        with pytest.raises(ga.GfxError):
+            assemble(refused)
+    assemble(c2)
+    assert plan.pattern_id() == pid
+    equal(plan, at(case, c2))
+    del views
+    assemble(c1)
+    equal(plan, at(case, c1))
