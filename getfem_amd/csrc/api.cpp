@@ -438,7 +438,7 @@ int gfx_plan_destroy(gfx_plan *p) {
   dfree(p->d_node_ok);
   dfree(p->d_nbr); dfree(p->d_mask);
   dfree(p->d_indptr); dfree(p->d_indices); dfree(p->d_vals); dfree(p->d_err);
-  dfree(p->d_gN); dfree(p->d_E); dfree(p->d_res); dfree(p->d_U); dfree(p->d_rhs); dfree(p->d_cg);
+  dfree(p->d_t1d); dfree(p->d_pd); dfree(p->d_full); dfree(p->d_E); dfree(p->d_res); dfree(p->d_U); dfree(p->d_rhs); dfree(p->d_cg);
   dfree(p->d_fixed); dfree(p->d_go);
   il_free(p->il);
   for (hipEvent_t e : p->ev) (void)hipEventDestroy(e);
@@ -551,12 +551,20 @@ int gfx_plan_create(gfx_mesh_fem *mf, gfx_mesh_im *mim, int term, const gfx_coef
           for (int b = 0; b < 3; ++b) R[((size_t)i * nd + j) * 9 + 3 * a + b] += w * g[3 * i + a] * g[3 * j + b];
   }
   p->eb = eb;
-  std::vector<double> gN((size_t)nq * m->nv * 3), Nv(m->nv);
-  for (int q = 0; q < nq; ++q) geotrans_eval(m->gt, &mim->rule.pts[3 * q], Nv.data(), &gN[(size_t)q * m->nv * 3]);
+  // the tensor rule's 1D points and the 1D base (FEM_QK(3,2) = its products):
+  // l_m(x_q) and its derivative, nodes 0, 1/2, 1
+  double t1d[18] = {0};
+  if (eb && nq == 27)
+    for (int q = 0; q < 3; ++q) {
+      const double x = p->xq[q] = mim->rule.pts[3 * q];
+      const double v[3] = {(1.0 - 2.0 * x) * (1.0 - x), 4.0 * x * (1.0 - x), x * (2.0 * x - 1.0)};
+      const double d[3] = {4.0 * x - 3.0, 4.0 - 8.0 * x, 4.0 * x - 1.0};
+      for (int b = 0; b < 3; ++b) { t1d[3 * b + q] = v[b]; t1d[9 + 3 * b + q] = d[b]; }
+    }
   hipError_t e = dalloc(&p->d_gref, gref.size());
   if (e == hipSuccess) e = dalloc(&p->d_qw, (size_t)nq);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_gN, gN.size());
-  if (e == hipSuccess && eb) e = hipMemcpy(p->d_gN, gN.data(), 8 * gN.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess && eb) e = dalloc(&p->d_t1d, 18);
+  if (e == hipSuccess && eb) e = hipMemcpy(p->d_t1d, t1d, sizeof t1d, hipMemcpyHostToDevice);
   if (e == hipSuccess && eb) e = dalloc(&p->d_E, (size_t)m->n_cv * p->nloc * p->nloc);
   if (e == hipSuccess && eb) e = dalloc(&p->d_res, (size_t)m->n_cv * p->nloc);
   if (e == hipSuccess && eb) e = dalloc(&p->d_U, (size_t)p->ndof);
@@ -675,19 +683,38 @@ static int plan_keep(gfx_plan *p, bool check) {
   return GFX_OK;
 }
 
-// the element kernel; with_keep (FP64): it also writes the keep bits
-static int plan_eb_elements(gfx_plan *p, int precision, bool with_keep = false) {
+static EbArgs eb_args(gfx_plan *p) {
   const gfx_mesh *m = p->mf->mesh;
-  gfx_ctx *c = p->ctx;
   EbArgs a{};
   a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx; a.dofs = p->mf->d_dofs; a.U = p->d_U;
   a.ca = p->coef[0].kind == GFX_COEF_PER_ELEMENT ? p->d_coef[0] : nullptr;
   a.cb = p->coef[1].kind == GFX_COEF_PER_ELEMENT ? p->d_coef[1] : nullptr;
   a.ca_c = p->coef[0].value; a.cb_c = p->coef[1].value;
-  a.gN = p->d_gN; a.gref = p->d_gref; a.qw = p->d_qw; a.nq = p->nq;
+  a.gref = p->d_gref; a.t1d = p->d_t1d; a.qw = p->d_qw; a.nq = p->nq;
+  for (int q = 0; q < 3; ++q) a.xq[q] = p->xq[q];
   a.E = p->d_E; a.res = p->d_res; a.thr = p->d_thr; a.err = p->d_err;
-  a.keep = with_keep ? p->d_keep : nullptr; a.kwords = p->kwords;
-  HIPCHK(c, launch_nh_element(c->stream, a, precision));
+  a.keep = p->d_keep; a.full = p->d_full; a.kwords = p->kwords;
+  return a;
+}
+
+// element residuals and, for the tangents that follow, the points' values
+static int plan_eb_points(gfx_plan *p, bool tangent) {
+  gfx_ctx *c = p->ctx;
+  const int64_t n_cv = p->mf->mesh->n_cv;
+  if (tangent && !p->d_pd) HIPCHK(c, dalloc(&p->d_pd, (size_t)nh_point_doubles(n_cv)));
+  EbArgs a = eb_args(p);
+  a.pd = tangent ? p->d_pd : nullptr;
+  HIPCHK(c, launch_nh_points(c->stream, a));
+  return GFX_OK;
+}
+
+// element matrices and thresholds from the points' values; keep: kNhKeep*
+static int plan_eb_tangent(gfx_plan *p, int precision, int keep) {
+  gfx_ctx *c = p->ctx;
+  if (keep && !p->d_full) HIPCHK(c, dalloc(&p->d_full, (size_t)p->mf->mesh->n_cv));
+  EbArgs a = eb_args(p);
+  a.pd = p->d_pd;
+  HIPCHK(c, launch_nh_tangent(c->stream, a, precision, keep));
   return GFX_OK;
 }
 
@@ -918,7 +945,7 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.keep = p->d_keep;
   a.inc_ptr = p->d_inc_ptr; a.inc = p->d_inc; a.err = p->d_err;
   if (p->eb) {
-    if ((r = plan_eb_elements(p, GFX_PREC_FP64, true))) return r;
+    if ((r = plan_eb_points(p, true)) || (r = plan_eb_tangent(p, GFX_PREC_FP64, kNhKeepWrite))) return r;
   } else {
     if ((r = plan_keep(p, false))) return r;
   }
@@ -977,14 +1004,14 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
 // The values behind the stored pattern changed (coefficients, node positions
 // or state): re-derive the per-element thresholds and keep bits at the new
 // values, as GetFEM's per-assembly threshold does, and see whether the
-// pattern they give is the stored one.  The keep bits of the affine terms are
-// compared with the stored ones first: the same bits give the same pattern.
+// pattern they give is the stored one.  The keep bits are compared with the
+// stored ones first: the same bits give the same pattern.
 // Where they differ the presence bits they give are compared with the stored
 // ones.  Equal: the pattern stands and the new thresholds are used.
 // Different: the pattern is rebuilt (refused while pinned).  A degenerate
 // element is reported here, like GetFEM's "Non invertible matrix" at every
-// assembly.  The records (affine terms) or FP64 element matrices computed here
-// serve the assembly that follows (*fresh).
+// assembly.  The records (affine terms) or the points' values and FP64 element
+// matrices computed here serve the assembly that follows (*fresh).
 static int plan_validate(gfx_plan *p, bool *fresh) {
   gfx_ctx *c = p->ctx;
   const gfx_mesh *m = p->mf->mesh;
@@ -1002,8 +1029,10 @@ static int plan_validate(gfx_plan *p, bool *fresh) {
     return GFX_OK;
   };
   HIPCHK(c, hipMemsetAsync(p->d_err, 0, 4, s));
-  if (!p->eb && p->keep_ok) {
-    if ((r = plan_keep(p, true)) || (r = read_flag())) return r;
+  if (p->eb && (r = plan_eb_points(p, true))) return r;
+  if (p->keep_ok) {
+    r = p->eb ? plan_eb_tangent(p, GFX_PREC_FP64, kNhKeepCheck) : plan_keep(p, true);
+    if (r || (r = read_flag())) return r;
     if (flag & 1) return fail(c, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
     if (!(flag & 32)) {
       p->pts_version = m->version;
@@ -1021,7 +1050,7 @@ static int plan_validate(gfx_plan *p, bool *fresh) {
   a.mask = p->d_mask; a.err = p->d_err;
   if (!p->d_node_ok) HIPCHK(c, dalloc(&p->d_node_ok, (size_t)std::max<int64_t>(p->n_nodes, 1)));
   a.node_ok = p->d_node_ok;
-  if ((r = p->eb ? plan_eb_elements(p, GFX_PREC_FP64, true) : plan_keep(p, false))) return r;
+  if ((r = p->eb ? plan_eb_tangent(p, GFX_PREC_FP64, kNhKeepWrite) : plan_keep(p, false))) return r;
   // nodes whose rows keep every entry are confirmed by one pass; the exact
   // check runs only when some node is not
   HIPCHK(c, launch_mask_fast(s, a));
@@ -1053,7 +1082,7 @@ int gfx_plan_assemble(gfx_plan *p) {
   if (p->nnz < 0) return fail(c, GFX_E_STATE, "build the pattern first");
   if (set_device(c)) return GFX_E_HIP;
   int r;
-  bool fresh = false;  // element-batched: E and thresholds already computed in FP64; else the records
+  bool fresh = false;  // element-batched: points, FP64 E and thresholds already computed; else the records
   if (p->values_changed || p->pts_version != p->mf->mesh->version)
     if ((r = plan_validate(p, &fresh))) return r;
   hipEvent_t *ev = nullptr;
@@ -1068,8 +1097,12 @@ int gfx_plan_assemble(gfx_plan *p) {
     p->n_timed++;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
   }
-  if (!fresh || (p->eb && p->precision != GFX_PREC_FP64))
-    if ((r = p->eb ? plan_eb_elements(p, p->precision) : plan_records(p))) return r;
+  if (!p->eb) {
+    if (!fresh && (r = plan_records(p))) return r;
+  } else if (!fresh || p->precision != GFX_PREC_FP64) {
+    if (!fresh && (r = plan_eb_points(p, true))) return r;
+    if ((r = plan_eb_tangent(p, p->precision, kNhKeepNone))) return r;
+  }
   const bool bdb = !p->eb && p->precision >= GFX_PREC_BF16X2;
   const bool bdb64 = bdb && p->precision == GFX_PREC_FP64_MFMA;
   if (bdb) {  // element matrices on the matrix cores, then the node-patch gather below
@@ -1195,7 +1228,7 @@ int gfx_plan_assemble_residual(gfx_plan *p) {
   if (p->nnz < 0) return fail(c, GFX_E_STATE, "build the pattern first");
   if (set_device(c)) return GFX_E_HIP;
   int r;
-  if ((r = plan_eb_elements(p, p->precision))) return r;
+  if ((r = plan_eb_points(p, false))) return r;
   HIPCHK(c, launch_gather_vec(c->stream, p->n_nodes, p->nd, p->qdim, p->d_inc_ptr, p->d_inc, p->d_res,
                               p->d_rhs));
   return GFX_OK;

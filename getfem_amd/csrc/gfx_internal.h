@@ -144,8 +144,9 @@ struct EbArgs {
   const double *U;          // state (ndof)
   const double *ca, *cb;    // per-element coefficients or null
   double ca_c, cb_c;
-  const double *gN;         // nq*8*3 transformation gradients
   const double *gref;       // nq*nd*3 base gradients
+  const double *t1d;        // 1D base l_m(x_q) then its derivative, [m][q]
+  double xq[3];             // 1D points
   const double *qw;
   int nq;
   double *E;                // n_cv * nl * nl element matrices, node-blocked: K[(i,a),(j,b)] at
@@ -153,7 +154,9 @@ struct EbArgs {
   double *res;              // n_cv * nl element residuals
   double *thr;              // n_cv thresholds
   int *err;
-  uint32_t *keep;           // FP64 form: when set, the keep bits (row-major, kwords words per element)
+  double *pd;               // the points' values for the tangent, or null: the residual alone
+  uint32_t *keep;           // keep bits (row-major, kwords words per element)
+  uint8_t *full;            // n_cv: 1 where every keep bit is set
   int kwords;
 };
 
@@ -310,7 +313,13 @@ hipError_t scan_exclusive_i32(hipStream_t s, const int32_t *in, int32_t *out,
 int64_t scan_tmp_elems(int64_t n);
 
 // kernels_eb.hip
-hipError_t launch_nh_element(hipStream_t s, const EbArgs &a, int precision);
+// element residuals and (a.pd set) the points' values, then the tangents; the
+// keep bits of a FP64 tangent are left, compared with the stored ones (bit 32
+// of the error flag) or written
+constexpr int kNhKeepNone = 0, kNhKeepCheck = 1, kNhKeepWrite = 2;
+int64_t nh_point_doubles(int64_t n_cv);
+hipError_t launch_nh_points(hipStream_t s, const EbArgs &a);
+hipError_t launch_nh_tangent(hipStream_t s, const EbArgs &a, int precision, int keep);
 hipError_t launch_elast_bdb_mfma(hipStream_t s, int64_t n_cv, int nd, int nq, const double *rec,
                                  const double *gref, const double *qw, float *E);
 hipError_t launch_elast_bdb_mfma_hp(hipStream_t s, int64_t n_cv, int nd, int nq, const double *rec,
@@ -492,7 +501,9 @@ struct gfx_plan {
   int precision = GFX_PREC_FP64;
   // element-batched plans (non-affine / nonlinear): buffered element matrices
   bool eb = false;
-  double *d_gN = nullptr, *d_E = nullptr, *d_res = nullptr, *d_U = nullptr, *d_rhs = nullptr;
+  double *d_t1d = nullptr, *d_pd = nullptr, *d_E = nullptr, *d_res = nullptr, *d_U = nullptr, *d_rhs = nullptr;
+  double xq[3] = {0, 0, 0};  // 1D points of the rule
+  uint8_t *d_full = nullptr; // elements whose keep bits are all set
   double *d_cg = nullptr;  // conjugate gradient work vectors (allocated on first solve)
   gfx::IldltData il;       // incomplete LDL^T preconditioner (built on first use)
   uint8_t *d_fixed = nullptr;  // dof constraints: mask and prescribed values

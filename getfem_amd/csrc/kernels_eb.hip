@@ -21,21 +21,27 @@ namespace {
 constexpr int kEbThreads = 256;
 constexpr int kNd = 27, kNl = 81, kNv = 8;
 
-// One workgroup per element.
-// Phase A, every integration point at once (FP64):
+// The Neo-Hookean element computations are two kernels.
+// k_nh_points, a wavefront per two elements (lane = point, then node):
 //   K_q = G grad(N)(q), J_q, B_q = K_q^{-T}, wJ_q = |J_q| w_q     (trilinear map)
-//   g[q][i] = B_q grad(phi_i)(q);  H_q = sum_i U_i (x) g[q][i];  F_q = I + H_q
-//   S_q = mu (I - C^-1) + lambda/2 ln(I3) C^-1,  A = dS/dE  (Bonet law)
-//   re[(i,a)] = sum_q wJ_q (F_q S_q g[q][i])_a
-// Phase B, the tangent K[(i,a),(j,b)] = sum_q g[q][i][c] D_q[(a,c),(b,n)]
-// g[q][j][n] with D_q[(a,c),(b,n)] = wJ_q (delta_ab S[n][c] + F[a][k]
-// A[k c m n] F[b][m]) (the GWFL derivative of the residual):
-//   in the spatial form (h = F^{-T} g, see k_nh_element): per node pair and
-//   point, two outer products of spatial gradients and a dot product of
-//   material ones, as products on the matrix cores in FP64 (FP64 form) or
-//   FP32 (FP32 form), upper tiles only (nh_phase_b_mfma).
+//   H_q = sum_i U_i (x) grad(phi_i)(q) B_q^T;  F_q = I + H_q
+//   S_q = mu (I - C^-1) + lambda/2 ln(I3) C^-1                    (Bonet law)
+//   re[(i,a)] = sum_q wJ_q (F_q S_q B_q grad(phi_i)(q))_a
+// and, for a tangent, the kNhPd values per point that k_nh_tangent needs.
+// k_nh_tangent, a workgroup per element, the tangent K[(i,a),(j,b)] =
+// sum_q g[q][i][c] D_q[(a,c),(b,n)] g[q][j][n] with D_q[(a,c),(b,n)] = wJ_q
+// (delta_ab S[n][c] + F[a][k] A[k c m n] F[b][m]) (the GWFL derivative of the
+// residual, A = dS/dE) in the spatial form (h = F^{-T} g): per node pair and
+// point, two outer products of spatial gradients and a dot product, as
+// products on the matrix cores in FP64 (FP64 form) or FP32 (FP32 form), upper
+// tiles only (nh_phase_b_mfma).
 constexpr int kNq = 27;
 constexpr int kKeepWords = (kNl * kNl + 31) / 32;  // keep-bit words per element (206)
+// k_nh_points' values per point, each kNq consecutive doubles of the element's
+// run: A = F^{-T} B row-major (h = A grad(phi)), alpha = wJ lambda, beta =
+// wJ (mu - lambda ln J), and the node term's symmetric kernel M (00, 01, 02,
+// 11, 12, 22)
+constexpr int kNhPd = 17;
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
@@ -209,10 +215,36 @@ __device__ __forceinline__ double nh_w_max(const typename BdbMfma<T>::v4 (&acc)[
   return nh_w_max_seq<T, T0>(std::make_integer_sequence<int, NT>{}, acc, k3);
 }
 
-template <typename T, bool KEEP>
-__device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double (*coef)[2], const double (*Mq)[9],
-                                                const T (*hC)[3][kNhN], T *stage, uint32_t *skeep, double *red,
-                                                const EbArgs &a) {
+// whether every entry of tiles T0 .. T0 + NT - 1 is above th (zero pads aside)
+template <typename T, int N>
+__device__ __forceinline__ bool nh_w_all1(int lr, int lg, double th, const typename BdbMfma<T>::v4 &acc,
+                                          const typename BdbMfma<T>::v4 &k3) {
+  typedef NhTile<N> D;
+  bool ok = true;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const bool in = 16 * D::I + BdbMfma<T>::row(lg, x) < kNd && 16 * D::J + lr < kNd;
+    ok &= !in || (double)fabs(D::diag ? acc[x] + k3[x] : acc[x]) > th;
+  }
+  return ok;
+}
+template <typename T, int T0, int... U>
+__device__ __forceinline__ bool nh_w_all_seq(std::integer_sequence<int, U...>, int lr, int lg, double th,
+                                             const typename BdbMfma<T>::v4 (&acc)[6],
+                                             const typename BdbMfma<T>::v4 &k3) {
+  return (nh_w_all1<T, T0 + U>(lr, lg, th, acc[U], k3) & ...);
+}
+template <typename T, int T0, int NT>
+__device__ __forceinline__ bool nh_w_all(int lr, int lg, double th, const typename BdbMfma<T>::v4 (&acc)[6],
+                                         const typename BdbMfma<T>::v4 &k3) {
+  return nh_w_all_seq<T, T0>(std::make_integer_sequence<int, NT>{}, lr, lg, th, acc, k3);
+}
+
+// KEEP: 0 no keep bits; 1 they are compared with the stored ones (bit 32 of
+// the error flag when any differs); 2 they are written
+template <typename T, int KEEP>
+__device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double *pd, const T (*hC)[3][kNhN], T *stage,
+                                                uint32_t *skeep, double *red, const EbArgs &a) {
   typedef typename BdbMfma<T>::v4 v4;
   // the wavefront index as a scalar: the branches on it are uniform
   const int w = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64, lr = l % 16, lg = l / 16;
@@ -225,11 +257,12 @@ __device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double (
 #pragma unroll
     for (int st = 0; st < kNhQ / 4; ++st) {
       const int q = 4 * st + lg;
-      const double *M = Mq[min(q, kNq - 1)];
+      const double *M = pd + 11 * kNq + min(q, kNq - 1);
       const T h0 = hC[q][0][j], h1 = hC[q][1][j], h2 = hC[q][2][j];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        const T m = (T)M[3 * c] * h0 + (T)M[3 * c + 1] * h1 + (T)M[3 * c + 2] * h2;
+        // row c of the symmetric M: its entries (c, 0), (c, 1), (c, 2)
+        const T m = (T)M[c * kNq] * h0 + (T)M[(c == 0 ? 1 : 2 + c) * kNq] * h1 + (T)M[(c == 0 ? 2 : 3 + c) * kNq] * h2;
         k3 = BdbMfma<T>::mma(hC[q][c][i], m, k3);
       }
     }
@@ -239,29 +272,42 @@ __device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double (
 #pragma unroll
   for (int st = 0; st < kNhQ / 4; ++st) {
     const int qc = min(4 * st + lg, kNq - 1);
-    al[st] = (T)coef[qc][0];
-    be[st] = (T)coef[qc][1];
+    al[st] = (T)pd[9 * kNq + qc];
+    be[st] = (T)pd[10 * kNq + qc];
   }
   v4 acc[6];
   if (w == 0) nh_w_tiles<T, 0, 5>(lr, lg, hC, al, be, acc);
   else if (w == 1) nh_w_tiles<T, 5, 5>(lr, lg, hC, al, be, acc);
   else if (w == 2) nh_w_tiles<T, 10, 5>(lr, lg, hC, al, be, acc);
   else nh_w_tiles<T, 15, 6>(lr, lg, hC, al, be, acc);
-  // threshold 1e-14 max|K| (all-zero element skipped): over the streamed
-  // entries, or, when the FP64 pass also sets the keep bits while it streams
-  // E (pattern build, re-validation), from the accumulators before any entry
-  // is written
-  constexpr bool kb = KEEP;
-  double mx = 0.0, th = 0.0;
-  if constexpr (kb) {
-    if (w == 0) mx = nh_w_max<T, 0, 5>(acc, k3);
-    else if (w == 1) mx = nh_w_max<T, 5, 5>(acc, k3);
-    else if (w == 2) mx = nh_w_max<T, 10, 5>(acc, k3);
-    else mx = nh_w_max<T, 15, 6>(acc, k3);
-    const double mxe = block_max(mx, red);
-    th = mxe > 0.0 ? 1e-14 * mxe : INFINITY;
-    if (t == 0) a.thr[e] = th;
-    for (int x = t; x < a.kwords; x += kEbThreads) skeep[x] = 0u;
+  // threshold 1e-14 max|K| (all-zero element skipped), from the accumulators
+  double mx = 0.0;
+  if (w == 0) mx = nh_w_max<T, 0, 5>(acc, k3);
+  else if (w == 1) mx = nh_w_max<T, 5, 5>(acc, k3);
+  else if (w == 2) mx = nh_w_max<T, 10, 5>(acc, k3);
+  else mx = nh_w_max<T, 15, 6>(acc, k3);
+  const double mxe = block_max(mx, red);
+  const double th = mxe > 0.0 ? 1e-14 * mxe : INFINITY;
+  if (t == 0) a.thr[e] = th;
+  // An element that keeps every entry (nearly all do) has words of ones: they
+  // are not formed.  full[e] says that of the stored words.
+  bool words = false;
+  if constexpr (KEEP != 0) {
+    bool all;
+    if (w == 0) all = nh_w_all<T, 0, 5>(lr, lg, th, acc, k3);
+    else if (w == 1) all = nh_w_all<T, 5, 5>(lr, lg, th, acc, k3);
+    else if (w == 2) all = nh_w_all<T, 10, 5>(lr, lg, th, acc, k3);
+    else all = nh_w_all<T, 15, 6>(lr, lg, th, acc, k3);
+    words = !__syncthreads_and(all);
+    if (KEEP == 1 && t == 0 && a.full[e] != (words ? 0 : 1)) atomicOr(a.err, 32);
+    if (KEEP == 2) {
+      if (t == 0) a.full[e] = words ? 0 : 1;
+      if (!words)
+        for (int x = t; x < kKeepWords; x += kEbThreads)
+          a.keep[e * kKeepWords + x] = x == kKeepWords - 1 ? (1u << (kNl * kNl % 32)) - 1u : 0xffffffffu;
+    }
+    if (words)
+      for (int x = t; x < kKeepWords; x += kEbThreads) skeep[x] = 0u;
   }
   T *E = reinterpret_cast<T *>(a.E) + e * kNl * kNl;
   // two stages: node rows 0-15, then 16-26; the trash row (a slot per lane)
@@ -282,12 +328,8 @@ __device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double (
     __syncthreads();
     const int len = 3 * (n1 - n0) * kNl;
     T *dst = E + 3 * n0 * kNl;
-    for (int x = t; x < len; x += kEbThreads) {
-      const T v = stage[x];
-      __builtin_nontemporal_store(v, dst + x);
-      if constexpr (!kb) mx = fmax(mx, (double)fabs(v));
-    }
-    if constexpr (kb) {
+    for (int x = t; x < len; x += kEbThreads) __builtin_nontemporal_store(stage[x], dst + x);
+    if (KEEP != 0 && words) {
       // keep bits, row-major (r, c) = (3 i + a, 3 j + b): one thread per
       // 32-bit word of this slab's rows reads its entries from the stage
       // (staged at ((3 i + a) 3 + b) 27 + j); the word shared with the other
@@ -311,76 +353,123 @@ __device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double (
       }
     }
   }
-  if constexpr (!kb) {
-    const double mxe = block_max(mx, red);
-    if (t == 0) a.thr[e] = mxe > 0.0 ? 1e-14 * mxe : INFINITY;
-  } else {
+  if (KEEP != 0 && words) {
     __syncthreads();
-    for (int x = t; x < a.kwords; x += kEbThreads) a.keep[e * a.kwords + x] = skeep[x];
+    bool same = true;
+    for (int x = t; x < kKeepWords; x += kEbThreads) {
+      if constexpr (KEEP == 2) a.keep[e * kKeepWords + x] = skeep[x];
+      else same &= a.keep[e * kKeepWords + x] == skeep[x];
+    }
+    if (!same) atomicOr(a.err, 32);
   }
 }
 
-// phase A's per-element arrays; the material gradients gq (phase A) and
-// then the spatial ones hC (phase B) share their space; phase B stages E
-// over all of it
-struct NhPhaseA {
-  double X[kNv][3], Ue[kNd][3];
-  double Bq[kNq][9], wJ[kNq], Fq[kNq][9], Sq[kNq][9], Cq[kNq][9], cf[kNq][2], Mq[kNq][9];
-};
-template <typename T>
-union NhGrad {
-  double gq[kNq][kNd][3];
-  T hC[kNhQ][3][kNhN];
-};
-template <typename T>
-union NhLds {
-  struct {
-    NhPhaseA A;
-    NhGrad<T> G;
-  } P;
-  T stage[3 * 16 * kNl + 64];  // the slab and the trash row
-};
+// Points and residual.  Bound by FP64 issue and the LDS.  A half wavefront
+// per element, 27 of its 32 lanes at work: the sums over nodes and over points
+// are tensor products, done one direction at a time (72 products a lane each
+// way instead of 243), so lane (x, y, z) is in turn a point or a node along
+// each direction and the partial sums pass through the element's own LDS
+// block; only the wavefront's own lanes read it, so no workgroup barrier is
+// needed.  NHPTIME
+constexpr int kNhHalf = 32;
 
-template <typename Real, bool KEEP>
-__global__ __launch_bounds__(kEbThreads, 4) void k_nh_element(EbArgs a) {
-  __shared__ NhLds<Real> L;
-  double(&X)[kNv][3] = L.P.A.X;
-  double(&Ue)[kNd][3] = L.P.A.Ue;
-  double(&Bq)[kNq][9] = L.P.A.Bq;
-  double(&wJ)[kNq] = L.P.A.wJ;
-  double(&Fq)[kNq][9] = L.P.A.Fq;
-  double(&Sq)[kNq][9] = L.P.A.Sq;
-  double(&Cq)[kNq][9] = L.P.A.Cq;
-  double(&cf)[kNq][2] = L.P.A.cf;
-  double(&Mq)[kNq][9] = L.P.A.Mq;
-  double(&gq)[kNq][kNd][3] = L.P.G.gq;
-  Real(&hC)[kNhQ][3][kNhN] = L.P.G.hC;  // phase B: the spatial gradients in the fragments' layout
-  __shared__ double red[kEbThreads];
-  __shared__ uint32_t skeep[KEEP ? kKeepWords : 1];  // the element's keep bits
-  const int64_t e = blockIdx.x;
-  if (e >= a.n_cv || a.nq != kNq) return;
-  const int t = threadIdx.x;
-  if (t < kNv * 3) X[t / 3][t % 3] = a.pts[3 * (int64_t)a.cvx[kNv * e + t / 3] + t % 3];
-  if (t < kNl) Ue[t / 3][t % 3] = a.U[(int64_t)a.dofs[kNd * e + t / 3] + t % 3];
-  const double lam = a.ca ? a.ca[e] : a.ca_c, mu = a.cb ? a.cb[e] : a.cb_c;
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool TANGENT>
+__global__ __launch_bounds__(kEbThreads) void k_nh_points(EbArgs a) {
+  __shared__ double T1[2][3][3];                                  // l_m(x_q), dl_m(x_q): [.][m][q]
+  __shared__ double bufA[kEbThreads / kNhHalf][9][kNhHalf];       // partial sums, component-major
+  __shared__ double bufB[kEbThreads / kNhHalf][9][kNhHalf];
+  if (threadIdx.x < 18) T1[threadIdx.x / 9][threadIdx.x % 9 / 3][threadIdx.x % 3] = a.t1d[threadIdx.x];
   __syncthreads();
-  // A1: geometry per point
-  if (t < kNq) {
-    const double *gn = a.gN + (int64_t)t * kNv * 3;
-    double k[9];  // column-major K(r,c)
-    for (int r = 0; r < 3; ++r)
-      for (int c = 0; c < 3; ++c) {
-        double s = X[0][r] * gn[c];
-        for (int v = 1; v < kNv; ++v) s += X[v][r] * gn[3 * v + c];
-        k[r + 3 * c] = s;
-      }
+  const int slot = threadIdx.x / kNhHalf, l = threadIdx.x % kNhHalf;
+  const bool on = l < kNq;
+  const int t = on ? l : 0, tx = t % 3, ty = t / 3 % 3, tz = t / 9;
+  const int64_t e0 = (int64_t)blockIdx.x * (kEbThreads / kNhHalf) + slot;
+  const bool live = e0 < a.n_cv;
+  const int64_t e = live ? e0 : a.n_cv - 1;  // past the last element: computed, not written
+  double (&A)[9][kNhHalf] = bufA[slot];
+  double (&Bf)[9][kNhHalf] = bufB[slot];
+  {  // the nodes' displacements, and the vertices behind them
+    const double *u = a.U + a.dofs[kNd * e + t];
+    const double *x = a.pts + 3 * (int64_t)a.cvx[kNv * e + l % kNv];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      A[c][l] = u[c];
+      A[3 + c][l] = x[c];
+    }
+  }
+  wave_lds_fence();
+  // K = sum_v X_v (x) grad N_v at this lane's point (vertex dx + 2 dy + 4 dz)
+  double k[9];  // column-major K(r,c)
+  {
+    const double x1 = a.xq[tx], y1 = a.xq[ty], z1 = a.xq[tz], x0 = 1.0 - x1, y0 = 1.0 - y1, z0 = 1.0 - z1;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const double *X = A[3 + r];
+      k[r] = y0 * z0 * (X[1] - X[0]) + y1 * z0 * (X[3] - X[2]) + y0 * z1 * (X[5] - X[4]) + y1 * z1 * (X[7] - X[6]);
+      k[r + 3] = x0 * z0 * (X[2] - X[0]) + x1 * z0 * (X[3] - X[1]) + x0 * z1 * (X[6] - X[4]) + x1 * z1 * (X[7] - X[5]);
+      k[r + 6] = x0 * y0 * (X[4] - X[0]) + x1 * y0 * (X[5] - X[1]) + x0 * y1 * (X[6] - X[2]) + x1 * y1 * (X[7] - X[3]);
+    }
+  }
+  const double lam = a.ca ? a.ca[e] : a.ca_c, mu = a.cb ? a.cb[e] : a.cb_c;
+  // H = sum_i U_i (x) grad(phi_i), one direction at a time:
+  // x: lane (point x, node y, node z) -> value and d/dx
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double v = 0.0, d = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const double u = A[c][m + 3 * ty + 9 * tz];
+      v += T1[0][m][tx] * u;
+      d += T1[1][m][tx] * u;
+    }
+    Bf[2 * c][l] = v;
+    Bf[2 * c + 1][l] = d;
+  }
+  wave_lds_fence();
+  // y: lane (point x, point y, node z) -> d/dx, d/dy, value
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double dx = 0.0, dy = 0.0, v = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const double w = Bf[2 * c][tx + 3 * m + 9 * tz];
+      dx += T1[0][m][ty] * Bf[2 * c + 1][tx + 3 * m + 9 * tz];
+      dy += T1[1][m][ty] * w;
+      v += T1[0][m][ty] * w;
+    }
+    A[3 * c][l] = dx;
+    A[3 * c + 1][l] = dy;
+    A[3 * c + 2][l] = v;
+  }
+  wave_lds_fence();
+  // z: lane = point
+  double Hr[9];  // row-major d u_c / d xi_d
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double dx = 0.0, dy = 0.0, dz = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const int o = tx + 3 * ty + 9 * m;
+      dx += T1[0][m][tz] * A[3 * c][o];
+      dy += T1[0][m][tz] * A[3 * c + 1][o];
+      dz += T1[1][m][tz] * A[3 * c + 2][o];
+    }
+    Hr[3 * c] = dx; Hr[3 * c + 1] = dy; Hr[3 * c + 2] = dz;
+  }
+  double B[9], F[9], wJ;
+  {
     const double a0 = k[4] * k[8] - k[5] * k[7];
     const double a1 = k[5] * k[6] - k[3] * k[8];
     const double a2 = k[3] * k[7] - k[4] * k[6];
     const double J = k[0] * a0 + k[1] * a1 + k[2] * a2;
-    if (J == 0.0) atomicOr(a.err, 1);
-    const double rJ = 1.0 / J;
-    double *B = Bq[t];  // row-major B(r,c)
+    if (J == 0.0 && live && on) atomicOr(a.err, 1);
+    const double rJ = 1.0 / J;  // B row-major B(r,c)
     B[0] = a0 * rJ; B[3] = a1 * rJ; B[6] = a2 * rJ;
     B[1] = (k[2] * k[7] - k[1] * k[8]) * rJ;
     B[4] = (k[0] * k[8] - k[2] * k[6]) * rJ;
@@ -388,32 +477,22 @@ __global__ __launch_bounds__(kEbThreads, 4) void k_nh_element(EbArgs a) {
     B[2] = (k[1] * k[5] - k[2] * k[4]) * rJ;
     B[5] = (k[2] * k[3] - k[0] * k[5]) * rJ;
     B[8] = (k[0] * k[4] - k[1] * k[3]) * rJ;
-    wJ[t] = fabs(J) * a.qw[t];
+    wJ = fabs(J) * a.qw[t];
   }
-  __syncthreads();
-  // A2: real gradients
-  for (int x = t; x < kNq * kNd; x += kEbThreads) {
-    const int q = x / kNd, i = x % kNd;
-    const double *h = a.gref + ((int64_t)q * kNd + i) * 3;
-    const double h0 = h[0], h1 = h[1], h2 = h[2];
-    const double *B = Bq[q];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) gq[q][i][c] = B[3 * c] * h0 + B[3 * c + 1] * h1 + B[3 * c + 2] * h2;
-  }
-  __syncthreads();
-  // A3: deformation gradient
-  for (int x = t; x < kNq * 9; x += kEbThreads) {
-    const int q = x / 9, r = (x % 9) / 3, c = x % 3;
-    double s = 0.0;
-    for (int i = 0; i < kNd; ++i) s += Ue[i][r] * gq[q][i][c];
-    Fq[q][3 * r + c] = s + (r == c ? 1.0 : 0.0);
-  }
-  __syncthreads();
-  // A4: the law at every point
-  if (t < kNq) {
-    const double *F = Fq[t];
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      F[3 * r + c] = Hr[3 * r] * B[3 * c] + Hr[3 * r + 1] * B[3 * c + 1] + Hr[3 * r + 2] * B[3 * c + 2] + (r == c ? 1.0 : 0.0);
+  // the law
+  const double f0 = F[4] * F[8] - F[5] * F[7], f1 = F[5] * F[6] - F[3] * F[8], f2 = F[3] * F[7] - F[4] * F[6];
+  const double detF = F[0] * f0 + F[1] * f1 + F[2] * f2;
+  double S[9], ln3;
+  {
     double C[9], Ci[9];
+#pragma unroll
     for (int i = 0; i < 3; ++i)
+#pragma unroll
       for (int j = 0; j < 3; ++j) C[3 * i + j] = F[i] * F[j] + F[3 + i] * F[3 + j] + F[6 + i] * F[6 + j];
     const double c0 = C[4] * C[8] - C[5] * C[7];
     const double c1 = C[5] * C[6] - C[3] * C[8];
@@ -427,19 +506,26 @@ __global__ __launch_bounds__(kEbThreads, 4) void k_nh_element(EbArgs a) {
     Ci[2] = (C[1] * C[5] - C[2] * C[4]) * rI3;
     Ci[5] = (C[2] * C[3] - C[0] * C[5]) * rI3;
     Ci[8] = (C[0] * C[4] - C[1] * C[3]) * rI3;
-    const double f0 = F[4] * F[8] - F[5] * F[7], f1 = F[5] * F[6] - F[3] * F[8], f2 = F[3] * F[7] - F[4] * F[6];
-    const double detF = F[0] * f0 + F[1] * f1 + F[2] * f2;
-    const double ln3 = log(I3);
+    ln3 = log(I3);
+#pragma unroll
     for (int i = 0; i < 9; ++i) {
-      double sv = mu * ((i % 4 == 0 ? 1.0 : 0.0) - Ci[i]) + 0.5 * lam * ln3 * Ci[i];
-      if (detF <= 0.0) sv += 1e200 * C[i];
-      Sq[t][i] = sv;
+      S[i] = mu * ((i % 4 == 0 ? 1.0 : 0.0) - Ci[i]) + 0.5 * lam * ln3 * Ci[i];
+      if (detF <= 0.0) S[i] += 1e200 * C[i];  // the law's penalty on inverted points
     }
-    // the spatial form's inputs of phase B: F^{-1} (row-major, into Cq) and
-    // the point's coefficients alpha = wJ lambda, beta = wJ (mu - lambda ln J),
-    // gamma = wJ mu and the penalty pen = 1e200 wJ where det F <= 0
+  }
+  // Q = wJ F S B (first Piola stress against the reference gradients), component-major
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    double P[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) P[c] = wJ * (F[3 * r] * S[c] + F[3 * r + 1] * S[3 + c] + F[3 * r + 2] * S[6 + c]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) Bf[3 * r + d][l] = P[0] * B[d] + P[1] * B[3 + d] + P[2] * B[6 + d];
+  }
+  if (TANGENT && live && on) {
+    double *pd = a.pd + e * (kNhPd * kNq) + t;
     const double rF = 1.0 / detF;
-    double *Fi = Cq[t];
+    double Fi[9];  // F^{-1}, row-major
     Fi[0] = f0 * rF; Fi[3] = f1 * rF; Fi[6] = f2 * rF;
     Fi[1] = (F[2] * F[7] - F[1] * F[8]) * rF;
     Fi[4] = (F[0] * F[8] - F[2] * F[6]) * rF;
@@ -447,82 +533,128 @@ __global__ __launch_bounds__(kEbThreads, 4) void k_nh_element(EbArgs a) {
     Fi[2] = (F[1] * F[5] - F[2] * F[4]) * rF;
     Fi[5] = (F[2] * F[3] - F[0] * F[5]) * rF;
     Fi[8] = (F[0] * F[4] - F[1] * F[3]) * rF;
-    const double w = wJ[t];
-    cf[t][0] = w * lam;
-    cf[t][1] = w * (mu - 0.5 * lam * ln3);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) pd[(3 * c + d) * kNq] = Fi[c] * B[d] + Fi[3 + c] * B[3 + d] + Fi[6 + c] * B[6 + d];
+    pd[9 * kNq] = wJ * lam;
+    pd[10 * kNq] = wJ * (mu - 0.5 * lam * ln3);
     // the node term's kernel in the spatial gradients: with g = F^T h,
     // gamma g_i . g_j + pen (F g_i) . (F g_j) = h_i^T M h_j, M = gamma b + pen b^2,
-    // b = F F^T (symmetric)
-    const double ga = w * mu, pen = detF <= 0.0 ? w * 1e200 : 0.0;
+    // b = F F^T (symmetric), gamma = wJ mu, pen = 1e200 wJ where det F <= 0
+    const double ga = wJ * mu, pen = detF <= 0.0 ? wJ * 1e200 : 0.0;
     double b[9];
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
       for (int c = 0; c < 3; ++c) b[3 * r + c] = F[3 * r] * F[3 * c] + F[3 * r + 1] * F[3 * c + 1] + F[3 * r + 2] * F[3 * c + 2];
+    int o = 11;
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
+      for (int c = r; c < 3; ++c, ++o) {
         double m = ga * b[3 * r + c];
         if (pen != 0.0) m += pen * (b[3 * r] * b[c] + b[3 * r + 1] * b[3 + c] + b[3 * r + 2] * b[6 + c]);
-        Mq[t][3 * r + c] = m;
+        pd[o * kNq] = m;
       }
   }
-  __syncthreads();
-  // A5: the residual re[(i,a)] = sum_q sum_c P_q[a][c] g[q][i][c] with
-  // P_q = wJ_q F_q S_q (first Piola stress times the weight, into Bq, which
-  // is free after A2), as three partial sums over 9 points each
-  if (t < kNq * 9) {
-    const int q = t / 9, ar = (t % 9) / 3, c = t % 3;
-    const double *F = Fq[q], *S = Sq[q];
-    Bq[q][t % 9] = wJ[q] * (F[3 * ar] * S[c] + F[3 * ar + 1] * S[3 + c] + F[3 * ar + 2] * S[6 + c]);
-  }
-  __syncthreads();
-  if (t < 3 * kNl) {
-    const int grp = t / kNl, o = t % kNl, i = o / 3, ar = o % 3;
-    double re = 0.0;
-    for (int q = 9 * grp; q < 9 * grp + 9; ++q)
-      re += Bq[q][3 * ar] * gq[q][i][0] + Bq[q][3 * ar + 1] * gq[q][i][1] + Bq[q][3 * ar + 2] * gq[q][i][2];
-    red[t] = re;
-  }
-  __syncthreads();
-  if (t < kNl) a.res[(int64_t)e * kNl + t] = red[t] + red[kNl + t] + red[2 * kNl + t];
-  // Phase B in the spatial form.  With h_qi = F_q^{-T} g_qi (spatial
-  // gradients), the push-forward of this law's material tangent is
-  // J c = lambda 1 x 1 + (mu - lambda ln J)(two symmetric identities), and
-  // F^{-1} b F^{-T} = I folds the stress term into mu g_qi . g_qj, so the
-  // (i, j) block of D's contraction is, per point,
-  //   wJ_q [lambda h_qi (x) h_qj + (mu - lambda ln J_q) h_qj (x) h_qi
-  //         + (mu g_qi . g_qj + pen_q (F g_qi) . (F g_qj)) I]
-  // (pen_q = 1e200 where det F <= 0: the derivative of the law's penalty
-  // term 1e200 C added to S there).  Same matrix as the material form
-  // D[(a,c),(b,n)] = wJ (delta_ab S_nc + F_ak A_kcmn F_bm) up to roundoff,
-  // without forming D or D g (nh_phase_b_mfma).
-  // hC[q][c][i] = h_qic in Real (zero for q = 27 and nodes i >= 27), over
-  // gq: formed in registers, written once every thread has read gq
-  constexpr int kHc = (kNhQ * kNhN + kEbThreads - 1) / kEbThreads;
-  Real hv[kHc][3];
+  wave_lds_fence();
+  // re = sum_q Q_q grad(phi_i)(q), the directions the other way round:
+  // z: lane (point x, point y, node z)
 #pragma unroll
-  for (int k = 0; k < kHc; ++k) {
-    const int x = t + k * kEbThreads, q = x / kNhN, i = x % kNhN;
-    hv[k][0] = hv[k][1] = hv[k][2] = Real(0);
+  for (int c = 0; c < 3; ++c) {
+    double r0 = 0.0, r1 = 0.0, r2 = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int o = tx + 3 * ty + 9 * q;
+      r0 += T1[0][tz][q] * Bf[3 * c][o];
+      r1 += T1[0][tz][q] * Bf[3 * c + 1][o];
+      r2 += T1[1][tz][q] * Bf[3 * c + 2][o];
+    }
+    A[3 * c][l] = r0;
+    A[3 * c + 1][l] = r1;
+    A[3 * c + 2][l] = r2;
+  }
+  wave_lds_fence();
+  // y: lane (point x, node y, node z)
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double r0 = 0.0, r1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int o = tx + 3 * q + 9 * tz;
+      r0 += T1[0][ty][q] * A[3 * c][o];
+      r1 += T1[1][ty][q] * A[3 * c + 1][o] + T1[0][ty][q] * A[3 * c + 2][o];
+    }
+    Bf[2 * c][l] = r0;
+    Bf[2 * c + 1][l] = r1;
+  }
+  wave_lds_fence();
+  // x: lane = node
+  double *re = a.res + e * kNl + 3 * t;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    double r = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int o = q + 3 * ty + 9 * tz;
+      r += T1[1][tx][q] * Bf[2 * c][o] + T1[0][tx][q] * Bf[2 * c + 1][o];
+    }
+    if (live && on) re[c] = r;
+  }
+}
+
+// The tangent in the spatial form.  With h_qi = F_q^{-T} g_qi (spatial
+// gradients), the push-forward of this law's material tangent is
+// J c = lambda 1 x 1 + (mu - lambda ln J)(two symmetric identities), and
+// F^{-1} b F^{-T} = I folds the stress term into mu g_qi . g_qj, so the
+// (i, j) block of D's contraction is, per point,
+//   wJ_q [lambda h_qi (x) h_qj + (mu - lambda ln J_q) h_qj (x) h_qi
+//         + (mu g_qi . g_qj + pen_q (F g_qi) . (F g_qj)) I]
+// (pen_q = 1e200 where det F <= 0: the derivative of the penalty term 1e200 C
+// that the law adds to S there).  Same matrix as the material form
+// D[(a,c),(b,n)] = wJ (delta_ab S_nc + F_ak A_kcmn F_bm) up to roundoff,
+// without forming D or D g (nh_phase_b_mfma).  h = A grad(phi) from the points'
+// values, which k_nh_points leaves in memory (3.7 KB an element): its serial
+// phases (27 of 256 threads at work) used to take as long here as the products.
+// NHTTIME
+template <typename T>
+union NhLds {
+  struct {
+    double pd[kNhPd * kNq];
+    T hC[kNhQ][3][kNhN];  // the spatial gradients in the fragments' layout
+  } P;
+  T stage[3 * 16 * kNl + 64];  // the slab and the trash row, over what phase B has read
+};
+
+template <typename Real, int KEEP>
+__global__ __launch_bounds__(kEbThreads, 4) void k_nh_tangent(EbArgs a) {
+  __shared__ NhLds<Real> L;
+  __shared__ double red[kEbThreads / 64];
+  __shared__ uint32_t skeep[KEEP ? kKeepWords : 1];  // the element's keep bits, where not all are set
+  const int64_t e = blockIdx.x;
+  const int t = threadIdx.x;
+  double *pd = L.P.pd;
+  Real(&hC)[kNhQ][3][kNhN] = L.P.hC;
+  const double *src = a.pd + e * (kNhPd * kNq);
+  for (int x = t; x < kNhPd * kNq; x += kEbThreads) pd[x] = src[x];
+  __syncthreads();
+  // hC[q][c][i] = h_qic in Real (zero for q = 27 and nodes i >= 27)
+  for (int x = t; x < kNhQ * kNhN; x += kEbThreads) {
+    const int q = x / kNhN, i = x % kNhN;
+    Real h[3] = {Real(0), Real(0), Real(0)};
     if (q < kNq && i < kNd) {
-      const double *Fi = Cq[q], *g = gq[q][i];
+      const double *g = a.gref + (q * kNd + i) * 3;
       const double g0 = g[0], g1 = g[1], g2 = g[2];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) hv[k][c] = (Real)(Fi[c] * g0 + Fi[3 + c] * g1 + Fi[6 + c] * g2);
+      for (int c = 0; c < 3; ++c)
+        h[c] = (Real)(pd[3 * c * kNq + q] * g0 + pd[(3 * c + 1) * kNq + q] * g1 + pd[(3 * c + 2) * kNq + q] * g2);
     }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) hC[q][c][i] = h[c];
   }
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kHc; ++k) {
-    const int x = t + k * kEbThreads, q = x / kNhN, i = x % kNhN;
-    if (x < kNhQ * kNhN)
-#pragma unroll
-      for (int c = 0; c < 3; ++c) hC[q][c][i] = hv[k][c];
-  }
-  __syncthreads();
-  nh_phase_b_mfma<Real, KEEP>(t, e, cf, Mq, hC, L.stage, skeep, red, a);
+  nh_phase_b_mfma<Real, KEEP>(t, e, pd, hC, L.stage, skeep, red, a);
 }
 
 // node-patch gather of the rows of buffered element matrices: the Q rows of
@@ -931,38 +1063,48 @@ __global__ __launch_bounds__(256) void k_elast_bdb_mfma(int64_t n_cv, int nq, co
   }
 }
 
-// V[node*Q + x] = sum over incidences (e, i) of res[(e*nd + i)*Q + x]
-__global__ __launch_bounds__(256) void k_gather_vec(int64_t n_nodes, int nd, int Q,
-                                                    const int32_t *__restrict__ inc_ptr,
+// V[node*Q + x] = sum over incidences (e, i) of res[(e*nd + i)*Q + x]; one
+// thread per dof, so that the Q threads of a node read consecutive values (one
+// thread per node read them Q times apart, one after another)
+template <int Q>
+__global__ __launch_bounds__(256) void k_gather_vec(int64_t n_dof, int nd, const int32_t *__restrict__ inc_ptr,
                                                     const uint32_t *__restrict__ inc,
                                                     const double *__restrict__ res,
                                                     double *__restrict__ V) {
-  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= n_nodes) return;
-  for (int x = 0; x < Q; ++x) {
-    double s = 0.0;
-    for (int k = inc_ptr[n]; k < inc_ptr[n + 1]; ++k) {
-      const uint32_t c = inc[k];
-      s += res[((int64_t)(c >> 5) * nd + (c & 31)) * Q + x];
-    }
-    V[n * Q + x] = s;
+  const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (d >= n_dof) return;
+  const int64_t n = d / Q;
+  const int x = (int)(d - n * Q), k1 = inc_ptr[n + 1];
+  double s = 0.0;
+  for (int k = inc_ptr[n]; k < k1; ++k) {
+    const uint32_t c = inc[k];
+    s += res[((int64_t)(c >> 5) * nd + (c & 31)) * Q + x];
   }
+  V[d] = s;
 }
 
 }  // namespace
 
-hipError_t launch_nh_element(hipStream_t s, const EbArgs &a, int precision) {
+int64_t nh_point_doubles(int64_t n_cv) { return n_cv * kNhPd * kNq; }
+
+hipError_t launch_nh_points(hipStream_t s, const EbArgs &a) {
   if (a.n_cv == 0) return hipSuccess;
   if (a.nq != kNq) return hipErrorInvalidValue;
-  if (precision == GFX_PREC_FP32) {
-    if (a.keep) return hipErrorInvalidValue;  // keep bits come from the FP64 pass
-    k_nh_element<float, false><<<(unsigned)a.n_cv, kEbThreads, 0, s>>>(a);
-  } else if (a.keep) {
-    if (a.kwords != kKeepWords) return hipErrorInvalidValue;
-    k_nh_element<double, true><<<(unsigned)a.n_cv, kEbThreads, 0, s>>>(a);
-  } else {
-    k_nh_element<double, false><<<(unsigned)a.n_cv, kEbThreads, 0, s>>>(a);
-  }
+  const unsigned grid = (unsigned)((a.n_cv + kEbThreads / kNhHalf - 1) / (kEbThreads / kNhHalf));
+  if (a.pd) k_nh_points<true><<<grid, kEbThreads, 0, s>>>(a);
+  else k_nh_points<false><<<grid, kEbThreads, 0, s>>>(a);
+  return hipGetLastError();
+}
+
+hipError_t launch_nh_tangent(hipStream_t s, const EbArgs &a, int precision, int keep) {
+  if (a.n_cv == 0) return hipSuccess;
+  if (a.nq != kNq || !a.pd || (keep && (precision != GFX_PREC_FP64 || a.kwords != kKeepWords)))
+    return hipErrorInvalidValue;  // keep bits come from the FP64 pass
+  const unsigned grid = (unsigned)a.n_cv;
+  if (precision == GFX_PREC_FP32) k_nh_tangent<float, 0><<<grid, kEbThreads, 0, s>>>(a);
+  else if (keep == kNhKeepCheck) k_nh_tangent<double, 1><<<grid, kEbThreads, 0, s>>>(a);
+  else if (keep == kNhKeepWrite) k_nh_tangent<double, 2><<<grid, kEbThreads, 0, s>>>(a);
+  else k_nh_tangent<double, 0><<<grid, kEbThreads, 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -1156,7 +1298,12 @@ hipError_t launch_gather_emat(hipStream_t s, const PatchArgs &a0, const void *E,
 hipError_t launch_gather_vec(hipStream_t s, int64_t n_nodes, int nd, int Q, const int32_t *inc_ptr,
                              const uint32_t *inc, const double *res, double *V) {
   if (n_nodes == 0) return hipSuccess;
-  k_gather_vec<<<(unsigned)((n_nodes + 255) / 256), 256, 0, s>>>(n_nodes, nd, Q, inc_ptr, inc, res, V);
+  const int64_t n = n_nodes * Q;
+  const unsigned grid = (unsigned)((n + 255) / 256);
+  if (Q == 3) k_gather_vec<3><<<grid, 256, 0, s>>>(n, nd, inc_ptr, inc, res, V);
+  else if (Q == 2) k_gather_vec<2><<<grid, 256, 0, s>>>(n, nd, inc_ptr, inc, res, V);
+  else if (Q == 1) k_gather_vec<1><<<grid, 256, 0, s>>>(n, nd, inc_ptr, inc, res, V);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
