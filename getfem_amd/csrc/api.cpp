@@ -1377,11 +1377,18 @@ int gfx_plan_solve_cg(gfx_plan *p, const double *d_b, double *d_x, double rtol, 
   gfx_ctx *c = p->ctx;
   if (p->nnz < 0) return fail(c, GFX_E_STATE, "build the pattern and assemble first");
   if (set_device(c)) return GFX_E_HIP;
-  if (!p->d_cg) HIPCHK(c, dalloc(&p->d_cg, cg_workspace_doubles(p->ndof)));
+  const size_t need = cg_workspace_doubles(p->ndof, p->nnz);
+  if (need > p->cg_cap) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    dfree(p->d_cg);
+    p->cg_cap = 0;
+    HIPCHK(c, dalloc(&p->d_cg, need));
+    p->cg_cap = need;
+  }
   // vector fields: 3x3 block Jacobi (a node's coupled components), else the diagonal
   const int qb = (p->qdim == 3 && p->ndof % 3 == 0) ? 3 : 1;
-  HIPCHK(c, cg_solve(c->stream, p->ndof, p->nnz, p->d_indptr, p->d_indices, p->d_vals, d_b, d_x, rtol, maxit,
-                     qb, p->d_cg, iters, rel_res));
+  HIPCHK(c, cg_solve(c->stream, p->ndof, p->nnz, p->d_indptr, p->d_indices, p->d_vals, p->d_nslots, d_b, d_x, rtol,
+                     maxit, qb, p->d_cg, iters, rel_res));
   return GFX_OK;
 }
 

@@ -351,15 +351,16 @@ hipError_t launch_fill_f64(hipStream_t s, int64_t n, double *p, double v);
 hipError_t launch_dof_constraints(hipStream_t s, int64_t n, const int64_t *indptr, const int32_t *indices,
                                   double *vals, const uint8_t *fixed, const double *go, const double *pr,
                                   double *rhs, int flags, int *err);
-size_t cg_workspace_doubles(int64_t n);
+size_t cg_workspace_doubles(int64_t n, int64_t nnz);
+// nslots (may be null; qb = 3): the nodes' slot counts with the bit of the full nodes
 size_t gmres_workspace_doubles(int64_t n, int m);
 struct IluData;
 hipError_t gmres_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
                        const double *vals, const double *b, double *x, double rtol, int maxit, int m,
                        double *work, const IluData *ilu, int *iters, double *rel_res);
 hipError_t cg_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
-                    const double *vals, const double *b, double *x, double rtol, int maxit, int qb, double *work,
-                    int *iters, double *rel_res);
+                    const double *vals, const uint16_t *nslots, const double *b, double *x, double rtol, int maxit,
+                    int qb, double *work, int *iters, double *rel_res);
 
 // adjoint.hip
 int64_t compliance_nblocks(int64_t n_cv);
@@ -505,6 +506,7 @@ struct gfx_plan {
   double xq[3] = {0, 0, 0};  // 1D points of the rule
   uint8_t *d_full = nullptr; // elements whose keep bits are all set
   double *d_cg = nullptr;  // conjugate gradient work vectors (allocated on first solve)
+  size_t cg_cap = 0;       // their size in doubles
   gfx::IldltData il;       // incomplete LDL^T preconditioner (built on first use)
   uint8_t *d_fixed = nullptr;  // dof constraints: mask and prescribed values
   double *d_go = nullptr;

@@ -370,7 +370,8 @@ __device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double *
 // way instead of 243), so lane (x, y, z) is in turn a point or a node along
 // each direction and the partial sums pass through the element's own LDS
 // block; only the wavefront's own lanes read it, so no workgroup barrier is
-// needed.  NHPTIME
+// needed.  Measured: 38 us at 31^3 elements (a residual alone took 720 us, with
+// the tangent kernel), 168 us with the points' values at 48^3 = 110,592.
 constexpr int kNhHalf = 32;
 
 __device__ __forceinline__ void wave_lds_fence() {
@@ -617,7 +618,8 @@ __global__ __launch_bounds__(kEbThreads) void k_nh_points(EbArgs a) {
 // without forming D or D g (nh_phase_b_mfma).  h = A grad(phi) from the points'
 // values, which k_nh_points leaves in memory (3.7 KB an element): its serial
 // phases (27 of 256 threads at work) used to take as long here as the products.
-// NHTTIME
+// Measured at 48^3 = 110,592 elements with the keep check: 2.66 ms (with those
+// phases inside and the keep words always formed 3.21 ms).
 template <typename T>
 union NhLds {
   struct {

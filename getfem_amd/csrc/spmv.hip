@@ -7,14 +7,16 @@
 // from the mean row length so that short rows (P1) do not leave most lanes
 // idle.
 //
-// CG: every scalar of the recurrence (alpha, beta, r.z, r.r) lives in device
-// memory and is produced by fixed-order block reductions, so an iteration
-// issues kernels only and the result does not depend on scheduling.  The host
-// reads r.r once per iteration for the stopping test.
+// CG: an iteration is three launches (product with p.q, update with r.z and
+// r.r, direction); every scalar of the recurrence lives in device memory and
+// comes from fixed-order reductions, and so does the stopping test, so the
+// host launches iterations in batches and looks once per batch; the result
+// does not depend on scheduling or on the batch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "gfx_internal.h"
@@ -24,7 +26,8 @@ namespace {
 
 constexpr int kSpmvThreads = 256;
 constexpr int kRedThreads = 256;   // threads of a reduction block
-constexpr int kRedBlocks = 1024;   // partial sums per dot product (fixed: deterministic order)
+constexpr int kRedBlocks = 1024;   // most partial sums of a vector kernel's dot product
+constexpr int kMaxProdBlocks = 2048;  // and of the product's (8 blocks a CU)
 
 template <int G, bool ACC>
 __global__ __launch_bounds__(kSpmvThreads) void k_spmv(int64_t n, const int64_t *__restrict__ indptr,
@@ -148,20 +151,53 @@ __global__ void k_fill_f64(int64_t n, double *__restrict__ p, double v) {
 }
 
 // ---------------------------------------------------------------- CG
+// The recurrence's scalars after an iteration; two of them, the launches of
+// an iteration reading one and writing the other.  done: the loop has ended
+// (the launches that follow in the batch do nothing but hand the state on).
 struct CgScal {
-  double rz, rr, bb, pq, alpha, beta;
+  double rz, rr, bb, pq;
+  int it, done;
 };
 
+// sum over the wavefront, every lane gets it: data-parallel moves within rows
+// of 16 lanes, then across them (a move costs a few cycles, a shuffle through
+// the LDS unit some fifty)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
+  return v + __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row has the row's sum
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3: lane 63 has the sum
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// sum over the block, every thread gets it; the wavefronts' sums, then those
+// in order through LDS
 __device__ __forceinline__ double block_sum(double v, double *sh) {
-  sh[threadIdx.x] = v;
+  v = wave_sum(v);
+  __syncthreads();  // the last use of sh
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int off = kRedThreads / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
-  }
-  const double r = sh[0];
-  __syncthreads();
+  double r = sh[0];
+  for (int w = 1; w < kRedThreads / 64; ++w) r += sh[w];
   return r;
+}
+
+// the sum of a launch's n partials, in a fixed order, by every block that needs it
+__device__ __forceinline__ double partials_sum(const double *__restrict__ part, int n, double *sh) {
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += kRedThreads) s += part[i];
+  return block_sum(s, sh);
 }
 
 // inverse diagonal (0 where the diagonal is absent or zero: that dof is left alone)
@@ -187,19 +223,29 @@ __global__ void k_inv_diag(int64_t n, const int64_t *__restrict__ indptr,
 // Dirichlet simplification) falls back to the inverse diagonal of that node
 __global__ void k_inv_block3(int64_t nn, const int64_t *__restrict__ indptr,
                              const int32_t *__restrict__ indices, const double *__restrict__ vals,
-                             double *__restrict__ minv) {
+                             const uint16_t *__restrict__ nslots, double *__restrict__ minv) {
   const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= nn) return;
   double M[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-  for (int a = 0; a < 3; ++a) {
-    const int64_t row = 3 * u + a;
+  auto first = [&](int64_t row) {  // first entry with a column >= 3u (sorted columns)
     int64_t lo = indptr[row], hi = indptr[row + 1];
-    while (lo < hi) {  // first column >= 3u (sorted columns)
+    while (lo < hi) {
       const int64_t mid = (lo + hi) / 2;
       if (indices[mid] < 3 * u) lo = mid + 1;
       else hi = mid;
     }
-    for (int64_t k = lo; k < indptr[row + 1] && indices[k] < 3 * u + 3; ++k) M[a][indices[k] - 3 * u] = vals[k];
+    return lo;
+  };
+  if (nslots && (nslots[u] & 0x8000)) {  // a full node: the three rows have the same columns
+    const int64_t len = 3 * (nslots[u] & 0x7fff), lo = first(3 * u);
+    if (lo < indptr[3 * u + 1] && indices[lo] == 3 * u)
+      for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) M[a][b] = vals[lo + a * len + b];
+  } else {
+    for (int a = 0; a < 3; ++a) {
+      const int64_t row = 3 * u + a;
+      for (int64_t k = first(row); k < indptr[row + 1] && indices[k] < 3 * u + 3; ++k) M[a][indices[k] - 3 * u] = vals[k];
+    }
   }
   const double c00 = M[1][1] * M[2][2] - M[1][2] * M[2][1], c01 = M[1][2] * M[2][0] - M[1][0] * M[2][2],
                c02 = M[1][0] * M[2][1] - M[1][1] * M[2][0];
@@ -239,9 +285,9 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_start(int64_t nu, const doub
                                                           const double *__restrict__ minv,
                                                           double *__restrict__ r, double *__restrict__ z,
                                                           double *__restrict__ p, double *__restrict__ part) {
-  __shared__ double sh[kRedThreads];
+  __shared__ double sh[kRedThreads / 64];
   double rz = 0, rr = 0, bb = 0;
-  for (int64_t u = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; u < nu; u += (int64_t)kRedBlocks * kRedThreads) {
+  for (int64_t u = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; u < nu; u += (int64_t)gridDim.x * kRedThreads) {
     double ri[QB], zi[QB];
     for (int a = 0; a < QB; ++a) ri[a] = b[QB * u + a] - r[QB * u + a];
     precond<QB>(minv, u, ri, zi);
@@ -253,56 +299,186 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_start(int64_t nu, const doub
   }
   rz = block_sum(rz, sh); rr = block_sum(rr, sh); bb = block_sum(bb, sh);
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = rz; part[kRedBlocks + blockIdx.x] = rr; part[2 * kRedBlocks + blockIdx.x] = bb;
+    part[blockIdx.x] = rz; part[gridDim.x + blockIdx.x] = rr; part[2 * gridDim.x + blockIdx.x] = bb;
   }
 }
 
-__global__ __launch_bounds__(kRedThreads) void k_dot(int64_t n, const double *__restrict__ x,
-                                                     const double *__restrict__ y, double *__restrict__ part) {
-  __shared__ double sh[kRedThreads];
-  double s = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (int64_t)kRedBlocks * kRedThreads)
-    s += x[i] * y[i];
-  s = block_sum(s, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
+// whether the loop stops at |r|^2 = rr: gmm::cg's test on |r| / |b|
+__device__ __forceinline__ bool cg_stops(double rr, double bb, double rtol) { return !(sqrt(rr) / sqrt(bb) > rtol); }
+
+__global__ __launch_bounds__(kRedThreads) void k_cg_first(const double *__restrict__ part, int n, double rtol,
+                                                          CgScal *__restrict__ sc) {
+  __shared__ double sh[kRedThreads / 64];
+  const double rz = partials_sum(part, n, sh), rr = partials_sum(part + n, n, sh);
+  const double bb = partials_sum(part + 2 * n, n, sh);
+  if (threadIdx.x == 0) *sc = CgScal{rz, rr, bb, 0.0, 0, bb == 0.0 || cg_stops(rr, bb, rtol)};
 }
 
-// sum `count` partial arrays of kRedBlocks entries in a fixed order;
-// mode 0: start (rz, rr, bb), 1: pq -> alpha, 2: (rz_new, rr) -> beta
-__global__ __launch_bounds__(kRedThreads) void k_cg_scalars(const double *__restrict__ part, int mode,
-                                                            CgScal *__restrict__ sc) {
-  __shared__ double sh[kRedThreads];
-  double v[3] = {0, 0, 0};
-  const int count = mode == 1 ? 1 : (mode == 0 ? 3 : 2);
-  for (int k = 0; k < count; ++k) {
-    double s = 0;
-    for (int i = threadIdx.x; i < kRedBlocks; i += kRedThreads) s += part[k * kRedBlocks + i];
-    v[k] = block_sum(s, sh);
-  }
-  if (threadIdx.x != 0) return;
-  if (mode == 0) {
-    sc->rz = v[0]; sc->rr = v[1]; sc->bb = v[2];
-  } else if (mode == 1) {
-    sc->pq = v[0];
-    sc->alpha = v[0] != 0.0 ? sc->rz / v[0] : 0.0;
-  } else {
-    sc->beta = sc->rz != 0.0 ? v[0] / sc->rz : 0.0;
-    sc->rz = v[0]; sc->rr = v[1];
-  }
+// Node lists of the full nodes (every component pair of every neighbour
+// stored): their three rows hold the same columns, whole triples in order, so
+// one int per neighbour node stands for nine column indices.  The list of the
+// node whose values start at b0 starts at b0 / 9, which leaves each its room.
+__global__ void k_cg_nodes(int64_t nn, const uint16_t *__restrict__ nslots, const int64_t *__restrict__ indptr,
+                           const int32_t *__restrict__ indices, int32_t *__restrict__ nodes) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, u = t / 8;
+  if (u >= nn || !(nslots[u] & 0x8000)) return;
+  const int64_t b0 = indptr[3 * u];
+  const int ns = nslots[u] & 0x7fff;
+  for (int s = (int)(t % 8); s < ns; s += 8) nodes[b0 / 9 + s] = indices[b0 + 3 * s] / 3;
 }
 
-// x += alpha p, r -= alpha q, z = M^-1 r; partials of r.z and r.r
+// q = K p and the partials of p.q: every launch writes one partial a block
+// (sc null: no iteration, the product of the start).
+// The blocks of an XCD sweep one eighth of the units, so that the x that
+// neighbouring rows share stays in its L2.
+// A row per G lanes (scalar fields and workspace matrices).
+template <int G>
+__global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv(int64_t n, int64_t chunk,
+                                                            const int64_t *__restrict__ indptr,
+                                                            const int32_t *__restrict__ indices,
+                                                            const double *__restrict__ vals,
+                                                            const double *__restrict__ p, double *__restrict__ q,
+                                                            const CgScal *__restrict__ sc,
+                                                            double *__restrict__ part) {
+  __shared__ double sh[kRedThreads / 64];
+  if (sc && sc->done) return;
+  constexpr int kPer = kRedThreads / G;
+  const int lane = threadIdx.x % G;
+  const int64_t first = (int64_t)(blockIdx.x & 7) * chunk, last = min(n, first + chunk);
+  const int64_t step = (int64_t)(gridDim.x >> 3) * kPer;
+  double pq = 0.0;
+  for (int64_t u = first + (int64_t)(blockIdx.x >> 3) * kPer + threadIdx.x / G; u < last; u += step) {
+    double s = 0.0;
+    const int64_t e = indptr[u + 1];
+    for (int64_t k = indptr[u] + lane; k < e; k += G) s += vals[k] * p[indices[k]];
+    for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
+    if (lane == 0) {
+      q[u] = s;
+      pq += p[u] * s;
+    }
+  }
+  pq = block_sum(pq, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = pq;
+}
+
+// A node's three rows per wavefront (3x3 block Jacobi's fields); a column's x
+// serves all three.  Bound by HBM: 8 bytes an entry and, in full nodes, 4/9
+// for its index.  A full node's columns go in tiles of 64; the next tile's
+// node ids and values are issued between this tile's x and its sums, so that
+// a tile costs one memory latency, not three (the loads of a wavefront return
+// in order: issued before the x they would have to arrive first).  The node's
+// start and slot count are the same for every lane and come by scalar loads,
+// a node ahead.
+// Measured at P2 elasticity, 24^3 x 6 (367,000 rows, 28.7 M entries): 72 us with
+// p.q (111 + 5 + 5 us for a row per 32 lanes, p.q and its sum apart: 12 bytes
+// an entry, two latencies a row); 82 us with the values loaded non-temporally
+// (rows share cache lines: they were fetched twice), 95-146 us with a node per
+// 16 or 32 lanes, 115 us at half the wavefronts.
+__global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t chunk,
+                                                             const int64_t *__restrict__ indptr,
+                                                             const int32_t *__restrict__ indices,
+                                                             const double *__restrict__ vals,
+                                                             const uint16_t *__restrict__ nslots,
+                                                             const int32_t *__restrict__ nodes,
+                                                             const double *__restrict__ p, double *__restrict__ q,
+                                                             const CgScal *__restrict__ sc,
+                                                             double *__restrict__ part) {
+  __shared__ double sh[kRedThreads / 64];
+  if (sc && sc->done) return;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t first = (int64_t)(blockIdx.x & 7) * chunk, last = min(nn, first + chunk);
+  const int64_t step = (int64_t)(gridDim.x >> 3) * (kRedThreads / 64);
+  struct Node {
+    int64_t b0;      // its first value
+    int r1, r2, r3;  // rows 1 and 2 and the end, from there
+    int len;         // columns of the longest row
+    bool full;
+  };
+  auto node = [&](int64_t v) {
+    const int64_t b0 = indptr[3 * v];
+    Node d{b0, (int)(indptr[3 * v + 1] - b0), (int)(indptr[3 * v + 2] - b0), (int)(indptr[3 * v + 3] - b0), 0,
+           (nslots[v] & 0x8000) != 0};
+    d.len = max(d.r1, max(d.r2 - d.r1, d.r3 - d.r2));
+    return d;
+  };
+  // a tile's columns and values; indices past a row's end are clamped to the
+  // node's last entry and their products left out of the sums
+  int c0 = 0, c1 = 0, c2 = 0;
+  double v0 = 0.0, v1 = 0.0, v2 = 0.0;
+  auto load = [&](const Node &d, int k0) {
+    const int k = k0 + lane;
+    const unsigned i0 = min(k, d.r3 - 1), i1 = min(d.r1 + k, d.r3 - 1), i2 = min(d.r2 + k, d.r3 - 1);
+    if (d.full) {
+      c0 = (nodes + d.b0 / 9)[(unsigned)min(k, d.len - 1) / 3];
+    } else {
+      const int32_t *ix = indices + d.b0;
+      c0 = ix[i0];
+      c1 = ix[i1];
+      c2 = ix[i2];
+    }
+    const double *v = vals + d.b0;
+    v0 = v[i0];
+    v1 = v[i1];
+    v2 = v[i2];
+  };
+  double pq = 0.0;
+  int64_t u = first + (int64_t)(blockIdx.x >> 3) * (kRedThreads / 64) + w;
+  Node cur{};
+  if (u < last) {
+    cur = node(u);
+    if (cur.len) load(cur, 0);
+  }
+  for (; u < last; u += step) {
+    const Node nxt = node(min(u + step, last - 1));
+    const double pu = p[3 * u + min(lane, 2)];
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    if (!cur.len && nxt.len) load(nxt, 0);
+    for (int k0 = 0; k0 < cur.len; k0 += 64) {
+      const int k = k0 + lane;
+      double x0, x1, x2;
+      if (cur.full) {
+        x0 = x1 = x2 = p[3 * (int64_t)c0 + (unsigned)min(k, cur.len - 1) % 3];
+      } else {
+        x0 = p[c0];
+        x1 = p[c1];
+        x2 = p[c2];
+      }
+      const double a0 = v0, a1 = v1, a2 = v2;
+      if (k0 + 64 < cur.len) load(cur, k0 + 64);
+      else if (nxt.len) load(nxt, 0);
+      s0 += k < cur.r1 ? a0 * x0 : 0.0;
+      s1 += k < cur.r2 - cur.r1 ? a1 * x1 : 0.0;
+      s2 += k < cur.r3 - cur.r2 ? a2 * x2 : 0.0;
+    }
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if (lane < 3) {
+      const double s = lane == 0 ? s0 : (lane == 1 ? s1 : s2);
+      q[3 * u + lane] = s;
+      pq += pu * s;
+    }
+    cur = nxt;
+  }
+  pq = block_sum(pq, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = pq;
+}
+
+// alpha = r.z / p.q; x += alpha p, r -= alpha q, z = M^-1 r; partials of r.z and r.r
 template <int QB>
-__global__ __launch_bounds__(kRedThreads) void k_cg_update(int64_t nu, const CgScal *__restrict__ sc,
+__global__ __launch_bounds__(kRedThreads) void k_cg_update(int64_t nu, CgScal *__restrict__ sc,
+                                                           const double *__restrict__ ppart, int np,
                                                            const double *__restrict__ p,
                                                            const double *__restrict__ q,
                                                            const double *__restrict__ minv,
                                                            double *__restrict__ x, double *__restrict__ r,
                                                            double *__restrict__ z, double *__restrict__ part) {
-  __shared__ double sh[kRedThreads];
-  const double alpha = sc->alpha;
+  __shared__ double sh[kRedThreads / 64];
+  if (sc->done) return;
+  const double pq = partials_sum(ppart, np, sh), alpha = pq != 0.0 ? sc->rz / pq : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->pq = pq;  // for the next launch; none of this one reads it
   double rz = 0, rr = 0;
-  for (int64_t u = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; u < nu; u += (int64_t)kRedBlocks * kRedThreads) {
+  for (int64_t u = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; u < nu; u += (int64_t)gridDim.x * kRedThreads) {
     double ri[QB], zi[QB];
     for (int a = 0; a < QB; ++a) {
       const int64_t i = QB * u + a;
@@ -317,14 +493,25 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_update(int64_t nu, const CgS
     }
   }
   rz = block_sum(rz, sh); rr = block_sum(rr, sh);
-  if (threadIdx.x == 0) { part[blockIdx.x] = rz; part[kRedBlocks + blockIdx.x] = rr; }
+  if (threadIdx.x == 0) { part[blockIdx.x] = rz; part[gridDim.x + blockIdx.x] = rr; }
 }
 
-// p = z + beta p
-__global__ void k_cg_direction(int64_t n, const CgScal *__restrict__ sc, const double *__restrict__ z,
-                               double *__restrict__ p) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = z[i] + sc->beta * p[i];
+// beta = (r.z) / (r.z before); p = z + beta p; the next iteration's scalars
+__global__ __launch_bounds__(kRedThreads) void k_cg_direction(int64_t n, const CgScal *__restrict__ sc,
+                                                              const double *__restrict__ part, int np, double rtol,
+                                                              const double *__restrict__ z, double *__restrict__ p,
+                                                              CgScal *__restrict__ next) {
+  __shared__ double sh[kRedThreads / 64];
+  if (sc->done) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *next = *sc;
+    return;
+  }
+  const double rz = partials_sum(part, np, sh), rr = partials_sum(part + np, np, sh);
+  const double beta = sc->rz != 0.0 ? rz / sc->rz : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0)  // p.q <= 0: K not positive definite along p
+    *next = CgScal{rz, rr, sc->bb, sc->pq, sc->it + 1, sc->pq <= 0.0 || cg_stops(rr, sc->bb, rtol)};
+  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRedThreads)
+    p[i] = z[i] + beta * p[i];
 }
 
 unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -428,8 +615,12 @@ hipError_t launch_fill_f64(hipStream_t s, int64_t n, double *p, double v) {
   return hipGetLastError();
 }
 
-// preconditioner storage (3 n: room for the 3x3 blocks) + r, z, p, q + partials
-size_t cg_workspace_doubles(int64_t n) { return 7 * (size_t)n + 3 * kRedBlocks + 8; }
+// preconditioner storage (3 n: room for the 3x3 blocks) + r, z, p, q +
+// partials + scalars, then the full nodes' lists (an int per 9 entries)
+static size_t cg_vector_doubles(int64_t n) {
+  return 7 * (size_t)n + 3 * kRedBlocks + kMaxProdBlocks + 2 * sizeof(CgScal) / sizeof(double);
+}
+size_t cg_workspace_doubles(int64_t n, int64_t nnz) { return cg_vector_doubles(n) + (size_t)nnz / 18 + 2; }
 
 // ------------------------------------------------------------------ GMRES
 namespace {
@@ -666,51 +857,98 @@ hipError_t gmres_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *ind
 }
 
 
+// the blocks of a product whose blocks do `per` units at a time, and the units of an XCD
+static int cg_prod_blocks(int64_t nu, int per, int64_t &chunk) {
+  chunk = (nu + 7) / 8;
+  return (int)std::min<int64_t>(8 * std::max<int64_t>(1, (chunk + per - 1) / per), kMaxProdBlocks);
+}
+
+static hipError_t cg_product(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
+                             const double *vals, const uint16_t *nslots, const int32_t *nodes, const double *p,
+                             double *q, const CgScal *sc, double *part, int *nblocks) {
+  int64_t chunk;
+  if (nslots) {
+    *nblocks = cg_prod_blocks(n / 3, kRedThreads / 64, chunk);
+    k_cg_spmv3<<<(unsigned)*nblocks, kRedThreads, 0, s>>>(n / 3, chunk, indptr, indices, vals, nslots, nodes, p, q, sc,
+                                                          part);
+    return hipGetLastError();
+  }
+  auto run = [&](auto g) {
+    constexpr int G = decltype(g)::value;
+    *nblocks = cg_prod_blocks(n, kRedThreads / G, chunk);
+    k_cg_spmv<G><<<(unsigned)*nblocks, kRedThreads, 0, s>>>(n, chunk, indptr, indices, vals, p, q, sc, part);
+  };
+  const double mean = (double)nnz / (double)n;  // as launch_spmv
+  if (mean <= 12) run(std::integral_constant<int, 4>{});
+  else if (mean <= 24) run(std::integral_constant<int, 8>{});
+  else if (mean <= 64) run(std::integral_constant<int, 16>{});
+  else run(std::integral_constant<int, 32>{});
+  return hipGetLastError();
+}
+
+// One iteration's launches; cur and next: the scalars before and after it.
+template <int QB>
+static hipError_t cg_iterations(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
+                                const double *vals, const uint16_t *nslots, const int32_t *nodes, const double *b,
+                                double *x, double rtol, int maxit, double *work, CgScal *h) {
+  double *minv = work, *r = work + 3 * n, *z = work + 4 * n, *p = work + 5 * n, *q = work + 6 * n;
+  double *part = work + 7 * n, *ppart = part + 3 * kRedBlocks;
+  CgScal *sc = reinterpret_cast<CgScal *>(ppart + kMaxProdBlocks);
+  const int64_t nu = n / QB;
+  const int nb = (int)std::min<int64_t>(kRedBlocks, (nu + kRedThreads - 1) / kRedThreads);
+  const int nd = (int)std::min<int64_t>(kRedBlocks, (n + kRedThreads - 1) / kRedThreads);
+  hipError_t e;
+  k_cg_start<QB><<<nb, kRedThreads, 0, s>>>(nu, b, minv, r, z, p, part);
+  k_cg_first<<<1, kRedThreads, 0, s>>>(part, nb, rtol, sc);
+  // batches: the host waits once for each; a batch is at most as long as all
+  // before it, so that the launches after the end are never the most of them
+  int it = 0, batch = 4;
+  do {
+    const int end = std::min(maxit, it + batch);
+    for (; it < end; ++it) {
+      CgScal *cur = sc + (it & 1), *next = sc + (~it & 1);
+      int np = 0;
+      if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, p, q, cur, ppart, &np)) != hipSuccess)
+        return e;
+      k_cg_update<QB><<<nb, kRedThreads, 0, s>>>(nu, cur, ppart, np, p, q, minv, x, r, z, part);
+      k_cg_direction<<<nd, kRedThreads, 0, s>>>(n, cur, part, nb, rtol, z, p, next);
+    }
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = hipMemcpyAsync(h, sc + (it & 1), sizeof *h, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+    batch = std::min(std::max(batch, it), 32);
+  } while (!h->done && it < maxit);
+  return hipSuccess;
+}
+
 hipError_t cg_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
-                    const double *vals, const double *b, double *x, double rtol, int maxit, int qb,
-                    double *work, int *iters, double *rel_res) {
+                    const double *vals, const uint16_t *nslots, const double *b, double *x, double rtol, int maxit,
+                    int qb, double *work, int *iters, double *rel_res) {
   *iters = 0;
   *rel_res = 0.0;
   if (n == 0) return hipSuccess;
   if (qb != 1 && (qb != 3 || n % 3 != 0)) return hipErrorInvalidValue;
-  double *minv = work, *r = work + 3 * n, *z = work + 4 * n, *p = work + 5 * n, *q = work + 6 * n;
-  double *part = work + 7 * n;
-  CgScal *sc = reinterpret_cast<CgScal *>(part + 3 * kRedBlocks);
+  double *minv = work, *r = work + 3 * n;
+  int32_t *nodes = reinterpret_cast<int32_t *>(work + cg_vector_doubles(n));
   const int64_t nu = n / qb;
   hipError_t e;
-  if (qb == 3) k_inv_block3<<<nb256(nu), 256, 0, s>>>(nu, indptr, indices, vals, minv);
+  if (qb == 3) k_inv_block3<<<nb256(nu), 256, 0, s>>>(nu, indptr, indices, vals, nslots, minv);
   else k_inv_diag<<<nb256(n), 256, 0, s>>>(n, indptr, indices, vals, minv);
-  if ((e = launch_spmv(s, n, nnz, indptr, indices, vals, x, r, false)) != hipSuccess) return e;
-  if (qb == 3) k_cg_start<3><<<kRedBlocks, kRedThreads, 0, s>>>(nu, b, minv, r, z, p, part);
-  else k_cg_start<1><<<kRedBlocks, kRedThreads, 0, s>>>(nu, b, minv, r, z, p, part);
-  k_cg_scalars<<<1, kRedThreads, 0, s>>>(part, 0, sc);
+  if (qb != 3) nslots = nullptr;
+  if (nslots) k_cg_nodes<<<nb256(8 * nu), 256, 0, s>>>(nu, nslots, indptr, indices, nodes);
+  int np = 0;
+  if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, x, r, nullptr, work + 7 * n, &np)) != hipSuccess)
+    return e;
   CgScal h{};
-  if ((e = hipMemcpyAsync(&h, sc, sizeof h, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
-  if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-  const double bn = sqrt(h.bb);
-  if (bn == 0.0) {  // b = 0: x = 0 is the solution
+  e = qb == 3 ? cg_iterations<3>(s, n, nnz, indptr, indices, vals, nslots, nodes, b, x, rtol, maxit, work, &h)
+              : cg_iterations<1>(s, n, nnz, indptr, indices, vals, nslots, nodes, b, x, rtol, maxit, work, &h);
+  if (e != hipSuccess) return e;
+  if (h.bb == 0.0) {  // b = 0: x = 0 is the solution
     if ((e = hipMemsetAsync(x, 0, 8 * (size_t)n, s)) != hipSuccess) return e;
     return hipStreamSynchronize(s);
   }
-  double res = sqrt(h.rr) / bn;
-  int it = 0;
-  while (res > rtol && it < maxit) {
-    if ((e = launch_spmv(s, n, nnz, indptr, indices, vals, p, q, false)) != hipSuccess) return e;
-    k_dot<<<kRedBlocks, kRedThreads, 0, s>>>(n, p, q, part);
-    k_cg_scalars<<<1, kRedThreads, 0, s>>>(part, 1, sc);
-    if (qb == 3) k_cg_update<3><<<kRedBlocks, kRedThreads, 0, s>>>(nu, sc, p, q, minv, x, r, z, part);
-    else k_cg_update<1><<<kRedBlocks, kRedThreads, 0, s>>>(nu, sc, p, q, minv, x, r, z, part);
-    k_cg_scalars<<<1, kRedThreads, 0, s>>>(part, 2, sc);
-    k_cg_direction<<<nb256(n), 256, 0, s>>>(n, sc, z, p);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(&h, sc, sizeof h, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
-    if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-    ++it;
-    res = sqrt(h.rr) / bn;
-    if (h.pq <= 0.0) break;  // K not positive definite along p
-  }
-  *iters = it;
-  *rel_res = res;
+  *iters = h.it;
+  *rel_res = sqrt(h.rr) / sqrt(h.bb);
   return hipSuccess;
 }
 

@@ -1377,11 +1377,11 @@ int gfx_ws_solve_cg(gfx_workspace *w, const double *d_b, double *d_x, double rto
   if (w->cg_n != n) {
     WHIP(w, hipStreamSynchronize(w->ctx->stream));
     wfree(w->d_cg);
-    if (hipMalloc((void **)&w->d_cg, 8 * cg_workspace_doubles(n)) != hipSuccess)
+    if (hipMalloc((void **)&w->d_cg, 8 * cg_workspace_doubles(n, 0)) != hipSuccess)
       return wfail(w, GFX_E_OOM, "CG vectors");
     w->cg_n = n;
   }
-  WHIP(w, cg_solve(w->ctx->stream, n, nnz, ip, ix, v, d_b, d_x, rtol, maxit, 1, w->d_cg, iters, rel_res));
+  WHIP(w, cg_solve(w->ctx->stream, n, nnz, ip, ix, v, nullptr, d_b, d_x, rtol, maxit, 1, w->d_cg, iters, rel_res));
   return GFX_OK;
 }
 
