@@ -221,21 +221,25 @@ struct PolyMatArgs {
   const int32_t *mptr;       // nout + 1: the monomials of output o
   const int32_t *moff;       // offsets into msym
   const int32_t *msym;
-  double *elem;              // n_cv * nr * nc, row r = i qt + a, column c = j qs + b
-  double *thr;               // n_cv: 1e-14 max|elem| (INFINITY: a zero element)
-  int64_t *cnt;              // n_cv: entries above the threshold
+  int nsym;                  // symbols of the table
+  bool varying;              // an output reads a fem field
+  int pmask, rmask;          // slots (bit 0 value, 1 + b gradient) of the test and trial function in use
+  double *elem;              // n_cv * nr * nc, row r = i qt + a, column c = j qs + b; entries at or
+                             // below the element's threshold are 0
   int *err;
 };
+constexpr uint32_t kPolyNone = 0xffffffffu;  // place of an entry that is not stored
 struct PolyEmitArgs {
   int64_t n_cv;
   int ndt, nds, qt, qs;
   const int32_t *dt, *ds;    // dof tables of the two fields (component 0 of each node)
   int64_t first_t, first_s;  // intervals of the two variables
   int64_t ncols;             // key = row * ncols + column
-  const double *elem, *thr;
+  const double *elem;
   const int64_t *off;        // n_cv: first slot of each element's entries
   uint64_t *keys;
   double *vals;
+  uint32_t *pos;             // launch_poly_keys: positions in the element matrices
 };
 // K = sum_v X_v grad(N_v) at point q (hexahedra) or the tetrahedron's edge
 // matrix; J = det K and B = K^{-T} row-major; false where J = 0
@@ -264,6 +268,28 @@ __device__ __forceinline__ bool poly_geometry(const double *pts, const int32_t *
   return true;
 }
 hipError_t launch_poly_mat(hipStream_t s, const PolyMatArgs &a);
+// The structure: every block's candidates (position base + index in the
+// element matrices), sorted by key (temporary storage: poly_structure_bytes)
+// with the heads of equal keys and their exclusive scan (n + 1; work:
+// scan_tmp_elems(n)), then the entries' candidate ranges, rows and columns.
+hipError_t launch_poly_keys(hipStream_t s, const PolyEmitArgs &a, int64_t base);
+size_t poly_structure_bytes(int64_t n, int end_bit);
+hipError_t poly_sort_candidates(hipStream_t s, void *tmp, size_t tmp_bytes, const uint64_t *keys, uint64_t *keys2,
+                                const uint32_t *pos, uint32_t *src, int64_t n, int end_bit, int64_t *head,
+                                int64_t *scan, int64_t *work);
+hipError_t launch_poly_entries(hipStream_t s, int64_t n, const uint64_t *keys, const int64_t *head,
+                               const int64_t *scan, int64_t ncols, uint32_t *start, int32_t *row, int32_t *col);
+// Sums into the stored entries; bit 4 of the error flag: other entries than
+// the stored ones have candidates.  Then poly_pattern makes the CSR's pattern
+// and the entries' places anew (work: 2 n + 1 + scan_tmp_elems(n) int64).
+hipError_t launch_poly_runs(hipStream_t s, int64_t n, const uint32_t *start, const uint32_t *src, const double *elem,
+                            const uint32_t *place, double *v, int *err);
+hipError_t poly_pattern(hipStream_t s, int64_t n, const uint32_t *start, const uint32_t *src, const double *elem,
+                        const int32_t *row, const int32_t *col, int64_t nrows, int64_t *work, uint32_t *place,
+                        int64_t *ip, int32_t *ix);
+hipError_t launch_poly_empty(hipStream_t s, int64_t nrows, int64_t *ip, int64_t *d_nnz);
+// beyond 2^31 candidates: entries above the threshold, counted and emitted
+hipError_t launch_poly_count(hipStream_t s, int64_t n_cv, int ne, const double *elem, int64_t *cnt);
 hipError_t launch_poly_emit(hipStream_t s, const PolyEmitArgs &a);
 // temporary storage of the stable key sort of n entries (bytes)
 size_t poly_sort_bytes(int64_t n, int end_bit);

@@ -59,6 +59,7 @@ struct ScProg {
   GwflScalarProgram prog;
   int vf = 0;                   // order 1: the field of the variable
   int nm = 0;
+  std::vector<int32_t> slots;   // table slots of the monomials' symbols
   double *d_coef = nullptr;
   int32_t *d_off = nullptr, *d_sym = nullptr, *d_out = nullptr;
   int32_t *d_mptr = nullptr;    // order 2: monomials of each output (sorted by output)
@@ -68,6 +69,10 @@ struct ScBlock {                // an order-2 block: test variable x trial varia
   std::string tv, sv;
   ScProg p;
   int vt = 0, vs = 0;           // their fields
+  bool varying = false;         // an output reads a fem field
+  int pmask = 0, rmask = 0;     // slots of the test and trial function in use
+  int ne = 0;                   // entries of an element matrix
+  int64_t base = 0;             // its element matrices in d_pelem
 };
 
 struct ScField {
@@ -116,9 +121,17 @@ struct ScalarRoute {
   // order 2 (polymat.hip): the blocks, or why they do not compile
   std::vector<ScBlock> blocks;
   std::string err2;
-  double *d_pelem = nullptr, *d_thr = nullptr;
-  int64_t *d_cnt = nullptr, *d_off = nullptr, *d_scan = nullptr, *d_nnz = nullptr;
-  // kept entries (keys, values and their sorted copies), sort and run work
+  double *d_pelem = nullptr;    // element matrices: every block's, or one block's beyond 2^31 candidates
+  int64_t *d_nnz = nullptr;
+  std::vector<double> h_consts;
+  // The structure (polymat.hip): n_cand candidates of n_ent matrix entries;
+  // n_ent < 0: not built yet.
+  int64_t n_cand = 0, n_ent = -1;
+  uint32_t *d_src = nullptr, *d_start = nullptr, *d_place = nullptr;
+  int32_t *d_row = nullptr, *d_col = nullptr;
+  // beyond 2^31 candidates: kept entries (keys, values and their sorted
+  // copies), sort and run work
+  int64_t *d_cnt = nullptr, *d_off = nullptr, *d_scan = nullptr;
   int64_t cap = 0;
   uint64_t *d_keys = nullptr, *d_keys2 = nullptr;
   double *d_vals = nullptr, *d_vals2 = nullptr;
@@ -486,11 +499,12 @@ void sc_release(ScalarRoute *sc) {
   wfree(sc->d_consts); wfree(sc->d_qw); wfree(sc->d_gN); wfree(sc->d_elem); wfree(sc->d_part); wfree(sc->d_sum);
   wfree(sc->d_V); wfree(sc->d_err);
   for (auto &b : sc->blocks) sc_free_prog(b.p);
-  wfree(sc->d_pelem); wfree(sc->d_thr); wfree(sc->d_cnt); wfree(sc->d_off); wfree(sc->d_scan);
+  wfree(sc->d_pelem); wfree(sc->d_src); wfree(sc->d_start); wfree(sc->d_place); wfree(sc->d_row); wfree(sc->d_col);
+  wfree(sc->d_cnt); wfree(sc->d_off); wfree(sc->d_scan);
   wfree(sc->d_nnz); wfree(sc->d_keys); wfree(sc->d_keys2); wfree(sc->d_vals); wfree(sc->d_vals2);
   wfree(sc->d_work); wfree(sc->d_sort); wfree(sc->d_ip); wfree(sc->d_ix); wfree(sc->d_v);
   sc->blocks.clear(); sc->err2.clear();
-  sc->cap = 0; sc->sort_cap = 0; sc->nnz = -1;
+  sc->cap = 0; sc->sort_cap = 0; sc->nnz = -1; sc->n_cand = 0; sc->n_ent = -1;
   sc->fields.clear(); sc->vars.clear(); sc->consts.clear();
   sc->p0 = ScProg();
   sc->mim = nullptr;
@@ -680,6 +694,7 @@ int sc_build(gfx_workspace *w) {
       out.push_back(mo.out);
     }
     p.nm = (int)coef.size();
+    p.slots = sym;
     if (upload(&p.d_coef, coef) != hipSuccess || upload(&p.d_off, offs) != hipSuccess ||
         upload(&p.d_sym, sym) != hipSuccess || upload(&p.d_out, out) != hipSuccess)
       return bail(GFX_E_OOM, "polynomial route programs");
@@ -697,18 +712,30 @@ int sc_build(gfx_workspace *w) {
         (int64_t)ft->fem.nd * ft->qdim * fs->fem.nd * fs->qdim > kPolyMaxEntries || b.p.prog.nout > kPolyMaxOut)
       return bail(GFX_E_UNSUPPORTED, "the order-2 block " + b.tv + " x " + b.sv +
                                          " is larger than the polynomial route's element matrices");
+    const int qt = ft->qdim, qs = fs->qdim;
+    for (auto &mo : b.p.prog.monos) {  // outputs: test slot * 4 qs + trial slot
+      const int ot = mo.out / (4 * qs), os = mo.out % (4 * qs);
+      b.pmask |= 1 << (ot < qt ? 0 : 1 + (ot - qt) % 3);
+      b.rmask |= 1 << (os < qs ? 0 : 1 + (os - qs) % 3);
+    }
+    for (int x : b.p.slots) b.varying |= x < sc->const_off;
+    b.ne = ft->fem.nd * qt * fs->fem.nd * qs;
+    b.base = sc->n_cand;
+    sc->n_cand += m->n_cv * b.ne;
     std::vector<int32_t> mptr((size_t)b.p.prog.nout + 1, 0);
     for (auto &mo : b.p.prog.monos) mptr[(size_t)mo.out + 1]++;
     for (size_t o = 0; o + 1 < mptr.size(); ++o) mptr[o + 1] += mptr[o];
     if (upload(&b.p.d_mptr, mptr) != hipSuccess) return bail(GFX_E_OOM, "order-2 route programs");
-    pelem = std::max(pelem, m->n_cv * (int64_t)ft->fem.nd * ft->qdim * fs->fem.nd * fs->qdim);
+    pelem = std::max(pelem, m->n_cv * b.ne);
   }
+  const bool structure = sc->n_cand <= INT32_MAX;
+  if (structure) pelem = sc->n_cand;
   if (!sc->blocks.empty() &&
       (hipMalloc((void **)&sc->d_pelem, 8 * (size_t)std::max<int64_t>(pelem, 1)) != hipSuccess ||
-       hipMalloc((void **)&sc->d_thr, 8 * (size_t)std::max<int64_t>(m->n_cv, 1)) != hipSuccess ||
-       hipMalloc((void **)&sc->d_cnt, 8 * (size_t)std::max<int64_t>(m->n_cv, 1)) != hipSuccess ||
-       hipMalloc((void **)&sc->d_off, 8 * (size_t)std::max<int64_t>(m->n_cv, 1)) != hipSuccess ||
-       hipMalloc((void **)&sc->d_scan, 8 * (size_t)std::max<int64_t>(scan_tmp_elems(m->n_cv), 1)) != hipSuccess))
+       (!structure &&
+        (hipMalloc((void **)&sc->d_cnt, 8 * (size_t)m->n_cv) != hipSuccess ||
+         hipMalloc((void **)&sc->d_off, 8 * (size_t)(m->n_cv + 1)) != hipSuccess ||
+         hipMalloc((void **)&sc->d_scan, 8 * (size_t)scan_tmp_elems(m->n_cv)) != hipSuccess))))
     return bail(GFX_E_OOM, "order-2 route buffers");
   int64_t elem = m->n_cv, nvec = 0;
   hipStream_t s = w->ctx->stream;
@@ -788,12 +815,13 @@ int sc_upload(gfx_workspace *w) {
     else
       WHIP(w, hipMemcpyAsync(f.d_U, v.V.data(), 8 * v.V.size(), hipMemcpyHostToDevice, s));
   }
-  std::vector<double> cv;
-  for (const std::string &n : sc->consts) cv.push_back(w->vars.at(n).V[0]);
-  if (!cv.empty()) WHIP(w, hipMemcpyAsync(sc->d_consts, cv.data(), 8 * cv.size(), hipMemcpyHostToDevice, s));
+  sc->h_consts.clear();
+  for (const std::string &n : sc->consts) sc->h_consts.push_back(w->vars.at(n).V[0]);
+  if (!sc->h_consts.empty())
+    WHIP(w, hipMemcpyAsync(sc->d_consts, sc->h_consts.data(), 8 * sc->h_consts.size(), hipMemcpyHostToDevice, s));
+  // the host buffers above are read before they can change: every assembly
+  // ends with a synchronisation of the stream
   WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
-  // the host buffers above are read before they can change
-  WHIP(w, hipStreamSynchronize(s));
   return GFX_OK;
 }
 
@@ -829,10 +857,163 @@ int sc_grow(gfx_workspace *w, int64_t need) {
   return GFX_OK;
 }
 
-// assembly(2) on the polynomial route: every block's element matrices, their
-// entries above the element threshold as keys in element order, then one
-// sort and sum into the nvec x nvec matrix (tested dofs x trial dofs at the
-// variables' intervals)
+// Device scratch for the duration of a call.
+struct Scratch {
+  std::vector<void *> p;
+  template <typename T>
+  T *get(size_t n) {
+    void *q = nullptr;
+    if (hipMalloc(&q, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) return nullptr;
+    p.push_back(q);
+    return static_cast<T *>(q);
+  }
+  ~Scratch() {
+    for (void *q : p) (void)hipFree(q);
+  }
+};
+
+PolyEmitArgs sc_emit_args(gfx_workspace *w, const ScBlock &b) {
+  const WsVar &vt = w->vars.at(b.tv), &vs = w->vars.at(b.sv);
+  PolyEmitArgs pe{};
+  pe.n_cv = w->sc->mim->mesh->n_cv;
+  pe.ndt = vt.mf->fem.nd; pe.nds = vs.mf->fem.nd; pe.qt = vt.mf->qdim; pe.qs = vs.mf->qdim;
+  pe.dt = vt.mf->d_dofs; pe.ds = vs.mf->d_dofs;
+  pe.first_t = vt.first; pe.first_s = vs.first; pe.ncols = w->sc->nvec;
+  return pe;
+}
+
+int sc_key_bits(int64_t n) {
+  int end_bit = 1;
+  while (end_bit < 64 && ((uint64_t)1 << end_bit) < (uint64_t)n * (uint64_t)n) ++end_bit;
+  return end_bit;
+}
+
+// Which candidates make up which matrix entry, from the dof tables: once per
+// set of registrations and expressions.
+int sc_structure(gfx_workspace *w) {
+  ScalarRoute *sc = w->sc;
+  hipStream_t s = w->ctx->stream;
+  const int64_t n = sc->n_cand;
+  if (n == 0) {
+    sc->n_ent = 0;
+    return GFX_OK;
+  }
+  const int bits = sc_key_bits(sc->nvec);
+  wfree(sc->d_src); wfree(sc->d_start); wfree(sc->d_row); wfree(sc->d_col); wfree(sc->d_place);  // of a failed attempt
+  wfree(sc->d_v); wfree(sc->d_ix);
+  Scratch t;
+  const size_t sb = poly_structure_bytes(n, bits);
+  uint64_t *keys = t.get<uint64_t>((size_t)n), *keys2 = t.get<uint64_t>((size_t)n);
+  uint32_t *pos = t.get<uint32_t>((size_t)n);
+  int64_t *head = t.get<int64_t>((size_t)n), *scan = t.get<int64_t>((size_t)n + 1);
+  int64_t *work = t.get<int64_t>((size_t)scan_tmp_elems(n));
+  void *tmp = t.get<char>(sb);
+  if (!keys || !keys2 || !pos || !head || !scan || !work || !tmp ||
+      hipMalloc((void **)&sc->d_src, 4 * (size_t)n) != hipSuccess)
+    return wfail(w, GFX_E_OOM, "order-2 route structure");
+  for (auto &b : sc->blocks) {
+    PolyEmitArgs pe = sc_emit_args(w, b);
+    pe.keys = keys + b.base;
+    pe.pos = pos + b.base;
+    WHIP(w, launch_poly_keys(s, pe, b.base));
+  }
+  WHIP(w, poly_sort_candidates(s, tmp, sb, keys, keys2, pos, sc->d_src, n, bits, head, scan, work));
+  int64_t n_ent = 0;
+  WHIP(w, hipMemcpyAsync(&n_ent, scan + n, 8, hipMemcpyDeviceToHost, s));
+  WHIP(w, hipStreamSynchronize(s));
+  if (hipMalloc((void **)&sc->d_start, 4 * (size_t)(n_ent + 1)) != hipSuccess ||
+      hipMalloc((void **)&sc->d_row, 4 * (size_t)n_ent) != hipSuccess ||
+      hipMalloc((void **)&sc->d_col, 4 * (size_t)n_ent) != hipSuccess ||
+      hipMalloc((void **)&sc->d_place, 4 * (size_t)n_ent) != hipSuccess ||
+      hipMalloc((void **)&sc->d_v, 8 * (size_t)n_ent) != hipSuccess ||
+      hipMalloc((void **)&sc->d_ix, 4 * (size_t)n_ent) != hipSuccess)
+    return wfail(w, GFX_E_OOM, "order-2 route matrix");
+  WHIP(w, launch_poly_entries(s, n, keys2, head, scan, sc->nvec, sc->d_start, sc->d_row, sc->d_col));
+  WHIP(w, hipMemsetAsync(sc->d_place, 0xff, 4 * (size_t)n_ent, s));  // nothing stored yet
+  WHIP(w, hipStreamSynchronize(s));
+  sc->n_ent = n_ent;
+  return GFX_OK;
+}
+
+// the matrix from the structure: sums into the stored entries, the pattern
+// anew where the element matrices give another
+int sc_matrix(gfx_workspace *w) {
+  ScalarRoute *sc = w->sc;
+  hipStream_t s = w->ctx->stream;
+  int flag = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    WHIP(w, launch_poly_runs(s, sc->n_ent, sc->d_start, sc->d_src, sc->d_pelem, sc->d_place, sc->d_v, sc->d_err));
+    WHIP(w, hipMemcpyAsync(&flag, sc->d_err, 4, hipMemcpyDeviceToHost, s));
+    WHIP(w, hipStreamSynchronize(s));
+    if (flag & 1) return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
+    if (sc->nnz >= 0 && !(flag & 4)) return GFX_OK;
+    sc->nnz = -1;
+    Scratch t;
+    int64_t *work = t.get<int64_t>((size_t)(2 * sc->n_ent + 1 + scan_tmp_elems(sc->n_ent)));
+    if (!work) return wfail(w, GFX_E_OOM, "order-2 route pattern");
+    int64_t nnz = 0;
+    if (sc->n_ent == 0) WHIP(w, launch_poly_empty(s, sc->nvec, sc->d_ip, sc->d_nnz));
+    else
+      WHIP(w, poly_pattern(s, sc->n_ent, sc->d_start, sc->d_src, sc->d_pelem, sc->d_row, sc->d_col, sc->nvec, work,
+                           sc->d_place, sc->d_ip, sc->d_ix));
+    WHIP(w, hipMemcpyAsync(&nnz, sc->d_ip + sc->nvec, 8, hipMemcpyDeviceToHost, s));
+    WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
+    WHIP(w, hipStreamSynchronize(s));
+    sc->nnz = nnz;
+  }
+  return GFX_OK;
+}
+
+// beyond 2^31 candidates: the kept entries of a block in element order
+int sc_emit(gfx_workspace *w, const ScBlock &b, int64_t &total) {
+  ScalarRoute *sc = w->sc;
+  hipStream_t s = w->ctx->stream;
+  const int64_t n_cv = sc->mim->mesh->n_cv;
+  WHIP(w, launch_poly_count(s, n_cv, b.ne, sc->d_pelem, sc->d_cnt));
+  WHIP(w, scan_exclusive_i64(s, sc->d_cnt, sc->d_off, n_cv, sc->d_scan));
+  int64_t nb = 0;
+  WHIP(w, hipMemcpyAsync(&nb, sc->d_off + n_cv, 8, hipMemcpyDeviceToHost, s));
+  WHIP(w, hipStreamSynchronize(s));
+  if (total + nb > INT32_MAX) return wfail(w, GFX_E_UNSUPPORTED, "more than 2^31 kept entries");
+  int r;
+  if ((r = sc_grow(w, total + nb))) return r;
+  PolyEmitArgs pe = sc_emit_args(w, b);
+  pe.elem = sc->d_pelem; pe.off = sc->d_off;
+  pe.keys = sc->d_keys + total; pe.vals = sc->d_vals + total;
+  WHIP(w, launch_poly_emit(s, pe));
+  total += nb;
+  return GFX_OK;
+}
+
+int sc_sorted_matrix(gfx_workspace *w, int64_t total) {
+  ScalarRoute *sc = w->sc;
+  hipStream_t s = w->ctx->stream;
+  const int64_t n = sc->nvec;
+  int r;
+  if ((r = sc_grow(w, std::max<int64_t>(total, 1)))) return r;
+  const int end_bit = sc_key_bits(n);
+  const size_t sb = poly_sort_bytes(total, end_bit);
+  if (sb > sc->sort_cap) {
+    WHIP(w, hipStreamSynchronize(s));
+    wfree(sc->d_sort);
+    if (hipMalloc(&sc->d_sort, sb) != hipSuccess) return wfail(w, GFX_E_OOM, "order-2 route sort");
+    sc->sort_cap = sb;
+  }
+  WHIP(w, poly_to_csr(s, sc->d_sort, sc->sort_cap, sc->d_keys, sc->d_vals, sc->d_keys2, sc->d_vals2, total,
+                      end_bit, n, n, sc->d_work, sc->d_ip, sc->d_ix, sc->d_v, sc->d_nnz));
+  int flag = 0;
+  int64_t nnz = 0;
+  WHIP(w, hipMemcpyAsync(&nnz, sc->d_nnz, 8, hipMemcpyDeviceToHost, s));
+  WHIP(w, hipMemcpyAsync(&flag, sc->d_err, 4, hipMemcpyDeviceToHost, s));
+  WHIP(w, hipStreamSynchronize(s));
+  if (flag & 1) return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
+  sc->nnz = nnz;
+  return GFX_OK;
+}
+
+// assembly(2) on the polynomial route: every block's element matrices, then
+// the nvec x nvec matrix (tested dofs x trial dofs at the variables'
+// intervals) from their entries above the element threshold
 int sc_run2(gfx_workspace *w) {
   if (!w->sc) w->sc = new (std::nothrow) ScalarRoute();
   if (!w->sc) return wfail(w, GFX_E_OOM, "workspace");
@@ -852,6 +1033,8 @@ int sc_run2(gfx_workspace *w) {
         hipMalloc((void **)&sc->d_nnz, 8) != hipSuccess)
       return wfail(w, GFX_E_OOM, "order-2 route matrix");
   }
+  const bool structure = sc->n_cand <= INT32_MAX;
+  if (structure && sc->n_ent < 0 && (r = sc_structure(w))) return r;
   PolyMatArgs a{};
   a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx; a.nv = m->nv; a.gN = sc->d_gN;
   a.nq = sc->mim->rule.n(); a.qw = sc->d_qw;
@@ -860,56 +1043,21 @@ int sc_run2(gfx_workspace *w) {
     const ScField &f = sc->fields[i];
     a.f[i] = ScalarField{f.mf->d_dofs, f.d_U, f.d_phi, f.d_gref, f.mf->fem.nd, f.mf->qdim, f.off};
   }
-  a.nconst = (int)sc->consts.size(); a.const_off = sc->const_off; a.consts = sc->d_consts;
-  a.elem = sc->d_pelem; a.thr = sc->d_thr; a.cnt = sc->d_cnt; a.err = sc->d_err;
+  a.nconst = (int)sc->consts.size(); a.const_off = sc->const_off; a.consts = sc->d_consts; a.nsym = sc->nsym;
+  a.err = sc->d_err;
   int64_t total = 0;
   for (auto &b : sc->blocks) {
     a.vt = b.vt; a.vs = b.vs;
-    a.nout = b.p.prog.nout;
+    a.nout = b.p.prog.nout; a.varying = b.varying; a.pmask = b.pmask; a.rmask = b.rmask;
     a.mcoef = b.p.d_coef; a.mptr = b.p.d_mptr; a.moff = b.p.d_off; a.msym = b.p.d_sym;
+    a.elem = sc->d_pelem + (structure ? b.base : 0);
     WHIP(w, launch_poly_mat(s, a));
-    WHIP(w, scan_exclusive_i64(s, sc->d_cnt, sc->d_off, m->n_cv, sc->d_scan));
-    int64_t tail[2] = {0, 0};
-    if (m->n_cv > 0) {
-      WHIP(w, hipMemcpyAsync(&tail[0], sc->d_off + m->n_cv - 1, 8, hipMemcpyDeviceToHost, s));
-      WHIP(w, hipMemcpyAsync(&tail[1], sc->d_cnt + m->n_cv - 1, 8, hipMemcpyDeviceToHost, s));
-    }
-    WHIP(w, hipStreamSynchronize(s));
-    const int64_t nb = tail[0] + tail[1];
-    if (total + nb > INT32_MAX) return wfail(w, GFX_E_UNSUPPORTED, "more than 2^31 kept entries");
-    if ((r = sc_grow(w, total + nb))) return r;
-    const WsVar &vt = w->vars.at(b.tv), &vs = w->vars.at(b.sv);
-    PolyEmitArgs pe{};
-    pe.n_cv = m->n_cv;
-    pe.ndt = vt.mf->fem.nd; pe.nds = vs.mf->fem.nd; pe.qt = vt.mf->qdim; pe.qs = vs.mf->qdim;
-    pe.dt = vt.mf->d_dofs; pe.ds = vs.mf->d_dofs;
-    pe.first_t = vt.first; pe.first_s = vs.first; pe.ncols = n;
-    pe.elem = sc->d_pelem; pe.thr = sc->d_thr; pe.off = sc->d_off;
-    pe.keys = sc->d_keys + total; pe.vals = sc->d_vals + total;
-    WHIP(w, launch_poly_emit(s, pe));
-    total += nb;
+    if (!structure && (r = sc_emit(w, b, total))) return r;
   }
-  if ((r = sc_grow(w, std::max<int64_t>(total, 1)))) return r;
-  int end_bit = 1;
-  while (end_bit < 64 && ((uint64_t)1 << end_bit) < (uint64_t)n * (uint64_t)n) ++end_bit;
-  const size_t sb = poly_sort_bytes(total, end_bit);
-  if (sb > sc->sort_cap) {
-    WHIP(w, hipStreamSynchronize(s));
-    wfree(sc->d_sort);
-    if (hipMalloc(&sc->d_sort, sb) != hipSuccess) return wfail(w, GFX_E_OOM, "order-2 route sort");
-    sc->sort_cap = sb;
-  }
-  WHIP(w, poly_to_csr(s, sc->d_sort, sc->sort_cap, sc->d_keys, sc->d_vals, sc->d_keys2, sc->d_vals2, total,
-                      end_bit, n, n, sc->d_work, sc->d_ip, sc->d_ix, sc->d_v, sc->d_nnz));
-  int flag = 0;
-  int64_t nnz = 0;
-  WHIP(w, hipMemcpyAsync(&nnz, sc->d_nnz, 8, hipMemcpyDeviceToHost, s));
-  WHIP(w, hipMemcpyAsync(&flag, sc->d_err, 4, hipMemcpyDeviceToHost, s));
-  WHIP(w, hipStreamSynchronize(s));
-  if (flag & 1) return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
-  sc->nnz = nnz;
+  if ((r = structure ? sc_matrix(w) : sc_sorted_matrix(w, total))) return r;
   if (w->ext) {
     if (w->ext_n != n) return wfail(w, GFX_E_INVALID, "target matrix of another size");
+    int flag = 0;
     WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
     WHIP(w, launch_add_into(s, w->ext_orient == GFX_CSC, n, sc->d_ip, sc->d_ix, sc->d_v, w->ext_ptr, w->ext_ind,
                             w->ext_vals, sc->d_err));
