@@ -5,96 +5,134 @@
 // src/getfem_generic_assembly_compile_and_exec.cc:4669-4735) for integrands
 // the compile stage turned into polynomial programs.
 //
-// k_scalar_elem: one thread per element (affine tetrahedra, or Q1 hexahedra
-// with the geometry at every point).  At
-// each integration point the thread fills its row of a symbol table in LDS
-// (values and gradients of the fem fields the program reads, then the
-// fixed-size constants), evaluates the program's monomials into its output
-// coefficients and integrates them: order 0, the potential's element value;
-// order 1, the element vector of the differentiated variable,
-//   elem[i, a] += w_q |J| (c_a phi_i + sum_b c_(q + 3a + b) (B grad phi_i)_b).
+// k_scalar_elem: G lanes per element (affine tetrahedra, or Q1 hexahedra with
+// the geometry at every point), a lane per integration point.
+// The lane fills its row of a symbol table in LDS (values and gradients of the
+// fem fields the program reads, from the element's nodal values in LDS, then
+// the fixed-size constants), evaluates the program's monomials into its output
+// coefficients and weights them; then the lanes take the results: order 0, the
+// potential's element value (one lane adds the points in order); order 1, the
+// element vector of the differentiated variable, a lane per dof,
+//   elem[i, a] = sum_q w_q |J| (c_a phi_i + sum_b c_(q + 3a + b) (B grad phi_i)_b),
+// with the B of a point taken to the coefficients' side.
 // The program is the same for every thread (uniform loads).  Element vectors
 // go to a buffer and are summed per dof over the node's incidences (no
 // atomics); element values are summed by a fixed-order two-stage reduction,
 // so both results are deterministic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "gfx_internal.h"
 
 namespace gfx {
 namespace {
 
-constexpr int kScThreads = 64;
+constexpr int kScThreads = 64;  // one wavefront
 constexpr int kScRedThreads = 256;
 constexpr int kScRedBlocks = 256;
 
-__global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a) {
-  __shared__ double tab[kScThreads][kScalarMaxSyms + 1];
-  __shared__ double oc[kScThreads][kScalarMaxOut + 1];
-  const int64_t e = (int64_t)blockIdx.x * kScThreads + threadIdx.x;
-  if (e >= a.n_cv) return;  // no barrier below
-  double *T = tab[threadIdx.x];
-  double *O = oc[threadIdx.x];
-  // geometry: once for an affine tetrahedron, at every point for a hexahedron
-  const int32_t *cv = a.cvx + (int64_t)a.nv * e;
-  double B[9], aJ = 0.0;
-  bool ok = poly_geometry(a.pts, cv, a.nv, a.gN, B, aJ);
-  for (int q = 1; ok && a.gN && q < a.nq; ++q) {
-    double Bq[9], aq;
-    ok = poly_geometry(a.pts, cv, a.nv, a.gN + (int64_t)q * a.nv * 3, Bq, aq);
-  }
-  if (!ok) {
-    atomicOr(a.err, 1);
-    return;
-  }
-  for (int c = 0; c < a.nconst; ++c) T[a.const_off + c] = a.consts[c];
-  const ScalarField &vf = a.f[a.vf];
-  const int nl = a.order == 1 ? vf.nd * vf.qdim : 0;
-  double *el = a.order == 1 ? a.elem + e * nl : nullptr;
-  for (int t = 0; t < nl; ++t) el[t] = 0.0;
-  double acc = 0.0;
-  for (int q = 0; q < a.nq; ++q) {
-    if (a.gN && q > 0) poly_geometry(a.pts, cv, a.nv, a.gN + (int64_t)q * a.nv * 3, B, aJ);
-    const double wJ = a.qw[q] * aJ;
+// Bound by latency (dependent loads and FP64 chains), so the points go side by
+// side: with a lane per element, 20,250 elements were 317 wavefronts for the
+// whole chip, each with 15 points one after another.  Measured there (u P2
+// vector + p P1): 58 us a variable, 222 us before.
+template <int G>
+__global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a, int nsym, int nvals) {
+  extern __shared__ double lds_sc[];
+  constexpr int kPer = kScThreads / G;
+  const int t = threadIdx.x, g = t / G, l = t % G;
+  double *T = lds_sc + t;                           // symbols, T[s * kScThreads]
+  double *O = T + nsym * kScThreads;                // outputs, then (order 1) the weighted coefficients
+  double *V = lds_sc + (nsym + max(a.nout, 12)) * kScThreads + g * nvals;  // nodal values, [field][node][component]
+  const int64_t e0 = (int64_t)blockIdx.x * kPer + g;
+  const bool live = e0 < a.n_cv;
+  const int64_t e = live ? e0 : a.n_cv - 1;  // past the last element: computed, not written
+  {
+    double *v = V;
     for (int fi = 0; fi < a.nf; ++fi) {
       const ScalarField &f = a.f[fi];
-      const int Q = f.qdim;
-      const int32_t *dofs = f.dofs + e * f.nd;
-      for (int c = 0; c < Q; ++c) {
-        double v = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
-        for (int i = 0; i < f.nd; ++i) {
-          const double u = f.U[(int64_t)dofs[i] + c];
-          const double *g = f.gref + ((int64_t)q * f.nd + i) * 3;
-          v += f.phi[q * f.nd + i] * u;
-          r0 += g[0] * u; r1 += g[1] * u; r2 += g[2] * u;
-        }
-        T[f.off + c] = v;
-        for (int b = 0; b < 3; ++b) T[f.off + Q + 3 * c + b] = B[3 * b] * r0 + B[3 * b + 1] * r1 + B[3 * b + 2] * r2;
+      const int n = f.nd * f.qdim;
+      for (int x = l; x < n; x += G) {
+        const int i = x / f.qdim;
+        v[x] = f.U[(int64_t)f.dofs[e * f.nd + i] + (x - i * f.qdim)];
       }
-    }
-    for (int o = 0; o < a.nout; ++o) O[o] = 0.0;
-    for (int m = 0; m < a.nm; ++m) {
-      double v = a.mcoef[m];
-      for (int s = a.moff[m]; s < a.moff[m + 1]; ++s) v *= T[a.msym[s]];
-      O[a.mout[m]] += v;
-    }
-    if (a.order == 0) {
-      acc += wJ * O[0];
-      continue;
-    }
-    const int Q = vf.qdim;
-    for (int i = 0; i < vf.nd; ++i) {
-      const double phi = vf.phi[q * vf.nd + i];
-      const double *h = vf.gref + ((int64_t)q * vf.nd + i) * 3;
-      double g[3];
-      for (int b = 0; b < 3; ++b) g[b] = B[3 * b] * h[0] + B[3 * b + 1] * h[1] + B[3 * b + 2] * h[2];
-      for (int c = 0; c < Q; ++c) {
-        const double *oc3 = O + Q + 3 * c;
-        el[i * Q + c] += wJ * (O[c] * phi + oc3[0] * g[0] + oc3[1] * g[1] + oc3[2] * g[2]);
-      }
+      v += n;
     }
   }
-  if (a.order == 0) a.elem[e] = acc;
+  for (int c = 0; c < a.nconst; ++c) T[(a.const_off + c) * kScThreads] = a.consts[c];
+  const int32_t *cv = a.cvx + (int64_t)a.nv * e;
+  const ScalarField &vf = a.f[a.vf];
+  const int Q = vf.qdim, nl = a.order == 1 ? vf.nd * Q : 0;
+  double acc = 0.0;
+  __syncthreads();
+  for (int q0 = 0; q0 < a.nq; q0 += G) {
+    const int q = min(q0 + l, a.nq - 1), nq = min(G, a.nq - q0);  // the points of this round
+    double B[9], aJ = 0.0;
+    const bool ok = poly_geometry(a.pts, cv, a.nv, a.gN ? a.gN + (int64_t)q * a.nv * 3 : nullptr, B, aJ);
+    if (!ok && live) atomicOr(a.err, 1);
+    const double wJ = ok ? a.qw[q] * aJ : 0.0;
+    const double *v0 = V;
+    for (int fi = 0; fi < a.nf; ++fi) {
+      const ScalarField &f = a.f[fi];
+      const double *phi = f.phi + q * f.nd, *gr = f.gref + (int64_t)q * f.nd * 3;
+      for (int c = 0; c < f.qdim; ++c) {
+        double v = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
+        for (int i = 0; i < f.nd; ++i) {
+          const double u = v0[i * f.qdim + c];
+          v += phi[i] * u;
+          r0 += gr[3 * i] * u; r1 += gr[3 * i + 1] * u; r2 += gr[3 * i + 2] * u;
+        }
+        T[(f.off + c) * kScThreads] = v;
+        for (int b = 0; b < 3; ++b)
+          T[(f.off + f.qdim + 3 * c + b) * kScThreads] = B[3 * b] * r0 + B[3 * b + 1] * r1 + B[3 * b + 2] * r2;
+      }
+      v0 += f.nd * f.qdim;
+    }
+    for (int o = 0; o < a.nout; ++o) O[o * kScThreads] = 0.0;
+    for (int m = 0; m < a.nm; ++m) {
+      double v = a.mcoef[m];
+      for (int s = a.moff[m]; s < a.moff[m + 1]; ++s) v *= T[a.msym[s] * kScThreads];
+      O[a.mout[m] * kScThreads] += v;
+    }
+    if (a.order == 0) {
+      O[0] = wJ * O[0];
+      __syncthreads();
+      if (l == 0)
+        for (int k = 0; k < nq; ++k) acc += O[k];
+    } else {
+      // w_q |J| times the value's and (against the reference gradients) the gradient's coefficients
+      double cw[3][4];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        if (c >= Q) break;
+        const double *oc = O + (Q + 3 * c) * kScThreads;
+        const double o0 = oc[0], o1 = oc[kScThreads], o2 = oc[2 * kScThreads];
+        cw[c][0] = wJ * O[c * kScThreads];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) cw[c][1 + d] = wJ * (o0 * B[d] + o1 * B[3 + d] + o2 * B[6 + d]);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        if (c < Q)
+#pragma unroll
+          for (int d = 0; d < 4; ++d) O[(4 * c + d) * kScThreads] = cw[c][d];
+      __syncthreads();
+      double *el = a.elem + e * nl;
+      for (int x = l; x < nl; x += G) {
+        const int i = x / Q, c = x - i * Q;
+        const double *w = lds_sc + (nsym + 4 * c) * kScThreads + g * G;  // point k: w[k]
+        double s = q0 && live ? el[x] : 0.0;
+        for (int k = 0; k < nq; ++k) {
+          const int p = (q0 + k) * vf.nd + i;
+          const double *h = vf.gref + (int64_t)p * 3;
+          s += w[k] * vf.phi[p] + w[kScThreads + k] * h[0] + w[2 * kScThreads + k] * h[1] + w[3 * kScThreads + k] * h[2];
+        }
+        if (live) el[x] = s;
+      }
+    }
+    __syncthreads();
+  }
+  if (a.order == 0 && l == 0 && live) a.elem[e] = acc;
 }
 
 __device__ __forceinline__ double sc_block_sum(double v, double *sh) {
@@ -135,10 +173,24 @@ int64_t scalar_partials() { return kScRedBlocks; }
 
 hipError_t launch_scalar_elem(hipStream_t s, const ScalarArgs &a) {
   if (a.n_cv == 0) return hipSuccess;
-  if (a.nf < 1 || a.nf > kScalarMaxFields || a.nout > kScalarMaxOut || a.vf < 0 || a.vf >= a.nf)
+  if (a.nf < 1 || a.nf > kScalarMaxFields || a.nout > kScalarMaxOut || a.vf < 0 || a.vf >= a.nf ||
+      a.f[a.vf].qdim > 3)
     return hipErrorInvalidValue;
-  const unsigned grid = (unsigned)((a.n_cv + kScThreads - 1) / kScThreads);
-  k_scalar_elem<<<grid, kScThreads, 0, s>>>(a);
+  int nvals = 0;
+  for (int i = 0; i < a.nf; ++i) nvals += a.f[i].nd * a.f[i].qdim;
+  const int nsym = a.const_off + a.nconst;
+  auto lds = [&](int g) {
+    return 8 * ((size_t)(nsym + std::max(a.nout, 12)) * kScThreads + (size_t)(kScThreads / g) * nvals);
+  };
+  auto grid = [&](int g) { return (unsigned)((a.n_cv + kScThreads / g - 1) / (kScThreads / g)); };
+  // as many lanes as the rule has points, and the elements of a wavefront
+  // must fit its LDS
+  if (a.nq <= 1 && lds(1) <= 48 * 1024) k_scalar_elem<1><<<grid(1), kScThreads, lds(1), s>>>(a, nsym, nvals);
+  else if (a.nq <= 4 && lds(4) <= 48 * 1024) k_scalar_elem<4><<<grid(4), kScThreads, lds(4), s>>>(a, nsym, nvals);
+  else if (a.nq <= 16 && lds(16) <= 64 * 1024) k_scalar_elem<16><<<grid(16), kScThreads, lds(16), s>>>(a, nsym, nvals);
+  else if (a.nq <= 32 && lds(32) <= 64 * 1024) k_scalar_elem<32><<<grid(32), kScThreads, lds(32), s>>>(a, nsym, nvals);
+  else if (lds(64) <= 64 * 1024) k_scalar_elem<64><<<grid(64), kScThreads, lds(64), s>>>(a, nsym, nvals);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 
