@@ -178,6 +178,8 @@ int gfx_ctx_destroy(gfx_ctx *c) {
 int gfx_ctx_set_stream(gfx_ctx *c, void *s) {
   if (!c) return GFX_E_INVALID;
   if (set_device(c)) return GFX_E_HIP;
+  // the stream that the context has already (its own one for NULL) stays
+  if (s ? c->stream == (hipStream_t)s : c->own_stream && c->stream) return GFX_OK;
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
   if (s) {
     c->stream = (hipStream_t)s;
@@ -1575,7 +1577,8 @@ int gfx_compliance_destroy(gfx_compliance *c) {
   if (!c) return GFX_E_INVALID;
   (void)hipSetDevice(c->ctx->device);
   dfree(c->d_vinc_ptr); dfree(c->d_dinc_ptr); dfree(c->d_vinc); dfree(c->d_dinc);
-  dfree(c->d_cX); dfree(c->d_cU); dfree(c->d_Jpart); dfree(c->d_err);
+  dfree(c->d_cX); dfree(c->d_cU); dfree(c->d_Jpart);
+  if (c->h_err) (void)hipHostFree(c->h_err);
   gfx_ctx *ctx = c->ctx;
   gfx_mesh_fem *mf = c->mf;
   delete c;
@@ -1611,8 +1614,9 @@ int gfx_compliance_create(gfx_mesh_fem *mf, gfx_mesh_im *mim, double lambda, dou
   if (e == hipSuccess) e = dalloc(&c->d_cX, (size_t)m->n_cv * 12);
   if (e == hipSuccess) e = dalloc(&c->d_cU, (size_t)m->n_cv * 12);
   if (e == hipSuccess) e = dalloc(&c->d_Jpart, 2 * (size_t)compliance_nblocks(m->n_cv));
-  if (e == hipSuccess) e = dalloc(&c->d_err, 1);
-  if (e == hipSuccess) e = hipMemset(c->d_err, 0, 4);  // sticky: set by any evaluation that meets J = 0
+  if (e == hipSuccess) e = hipHostMalloc((void **)&c->h_err, sizeof(int), hipHostMallocMapped);
+  if (e == hipSuccess) *c->h_err = 0;
+  if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->d_err, c->h_err, 0);
   if (e == hipSuccess) e = dalloc(&tmp, (size_t)(2 * big + scan_tmp_elems(big)));
   if (e == hipSuccess)
     e = launch_incidences(ctx->stream, m->n_cv, 4, 1, m->d_cvx, m->n_pts, c->d_vinc_ptr, c->d_vinc, tmp);
@@ -1632,12 +1636,10 @@ int gfx_compliance_status(gfx_compliance *c) {
   if (!c) return GFX_E_INVALID;
   gfx_ctx *ctx = c->ctx;
   if (set_device(ctx)) return GFX_E_HIP;
-  int flag = 0;
-  HIPCHK(ctx, hipMemcpyAsync(&flag, c->d_err, 4, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  if (flag) {
-    HIPCHK(ctx, hipMemsetAsync(c->d_err, 0, 4, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  volatile int *flag = c->h_err;
+  if (*flag) {
+    *flag = 0;
     return fail(ctx, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
   }
   return GFX_OK;

@@ -414,7 +414,9 @@ struct gfx_compliance {
   int32_t *d_vinc_ptr = nullptr, *d_dinc_ptr = nullptr;  // point / dof-node incidences
   uint32_t *d_vinc = nullptr, *d_dinc = nullptr;
   double *d_cX = nullptr, *d_cU = nullptr, *d_Jpart = nullptr;
-  int *d_err = nullptr;
+  // set by any evaluation that meets J = 0: pinned host memory that the
+  // kernel stores to, so that reading it takes a wait but no copy
+  int *h_err = nullptr, *d_err = nullptr;  // the host's and the device's address of it
 };
 
 namespace gfx {
