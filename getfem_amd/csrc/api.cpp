@@ -45,6 +45,33 @@ void dfree(T *&p) {
   p = nullptr;
 }
 
+// Arrays that live and die together in one allocation (an allocation and a
+// free each cost some 10 us and a wait for the device): add() them, then
+// alloc() sets their pointers, each 256-byte aligned.
+struct Carve {
+  std::vector<std::pair<void **, size_t>> parts;
+  size_t bytes = 0;
+  template <typename T>
+  void add(T **p, size_t n) {
+    *p = nullptr;
+    parts.push_back({(void **)p, bytes});
+    bytes += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+  }
+  hipError_t alloc(char **base) {
+    hipError_t e = dalloc(base, bytes);
+    if (e == hipSuccess)
+      for (auto &x : parts) *x.first = *base + x.second;
+    return e;
+  }
+};
+
+// a Carve for the duration of a call
+struct Scratch : Carve {
+  char *base = nullptr;
+  hipError_t alloc() { return Carve::alloc(&base); }
+  ~Scratch() { dfree(base); }
+};
+
 void il_free(gfx::IldltData &L) {
   dfree(L.d_dpos); dfree(L.d_fdeg); dfree(L.d_bdeg); dfree(L.d_flist); dfree(L.d_blist); dfree(L.d_counter);
   dfree(L.d_F); dfree(L.d_work); dfree(L.d_cg);
@@ -432,15 +459,9 @@ int gfx_plan_destroy(gfx_plan *p) {
   for (hipEvent_t e : p->join) (void)hipEventDestroy(e);
   if (p->fork) (void)hipEventDestroy(p->fork);
   dfree(p->d_coef[0]); dfree(p->d_coef[1]); dfree(p->d_coef[2]);
-  dfree(p->d_gref); dfree(p->d_qw); dfree(p->d_R);
-  dfree(p->d_rec); dfree(p->d_thr); dfree(p->d_keep); dfree(p->d_sig); dfree(p->d_Rp);
-  dfree(p->d_gref32); dfree(p->d_qw32); dfree(p->d_R32); dfree(p->d_rec32); dfree(p->d_Rq); dfree(p->d_E32);
-  dfree(p->d_E64);
-  dfree(p->d_inc_ptr); dfree(p->d_inc); dfree(p->d_slot); dfree(p->d_nslots); dfree(p->d_order); dfree(p->d_desc);
-  dfree(p->d_node_ok);
-  dfree(p->d_nbr); dfree(p->d_mask);
-  dfree(p->d_indptr); dfree(p->d_indices); dfree(p->d_vals); dfree(p->d_err);
-  dfree(p->d_t1d); dfree(p->d_pd); dfree(p->d_full); dfree(p->d_E); dfree(p->d_res); dfree(p->d_U); dfree(p->d_rhs); dfree(p->d_cg);
+  dfree(p->d_tab); dfree(p->d_elem); dfree(p->d_pat); dfree(p->d_order); dfree(p->d_desc); dfree(p->d_csr);
+  dfree(p->d_rec32); dfree(p->d_E32); dfree(p->d_E64); dfree(p->d_node_ok);
+  dfree(p->d_pd); dfree(p->d_full); dfree(p->d_E); dfree(p->d_cg);
   dfree(p->d_fixed); dfree(p->d_go);
   il_free(p->il);
   for (hipEvent_t e : p->ev) (void)hipEventDestroy(e);
@@ -563,48 +584,65 @@ int gfx_plan_create(gfx_mesh_fem *mf, gfx_mesh_im *mim, int term, const gfx_coef
       const double d[3] = {4.0 * x - 3.0, 4.0 - 8.0 * x, 4.0 * x - 1.0};
       for (int b = 0; b < 3; ++b) { t1d[3 * b + q] = v[b]; t1d[9 + 3 * b + q] = d[b]; }
     }
-  hipError_t e = dalloc(&p->d_gref, gref.size());
-  if (e == hipSuccess) e = dalloc(&p->d_qw, (size_t)nq);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_t1d, 18);
-  if (e == hipSuccess && eb) e = hipMemcpy(p->d_t1d, t1d, sizeof t1d, hipMemcpyHostToDevice);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_E, (size_t)m->n_cv * p->nloc * p->nloc);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_res, (size_t)m->n_cv * p->nloc);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_U, (size_t)p->ndof);
-  if (e == hipSuccess && eb) e = dalloc(&p->d_rhs, (size_t)p->ndof);
-  if (e == hipSuccess && eb) e = hipMemset(p->d_U, 0, 8 * (size_t)p->ndof);
-  if (e == hipSuccess) e = dalloc(&p->d_R, R.size());
-  if (e == hipSuccess) e = dalloc(&p->d_rec, (size_t)kRecStride * m->n_cv);
-  if (e == hipSuccess) e = dalloc(&p->d_thr, (size_t)m->n_cv);
-  if (e == hipSuccess) e = dalloc(&p->d_err, 4);
-  if (e == hipSuccess) e = hipMemcpy(p->d_gref, gref.data(), 8 * gref.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->d_qw, mim->rule.w.data(), 8 * (size_t)nq, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(p->d_R, R.data(), 8 * R.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(p->d_err, 0, 4);
-  if (!eb) {  // integer reference tensor, if R has one
-    std::vector<uint8_t> rq;
-    detect_int_reference(R, nd * nd, p->rk, p->r_L, rq);
-    if (p->rk && e == hipSuccess) e = dalloc(&p->d_Rq, rq.size());
-    if (p->rk && e == hipSuccess) e = hipMemcpy(p->d_Rq, rq.data(), rq.size(), hipMemcpyHostToDevice);
+  // the tables in one allocation, filled by one copy
+  std::vector<uint8_t> rq;
+  std::vector<double> Rp;
+  std::vector<float> gref32, R32, qw32;
+  if (!eb) {
+    detect_int_reference(R, nd * nd, p->rk, p->r_L, rq);  // integer reference tensor, if R has one
     // upper pairs for the threshold pass (the integers N where R has that form)
-    std::vector<double> Rp;
     for (int i = 0; i < nd; ++i)
       for (int j = i; j < nd; ++j)
         for (int t = 0; t < 9; ++t) {
           const double r = R[((size_t)i * nd + j) * 9 + t];
           Rp.push_back(p->rk ? std::nearbyint(r * p->r_L) : r);
         }
-    if (e == hipSuccess) e = dalloc(&p->d_Rp, Rp.size());
-    if (e == hipSuccess) e = hipMemcpy(p->d_Rp, Rp.data(), 8 * Rp.size(), hipMemcpyHostToDevice);
+    gref32.assign(gref.begin(), gref.end());  // FP32 copies for the FP32 contraction form
+    R32.assign(R.begin(), R.end());
+    qw32.assign(mim->rule.w.begin(), mim->rule.w.end());
   }
-  if (!eb) {  // FP32 copies of the tables for the FP32 contraction form
-    std::vector<float> gref32(gref.begin(), gref.end()), R32(R.begin(), R.end());
-    std::vector<float> qw32(mim->rule.w.begin(), mim->rule.w.end());
-    if (e == hipSuccess) e = dalloc(&p->d_gref32, gref32.size());
-    if (e == hipSuccess) e = dalloc(&p->d_qw32, qw32.size());
-    if (e == hipSuccess) e = dalloc(&p->d_R32, R32.size());
-    if (e == hipSuccess) e = hipMemcpy(p->d_gref32, gref32.data(), 4 * gref32.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_qw32, qw32.data(), 4 * qw32.size(), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_R32, R32.data(), 4 * R32.size(), hipMemcpyHostToDevice);
+  Carve tab, elem;
+  tab.add(&p->d_gref, gref.size());
+  tab.add(&p->d_qw, (size_t)nq);
+  tab.add(&p->d_R, R.size());
+  if (eb) tab.add(&p->d_t1d, 18);
+  if (p->rk) tab.add(&p->d_Rq, rq.size());
+  if (!eb) {
+    tab.add(&p->d_Rp, Rp.size());
+    tab.add(&p->d_gref32, gref32.size());
+    tab.add(&p->d_qw32, qw32.size());
+    tab.add(&p->d_R32, R32.size());
+  }
+  elem.add(&p->d_rec, eb ? 0 : (size_t)kRecStride * m->n_cv);
+  elem.add(&p->d_thr, (size_t)m->n_cv);
+  elem.add(&p->d_err, 4);
+  if (eb) {
+    elem.add(&p->d_res, (size_t)m->n_cv * p->nloc);
+    elem.add(&p->d_U, (size_t)p->ndof);
+    elem.add(&p->d_rhs, (size_t)p->ndof);
+  }
+  hipError_t e = tab.alloc(&p->d_tab);
+  if (e == hipSuccess) e = elem.alloc(&p->d_elem);
+  if (e == hipSuccess && eb) e = dalloc(&p->d_E, (size_t)m->n_cv * p->nloc * p->nloc);
+  if (e == hipSuccess && eb) e = hipMemset(p->d_U, 0, 8 * (size_t)p->ndof);
+  if (e == hipSuccess) e = hipMemset(p->d_err, 0, 4);
+  if (e == hipSuccess) {
+    std::vector<char> h(tab.bytes, 0);
+    auto put = [&](const void *d, const void *src, size_t n) {
+      std::memcpy(h.data() + ((const char *)d - p->d_tab), src, n);
+    };
+    put(p->d_gref, gref.data(), 8 * gref.size());
+    put(p->d_qw, mim->rule.w.data(), 8 * (size_t)nq);
+    put(p->d_R, R.data(), 8 * R.size());
+    if (eb) put(p->d_t1d, t1d, sizeof t1d);
+    if (p->rk) put(p->d_Rq, rq.data(), rq.size());
+    if (!eb) {
+      put(p->d_Rp, Rp.data(), 8 * Rp.size());
+      put(p->d_gref32, gref32.data(), 4 * gref32.size());
+      put(p->d_qw32, qw32.data(), 4 * qw32.size());
+      put(p->d_R32, R32.data(), 4 * R32.size());
+    }
+    e = hipMemcpy(p->d_tab, h.data(), h.size(), hipMemcpyHostToDevice);
   }
   if (e != hipSuccess) { gfx_plan_destroy(p); return hipfail(c, e, "gfx_plan_create"); }
   *out = p;
@@ -675,11 +713,9 @@ static int plan_records(gfx_plan *p) {
 // signature is compared with the stored one, not written.
 static int plan_keep(gfx_plan *p, bool check) {
   gfx_ctx *c = p->ctx;
-  const int64_t n_cv = p->mf->mesh->n_cv;
   RecordArgs a = record_args(p);
   int r;
   if ((r = records32(p, a))) return r;
-  if (!p->d_sig) HIPCHK(c, dalloc(&p->d_sig, (size_t)keep_sig_words(p->term, p->nd, p->qdim, n_cv)));
   HIPCHK(c, launch_keep(c->stream, p->term, p->nd, p->qdim, a, p->d_Rp, p->d_sig, check, p->d_thr, p->d_keep,
                         p->kwords));
   return GFX_OK;
@@ -898,21 +934,22 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   hipStream_t s = c->stream;
   int r;
   HIPCHK(c, hipMemsetAsync(p->d_err, 0, 4, s));
-  // incidences
-  dfree(p->d_inc_ptr); dfree(p->d_inc); dfree(p->d_slot); dfree(p->d_nslots); dfree(p->d_order); dfree(p->d_desc);
-  dfree(p->d_node_ok);
-  dfree(p->d_nbr); dfree(p->d_mask); dfree(p->d_indptr); dfree(p->d_indices); dfree(p->d_vals);
-  dfree(p->d_keep); dfree(p->d_sig);
+  dfree(p->d_pat); dfree(p->d_order); dfree(p->d_desc); dfree(p->d_csr); dfree(p->d_node_ok);
+  p->d_inc_ptr = nullptr; p->d_inc = nullptr; p->d_slot = nullptr; p->d_nslots = nullptr; p->d_mask = nullptr;
+  p->d_keep = nullptr; p->d_sig = nullptr; p->d_indptr = nullptr; p->d_indices = nullptr; p->d_vals = nullptr;
   p->keep_ok = false;
   p->nnz = -1;
   p->bins.clear();
   p->n_inc = n_cv * nd;
   if (p->n_inc >= INT32_MAX) return fail(c, GFX_E_INVALID, "too many element-node incidences");
   if (n_cv == 0 || nn == 0) {  // no element: an empty matrix (all rows empty)
-    HIPCHK(c, dalloc(&p->d_indptr, (size_t)p->ndof + 1));
+    Carve pat, csr;
+    pat.add(&p->d_indptr, (size_t)p->ndof + 1);
+    csr.add(&p->d_vals, 1);
+    csr.add(&p->d_indices, 1);
+    HIPCHK(c, pat.alloc(&p->d_pat));
+    HIPCHK(c, csr.alloc(&p->d_csr));
     HIPCHK(c, hipMemsetAsync(p->d_indptr, 0, 8 * ((size_t)p->ndof + 1), s));
-    HIPCHK(c, dalloc(&p->d_indices, 1));
-    HIPCHK(c, dalloc(&p->d_vals, 1));
     if (p->eb && p->ndof) HIPCHK(c, hipMemsetAsync(p->d_rhs, 0, 8 * (size_t)p->ndof, s));
     HIPCHK(c, hipStreamSynchronize(s));
     p->nnz = 0;
@@ -922,18 +959,32 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
     if (nnz_out) *nnz_out = 0;
     return GFX_OK;
   }
-  int32_t *tmp32 = nullptr;
-  HIPCHK(c, dalloc(&p->d_inc_ptr, (size_t)nn + 1));
-  HIPCHK(c, dalloc(&p->d_inc, (size_t)p->n_inc));
-  HIPCHK(c, dalloc(&tmp32, (size_t)(2 * nn + scan_tmp_elems(nn))));
-  hipError_t he = launch_incidences(s, n_cv, nd, Q, p->mf->d_dofs, nn, p->d_inc_ptr, p->d_inc, tmp32);
-  if (he != hipSuccess) { dfree(tmp32); return hipfail(c, he, "incidences"); }
+  // the patch kernel addresses presence words and slot pairs with 32-bit word offsets
+  if ((int64_t)p->n_inc * std::max(p->mwpi, nd / 2) >= (int64_t(1) << 32))
+    return fail(c, GFX_E_UNSUPPORTED, "mesh too large for one plan (presence/slot maps beyond 2^32 words)");
+  int32_t *tmp32, *nbr;
+  int64_t *rowcnt, *tmp64;
+  Carve pat;
+  pat.add(&p->d_inc_ptr, (size_t)nn + 1);
+  pat.add(&p->d_inc, (size_t)p->n_inc);
+  pat.add(&p->d_slot, (size_t)p->n_inc * nd);
+  pat.add(&p->d_nslots, (size_t)nn);
+  pat.add(&p->d_mask, (size_t)p->n_inc * p->mwpi);
+  pat.add(&p->d_keep, (size_t)n_cv * p->kwords);
+  if (!p->eb) pat.add(&p->d_sig, (size_t)keep_sig_words(p->term, nd, Q, n_cv));
+  pat.add(&p->d_indptr, (size_t)p->ndof + 1);
+  HIPCHK(c, pat.alloc(&p->d_pat));
+  Scratch scr;
+  scr.add(&tmp32, (size_t)(2 * nn + scan_tmp_elems(nn)));
+  scr.add(&nbr, (size_t)p->n_inc * nd);
+  scr.add(&rowcnt, (size_t)p->ndof);
+  scr.add(&tmp64, (size_t)scan_tmp_elems(p->ndof));
+  HIPCHK(c, scr.alloc());
+  HIPCHK(c, launch_incidences(s, n_cv, nd, Q, p->mf->d_dofs, nn, p->d_inc_ptr, p->d_inc, tmp32));
   // largest patch (LDS sort size) on the host
   std::vector<int32_t> iptr((size_t)nn + 1);
-  he = hipMemcpyAsync(iptr.data(), p->d_inc_ptr, 4 * ((size_t)nn + 1), hipMemcpyDeviceToHost, s);
-  if (he == hipSuccess) he = hipStreamSynchronize(s);
-  dfree(tmp32);
-  if (he != hipSuccess) return hipfail(c, he, "incidence copy");
+  HIPCHK(c, hipMemcpyAsync(iptr.data(), p->d_inc_ptr, 4 * ((size_t)nn + 1), hipMemcpyDeviceToHost, s));
+  HIPCHK(c, hipStreamSynchronize(s));
   int maxinc = 0;
   for (int64_t n = 0; n < nn; ++n) maxinc = std::max(maxinc, iptr[n + 1] - iptr[n]);
   p->max_cand = maxinc * nd;
@@ -941,7 +992,6 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   if (p->max_cand > 4096)
     return fail(c, GFX_E_PATTERN, "a node belongs to too many elements for the patch kernels");
   // thresholds and keep bits
-  HIPCHK(c, dalloc(&p->d_keep, (size_t)n_cv * p->kwords));
   PatternArgs a{};
   a.n_cv = n_cv; a.n_nodes = nn; a.nd = nd; a.qdim = Q; a.nloc = p->nloc;
   a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.keep = p->d_keep;
@@ -951,28 +1001,12 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   } else {
     if ((r = plan_keep(p, false))) return r;
   }
-  // patches (the patch kernel addresses presence words and slot pairs with
-  // 32-bit word offsets)
-  if ((int64_t)p->n_inc * std::max(p->mwpi, nd / 2) >= (int64_t(1) << 32))
-    return fail(c, GFX_E_UNSUPPORTED, "mesh too large for one plan (presence/slot maps beyond 2^32 words)");
-  HIPCHK(c, dalloc(&p->d_slot, (size_t)p->n_inc * nd));
-  HIPCHK(c, dalloc(&p->d_nslots, (size_t)nn));
-  HIPCHK(c, dalloc(&p->d_nbr, (size_t)p->n_inc * nd));
-  HIPCHK(c, dalloc(&p->d_mask, (size_t)p->n_inc * p->mwpi));
-  int64_t *rowcnt = nullptr, *tmp64 = nullptr;
-  HIPCHK(c, dalloc(&rowcnt, (size_t)p->ndof));
-  HIPCHK(c, dalloc(&p->d_indptr, (size_t)p->ndof + 1));
-  a.slot = p->d_slot; a.nslots = p->d_nslots; a.nbr = p->d_nbr; a.mask = p->d_mask;
+  a.slot = p->d_slot; a.nslots = p->d_nslots; a.nbr = nbr; a.mask = p->d_mask;
   a.rowcnt = rowcnt; a.indptr = p->d_indptr;
-  he = launch_patch_build(s, a, p->max_cand);
-  if (he == hipSuccess) he = dalloc(&tmp64, (size_t)scan_tmp_elems(p->ndof));
-  if (he == hipSuccess) he = scan_exclusive_i64(s, rowcnt, p->d_indptr, p->ndof, tmp64);
+  HIPCHK(c, launch_patch_build(s, a, p->max_cand));
+  HIPCHK(c, scan_exclusive_i64(s, rowcnt, p->d_indptr, p->ndof, tmp64));
   int64_t nnz = 0;
-  if (he == hipSuccess)
-    he = hipMemcpyAsync(&nnz, p->d_indptr + p->ndof, 8, hipMemcpyDeviceToHost, s);
-  if (he == hipSuccess) he = hipStreamSynchronize(s);
-  dfree(rowcnt); dfree(tmp64);
-  if (he != hipSuccess) return hipfail(c, he, "patch build");
+  HIPCHK(c, hipMemcpyAsync(&nnz, p->d_indptr + p->ndof, 8, hipMemcpyDeviceToHost, s));
   if ((r = check_err_flag(p))) return r;
   // nslots maximum for the assembly kernel's LDS
   std::vector<uint16_t> ns((size_t)nn);
@@ -986,12 +1020,13 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   dfree(p->d_desc);
   HIPCHK(c, dalloc(&p->d_desc, (size_t)p->n_order));
   HIPCHK(c, launch_fill_desc(s, p->n_order, Q, p->d_order, p->d_inc_ptr, p->d_nslots, p->d_indptr, p->d_desc));
-  HIPCHK(c, dalloc(&p->d_indices, (size_t)nnz));
-  HIPCHK(c, dalloc(&p->d_vals, (size_t)nnz));
+  Carve csr;
+  csr.add(&p->d_vals, (size_t)nnz);
+  csr.add(&p->d_indices, (size_t)nnz);
+  HIPCHK(c, csr.alloc(&p->d_csr));
   a.indices = p->d_indices;
   HIPCHK(c, launch_fill_columns(s, a));
   HIPCHK(c, hipStreamSynchronize(s));
-  dfree(p->d_nbr);
   // the keep bits stay: re-validation after a change of values compares
   // the pattern they give with this one
   p->nnz = nnz;
@@ -1044,7 +1079,6 @@ static int plan_validate(gfx_plan *p, bool *fresh) {
     }
   }
   p->keep_ok = false;  // until the new bits' pattern is confirmed or built
-  if (!p->d_keep) HIPCHK(c, dalloc(&p->d_keep, (size_t)m->n_cv * p->kwords));
   PatternArgs a{};
   a.n_cv = m->n_cv; a.n_nodes = p->n_nodes; a.nd = p->nd; a.qdim = p->qdim; a.nloc = p->nloc;
   a.kwords = p->kwords; a.mwpi = p->mwpi; a.dofs = p->mf->d_dofs; a.keep = p->d_keep;
@@ -1522,24 +1556,10 @@ int gfx_plan_export_csr(gfx_plan *p, int64_t *h_indptr, int32_t *h_indices, doub
 
 int gfx_plan_export_csc(gfx_plan *p, int64_t *h_colptr, uint32_t *h_rows, double *h_vals) {
   if (!p || !h_colptr) return GFX_E_INVALID;
-  const int64_t n = p->ndof, nnz = p->nnz;
-  if (nnz < 0) return fail(p->ctx, GFX_E_STATE, "build the pattern first");
-  std::vector<int64_t> ip((size_t)n + 1);
-  std::vector<int32_t> ix((size_t)nnz);
-  std::vector<double> v(h_vals ? (size_t)nnz : 0);
-  int r = gfx_plan_export_csr(p, ip.data(), ix.data(), h_vals ? v.data() : nullptr);
-  if (r) return r;
-  // transpose (counting sort by column keeps rows sorted)
-  std::vector<int64_t> cnt((size_t)n + 1, 0);
-  for (int64_t k = 0; k < nnz; ++k) cnt[ix[k] + 1]++;
-  for (int64_t j = 0; j < n; ++j) cnt[j + 1] += cnt[j];
-  std::copy(cnt.begin(), cnt.end(), h_colptr);
-  for (int64_t row = 0; row < n; ++row)
-    for (int64_t k = ip[row]; k < ip[row + 1]; ++k) {
-      const int64_t d = cnt[ix[k]]++;
-      if (h_rows) h_rows[d] = (uint32_t)row;
-      if (h_vals) h_vals[d] = v[k];
-    }
+  gfx_ctx *c = p->ctx;
+  if (p->nnz < 0) return fail(c, GFX_E_STATE, "build the pattern first");
+  if (set_device(c)) return GFX_E_HIP;
+  HIPCHK(c, export_csc(c->stream, p->ndof, p->nnz, p->d_indptr, p->d_indices, p->d_vals, h_colptr, h_rows, h_vals));
   return GFX_OK;
 }
 
@@ -1569,6 +1589,73 @@ int gfx_plan_last_timings(gfx_plan *p, float *ms_geometry, float *ms_assemble) {
 }
 
 }  // extern "C"
+
+namespace gfx {
+
+// On the host the transposition reads the matrix and scatters it entry by
+// entry through the caches on one core; beyond 2^31 entries, or without the
+// device memory for the sort, it is still done there.
+static hipError_t export_csc_host(hipStream_t s, int64_t n, int64_t nnz, const int64_t *ip, const int32_t *ix,
+                                  const double *v, int64_t *h_colptr, uint32_t *h_rows, double *h_vals) {
+  std::vector<int64_t> hp, cnt;
+  std::vector<int32_t> hx;
+  std::vector<double> hv;
+  try {
+    hp.resize((size_t)n + 1);
+    cnt.resize((size_t)n + 1);
+    hx.resize((size_t)nnz);
+    hv.resize(h_vals ? (size_t)nnz : 0);
+  } catch (const std::bad_alloc &) {
+    return hipErrorOutOfMemory;
+  }
+  hipError_t e = hipMemcpyAsync(hp.data(), ip, 8 * ((size_t)n + 1), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && nnz) e = hipMemcpyAsync(hx.data(), ix, 4 * (size_t)nnz, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && nnz && h_vals) e = hipMemcpyAsync(hv.data(), v, 8 * (size_t)nnz, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) return e;
+  // counting sort by column keeps the rows sorted
+  for (int64_t k = 0; k < nnz; ++k) cnt[hx[k] + 1]++;
+  for (int64_t j = 0; j < n; ++j) cnt[j + 1] += cnt[j];
+  std::copy(cnt.begin(), cnt.end(), h_colptr);
+  for (int64_t row = 0; row < n; ++row)
+    for (int64_t k = hp[row]; k < hp[row + 1]; ++k) {
+      const int64_t d = cnt[hx[k]]++;
+      if (h_rows) h_rows[d] = (uint32_t)row;
+      if (h_vals) h_vals[d] = hv[k];
+    }
+  return hipSuccess;
+}
+
+hipError_t export_csc(hipStream_t s, int64_t n, int64_t nnz, const int64_t *ip, const int32_t *ix, const double *v,
+                      int64_t *h_colptr, uint32_t *h_rows, double *h_vals) {
+  if (nnz <= 0 || nnz > INT32_MAX) return export_csc_host(s, n, nnz, ip, ix, v, h_colptr, h_rows, h_vals);
+  int bits = 1;
+  while (bits < 31 && (int64_t(1) << bits) < n) ++bits;
+  const size_t z = (size_t)nnz, sb = csc_sort_bytes(nnz, bits);
+  // one allocation: values, column pointers, rows, entry rows, positions, columns, sort storage
+  auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t b8 = up(8 * z), b4 = up(4 * z), bp = up(8 * ((size_t)n + 1));
+  char *d = nullptr;
+  if (hipMalloc((void **)&d, b8 + bp + 5 * b4 + up(sb)) != hipSuccess) {
+    (void)hipGetLastError();
+    return export_csc_host(s, n, nnz, ip, ix, v, h_colptr, h_rows, h_vals);
+  }
+  double *vals = (double *)d;
+  int64_t *cp = (int64_t *)(d + b8);
+  char *q = d + b8 + bp;
+  uint32_t *rows = (uint32_t *)q, *pos = (uint32_t *)(q + b4), *pos2 = (uint32_t *)(q + 2 * b4);
+  int32_t *row = (int32_t *)(q + 3 * b4), *col = (int32_t *)(q + 4 * b4);
+  hipError_t e = csr_to_csc(s, n, nnz, bits, ip, ix, v, q + 5 * b4, sb, row, pos, col, pos2, cp, rows,
+                            h_vals ? vals : nullptr);
+  if (e == hipSuccess) e = hipMemcpyAsync(h_colptr, cp, 8 * ((size_t)n + 1), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && h_rows) e = hipMemcpyAsync(h_rows, rows, 4 * z, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && h_vals) e = hipMemcpyAsync(h_vals, vals, 8 * z, hipMemcpyDeviceToHost, s);
+  const hipError_t w = hipStreamSynchronize(s);  // also where a copy failed: the buffer is freed next
+  (void)hipFree(d);
+  return e != hipSuccess ? e : w;
+}
+
+}  // namespace gfx
 
 // ----------------------------------------------------------- compliance
 extern "C" {

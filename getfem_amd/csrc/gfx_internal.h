@@ -379,6 +379,16 @@ hipError_t launch_dof_constraints(hipStream_t s, int64_t n, const int64_t *indpt
                                   double *rhs, int flags, int *err);
 size_t cg_workspace_doubles(int64_t n, int64_t nnz);
 // nslots (may be null; qb = 3): the nodes' slot counts with the bit of the full nodes
+// Transposition of a CSR matrix with sorted columns (0 < nnz < 2^31) into CSC
+// with sorted rows: a stable sort by column (bits: of the largest column; tmp:
+// csc_sort_bytes).  row, pos, col, pos2: nnz each; vals may be null.
+size_t csc_sort_bytes(int64_t nnz, int bits);
+hipError_t csr_to_csc(hipStream_t s, int64_t n, int64_t nnz, int bits, const int64_t *ip, const int32_t *ix,
+                      const double *v, void *tmp, size_t tmp_bytes, int32_t *row, uint32_t *pos, int32_t *col,
+                      uint32_t *pos2, int64_t *cp, uint32_t *rows, double *vals);
+// The same of a device matrix into host arrays (h_rows, h_vals may be null).
+hipError_t export_csc(hipStream_t s, int64_t n, int64_t nnz, const int64_t *ip, const int32_t *ix, const double *v,
+                      int64_t *h_colptr, uint32_t *h_rows, double *h_vals);
 size_t gmres_workspace_doubles(int64_t n, int m);
 struct IluData;
 hipError_t gmres_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
@@ -483,6 +493,10 @@ struct gfx_plan {
   bool values_changed = false;
   bool pinned = false;       // callers hold the CSR arrays: a rebuild is refused
   int64_t pattern_id = 0;    // incremented by every pattern (re)build
+  // allocations that hold several of the arrays below: tables; per-element and
+  // state arrays; what a pattern build makes before its size is known; the
+  // CSR's values and indices
+  char *d_tab = nullptr, *d_elem = nullptr, *d_pat = nullptr, *d_csr = nullptr;
   double *d_gref = nullptr, *d_qw = nullptr, *d_R = nullptr;
   double *d_rec = nullptr, *d_thr = nullptr;
   // FP32 contraction form: the tables and the element records in FP32
@@ -507,7 +521,6 @@ struct gfx_plan {
   uint32_t *d_inc = nullptr;
   uint16_t *d_slot = nullptr, *d_nslots = nullptr;
   uint8_t *d_node_ok = nullptr;   // pattern check scratch (n_nodes)
-  int32_t *d_nbr = nullptr;
   uint32_t *d_mask = nullptr;
   int max_nslots = 0, max_cand = 0, max_inc = 0;
   // element-batched plans: nodes grouped by patch size so each gather launch

@@ -14,6 +14,8 @@
 // does not depend on scheduling or on the batch.
 #include <hip/hip_runtime.h>
 
+#include <hipcub/hipcub.hpp>
+
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -143,6 +145,35 @@ __global__ void k_gather_i64(int64_t n, const int64_t *__restrict__ map, const i
                              int64_t *__restrict__ dst) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) dst[k] = src[map[k]];
+}
+
+// ---------------------------------------------- transposition (CSC export)
+// the entries' rows and positions, before their stable sort by column; a
+// group of 8 lanes per row
+__global__ void k_csc_entries(int64_t n, const int64_t *__restrict__ ip, int32_t *__restrict__ row,
+                              uint32_t *__restrict__ pos) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, r = t / 8;
+  if (r >= n) return;
+  const int64_t e = ip[r + 1];
+  for (int64_t k = ip[r] + t % 8; k < e; k += 8) {
+    row[k] = (int32_t)r;
+    pos[k] = (uint32_t)k;
+  }
+}
+
+// the sorted entries' rows and values, and the column pointers: an entry opens
+// the columns after the previous entry's up to its own
+__global__ void k_csc_fill(int64_t n, int64_t nnz, const int32_t *__restrict__ col, const uint32_t *__restrict__ pos,
+                           const int32_t *__restrict__ row, const double *__restrict__ v, int64_t *__restrict__ cp,
+                           uint32_t *__restrict__ rows, double *__restrict__ vals) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= nnz) return;
+  const uint32_t p = pos[k];
+  rows[k] = (uint32_t)row[p];
+  if (vals) vals[k] = v[p];
+  for (int64_t c = k ? (int64_t)col[k - 1] + 1 : 0; c <= col[k]; ++c) cp[c] = k;
+  if (k == nnz - 1)
+    for (int64_t c = (int64_t)col[k] + 1; c <= n; ++c) cp[c] = nnz;
 }
 
 __global__ void k_fill_f64(int64_t n, double *__restrict__ p, double v) {
@@ -612,6 +643,25 @@ hipError_t launch_gather_i64(hipStream_t s, int64_t n, const int64_t *map, const
 hipError_t launch_fill_f64(hipStream_t s, int64_t n, double *p, double v) {
   if (n == 0) return hipSuccess;
   k_fill_f64<<<nb256(n), 256, 0, s>>>(n, p, v);
+  return hipGetLastError();
+}
+
+size_t csc_sort_bytes(int64_t nnz, int bits) {
+  size_t bytes = 0;
+  if (hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (const int32_t *)nullptr, (int32_t *)nullptr,
+                                         (const uint32_t *)nullptr, (uint32_t *)nullptr, (int)nnz, 0, bits) !=
+      hipSuccess)
+    return 0;
+  return bytes;
+}
+
+hipError_t csr_to_csc(hipStream_t s, int64_t n, int64_t nnz, int bits, const int64_t *ip, const int32_t *ix,
+                      const double *v, void *tmp, size_t tmp_bytes, int32_t *row, uint32_t *pos, int32_t *col,
+                      uint32_t *pos2, int64_t *cp, uint32_t *rows, double *vals) {
+  k_csc_entries<<<nb256(8 * n), 256, 0, s>>>(n, ip, row, pos);
+  hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, ix, col, pos, pos2, (int)nnz, 0, bits, s);
+  if (e != hipSuccess) return e;
+  k_csc_fill<<<nb256(nnz), 256, 0, s>>>(n, nnz, col, pos2, row, v, cp, rows, vals);
   return hipGetLastError();
 }
 

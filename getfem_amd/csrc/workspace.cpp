@@ -1489,24 +1489,14 @@ int gfx_ws_export_csr(gfx_workspace *w, int64_t *h_indptr, int32_t *h_indices, d
 
 int gfx_ws_export_csc(gfx_workspace *w, int64_t *h_colptr, uint32_t *h_rows, double *h_vals) {
   int64_t n = 0, nnz = 0;
-  int r = gfx_ws_matrix_dims(w, &n, &nnz);
+  const int64_t *ip = nullptr;
+  const int32_t *ix = nullptr;
+  double *v = nullptr;
+  int r = gfx_ws_device_csr(w, &n, &nnz, &ip, &ix, &v);
   if (r) return r;
   if (!h_colptr) return GFX_E_INVALID;
-  std::vector<int64_t> ip((size_t)n + 1);
-  std::vector<int32_t> ix((size_t)nnz);
-  std::vector<double> v(h_vals ? (size_t)nnz : 0);
-  if ((r = gfx_ws_export_csr(w, ip.data(), ix.data(), h_vals ? v.data() : nullptr))) return r;
-  // transpose (counting sort by column keeps the rows sorted)
-  std::vector<int64_t> cnt((size_t)n + 1, 0);
-  for (int64_t k = 0; k < nnz; ++k) cnt[ix[k] + 1]++;
-  for (int64_t j = 0; j < n; ++j) cnt[j + 1] += cnt[j];
-  std::copy(cnt.begin(), cnt.end(), h_colptr);
-  for (int64_t row = 0; row < n; ++row)
-    for (int64_t k = ip[row]; k < ip[row + 1]; ++k) {
-      const int64_t d = cnt[ix[k]]++;
-      if (h_rows) h_rows[d] = (uint32_t)row;
-      if (h_vals) h_vals[d] = v[k];
-    }
+  if (hipSetDevice(w->ctx->device) != hipSuccess) return wfail(w, GFX_E_HIP, "hipSetDevice");
+  WHIP(w, export_csc(w->ctx->stream, n, nnz, ip, ix, v, h_colptr, h_rows, h_vals));
   return GFX_OK;
 }
 

@@ -161,9 +161,13 @@ class GaWorkspace:
         import scipy.sparse as sp
         n, z = self._dims()
         cp = np.zeros(n + 1, dtype=np.int64)
-        r = np.zeros(z, dtype=np.uint32)
-        v = np.zeros(z)
+        # rows as the int32 that scipy stores (they are below 2^31): it would
+        # look through uint32 ones and copy them
+        r = np.empty(z, dtype=np.int32)
+        v = np.empty(z)
         check(lib().gfx_ws_export_csc(self.h, _ptr(cp), _ptr(r), _ptr(v)), self.ctx.h)
+        if z <= np.iinfo(np.int32).max:
+            cp = cp.astype(np.int32)
         return sp.csc_matrix((v, r, cp), shape=(n, n))
 
     def __del__(self):
