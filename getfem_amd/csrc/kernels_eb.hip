@@ -34,7 +34,7 @@ constexpr int kNd = 27, kNl = 81, kNv = 8;
 // residual, A = dS/dE) in the spatial form (h = F^{-T} g): per node pair and
 // point, two outer products of spatial gradients and a dot product, as
 // products on the matrix cores in FP64 (FP64 form) or FP32 (FP32 form), upper
-// tiles only (nh_phase_b_mfma).
+// tiles only (nh_phase_b).
 constexpr int kNq = 27;
 constexpr int kKeepWords = (kNl * kNl + 31) / 32;  // keep-bit words per element (206)
 // k_nh_points' values per point, each kNq consecutive doubles of the element's
@@ -46,16 +46,22 @@ constexpr int kNhPd = 17;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
-// maximum over the workgroup's threads: shuffles within each wavefront, then
-// the wavefronts' maxima through LDS (one barrier instead of a tree)
-__device__ __forceinline__ double block_max(double v, double *red) {
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  const int t = threadIdx.x;
-  if ((t & 63) == 0) red[t >> 6] = v;
-  __syncthreads();
-  double m = red[0];
-  for (int w = 1; w < kEbThreads / 64; ++w) m = fmax(m, red[w]);
-  return m;
+// maximum over a wavefront in its lane 63: VALU lane moves, no trip through
+// the LDS (a lane without a source keeps its own value)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_max(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return fmax(v, __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo));
+}
+__device__ __forceinline__ double wave_max(double v) {
+  v = dpp_max<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row has the row's maximum
+  v = dpp_max<0x112, 0xf>(v);
+  v = dpp_max<0x114, 0xf>(v);
+  v = dpp_max<0x118, 0xf>(v);
+  v = dpp_max<0x142, 0xa>(v);     // row_bcast 15 into rows 1 and 3
+  return dpp_max<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
 }
 
 // Lane layout of the 16x16x4 matrix-core products (v_mfma_f64_16x16x4_f64,
@@ -82,28 +88,29 @@ struct BdbMfma<float> {
   static __device__ __forceinline__ int row(int g, int r) { return 4 * g + r; }
 };
 
-// Phase B in the spatial form (see k_nh_element) on the matrix cores, in T
+// Phase B in the spatial form (see k_nh_tangent) on the matrix cores, in T
 // (FP64: v_mfma_f64_16x16x4_f64; FP32: v_mfma_f32_16x16x4_f32, exact
 // products and FP32 sums).  With H_c[i][q] = h_qic (node i, point q), the
 // (a, b) component block of K over the node pairs is
 //   K_ab = H_a diag(alpha) H_b^T + H_b diag(beta) H_a^T + delta_ab K3,
-//   K3 = sum_c G_c M_c^T,  G_c[i][q] = g_qic,  M_c[j][q] = (gamma_q g_qj + pen_q C_q g_qj)_c,
+//   K3 = sum_c H_c M_c^T,  M_c[j][q] = (M_q h_qj)_c,
 // so both outer-product terms of a block go into one accumulator and no
-// value moves between lanes.  A tile is a 16 x 16 node tile (I, J) in
+// value moves between lanes; for a = b they are one product, with alpha + beta.  A tile is a 16 x 16 node tile (I, J) in
 // {0, 1}^2 (27 nodes and 5 zero pads) of one component pair (a, b); the k
-// axis is the 27 points and one zero (7 steps of 4).  hC ([q][c][32 nodes],
-// zero pads) holds h as the fragments read it: one LDS read per value.
+// axis is the 27 points and one zero (7 steps of 4).  hC (point q's row of
+// kNhRow values: [c][32 nodes], zero pads) holds h as the fragments read it:
+// one LDS read per value; the row's 16 spare values keep the four points of a
+// fragment in different banks.
 // K is symmetric: with P = 2 a + I and Q = 2 b + J only the 21 tiles P <= Q
 // are formed (the others are their transposes), and of K3 the node tiles
-// (0, 0), (0, 1), (1, 1).  Wavefront w < 3 forms K3 tile w and keeps it in
-// its accumulators beside the three tiles (a, a) of the same node tiles, to
-// which it is added, and two of the twelve tiles with a < b; wavefront 3
-// forms the other six (91, 91, 91, 84 products).  The tiles stay in the
-// accumulators until phase A's arrays and hC are free; then E is staged in
-// LDS over them (node rows 0-15, then 16-26), each tile written with its
-// transpose, and each staged run, contiguous in E, is streamed by the
-// workgroup.
-constexpr int kNhQ = 28, kNhN = 32;
+// (0, 0), (0, 1), (1, 1).  Wavefront w < 3 forms K3 tile w beside the three
+// tiles (a, a) of the same node tiles, to which it is added, from the same
+// fragments, and two of the twelve tiles with a < b; wavefront 3 forms the
+// other six (70, 70, 70, 84 products).  Each tile is stored from its
+// accumulators: 16-value runs of its own rows, 4-value runs of its
+// transpose's, which the L2 joins (plain stores: as non-temporal ones the
+// short runs took twice the time).
+constexpr int kNhQ = 28, kNhN = 32, kNhRow = 3 * kNhN + 16;
 
 // tile N (0..20): wavefront N / 5 (N < 15) takes N % 5 = 0..2 as the (a, a)
 // tiles of its K3 node tile and 3..4 as with-a<b tiles 2 (N / 5) + (N % 5 - 3);
@@ -130,8 +137,12 @@ static_assert(NhTile<0>::P == 0 && NhTile<0>::Q == 0 && NhTile<5>::P == 0 && NhT
 template <typename T, int N>
 __device__ __forceinline__ void nh_w_mma(typename BdbMfma<T>::v4 &acc, T al, T be, const T (&f)[3][2]) {
   typedef NhTile<N> D;
-  acc = BdbMfma<T>::mma(al * f[D::a][D::I], f[D::b][D::J], acc);
-  acc = BdbMfma<T>::mma(be * f[D::b][D::I], f[D::a][D::J], acc);
+  if constexpr (D::diag) {  // both terms are the same product
+    acc = BdbMfma<T>::mma((al + be) * f[D::a][D::I], f[D::a][D::J], acc);
+  } else {
+    acc = BdbMfma<T>::mma(al * f[D::a][D::I], f[D::b][D::J], acc);
+    acc = BdbMfma<T>::mma(be * f[D::b][D::I], f[D::a][D::J], acc);
+  }
 }
 template <typename T, int T0, int... U>
 __device__ __forceinline__ void nh_w_step(std::integer_sequence<int, U...>, typename BdbMfma<T>::v4 (&acc)[6], T al,
@@ -139,59 +150,86 @@ __device__ __forceinline__ void nh_w_step(std::integer_sequence<int, U...>, type
   (nh_w_mma<T, T0 + U>(acc[U], al, be, f), ...);
 }
 
-// the products of tiles T0 .. T0 + NT - 1 (accumulators acc[0 .. NT - 1])
+// the products of tiles T0 .. T0 + NT - 1 (accumulators acc[0 .. NT - 1]) and,
+// for the wavefronts that have diagonal tiles, of their K3 node tile:
+// K3[i][j] = sum_q h_qi^T M_q h_qj, k = (c, q): A = h_qic, B = (M_q h_qj)_c
 template <typename T, int T0, int NT>
-__device__ __forceinline__ void nh_w_tiles(int lr, int lg, const T (*hC)[3][kNhN], const T (&al)[kNhQ / 4],
-                                           const T (&be)[kNhQ / 4], typename BdbMfma<T>::v4 (&acc)[6]) {
+__device__ __forceinline__ void nh_w_tiles(int lr, int lg, const T *hC, const double *pd,
+                                           typename BdbMfma<T>::v4 (&acc)[6], typename BdbMfma<T>::v4 &k3) {
+  constexpr int w = T0 / 5, I3 = w / 2, J3 = (w + 1) / 2;
 #pragma unroll
   for (int u = 0; u < 6; ++u) acc[u] = typename BdbMfma<T>::v4{T(0), T(0), T(0), T(0)};
-#pragma unroll
+  k3 = typename BdbMfma<T>::v4{T(0), T(0), T(0), T(0)};
+#pragma unroll 1  // (in full it takes 104 registers, a wavefront less per SIMD, for nothing)
   for (int st = 0; st < kNhQ / 4; ++st) {
     T f[3][2];
+    const int q = 4 * st + lg;
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int I = 0; I < 2; ++I) f[c][I] = hC[4 * st + lg][c][16 * I + lr];
-    nh_w_step<T, T0>(std::make_integer_sequence<int, NT>{}, acc, al[st], be[st], f);
+      for (int I = 0; I < 2; ++I) f[c][I] = hC[q * kNhRow + c * kNhN + 16 * I + lr];
+    const double *pq = pd + min(q, kNq - 1);  // (hC is zero at q = 27)
+    const T al = (T)pq[9 * kNq], be = (T)pq[10 * kNq];
+    nh_w_step<T, T0>(std::make_integer_sequence<int, NT>{}, acc, al, be, f);
+    if constexpr (w < 3) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        // row c of the symmetric M: its entries (c, 0), (c, 1), (c, 2)
+        const T m = (T)pq[(11 + c) * kNq] * f[0][J3] + (T)pq[(11 + (c == 0 ? 1 : 2 + c)) * kNq] * f[1][J3] +
+                    (T)pq[(11 + (c == 0 ? 2 : 3 + c)) * kNq] * f[2][J3];
+        k3 = BdbMfma<T>::mma(f[c][I3], m, k3);
+      }
+    }
   }
 }
 
-// tile N's entries in node rows [n0, n1) of E into the stage (E's
-// node-blocked layout, entry ((3 (i - n0) + a) 3 + b) 27 + j for K[(i,a),(j,b)]),
-// K3 added to (a, a) tiles, the transpose written for P < Q.  Branch-free:
-// a lane whose entry is outside the slab (or a zero pad) writes its own slot
-// of the trash row behind the stage instead.
+// tile N's entries into E (node-blocked: entry ((3 i + a) 3 + b) 27 + j for
+// K[(i,a),(j,b)]), K3 added to (a, a) tiles, the transpose written for P < Q
 template <typename T, int N>
-__device__ __forceinline__ void nh_w_store1(int lr, int lg, int n0, int n1, int trash,
-                                            const typename BdbMfma<T>::v4 &acc,
-                                            const typename BdbMfma<T>::v4 &k3, T *stage) {
+__device__ __forceinline__ void nh_w_store1(int lr, int lg, const typename BdbMfma<T>::v4 &acc,
+                                            const typename BdbMfma<T>::v4 &k3, T *E) {
   typedef NhTile<N> D;
   const int j = 16 * D::J + lr;
-  const bool jv = j < kNd, jin = jv && j >= n0 && j < n1;
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const int i = 16 * D::I + BdbMfma<T>::row(lg, x);
-    const bool iv = i < kNd, iin = iv && i >= n0 && i < n1;
     const T v = D::diag ? acc[x] + k3[x] : acc[x];
-    stage[iin && jv ? ((3 * (i - n0) + D::a) * 3 + D::b) * kNd + j : trash] = v;
-    if (D::P != D::Q) stage[jin && iv ? ((3 * (j - n0) + D::b) * 3 + D::a) * kNd + i : trash] = v;
+    if (i < kNd && j < kNd) {
+      E[((3 * i + D::a) * 3 + D::b) * kNd + j] = v;
+      if (D::P != D::Q) E[((3 * j + D::b) * 3 + D::a) * kNd + i] = v;
+    }
+  }
+}
+// the keep bits (row-major over (3 i + a, 3 j + b)) of the same entries
+template <typename T, int N>
+__device__ __forceinline__ void nh_w_bits1(int lr, int lg, double th, const typename BdbMfma<T>::v4 &acc,
+                                           const typename BdbMfma<T>::v4 &k3, uint32_t *skeep) {
+  typedef NhTile<N> D;
+  const int j = 16 * D::J + lr;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int i = 16 * D::I + BdbMfma<T>::row(lg, x);
+    const T v = D::diag ? acc[x] + k3[x] : acc[x];
+    if (i < kNd && j < kNd && (double)fabs(v) > th) {
+      const int d = (3 * i + D::a) * kNl + 3 * j + D::b, m = (3 * j + D::b) * kNl + 3 * i + D::a;
+      atomicOr(&skeep[d >> 5], 1u << (d & 31));
+      if (D::P != D::Q) atomicOr(&skeep[m >> 5], 1u << (m & 31));
+    }
   }
 }
 template <typename T, int T0, int... U>
-__device__ __forceinline__ void nh_w_store_seq(std::integer_sequence<int, U...>, int lr, int lg, int n0, int n1,
-                                               int trash, const typename BdbMfma<T>::v4 (&acc)[6],
-                                               const typename BdbMfma<T>::v4 &k3, T *stage) {
-  (nh_w_store1<T, T0 + U>(lr, lg, n0, n1, trash, acc[U], k3, stage), ...);
-}
-template <typename T, int T0, int NT>
-__device__ __forceinline__ void nh_w_store(int lr, int lg, int n0, int n1, int trash,
+__device__ __forceinline__ void nh_w_store(std::integer_sequence<int, U...>, int lr, int lg,
                                            const typename BdbMfma<T>::v4 (&acc)[6],
-                                           const typename BdbMfma<T>::v4 &k3, T *stage) {
-  nh_w_store_seq<T, T0>(std::make_integer_sequence<int, NT>{}, lr, lg, n0, n1, trash, acc, k3, stage);
+                                           const typename BdbMfma<T>::v4 &k3, T *E) {
+  (nh_w_store1<T, T0 + U>(lr, lg, acc[U], k3, E), ...);
+}
+template <typename T, int T0, int... U>
+__device__ __forceinline__ void nh_w_bits(std::integer_sequence<int, U...>, int lr, int lg, double th,
+                                          const typename BdbMfma<T>::v4 (&acc)[6],
+                                          const typename BdbMfma<T>::v4 &k3, uint32_t *skeep) {
+  (nh_w_bits1<T, T0 + U>(lr, lg, th, acc[U], k3, skeep), ...);
 }
 
-// the stage aliases phase A's arrays and hC: written only after the
-// workgroup barrier that follows the last read of them
 // this lane's largest |entry| of tiles T0 .. T0 + NT - 1 (K3 added to the
 // (a, a) tiles; the zero pads add nothing)
 template <typename T, int N>
@@ -215,150 +253,84 @@ __device__ __forceinline__ double nh_w_max(const typename BdbMfma<T>::v4 (&acc)[
   return nh_w_max_seq<T, T0>(std::make_integer_sequence<int, NT>{}, acc, k3);
 }
 
-// whether every entry of tiles T0 .. T0 + NT - 1 is above th (zero pads aside)
+// this lane's smallest |entry| of tiles T0 .. T0 + NT - 1 (zero pads aside), 0
+// where one is not a number: every entry is kept where it is above the threshold
 template <typename T, int N>
-__device__ __forceinline__ bool nh_w_all1(int lr, int lg, double th, const typename BdbMfma<T>::v4 &acc,
-                                          const typename BdbMfma<T>::v4 &k3) {
+__device__ __forceinline__ double nh_w_min1(int lr, int lg, const typename BdbMfma<T>::v4 &acc,
+                                            const typename BdbMfma<T>::v4 &k3) {
   typedef NhTile<N> D;
-  bool ok = true;
+  double m = INFINITY;
+  bool nan = false;
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const bool in = 16 * D::I + BdbMfma<T>::row(lg, x) < kNd && 16 * D::J + lr < kNd;
-    ok &= !in || (double)fabs(D::diag ? acc[x] + k3[x] : acc[x]) > th;
+    const double v = (double)fabs(D::diag ? acc[x] + k3[x] : acc[x]);
+    m = fmin(m, in ? v : INFINITY);
+    nan |= v != v;
   }
-  return ok;
+  return nan ? 0.0 : m;
 }
 template <typename T, int T0, int... U>
-__device__ __forceinline__ bool nh_w_all_seq(std::integer_sequence<int, U...>, int lr, int lg, double th,
-                                             const typename BdbMfma<T>::v4 (&acc)[6],
-                                             const typename BdbMfma<T>::v4 &k3) {
-  return (nh_w_all1<T, T0 + U>(lr, lg, th, acc[U], k3) & ...);
+__device__ __forceinline__ double nh_w_min_seq(std::integer_sequence<int, U...>, int lr, int lg,
+                                               const typename BdbMfma<T>::v4 (&acc)[6],
+                                               const typename BdbMfma<T>::v4 &k3) {
+  double m = INFINITY;
+  ((m = fmin(m, nh_w_min1<T, T0 + U>(lr, lg, acc[U], k3))), ...);
+  return m;
 }
 template <typename T, int T0, int NT>
-__device__ __forceinline__ bool nh_w_all(int lr, int lg, double th, const typename BdbMfma<T>::v4 (&acc)[6],
-                                         const typename BdbMfma<T>::v4 &k3) {
-  return nh_w_all_seq<T, T0>(std::make_integer_sequence<int, NT>{}, lr, lg, th, acc, k3);
+__device__ __forceinline__ double nh_w_min(int lr, int lg, const typename BdbMfma<T>::v4 (&acc)[6],
+                                           const typename BdbMfma<T>::v4 &k3) {
+  return nh_w_min_seq<T, T0>(std::make_integer_sequence<int, NT>{}, lr, lg, acc, k3);
 }
 
-// KEEP: 0 no keep bits; 1 they are compared with the stored ones (bit 32 of
-// the error flag when any differs); 2 they are written
-template <typename T, int KEEP>
-__device__ __forceinline__ void nh_phase_b_mfma(int t, int64_t e, const double *pd, const T (*hC)[3][kNhN], T *stage,
-                                                uint32_t *skeep, double *red, const EbArgs &a) {
+// One wavefront's part, tiles T0 .. T0 + NT - 1.  KEEP: 0 no keep bits; 1 they
+// are compared with the stored ones (bit 32 of the error flag when any
+// differs); 2 they are written.
+template <typename T, int KEEP, int T0, int NT>
+__device__ __forceinline__ void nh_phase_b(int t, int64_t e, const double *pd, const T *hC, uint32_t *skeep,
+                                           double *red, int was_full, const EbArgs &a) {
   typedef typename BdbMfma<T>::v4 v4;
-  // the wavefront index as a scalar: the branches on it are uniform
-  const int w = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64, lr = l % 16, lg = l / 16;
-  // K3 node tile (w / 2, (w + 1) / 2) for wavefronts 0-2, in the spatial
-  // gradients: K3[i][j] = sum_q h_qi^T M_q h_qj, k = (c, q): A = h_qic,
-  // B = (M_q h_qj)_c (zero pads in hC make the pads' products zero)
-  v4 k3 = v4{T(0), T(0), T(0), T(0)};
-  if (w < 3) {
-    const int i = 16 * (w / 2) + lr, j = 16 * ((w + 1) / 2) + lr;
-#pragma unroll
-    for (int st = 0; st < kNhQ / 4; ++st) {
-      const int q = 4 * st + lg;
-      const double *M = pd + 11 * kNq + min(q, kNq - 1);
-      const T h0 = hC[q][0][j], h1 = hC[q][1][j], h2 = hC[q][2][j];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        // row c of the symmetric M: its entries (c, 0), (c, 1), (c, 2)
-        const T m = (T)M[c * kNq] * h0 + (T)M[(c == 0 ? 1 : 2 + c) * kNq] * h1 + (T)M[(c == 0 ? 2 : 3 + c) * kNq] * h2;
-        k3 = BdbMfma<T>::mma(hC[q][c][i], m, k3);
-      }
-    }
+  constexpr int w = T0 / 5, kWaves = kEbThreads / 64;
+  constexpr auto tiles = std::make_integer_sequence<int, NT>{};
+  const int l = t % 64, lr = l % 16, lg = l / 16;
+  v4 acc[6], k3;
+  nh_w_tiles<T, T0, NT>(lr, lg, hC, pd, acc, k3);
+  // threshold 1e-14 max|K| (all-zero element skipped), from the accumulators,
+  // and (negated) the smallest |entry|, one barrier for both
+  const double mx = wave_max(nh_w_max<T, T0, NT>(acc, k3));
+  double mn = 0.0;
+  if constexpr (KEEP != 0) mn = wave_max(-nh_w_min<T, T0, NT>(lr, lg, acc, k3));
+  if (l == 63) {
+    red[w] = mx;
+    if (KEEP != 0) red[kWaves + w] = mn;
   }
-  // this lane's alpha_q and beta_q at q = 4 st + lg (hC is zero at q = 27)
-  T al[kNhQ / 4], be[kNhQ / 4];
-#pragma unroll
-  for (int st = 0; st < kNhQ / 4; ++st) {
-    const int qc = min(4 * st + lg, kNq - 1);
-    al[st] = (T)pd[9 * kNq + qc];
-    be[st] = (T)pd[10 * kNq + qc];
-  }
-  v4 acc[6];
-  if (w == 0) nh_w_tiles<T, 0, 5>(lr, lg, hC, al, be, acc);
-  else if (w == 1) nh_w_tiles<T, 5, 5>(lr, lg, hC, al, be, acc);
-  else if (w == 2) nh_w_tiles<T, 10, 5>(lr, lg, hC, al, be, acc);
-  else nh_w_tiles<T, 15, 6>(lr, lg, hC, al, be, acc);
-  // threshold 1e-14 max|K| (all-zero element skipped), from the accumulators
-  double mx = 0.0;
-  if (w == 0) mx = nh_w_max<T, 0, 5>(acc, k3);
-  else if (w == 1) mx = nh_w_max<T, 5, 5>(acc, k3);
-  else if (w == 2) mx = nh_w_max<T, 10, 5>(acc, k3);
-  else mx = nh_w_max<T, 15, 6>(acc, k3);
-  const double mxe = block_max(mx, red);
+  if (KEEP != 0)  // (where they are needed; before the barrier that their use is behind)
+    for (int x = t; x < kKeepWords; x += kEbThreads) skeep[x] = 0u;
+  __syncthreads();
+  double mxe = red[0];
+  for (int v = 1; v < kWaves; ++v) mxe = fmax(mxe, red[v]);
   const double th = mxe > 0.0 ? 1e-14 * mxe : INFINITY;
   if (t == 0) a.thr[e] = th;
-  // An element that keeps every entry (nearly all do) has words of ones: they
-  // are not formed.  full[e] says that of the stored words.
-  bool words = false;
+  nh_w_store<T, T0>(tiles, lr, lg, acc, k3, reinterpret_cast<T *>(a.E) + e * kNl * kNl);
   if constexpr (KEEP != 0) {
-    bool all;
-    if (w == 0) all = nh_w_all<T, 0, 5>(lr, lg, th, acc, k3);
-    else if (w == 1) all = nh_w_all<T, 5, 5>(lr, lg, th, acc, k3);
-    else if (w == 2) all = nh_w_all<T, 10, 5>(lr, lg, th, acc, k3);
-    else all = nh_w_all<T, 15, 6>(lr, lg, th, acc, k3);
-    words = !__syncthreads_and(all);
-    if (KEEP == 1 && t == 0 && a.full[e] != (words ? 0 : 1)) atomicOr(a.err, 32);
-    if (KEEP == 2) {
-      if (t == 0) a.full[e] = words ? 0 : 1;
-      if (!words)
-        for (int x = t; x < kKeepWords; x += kEbThreads)
-          a.keep[e * kKeepWords + x] = x == kKeepWords - 1 ? (1u << (kNl * kNl % 32)) - 1u : 0xffffffffu;
+    // An element that keeps every entry (nearly all do) has words of ones: they
+    // are not formed.  full[e] says that of the stored words.
+    double mne = red[kWaves];
+    for (int v = 1; v < kWaves; ++v) mne = fmax(mne, red[kWaves + v]);
+    const bool full = -mne > th;  // (uniform)
+    if (KEEP == 1 && t == 0 && was_full != (full ? 1 : 0)) atomicOr(a.err, 32);
+    if (KEEP == 2 && t == 0) a.full[e] = full ? 1 : 0;
+    if (KEEP == 1 && full) return;
+    if (!full) {
+      nh_w_bits<T, T0>(tiles, lr, lg, th, acc, k3, skeep);
+      __syncthreads();
     }
-    if (words)
-      for (int x = t; x < kKeepWords; x += kEbThreads) skeep[x] = 0u;
-  }
-  T *E = reinterpret_cast<T *>(a.E) + e * kNl * kNl;
-  // two stages: node rows 0-15, then 16-26; the trash row (a slot per lane)
-  // behind the larger one.  (FP32 would fit one stage of all 27 node rows;
-  // that variant gave wrong values with this compiler at -O3, with a fill of
-  // the stage before the tile stores or at -O1 it did not, and the cause was
-  // not found: both precisions use the two stages, which are checked.)
-  constexpr int kSlabs = 2;
-  const int trash = 3 * 16 * kNl + l;
-#pragma unroll
-  for (int sl = 0; sl < kSlabs; ++sl) {
-    const int n0 = 16 * sl, n1 = sl == 1 ? kNd : 16;
-    __syncthreads();  // the last reads of what the stage overlays (or of the previous slab) are done
-    if (w == 0) nh_w_store<T, 0, 5>(lr, lg, n0, n1, trash, acc, k3, stage);
-    else if (w == 1) nh_w_store<T, 5, 5>(lr, lg, n0, n1, trash, acc, k3, stage);
-    else if (w == 2) nh_w_store<T, 10, 5>(lr, lg, n0, n1, trash, acc, k3, stage);
-    else nh_w_store<T, 15, 6>(lr, lg, n0, n1, trash, acc, k3, stage);
-    __syncthreads();
-    const int len = 3 * (n1 - n0) * kNl;
-    T *dst = E + 3 * n0 * kNl;
-    for (int x = t; x < len; x += kEbThreads) __builtin_nontemporal_store(stage[x], dst + x);
-    if (KEEP != 0 && words) {
-      // keep bits, row-major (r, c) = (3 i + a, 3 j + b): one thread per
-      // 32-bit word of this slab's rows reads its entries from the stage
-      // (staged at ((3 i + a) 3 + b) 27 + j); the word shared with the other
-      // slab gets its two halves from the same thread, a barrier apart
-      const int b0 = 3 * n0 * kNl, b1 = 3 * n1 * kNl;
-      const int w0 = b0 >> 5, w1 = (b1 + 31) >> 5;
-      // two lanes per word (16 bits each, lanes 2m and 2m + 1: both in the
-      // loop, since the bound is even), combined by a lane exchange
-      for (int id = t; id < 2 * (w1 - w0); id += kEbThreads) {
-        const int wd = w0 + (id >> 1), k0 = 16 * (id & 1);
-        uint32_t bits = 0u;
-        for (int k = k0; k < k0 + 16; ++k) {
-          const int bit = 32 * wd + k;
-          if (bit < b0 || bit >= b1) continue;
-          const int r = bit / kNl, c = bit - r * kNl, j = c / 3;
-          const int x = (3 * r + (c - 3 * j)) * kNd + j - b0;  // the slab starts at entry b0
-          if (fabs((double)stage[x]) > th) bits |= 1u << k;
-        }
-        bits |= __shfl_xor(bits, 1);
-        if ((id & 1) == 0) skeep[wd] |= bits;
-      }
-    }
-  }
-  if (KEEP != 0 && words) {
-    __syncthreads();
     bool same = true;
     for (int x = t; x < kKeepWords; x += kEbThreads) {
-      if constexpr (KEEP == 2) a.keep[e * kKeepWords + x] = skeep[x];
-      else same &= a.keep[e * kKeepWords + x] == skeep[x];
+      const uint32_t bits = !full ? skeep[x] : (x == kKeepWords - 1 ? (1u << (kNl * kNl % 32)) - 1u : 0xffffffffu);
+      if constexpr (KEEP == 2) a.keep[e * kKeepWords + x] = bits;
+      else same &= a.keep[e * kKeepWords + x] == bits;
     }
     if (!same) atomicOr(a.err, 32);
   }
@@ -615,48 +587,69 @@ __global__ __launch_bounds__(kEbThreads) void k_nh_points(EbArgs a) {
 // (pen_q = 1e200 where det F <= 0: the derivative of the penalty term 1e200 C
 // that the law adds to S there).  Same matrix as the material form
 // D[(a,c),(b,n)] = wJ (delta_ab S_nc + F_ak A_kcmn F_bm) up to roundoff,
-// without forming D or D g (nh_phase_b_mfma).  h = A grad(phi) from the points'
+// without forming D or D g (nh_phase_b).  h = A grad(phi) from the points'
 // values, which k_nh_points leaves in memory (3.7 KB an element): its serial
 // phases (27 of 256 threads at work) used to take as long here as the products.
-// Measured at 48^3 = 110,592 elements with the keep check: 2.66 ms (with those
-// phases inside and the keep words always formed 3.21 ms).
-template <typename T>
-union NhLds {
-  struct {
-    double pd[kNhPd * kNq];
-    T hC[kNhQ][3][kNhN];  // the spatial gradients in the fragments' layout
-  } P;
-  T stage[3 * 16 * kNl + 64];  // the slab and the trash row, over what phase B has read
-};
-
+// Bound by no single unit: the matrix cores are 49 % busy, the VALU 24 %, the
+// stores of E (5.8 GB) run at 3 TB/s; a workgroup is 2 us at the points' values
+// and gradients (issued together, before anything waits), 4 us at the products
+// and 4 us at the maximum and the stores, five workgroups a CU taking turns.
+// Measured at 48^3 = 110,592 elements with the keep check: 1.93 ms.  2.64 ms
+// with the gradients loaded after the points' values, a barrier each for the
+// maximum and for the keep check, K3 in a pass of its own, two products for
+// a = b and E staged in the LDS (four more barriers); 3.21 ms with the serial
+// phases inside and the keep words always formed.  Workgroups that stay for
+// many elements and fetch the next one's values ahead took 2.2 ms.
 template <typename Real, int KEEP>
-__global__ __launch_bounds__(kEbThreads, 4) void k_nh_tangent(EbArgs a) {
-  __shared__ NhLds<Real> L;
-  __shared__ double red[kEbThreads / 64];
+__global__ __launch_bounds__(kEbThreads, 5) void k_nh_tangent(EbArgs a) {
+  __shared__ double pd[kNhPd * kNq];
+  __shared__ Real hC[kNhQ * kNhRow];  // the spatial gradients in the fragments' layout
+  __shared__ double red[2 * (kEbThreads / 64)];
   __shared__ uint32_t skeep[KEEP ? kKeepWords : 1];  // the element's keep bits, where not all are set
   const int64_t e = blockIdx.x;
   const int t = threadIdx.x;
-  double *pd = L.P.pd;
-  Real(&hC)[kNhQ][3][kNhN] = L.P.hC;
   const double *src = a.pd + e * (kNhPd * kNq);
-  for (int x = t; x < kNhPd * kNq; x += kEbThreads) pd[x] = src[x];
+  constexpr int kPd = (kNhPd * kNq + kEbThreads - 1) / kEbThreads;
+  double pv[kPd];
+#pragma unroll
+  for (int r = 0; r < kPd; ++r) pv[r] = src[min(t + r * kEbThreads, kNhPd * kNq - 1)];
+  const int was_full = KEEP == 1 && t == 0 ? a.full[e] : 0;
+  // hC[q][c][i] = h_qic in Real (zero for q = 27 and nodes i >= 27): thread
+  // (i, q mod 8) takes every eighth point; its gradients are on the way while
+  // the points' values are
+  static_assert(kNhN * 8 == kEbThreads, "a thread per (node, point mod 8)");
+  constexpr int kHq = (kNhQ + 7) / 8;
+  const int i = t % kNhN, q0 = t / kNhN;
+  double g[kHq][3];
+#pragma unroll
+  for (int r = 0; r < kHq; ++r) {
+    const double *gp = a.gref + (min(q0 + 8 * r, kNq - 1) * kNd + min(i, kNd - 1)) * 3;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) g[r][c] = gp[c];
+  }
+#pragma unroll
+  for (int r = 0; r < kPd; ++r)
+    if (t + r * kEbThreads < kNhPd * kNq) pd[t + r * kEbThreads] = pv[r];
   __syncthreads();
-  // hC[q][c][i] = h_qic in Real (zero for q = 27 and nodes i >= 27)
-  for (int x = t; x < kNhQ * kNhN; x += kEbThreads) {
-    const int q = x / kNhN, i = x % kNhN;
-    Real h[3] = {Real(0), Real(0), Real(0)};
-    if (q < kNq && i < kNd) {
-      const double *g = a.gref + (q * kNd + i) * 3;
-      const double g0 = g[0], g1 = g[1], g2 = g[2];
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        h[c] = (Real)(pd[3 * c * kNq + q] * g0 + pd[(3 * c + 1) * kNq + q] * g1 + pd[(3 * c + 2) * kNq + q] * g2);
+  for (int r = 0; r < kHq; ++r) {
+    const int q = q0 + 8 * r, qc = min(q, kNq - 1);
+    const bool in = q < kNq && i < kNd;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const double h = pd[3 * c * kNq + qc] * g[r][0] + pd[(3 * c + 1) * kNq + qc] * g[r][1] +
+                       pd[(3 * c + 2) * kNq + qc] * g[r][2];
+      if (q < kNhQ) hC[q * kNhRow + c * kNhN + i] = in ? (Real)h : Real(0);
     }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) hC[q][c][i] = h[c];
   }
   __syncthreads();
-  nh_phase_b_mfma<Real, KEEP>(t, e, pd, hC, L.stage, skeep, red, a);
+  // the wavefront index as a scalar: the branches on it are uniform (each
+  // branch meets the same barriers)
+  const int w = __builtin_amdgcn_readfirstlane(t / 64);
+  if (w == 0) nh_phase_b<Real, KEEP, 0, 5>(t, e, pd, hC, skeep, red, was_full, a);
+  else if (w == 1) nh_phase_b<Real, KEEP, 5, 5>(t, e, pd, hC, skeep, red, was_full, a);
+  else if (w == 2) nh_phase_b<Real, KEEP, 10, 5>(t, e, pd, hC, skeep, red, was_full, a);
+  else nh_phase_b<Real, KEEP, 15, 6>(t, e, pd, hC, skeep, red, was_full, a);
 }
 
 // node-patch gather of the rows of buffered element matrices: the Q rows of
