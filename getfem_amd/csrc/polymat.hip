@@ -13,6 +13,8 @@
 //              element's threshold 1e-14 max|elem| (a zero element adds
 //              nothing): entries at or below it are written as 0, so that
 //              what is stored and not zero is what add_elem_matrix inserts.
+// k_poly_ref   the same for affine elements and outputs without fem fields,
+//              through the reference tensor.
 // The matrix.  Which entries of which elements meet in a matrix entry depends
 // on the dof tables alone, so it is worked out once per set of expressions
 // (poly_structure): every candidate (block, element, entry) sorted by (row,
@@ -25,6 +27,8 @@
 // Beyond 2^31 candidates the kept entries are sorted at every assembly instead
 // (k_poly_emit, poly_to_csr).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include <hipcub/hipcub.hpp>
 
@@ -218,6 +222,146 @@ __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
         }
 }
 
+// Affine elements whose outputs read no fem field: the point sum goes through
+// the reference tensor of a pair of base functions,
+//   E[(i, a), (j, b)] = |J| sum_{p, r} O[(a, p), (b, r)] (B' R_ij B'^T)_{p r},
+//   R_ij[p][r] = sum_q w_q phi_i^p psi_j^r  (p, r: value, reference gradient),
+// B' = 1 for the value and B for the gradient: 54 + 81 products a pair of vector
+// base functions instead of 45 and a share of U at each of the points.
+// A lane keeps its pair (i, j), and with it R_ij in registers, for all the
+// elements that its workgroup passes over, `epb` side by side; a chunk's
+// geometry is formed first, a lane an element.  Bound by FP64 issue and the
+// latency of the start (R is formed by every workgroup: the points' base
+// functions are read from the L2).
+// Measured, u P2 vector + p P1 on 15^3 x 6 = 20,250 elements: the four blocks
+// 0.154 ms (67 us for the 30 x 30 one), through the points (k_poly_mat) 0.59 ms.
+constexpr int kPrIters = 8;      // passes of a workgroup where the elements are enough to fill the card
+constexpr int kPrMaxChunk = 512; // elements of a workgroup
+
+template <int QT, int QS>
+__global__ __launch_bounds__(512) void k_poly_ref(PolyMatArgs a, int epb, int iters) {
+  extern __shared__ double lds_pr[];
+  const ScalarField &ft = a.f[a.vt], &fs = a.f[a.vs];
+  const int ndt = ft.nd, nds = fs.nd, pairs = ndt * nds, nc = nds * QS, ne = ndt * QT * nc, chunk = epb * iters;
+  constexpr int w4 = 4 * QS;
+  double *T = lds_pr;                                            // symbols
+  double *O = T + a.nsym;                                        // outputs
+  double *geo = O + a.nout;                                      // [element][10]: B, |J|
+  unsigned long long *smax = reinterpret_cast<unsigned long long *>(geo + 10 * chunk);  // max |entry|, as its bits
+  const int t = threadIdx.x, lane = t & 63;
+  const int64_t e0 = (int64_t)blockIdx.x * chunk;
+  for (int c = t; c < a.nconst; c += blockDim.x) T[a.const_off + c] = a.consts[c];
+  for (int x = t; x < chunk; x += blockDim.x) {
+    double B[9], aJ;
+    smax[x] = 0;
+    if (e0 + x < a.n_cv) {
+      if (!poly_geometry(a.pts, a.cvx + (int64_t)a.nv * (e0 + x), a.nv, nullptr, B, aJ)) {  // its entries are 0
+        atomicOr(a.err, 1);
+        aJ = 0.0;
+        for (int c = 0; c < 9; ++c) B[c] = 0.0;
+      }
+      for (int c = 0; c < 9; ++c) geo[10 * x + c] = B[c];
+      geo[10 * x + 9] = aJ;
+    }
+  }
+  const int slot = t / pairs, pr = t - slot * pairs, i = pr / nds, j = pr - i * nds;
+  const bool on = slot < epb;
+  const bool t0 = a.pmask & 1, t1 = a.pmask & 14, s0 = a.rmask & 1, s1 = a.rmask & 14;  // slots in use
+  double R[4][4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) R[p][r] = 0.0;
+  for (int q = 0; on && q < a.nq; ++q) {
+    const double *gt = ft.gref + ((int64_t)q * ndt + i) * 3, *gs = fs.gref + ((int64_t)q * nds + j) * 3;
+    const double w = a.qw[q];
+    const double f[4] = {ft.phi[q * ndt + i], gt[0], gt[1], gt[2]};
+    const double g[4] = {w * fs.phi[q * nds + j], w * gs[0], w * gs[1], w * gs[2]};
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) R[p][r] += f[p] * g[r];
+  }
+  __syncthreads();
+  for (int o = t; o < a.nout; o += blockDim.x) {  // its monomials in a fixed order
+    double s = 0.0;
+    for (int m = a.mptr[o]; m < a.mptr[o + 1]; ++m) {
+      double v = a.mcoef[m];
+      for (int x = a.moff[m]; x < a.moff[m + 1]; ++x) v *= T[a.msym[x]];
+      s += v;
+    }
+    O[o] = s;
+  }
+  __syncthreads();
+  for (int it = 0; it < iters; ++it) {
+    const int x = it * epb + slot;
+    const int64_t e = e0 + x;
+    const bool live = on && e < a.n_cv;
+    double v[QT][QS];
+#pragma unroll
+    for (int c = 0; c < QT; ++c)
+#pragma unroll
+      for (int b = 0; b < QS; ++b) v[c][b] = 0.0;
+    double mx = 0.0;
+    if (live) {
+      double B[9];
+#pragma unroll
+      for (int c = 0; c < 9; ++c) B[c] = geo[10 * x + c];
+      const double aJ = geo[10 * x + 9];
+      // adds O[.][p][.][r] S, with S the (p, r) entry of |J| B' R B'^T
+      auto add = [&](int p, int r, double S) {
+#pragma unroll
+        for (int c = 0; c < QT; ++c)
+#pragma unroll
+          for (int b = 0; b < QS; ++b)
+            v[c][b] += O[(p == 0 ? c : QT + 3 * c + p - 1) * w4 + (r == 0 ? b : QS + 3 * b + r - 1)] * S;
+      };
+      if (t0 && s0) add(0, 0, aJ * R[0][0]);
+      if (t0 && s1) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+          add(0, 1 + r, aJ * (R[0][1] * B[3 * r] + R[0][2] * B[3 * r + 1] + R[0][3] * B[3 * r + 2]));
+      }
+      if (t1 && s0) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          add(1 + p, 0, aJ * (B[3 * p] * R[1][0] + B[3 * p + 1] * R[2][0] + B[3 * p + 2] * R[3][0]));
+      }
+      if (t1 && s1) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+          double W[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            W[c] = aJ * (R[1 + c][1] * B[3 * r] + R[1 + c][2] * B[3 * r + 1] + R[1 + c][3] * B[3 * r + 2]);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) add(1 + p, 1 + r, B[3 * p] * W[0] + B[3 * p + 1] * W[1] + B[3 * p + 2] * W[2]);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < QT; ++c)
+#pragma unroll
+        for (int b = 0; b < QS; ++b) mx = fmax(mx, fabs(v[c][b]));
+    }
+    // the elements that meet in this wavefront, one after the other
+    const int k1 = min((t | 63) / pairs, epb - 1);
+    for (int k = (t & ~63) / pairs; k <= k1; ++k) {
+      const double m = pm_wave_max(slot == k ? mx : 0.0);
+      if (lane == 0) atomicMax(&smax[it * epb + k], (unsigned long long)__double_as_longlong(m));
+    }
+    __syncthreads();
+    if (live) {
+      const double m = __longlong_as_double((long long)smax[x]);
+      const double th = m > 0.0 ? 1e-14 * m : INFINITY;
+      double *dst = a.elem + e * ne + (int64_t)i * QT * nc + j * QS;
+#pragma unroll
+      for (int c = 0; c < QT; ++c)
+#pragma unroll
+        for (int b = 0; b < QS; ++b) dst[c * nc + b] = fabs(v[c][b]) > th ? v[c][b] : 0.0;
+    }
+  }
+}
+
 // ------------------------------------------------------------ structure
 // (row, column) key and position in the element matrices of every candidate
 // of a block
@@ -406,6 +550,20 @@ static hipError_t launch_poly_mat_q(hipStream_t s, const PolyMatArgs &a, size_t 
   return hipGetLastError();
 }
 
+template <int QT, int QS>
+static hipError_t launch_poly_ref(hipStream_t s, const PolyMatArgs &a) {
+  const int pairs = a.f[a.vt].nd * a.f[a.vs].nd;
+  const int threads = pairs <= 256 ? 256 : 512;
+  const int epb = threads / pairs;
+  int64_t iters = a.n_cv / ((int64_t)epb * 1024);  // four workgroups a CU before any takes a second pass
+  iters = std::min<int64_t>({std::max<int64_t>(iters, 1), kPrIters, kPrMaxChunk / epb});
+  const int chunk = epb * (int)iters;
+  const size_t lds = 8 * (size_t)(a.nsym + a.nout + 11 * chunk);
+  if (lds > 64 * 1024) return hipErrorInvalidValue;
+  k_poly_ref<QT, QS><<<(unsigned)((a.n_cv + chunk - 1) / chunk), threads, lds, s>>>(a, epb, (int)iters);
+  return hipGetLastError();
+}
+
 hipError_t launch_poly_mat(hipStream_t s, const PolyMatArgs &a) {
   if (a.n_cv == 0) return hipSuccess;
   if (a.nf < 1 || a.nf > kScalarMaxFields || a.vt < 0 || a.vt >= a.nf || a.vs < 0 || a.vs >= a.nf ||
@@ -422,6 +580,24 @@ hipError_t launch_poly_mat(hipStream_t s, const PolyMatArgs &a) {
   const size_t lds = 8 * (size_t)(a.nsym + a.nout + 4 * (a.f[a.vt].nd + a.f[a.vs].nd) + 4 * qt * nc +
                                   (a.varying ? vals : 0));
   if (lds > 64 * 1024) return hipErrorInvalidValue;
+  // tetrahedra and a program without fem fields: one reference tensor a pair
+  // serves every element (a field's values or a hexahedron's points make the
+  // integrand another one in each)
+  if (!a.gN && !a.varying && a.f[a.vt].nd * a.f[a.vs].nd <= 512) {
+    const int qs = a.f[a.vs].qdim;
+#define GFX_REF(QT, QS) \
+  if (qt == QT && qs == QS) return launch_poly_ref<QT, QS>(s, a)
+    GFX_REF(1, 1);
+    GFX_REF(1, 2);
+    GFX_REF(1, 3);
+    GFX_REF(2, 1);
+    GFX_REF(2, 2);
+    GFX_REF(2, 3);
+    GFX_REF(3, 1);
+    GFX_REF(3, 2);
+    GFX_REF(3, 3);
+#undef GFX_REF
+  }
   if (qt == 1) return launch_poly_mat_q<1>(s, a, lds);
   if (qt == 2) return launch_poly_mat_q<2>(s, a, lds);
   if (qt == 3) return launch_poly_mat_q<3>(s, a, lds);
