@@ -1133,8 +1133,9 @@ int gfx_plan_assemble(gfx_plan *p) {
     p->n_timed++;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
   }
+  const bool fused = !p->eb && !fresh && fused_records(p->nd, p->qdim, p->form, p->precision, p->mf->mesh->n_cv);
   if (!p->eb) {
-    if (!fresh && (r = plan_records(p))) return r;
+    if (!fresh && !fused && (r = plan_records(p))) return r;
   } else if (!fresh || p->precision != GFX_PREC_FP64) {
     if (!fresh && (r = plan_eb_points(p, true))) return r;
     if ((r = plan_eb_tangent(p, p->precision, kNhKeepNone))) return r;
@@ -1171,6 +1172,10 @@ int gfx_plan_assemble(gfx_plan *p) {
   a.qw = p->d_qw; a.R = p->d_R; a.vals = p->d_vals; a.max_inc = p->max_inc;
   a.rec32 = p->d_rec32; a.gref32 = p->d_gref32; a.qw32 = p->d_qw32; a.R32 = p->d_R32;
   a.Rq = p->d_Rq; a.rk = p->rk;
+  if (fused) {
+    a.geo = record_args(p);
+    a.thr = p->d_thr;
+  }
   // The launches (patch plans: large-patch size classes and the packed
   // waves; element-batched plans: gather bins) write disjoint rows: they run
   // concurrently, each on its own stream (up to seven auxiliary streams forked

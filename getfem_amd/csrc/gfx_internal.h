@@ -71,6 +71,19 @@ struct PatchDesc {
   uint32_t ninc_ns;         // incidences (low 16 bits) | nslots (high 16 bits)
 };
 
+// What the element records are formed from, and where they go.
+struct RecordArgs {
+  int64_t n_cv;
+  const double *pts;
+  const int32_t *cvx;
+  const double *ca, *cb, *cc;  // per-element coefficients or null (then ca_c, ...)
+  double ca_c, cb_c, cc_c;
+  double r_scale;              // scale of the reference tensor
+  double *rec;                 // kRecStride doubles per element
+  float *rec32;                // the FP32 form's records, or null
+  int *err;                    // bit 1: det K = 0
+};
+
 struct PatchArgs {
   int64_t n_nodes;
   const int32_t *order;     // node ids of this launch's bin
@@ -103,19 +116,10 @@ struct PatchArgs {
   // staging run (4-byte words) of any of the launch's waves
   int64_t n_waves;
   int lds_flat;
-};
-
-// What the element records are formed from, and where they go.
-struct RecordArgs {
-  int64_t n_cv;
-  const double *pts;
-  const int32_t *cvx;
-  const double *ca, *cb, *cc;  // per-element coefficients or null (then ca_c, ...)
-  double ca_c, cb_c, cc_c;
-  double r_scale;              // scale of the reference tensor
-  double *rec;                 // kRecStride doubles per element
-  float *rec32;                // the FP32 form's records, or null
-  int *err;                    // bit 1: det K = 0
+  // patch kernel, where the lanes form the records: their geometry and
+  // coefficients, and the elements' thresholds (else null)
+  RecordArgs geo;
+  const double *thr;
 };
 
 struct PatternArgs {
@@ -331,6 +335,8 @@ hipError_t launch_mask_fast(hipStream_t s, const PatternArgs &a);
 hipError_t launch_mask_exact(hipStream_t s, const PatternArgs &a, int max_nslots);
 hipError_t launch_fill_desc(hipStream_t s, int64_t n, int qdim, const int32_t *order, const int32_t *inc_ptr,
                             const uint16_t *nslots, const int64_t *indptr, PatchDesc *desc);
+// whether an assembly leaves the records to the patch kernel
+bool fused_records(int nd, int qdim, int form, int prec, int64_t n_cv);
 hipError_t launch_assemble_patch(hipStream_t s, int term, int form, int prec, const PatchArgs &a);
 hipError_t scan_exclusive_i64(hipStream_t s, const int64_t *in, int64_t *out,
                               int64_t n, int64_t *tmp);

@@ -633,7 +633,9 @@ __device__ __forceinline__ T pick4(const T (&v)[kMaxNpw], int k) {
   return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3]));
 }
 
-template <int ND, int Q, int TERM, int FORM, typename Real, int RK>
+// GEO: the lanes form the records themselves (small meshes, see
+// fused_records), which saves the launch of k_records_tet and a round trip.
+template <int ND, int Q, int TERM, int FORM, typename Real, int RK, bool GEO = false>
 __global__ __launch_bounds__(kWave) void k_assemble_patch(PatchArgs a) {
   static_assert(ND % 2 == 0, "slot maps are staged as u16 pairs");
   extern __shared__ double lds[];
@@ -758,6 +760,14 @@ __global__ __launch_bounds__(kWave) void k_assemble_patch(PatchArgs a) {
       const int64_t e = inc >> 5;
       const int i = inc & 31;
       const Real *rec = tab_rec + (int64_t)kRecStride * e;
+      Real own[16];
+      if constexpr (GEO) {
+        double o[16];
+        if (!tet_record(e, a.geo, o)) atomicOr(a.geo.err, 1);
+        o[11] = a.thr[e];
+        for (int t = 0; t < 16; ++t) own[t] = (Real)o[t];
+        rec = own;
+      }
       const double thr = (double)rec[11];
 #pragma unroll 1
       for (int jb = 0; jb < JB; ++jb) {
@@ -1037,12 +1047,40 @@ hipError_t launch_fill_columns(hipStream_t s, const PatternArgs &a) {
   return hipGetLastError();
 }
 
+// P1 elements: a lane's record is a row of loads and some 250 instructions for
+// the one pair block it is used for, against a launch, the records' way through
+// memory and a round trip.  Vector fields gain at every size (FP64 elasticity:
+// 384 elements 9.3 -> 7.8 us, 48,000 21.5 -> 17.8, 3.07 M 692 -> 645), scalar
+// ones, with less to do per record, up to where the launch no longer counts
+// (FP64 Poisson: 384 elements 8.4 -> 6.9 us, 48,000 15.0 -> 13.7, 131,712 29.0
+// -> 28.5, 279,936 43.6 -> 50.0; FP32, whose records are half as long: 24,576
+// 10.0 -> 9.6, 48,000 12.1 -> 12.7).
+bool fused_records(int nd, int qdim, int form, int prec, int64_t n_cv) {
+  if (nd != 4 || form != GFX_FORM_FACTORIZED || prec > GFX_PREC_FP32) return false;
+  return qdim > 1 || n_cv <= (prec == GFX_PREC_FP64 ? 131072 : 32768);
+}
+
 template <int ND, int Q, int TERM>
 static hipError_t launch_asm3(hipStream_t s, int form, int prec, const PatchArgs &a,
                               unsigned grid, size_t lds) {
   constexpr int F = GFX_FORM_FACTORIZED, P = GFX_FORM_PERQP;
   if (form == F) {
     const bool d = prec == GFX_PREC_FP64;
+    if constexpr (ND == 4) {
+      if (a.thr) {  // the records are formed by the lanes
+        if (a.rk == 1) {
+          if (d) k_assemble_patch<ND, Q, TERM, F, double, 1, true><<<grid, kWave, lds, s>>>(a);
+          else k_assemble_patch<ND, Q, TERM, F, float, 1, true><<<grid, kWave, lds, s>>>(a);
+        } else if (a.rk == 2) {
+          if (d) k_assemble_patch<ND, Q, TERM, F, double, 2, true><<<grid, kWave, lds, s>>>(a);
+          else k_assemble_patch<ND, Q, TERM, F, float, 2, true><<<grid, kWave, lds, s>>>(a);
+        } else {
+          if (d) k_assemble_patch<ND, Q, TERM, F, double, 0, true><<<grid, kWave, lds, s>>>(a);
+          else k_assemble_patch<ND, Q, TERM, F, float, 0, true><<<grid, kWave, lds, s>>>(a);
+        }
+        return hipGetLastError();
+      }
+    }
     if (a.rk == 1) {
       if (d) k_assemble_patch<ND, Q, TERM, F, double, 1><<<grid, kWave, lds, s>>>(a);
       else k_assemble_patch<ND, Q, TERM, F, float, 1><<<grid, kWave, lds, s>>>(a);

@@ -1,0 +1,38 @@
+"""P1 assembly with the element records formed by the patch kernel's lanes: bit
+for bit what the records kernel gives, for every term, both precisions,
+constant and per-element coefficients, and after the points moved."""
+import numpy as np
+import pytest
+
+import getfem_amd as ga
+from getfem_amd import meshes
+
+pytestmark = pytest.mark.gpu
+
+TERMS = {"laplace1": (ga.TERM_LAPLACE, 1, 1), "laplace3": (ga.TERM_LAPLACE, 3, 1),
+         "elast": (ga.TERM_ISO_ELAST, 3, 2), "isotropic": (ga.TERM_ISOTROPIC, 3, 3)}
+
+
+@pytest.mark.parametrize("n", [1, 3, 10])
+@pytest.mark.parametrize("prec", [ga.PREC_FP64, ga.PREC_FP32])
+@pytest.mark.parametrize("name", sorted(TERMS))
+def test_same_as_records(ctx, name, prec, n):
+    print("case: records formed by the lanes", name, prec, n, flush=True)
+    term, q, nc = TERMS[name]
+    pts, cvx = meshes.regular_unit_mesh(n, "GT_PK(3,1)")
+    pts = meshes.jitter(pts, n)
+    rng = np.random.default_rng(n)
+    coefs = [rng.uniform(0.5, 2.0, cvx.shape[0]) if k == 0 else 1.25 for k in range(nc)]
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", pts, cvx)
+    plan = ga.Plan(ga.MeshFem(mesh, "FEM_PK(3,1)", q), ga.MeshIm(mesh, "IM_TETRAHEDRON(2)"), term, coefs)
+    plan.set_form(ga.FORM_FACTORIZED, prec)
+    plan.build_pattern()
+    for moved in (False, True):
+        if moved:
+            mesh.set_points(pts + 0.01 / n * np.sin(5.0 * pts[:, ::-1]))
+        plan.set_coef(0, coefs[0])
+        plan.assemble()  # new values: the records come from the check of the pattern
+        ref = plan.csr()
+        plan.assemble()  # the same values again: from the lanes
+        for a, b in zip(ref, plan.csr()):
+            assert np.array_equal(a, b)
