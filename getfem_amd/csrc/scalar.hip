@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gfx_internal.h"
 
@@ -35,7 +36,8 @@ constexpr int kScRedBlocks = 256;
 // Bound by latency (dependent loads and FP64 chains), so the points go side by
 // side: with a lane per element, 20,250 elements were 317 wavefronts for the
 // whole chip, each with 15 points one after another.  Measured there (u P2
-// vector + p P1): 58 us a variable, 222 us before.
+// vector + p P1): 43 us a variable (58 us with a node's base function loaded
+// again for each component), 222 us with a lane per element.
 template <int G>
 __global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a, int nsym, int nvals) {
   extern __shared__ double lds_sc[];
@@ -75,17 +77,31 @@ __global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a, int ns
     for (int fi = 0; fi < a.nf; ++fi) {
       const ScalarField &f = a.f[fi];
       const double *phi = f.phi + q * f.nd, *gr = f.gref + (int64_t)q * f.nd * 3;
-      for (int c = 0; c < f.qdim; ++c) {
-        double v = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
+      const auto field = [&](auto qd) {  // a node's base function and gradient serve the components together
+        constexpr int QD = decltype(qd)::value;
+        double v[QD], r0[QD], r1[QD], r2[QD];
+#pragma unroll
+        for (int c = 0; c < QD; ++c) v[c] = r0[c] = r1[c] = r2[c] = 0.0;
+#pragma unroll 2
         for (int i = 0; i < f.nd; ++i) {
-          const double u = v0[i * f.qdim + c];
-          v += phi[i] * u;
-          r0 += gr[3 * i] * u; r1 += gr[3 * i + 1] * u; r2 += gr[3 * i + 2] * u;
+          const double h = phi[i], g0 = gr[3 * i], g1 = gr[3 * i + 1], g2 = gr[3 * i + 2];
+#pragma unroll
+          for (int c = 0; c < QD; ++c) {
+            const double u = v0[i * QD + c];
+            v[c] += h * u;
+            r0[c] += g0 * u; r1[c] += g1 * u; r2[c] += g2 * u;
+          }
         }
-        T[(f.off + c) * kScThreads] = v;
-        for (int b = 0; b < 3; ++b)
-          T[(f.off + f.qdim + 3 * c + b) * kScThreads] = B[3 * b] * r0 + B[3 * b + 1] * r1 + B[3 * b + 2] * r2;
-      }
+#pragma unroll
+        for (int c = 0; c < QD; ++c) {
+          T[(f.off + c) * kScThreads] = v[c];
+          for (int b = 0; b < 3; ++b)
+            T[(f.off + QD + 3 * c + b) * kScThreads] = B[3 * b] * r0[c] + B[3 * b + 1] * r1[c] + B[3 * b + 2] * r2[c];
+        }
+      };
+      if (f.qdim == 1) field(std::integral_constant<int, 1>{});
+      else if (f.qdim == 2) field(std::integral_constant<int, 2>{});
+      else field(std::integral_constant<int, 3>{});  // (a mesh_fem has at most three)
       v0 += f.nd * f.qdim;
     }
     for (int o = 0; o < a.nout; ++o) O[o * kScThreads] = 0.0;
