@@ -241,7 +241,9 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 // (i <= j: the matrix is symmetric) are shared out between the workgroup's
 // kKeepWaves wavefronts.  Pass 1 takes the largest entry (threshold 1e-14
 // max|elem|, an all-zero element gets infinity: GetFEM skips it,
-// compile_and_exec.cc:5441-5442), pass 2 forms the blocks again and compares.
+// compile_and_exec.cc:5441-5442), pass 2 forms the blocks again and compares
+// (a check of finite values needs no pass 2: it takes the smallest entry of
+// those that are stored as kept and the largest of the others in pass 1).
 // The blocks are those of the factorized form, G = B R_ij B^T: an integral
 // instead of a sum over the points (P2: 63 products a block instead of 600),
 // and the reference blocks are the same for every lane, so they come through
@@ -253,9 +255,10 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 // scalar unit.  The element records, needed with the threshold by the
 // assembly that follows, are formed here too (they would cost a launch and a
 // pass over the elements before and after).
-// Bound by FP64 issue: 8,000 products and sums a lane, 0.57 of the rate.
-// Measured at P2 elasticity, 40^3 x 6 = 384,000 elements: 146 us, and no
-// pattern pass where the bits stay, against 3,553 us of per-point blocks (a
+// Bound by FP64 issue (4,000 products and sums a lane) and the wait for the
+// scalars.  Measured at P2 elasticity, 40^3 x 6 = 384,000 elements: 131 us (143
+// with the second pass; P2 Laplacian on 55,566 moved elements 14 us, 18 with
+// it), and no pattern pass where the bits stay, against 3,553 us of per-point blocks (a
 // wavefront per element, all pairs, twice) with 394 us of presence-bit passes
 // after them and 15 us of records before and after; an assembly with new
 // coefficients 4.91 -> 0.59 ms.
@@ -312,12 +315,30 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
     for (int t = 0; t < 9; ++t) B[t] = live ? o[t] : 0.0;
     if (live) { sa = o[9]; sb = o[10]; sc = o[15]; }
   }
-  double mx = 0.0;
+  const uint64_t *sg = sig + g * (NP * NV);
+  // CHECK: the smallest of the entries whose stored bit is set, the largest of
+  // the others (mn > thr and md <= thr: the bits are the stored ones), and
+  // whether every value is finite, where both say what the bits would
+  const uint64_t full = nblk == kWave ? ~0ull : (1ull << nblk) - 1ull;
+  double mx = 0.0, mn = INFINITY, md = 0.0, fin = 0.0;
   for (int p = w; p < NP; p += kKeepWaves) {
     double v[NV];
     keep_block<Q, TERM>(Rp + 9 * p, B, sa, sb, sc, v);
 #pragma unroll
-    for (int x = 0; x < NV; ++x) mx = fmax(mx, fabs(v[x]));
+    for (int x = 0; x < NV; ++x) {
+      const double m = fabs(v[x]);
+      mx = fmax(mx, m);
+      if constexpr (CHECK) {
+        const uint64_t k = sg[p * NV + x];
+        fin += 0.0 * v[x];
+        if (k == full) mn = fmin(mn, m);
+        else if (k == 0) md = fmax(md, m);
+        else {
+          mn = fmin(mn, k >> lane & 1 ? m : INFINITY);
+          md = fmax(md, k >> lane & 1 ? 0.0 : m);
+        }
+      }
+    }
   }
   red[w][lane] = mx;
   __syncthreads();
@@ -328,9 +349,14 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
     thr_out[e0 + lane] = thr;
     reinterpret_cast<double *>(stage + 9 * lane)[11] = thr;
   }
-  const uint64_t *sg = sig + g * (NP * NV);
   uint64_t diff = 0;
-  for (int p = w; p < NP; p += kKeepWaves) {
+  bool pass2 = true;
+  if constexpr (CHECK) {
+    pass2 = __ballot(fin != 0.0) != 0;  // not a number: the bits themselves are compared
+    diff = __ballot(lane < nblk && !(mn > thr && md <= thr));
+  }
+  if (CHECK && pass2) diff = 0;
+  for (int p = pass2 ? w : NP; p < NP; p += kKeepWaves) {
     double v[NV];
     keep_block<Q, TERM>(Rp + 9 * p, B, sa, sb, sc, v);
 #pragma unroll
