@@ -64,7 +64,7 @@ WORKLOAD = {
           "u = sum of 8 sine modes (max |u| = 0.05)",
 }
 # kernels whose HBM traffic the PMC passes measure, per config
-PMC_KERNELS = {"c2": "k_assemble_patch", "c5": "k_assemble_patch", "c3": "k_nh_element|k_gather"}
+PMC_KERNELS = {"c2": "k_assemble_patch", "c5": "k_assemble_patch", "c3": "k_nh_points|k_nh_tangent|k_gather"}
 
 
 def log(*a):
@@ -342,17 +342,18 @@ def run_gpu(args):
             out["mfma_note"] = ("the FP64 node-patch form (factorized 3x3 pair blocks on the vector ALUs) stays the "
                                 "headline; the element-batched forms buffer n_loc^2 values per element and gather them")
     if hexes:
-        # The step is two launches: k_nh_element (element matrices and residuals,
-        # the tangent on the matrix cores, E to HBM) and k_gather_emat (node
-        # gathers of E into the CSR).  The HBM roofline takes the compulsory
-        # bytes over both kernels' time (traffic over the same two kernels);
-        # the compute side is the element kernel's matrix-core rate.
+        # The step is three launches: k_nh_points (the points' values and the
+        # residuals), k_nh_tangent (element matrices on the matrix cores, E to
+        # HBM) and k_gather_emat (node gathers of E into the CSR).  The HBM
+        # roofline takes the compulsory bytes over the kernels' time (traffic
+        # over the same kernels); the compute side is the matrix-core rate over
+        # the first two.
         t2 = head["ms_geometry_kernel"] + head["ms_assemble_kernel"]
         r = out["roofline"]
-        r.update(kernel="k_nh_element + k_gather_emat", kernel_ms=t2,
+        r.update(kernel="k_nh_points + k_nh_tangent + k_gather_emat", kernel_ms=t2,
                  kernel_ms_min=None, achieved=compulsory / (t2 * 1e-3) / 1e9,
                  frac=compulsory / (t2 * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                 kernel_ms_stat="sum of the two kernels' medians over the timed steps (HIP events on the "
+                 kernel_ms_stat="sum of the element and the gather kernels' medians over the timed steps (HIP events on the "
                                 "launch stream)",
                  element_kernel_ms=head["ms_geometry_kernel"], gather_kernel_ms=head["ms_assemble_kernel"])
         r["element_scatter_model"]["note"] = ("SURVEY-style element-scatter count (a read, a write and a "
@@ -361,10 +362,10 @@ def run_gpu(args):
         r["element_scatter_model"]["bytes_per_element"] = b_patch + 16 * n_loc
         r["element_scatter_model"]["gb_per_assembly"] = (b_patch + 16 * n_loc) * n_cv / 1e9
         # matrix-core products per element (both forms): 3 K3 node tiles x 21 and
-        # 21 upper (component pair, node tile pair) tiles x 14 products of
-        # 16x16x4 (2048 FLOP each), zero pads included; the spatial form's useful
-        # FLOP: 48 per upper node-pair block and point
-        n_mfma = 3 * 21 + 21 * 14
+        # 21 upper (component pair, node tile pair) tiles x 14 (the 9 of equal
+        # components 7) products of 16x16x4 (2048 FLOP each), zero pads included;
+        # the spatial form's useful FLOP: 48 per upper node-pair block and point
+        n_mfma = 3 * 21 + 12 * 14 + 9 * 7
         useful = 48 * (27 * 28 // 2) * 27
         mf = {}
         for fname, instr, peak in (("fp64_element_batched", "v_mfma_f64_16x16x4_f64", FP64_PEAK_TFLOPS),
@@ -374,7 +375,7 @@ def run_gpu(args):
                 continue
             t_el = f["ms_geometry_kernel"] * 1e-3
             issued = n_mfma * 2048 * n_cv / t_el / 1e12
-            mf[fname] = {"kernel": "k_nh_element", "instruction": instr, "mfma_per_element": n_mfma,
+            mf[fname] = {"kernel": "k_nh_points + k_nh_tangent", "instruction": instr, "mfma_per_element": n_mfma,
                          "issued_tflops": issued, "peak_tflops": peak, "frac": issued / peak,
                          "useful_flop_per_element": useful,
                          "useful_tflops": useful * n_cv / t_el / 1e12,
