@@ -806,21 +806,17 @@ static int plan_bins(gfx_plan *p, const std::vector<uint16_t> &ns, const std::ve
       gmax = 0;
     }
   }
-  // patches per wavefront: small patches are packed so that one wave's
-  // incidences fill about three passes of its lanes
+  // patches per workgroup
   std::vector<int> bmax(p->bins.size(), 0);
   for (int64_t n = 0; n < nn; ++n) {
     const int b = group[cls[n]];
     bmax[b] = std::max(bmax[b], iptr[n + 1] - iptr[n]);
   }
-  const int lanes = (64 / p->nd) * p->nd;
-  for (size_t b = 0; b < p->bins.size(); ++b) {
-    const int per = std::max(1, bmax[b]) * p->nd;
-    if (p->eb)  // gather workgroups stream ~4 incidences each
-      p->bins[b].npw = std::max(1, std::min({4, 4 / std::max(1, bmax[b]), 64 / std::max(1, p->max_inc)}));
-    else
-      p->bins[b].npw = std::max(1, std::min(4, 3 * lanes / per));
-  }
+  // a workgroup streams about eight incidences, all in flight at once (an
+  // assembly at 48^3: 4.26 ms; with two 4.62, four 4.42, sixteen 4.32); its
+  // accumulators hold at most npw x 27 bmax slots, 216 by this rule
+  for (size_t b = 0; b < p->bins.size(); ++b)
+    p->bins[b].npw = std::max(1, std::min({4, 8 / std::max(1, bmax[b]), 64 / std::max(1, p->max_inc)}));
   std::vector<int64_t> cur(p->bins.size());
   for (size_t b = 0; b < p->bins.size(); ++b) cur[b] = p->bins[b].off;
   std::vector<int32_t> order((size_t)nn);
