@@ -400,8 +400,11 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv(int64_t n, int64_t c
 // in order: issued before the x they would have to arrive first).  The node's
 // start and slot count are the same for every lane and come by scalar loads,
 // a node ahead.
-// Measured at P2 elasticity, 24^3 x 6 (367,000 rows, 28.7 M entries): 72 us with
-// p.q (111 + 5 + 5 us for a row per 32 lanes, p.q and its sum apart: 12 bytes
+// Every other product goes through the matrix backwards (`back`), so that it
+// begins with what the last one left in the memory-side cache (256 MB): a matrix
+// of about that size, swept one way, would find none of it.
+// Measured at P2 elasticity, 24^3 x 6 (367,000 rows, 28.7 M entries, 242 MB): 68 us
+// (one way 72) with p.q (111 + 5 + 5 us for a row per 32 lanes, p.q and its sum apart: 12 bytes
 // an entry, two latencies a row); 82 us with the values loaded non-temporally
 // (rows share cache lines: they were fetched twice), 95-146 us with a node per
 // 16 or 32 lanes, 115 us at half the wavefronts.
@@ -413,12 +416,12 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
                                                              const int32_t *__restrict__ nodes,
                                                              const double *__restrict__ p, double *__restrict__ q,
                                                              const CgScal *__restrict__ sc,
-                                                             double *__restrict__ part) {
+                                                             double *__restrict__ part, bool back) {
   __shared__ double sh[kRedThreads / 64];
   if (sc && sc->done) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t first = (int64_t)(blockIdx.x & 7) * chunk, last = min(nn, first + chunk);
-  const int64_t step = (int64_t)(gridDim.x >> 3) * (kRedThreads / 64);
+  int64_t step = (int64_t)(gridDim.x >> 3) * (kRedThreads / 64);
   struct Node {
     int64_t b0;      // its first value
     int r1, r2, r3;  // rows 1 and 2 and the end, from there
@@ -454,13 +457,17 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
   };
   double pq = 0.0;
   int64_t u = first + (int64_t)(blockIdx.x >> 3) * (kRedThreads / 64) + w;
+  if (back && u < last) {  // the same nodes, last to first
+    u += (last - 1 - u) / step * step;
+    step = -step;
+  }
   Node cur{};
   if (u < last) {
     cur = node(u);
     if (cur.len) load(cur, 0);
   }
-  for (; u < last; u += step) {
-    const Node nxt = node(min(u + step, last - 1));
+  for (; u >= first && u < last; u += step) {
+    const Node nxt = node(max(first, min(u + step, last - 1)));
     const double pu = p[3 * u + min(lane, 2)];
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     if (!cur.len && nxt.len) load(nxt, 0);
@@ -915,12 +922,12 @@ static int cg_prod_blocks(int64_t nu, int per, int64_t &chunk) {
 
 static hipError_t cg_product(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
                              const double *vals, const uint16_t *nslots, const int32_t *nodes, const double *p,
-                             double *q, const CgScal *sc, double *part, int *nblocks) {
+                             double *q, const CgScal *sc, double *part, int *nblocks, bool back) {
   int64_t chunk;
   if (nslots) {
     *nblocks = cg_prod_blocks(n / 3, kRedThreads / 64, chunk);
     k_cg_spmv3<<<(unsigned)*nblocks, kRedThreads, 0, s>>>(n / 3, chunk, indptr, indices, vals, nslots, nodes, p, q, sc,
-                                                          part);
+                                                          part, back);
     return hipGetLastError();
   }
   auto run = [&](auto g) {
@@ -958,7 +965,8 @@ static hipError_t cg_iterations(hipStream_t s, int64_t n, int64_t nnz, const int
     for (; it < end; ++it) {
       CgScal *cur = sc + (it & 1), *next = sc + (~it & 1);
       int np = 0;
-      if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, p, q, cur, ppart, &np)) != hipSuccess)
+      if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, p, q, cur, ppart, &np, it & 1)) !=
+          hipSuccess)
         return e;
       k_cg_update<QB><<<nb, kRedThreads, 0, s>>>(nu, cur, ppart, np, p, q, minv, x, r, z, part);
       k_cg_direction<<<nd, kRedThreads, 0, s>>>(n, cur, part, nb, rtol, z, p, next);
@@ -987,7 +995,8 @@ hipError_t cg_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr
   if (qb != 3) nslots = nullptr;
   if (nslots) k_cg_nodes<<<nb256(8 * nu), 256, 0, s>>>(nu, nslots, indptr, indices, nodes);
   int np = 0;
-  if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, x, r, nullptr, work + 7 * n, &np)) != hipSuccess)
+  if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, x, r, nullptr, work + 7 * n, &np, false)) !=
+      hipSuccess)
     return e;
   CgScal h{};
   e = qb == 3 ? cg_iterations<3>(s, n, nnz, indptr, indices, vals, nslots, nodes, b, x, rtol, maxit, work, &h)
