@@ -80,6 +80,7 @@ struct ScField {
   gfx_mesh_fem *mf = nullptr;
   int off = 0;
   double *d_U = nullptr, *d_phi = nullptr, *d_gref = nullptr;
+  const double *u = nullptr;    // the values that an assembly reads: d_U or the variable's device copy
 };
 
 struct ScVar {                  // a fem variable's order-1 block
@@ -774,6 +775,7 @@ int sc_build(gfx_workspace *w) {
       hipMalloc((void **)&sc->d_err, 4) != hipSuccess ||
       hipMalloc((void **)&sc->d_consts, 8 * std::max<size_t>(sc->consts.size(), 1)) != hipSuccess)
     return bail(GFX_E_OOM, "polynomial route buffers");
+  sc->h_consts.clear();  // nothing is on the device yet
   return GFX_OK;
 }
 
@@ -808,17 +810,20 @@ bool sc_zero_ok(gfx_workspace *w, const GwflScalarProgram &p) {
 int sc_upload(gfx_workspace *w) {
   ScalarRoute *sc = w->sc;
   hipStream_t s = w->ctx->stream;
-  for (auto &f : sc->fields) {
+  for (auto &f : sc->fields) {  // device values are read where they are
     const WsVar &v = w->vars.at(f.name);
-    if (v.dev)
-      WHIP(w, hipMemcpyAsync(f.d_U, v.d_val, 8 * v.V.size(), hipMemcpyDeviceToDevice, s));
-    else
-      WHIP(w, hipMemcpyAsync(f.d_U, v.V.data(), 8 * v.V.size(), hipMemcpyHostToDevice, s));
+    f.u = v.dev ? v.d_val : f.d_U;
+    if (!v.dev) WHIP(w, hipMemcpyAsync(f.d_U, v.V.data(), 8 * v.V.size(), hipMemcpyHostToDevice, s));
   }
-  sc->h_consts.clear();
-  for (const std::string &n : sc->consts) sc->h_consts.push_back(w->vars.at(n).V[0]);
-  if (!sc->h_consts.empty())
-    WHIP(w, hipMemcpyAsync(sc->d_consts, sc->h_consts.data(), 8 * sc->h_consts.size(), hipMemcpyHostToDevice, s));
+  std::vector<double> consts;
+  for (const std::string &n : sc->consts) consts.push_back(w->vars.at(n).V[0]);
+  const size_t cb = 8 * consts.size();
+  if (cb && (sc->h_consts.size() != consts.size() || memcmp(sc->h_consts.data(), consts.data(), cb) != 0)) {
+    sc->h_consts = consts;  // what the device holds
+    const hipError_t e = hipMemcpyAsync(sc->d_consts, sc->h_consts.data(), cb, hipMemcpyHostToDevice, s);
+    if (e != hipSuccess) sc->h_consts.clear();
+    WHIP(w, e);
+  }
   // the host buffers above are read before they can change: every assembly
   // ends with a synchronisation of the stream
   WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
@@ -1041,7 +1046,7 @@ int sc_run2(gfx_workspace *w) {
   a.nf = (int)sc->fields.size();
   for (int i = 0; i < a.nf; ++i) {
     const ScField &f = sc->fields[i];
-    a.f[i] = ScalarField{f.mf->d_dofs, f.d_U, f.d_phi, f.d_gref, f.mf->fem.nd, f.mf->qdim, f.off};
+    a.f[i] = ScalarField{f.mf->d_dofs, f.u, f.d_phi, f.d_gref, f.mf->fem.nd, f.mf->qdim, f.off};
   }
   a.nconst = (int)sc->consts.size(); a.const_off = sc->const_off; a.consts = sc->d_consts; a.nsym = sc->nsym;
   a.err = sc->d_err;
@@ -1089,7 +1094,7 @@ int sc_run(gfx_workspace *w, int order) {
   a.nf = (int)sc->fields.size();
   for (int i = 0; i < a.nf; ++i) {
     const ScField &f = sc->fields[i];
-    a.f[i] = ScalarField{f.mf->d_dofs, f.d_U, f.d_phi, f.d_gref, f.mf->fem.nd, f.mf->qdim, f.off};
+    a.f[i] = ScalarField{f.mf->d_dofs, f.u, f.d_phi, f.d_gref, f.mf->fem.nd, f.mf->qdim, f.off};
   }
   a.nconst = (int)sc->consts.size(); a.const_off = sc->const_off; a.consts = sc->d_consts;
   a.elem = sc->d_elem; a.err = sc->d_err;
