@@ -7,11 +7,12 @@
 // from the mean row length so that short rows (P1) do not leave most lanes
 // idle.
 //
-// CG: an iteration is three launches (product with p.q, update with r.z and
-// r.r, direction); every scalar of the recurrence lives in device memory and
+// CG: an iteration is four launches (product, p.q, update with r.z and r.r,
+// direction); every scalar of the recurrence lives in device memory and
 // comes from fixed-order reductions, and so does the stopping test, so the
 // host launches iterations in batches and looks once per batch; the result
-// does not depend on scheduling or on the batch.
+// does not depend on scheduling or on the batch, nor on which of the products'
+// kernels runs: all of them sum a row in k_spmv's order.
 #include <hip/hip_runtime.h>
 
 #include <hipcub/hipcub.hpp>
@@ -28,8 +29,8 @@ namespace {
 
 constexpr int kSpmvThreads = 256;
 constexpr int kRedThreads = 256;   // threads of a reduction block
-constexpr int kRedBlocks = 1024;   // most partial sums of a vector kernel's dot product
-constexpr int kMaxProdBlocks = 2048;  // and of the product's (8 blocks a CU)
+constexpr int kRedBlocks = 1024;   // most partial sums of a dot product
+constexpr int kMaxProdBlocks = 2048;  // most blocks of a CG product (8 a CU)
 
 template <int G, bool ACC>
 __global__ __launch_bounds__(kSpmvThreads) void k_spmv(int64_t n, const int64_t *__restrict__ indptr,
@@ -190,38 +191,59 @@ struct CgScal {
   int it, done;
 };
 
-// sum over the wavefront, every lane gets it: data-parallel moves within rows
-// of 16 lanes, then across them (a move costs a few cycles, a shuffle through
-// the LDS unit some fifty)
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
-  return v + __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-__device__ __forceinline__ double wave_sum(double v) {
-  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row has the row's sum
-  v = dpp_add<0x112, 0xf>(v);
-  v = dpp_add<0x114, 0xf>(v);
-  v = dpp_add<0x118, 0xf>(v);
-  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
-  v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3: lane 63 has the sum
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+// Lane exchanges of doubles: data-parallel moves within rows of 16 lanes, swaps
+// across them (a move costs a few cycles, a shuffle through the LDS unit some fifty).
+struct Dbl2 {
+  double a, b;
+};
+__device__ __forceinline__ uint32_t lo32(double v) { return (uint32_t)__builtin_bit_cast(uint64_t, v); }
+__device__ __forceinline__ uint32_t hi32(double v) { return (uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32); }
+__device__ __forceinline__ double dbl(uint32_t lo, uint32_t hi) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
+// {a's lower 32 lanes, b's lower}, {a's upper, b's upper}
+__device__ __forceinline__ Dbl2 swap32(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane32_swap(lo32(a), lo32(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(hi32(a), hi32(b), false, false);
+  return {dbl(l[0], h[0]), dbl(l[1], h[1])};
+}
+// by rows of 16 lanes: {a0 b0 a2 b2}, {a1 b1 a3 b3}
+__device__ __forceinline__ Dbl2 swap16(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane16_swap(lo32(a), lo32(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(hi32(a), hi32(b), false, false);
+  return {dbl(l[0], h[0]), dbl(l[1], h[1])};
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  return v + dbl(__builtin_amdgcn_update_dpp(0, (int)lo32(v), CTRL, 0xf, 0xf, true),
+                 __builtin_amdgcn_update_dpp(0, (int)hi32(v), CTRL, 0xf, 0xf, true));
+}
+// sum over each G lanes (16, 32 or 64), every lane gets its group's: the tree
+// of lane ^ G/2, ..., lane ^ 1
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+  if constexpr (G == 64) {
+    const Dbl2 r = swap32(v, v);
+    v = r.a + r.b;
+  }
+  if constexpr (G >= 32) {
+    const Dbl2 r = swap16(v, v);
+    v = r.a + r.b;
+  }
+  v = dpp_add<0x128>(v);  // row_ror 8
+  v = dpp_add<0x124>(v);  // row_ror 4: the same as lane ^ 4, the sums repeat every 8 lanes
+  v = dpp_add<0x4e>(v);   // quad_perm 2 3 0 1
+  return dpp_add<0xb1>(v);  // quad_perm 1 0 3 2
+}
 
-// sum over the block, every thread gets it; the wavefronts' sums, then those
-// in order through LDS
+// sum over the block, every thread gets it: thread t and t + 128, then t + 64,
+// t + 32, ..., t + 1
 __device__ __forceinline__ double block_sum(double v, double *sh) {
-  v = wave_sum(v);
   __syncthreads();  // the last use of sh
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  sh[threadIdx.x] = v;
   __syncthreads();
-  double r = sh[0];
-  for (int w = 1; w < kRedThreads / 64; ++w) r += sh[w];
-  return r;
+  const int l = threadIdx.x & 63;
+  return group_sum<64>((sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]));
 }
 
 // the sum of a launch's n partials, in a fixed order, by every block that needs it
@@ -316,7 +338,7 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_start(int64_t nu, const doub
                                                           const double *__restrict__ minv,
                                                           double *__restrict__ r, double *__restrict__ z,
                                                           double *__restrict__ p, double *__restrict__ part) {
-  __shared__ double sh[kRedThreads / 64];
+  __shared__ double sh[kRedThreads];
   double rz = 0, rr = 0, bb = 0;
   for (int64_t u = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; u < nu; u += (int64_t)gridDim.x * kRedThreads) {
     double ri[QB], zi[QB];
@@ -339,7 +361,7 @@ __device__ __forceinline__ bool cg_stops(double rr, double bb, double rtol) { re
 
 __global__ __launch_bounds__(kRedThreads) void k_cg_first(const double *__restrict__ part, int n, double rtol,
                                                           CgScal *__restrict__ sc) {
-  __shared__ double sh[kRedThreads / 64];
+  __shared__ double sh[kRedThreads];
   const double rz = partials_sum(part, n, sh), rr = partials_sum(part + n, n, sh);
   const double bb = partials_sum(part + 2 * n, n, sh);
   if (threadIdx.x == 0) *sc = CgScal{rz, rr, bb, 0.0, 0, bb == 0.0 || cg_stops(rr, bb, rtol)};
@@ -358,38 +380,29 @@ __global__ void k_cg_nodes(int64_t nn, const uint16_t *__restrict__ nslots, cons
   for (int s = (int)(t % 8); s < ns; s += 8) nodes[b0 / 9 + s] = indices[b0 + 3 * s] / 3;
 }
 
-// q = K p and the partials of p.q: every launch writes one partial a block
-// (sc null: no iteration, the product of the start).
+// q = K p (sc null: no iteration, the product of the start).
 // The blocks of an XCD sweep one eighth of the units, so that the x that
 // neighbouring rows share stays in its L2.
-// A row per G lanes (scalar fields and workspace matrices).
+// A row per G lanes (scalar fields, workspace matrices and short rows).
 template <int G>
 __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv(int64_t n, int64_t chunk,
                                                             const int64_t *__restrict__ indptr,
                                                             const int32_t *__restrict__ indices,
                                                             const double *__restrict__ vals,
                                                             const double *__restrict__ p, double *__restrict__ q,
-                                                            const CgScal *__restrict__ sc,
-                                                            double *__restrict__ part) {
-  __shared__ double sh[kRedThreads / 64];
+                                                            const CgScal *__restrict__ sc) {
   if (sc && sc->done) return;
   constexpr int kPer = kRedThreads / G;
   const int lane = threadIdx.x % G;
   const int64_t first = (int64_t)(blockIdx.x & 7) * chunk, last = min(n, first + chunk);
   const int64_t step = (int64_t)(gridDim.x >> 3) * kPer;
-  double pq = 0.0;
   for (int64_t u = first + (int64_t)(blockIdx.x >> 3) * kPer + threadIdx.x / G; u < last; u += step) {
     double s = 0.0;
     const int64_t e = indptr[u + 1];
     for (int64_t k = indptr[u] + lane; k < e; k += G) s += vals[k] * p[indices[k]];
     for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
-    if (lane == 0) {
-      q[u] = s;
-      pq += p[u] * s;
-    }
+    if (lane == 0) q[u] = s;
   }
-  pq = block_sum(pq, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = pq;
 }
 
 // A node's three rows per wavefront (3x3 block Jacobi's fields); a column's x
@@ -400,14 +413,21 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv(int64_t n, int64_t c
 // in order: issued before the x they would have to arrive first).  The node's
 // start and slot count are the same for every lane and come by scalar loads,
 // a node ahead.
+// G: lanes of a row's sum, k_spmv's (16 or 32).  A row's sum there is G chains
+// and a tree, and 40 unconverged iterations turn another order's last bits into
+// differences of up to 1e-9 (seen over random right-hand sides), so the tile's
+// 64 products are dealt to the same G chains: lane swaps put a row's tile, G
+// columns after G columns, on the row's own G lanes (two rows share a register
+// at 32, all three at 16).
 // Every other product goes through the matrix backwards (`back`), so that it
 // begins with what the last one left in the memory-side cache (256 MB): a matrix
 // of about that size, swept one way, would find none of it.
 // Measured at P2 elasticity, 24^3 x 6 (367,000 rows, 28.7 M entries, 242 MB): 68 us
-// (one way 72) with p.q (111 + 5 + 5 us for a row per 32 lanes, p.q and its sum apart: 12 bytes
-// an entry, two latencies a row); 82 us with the values loaded non-temporally
-// (rows share cache lines: they were fetched twice), 95-146 us with a node per
-// 16 or 32 lanes, 115 us at half the wavefronts.
+// (one way 72; the same with 64 chains a row) against 111 us for a row per 32
+// lanes (12 bytes an entry, two latencies a row); 82 us with the values loaded
+// non-temporally (rows share cache lines: they were fetched twice), 95-146 us
+// with a node per 16 or 32 lanes, 115 us at half the wavefronts.
+template <int G>
 __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t chunk,
                                                              const int64_t *__restrict__ indptr,
                                                              const int32_t *__restrict__ indices,
@@ -415,9 +435,7 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
                                                              const uint16_t *__restrict__ nslots,
                                                              const int32_t *__restrict__ nodes,
                                                              const double *__restrict__ p, double *__restrict__ q,
-                                                             const CgScal *__restrict__ sc,
-                                                             double *__restrict__ part, bool back) {
-  __shared__ double sh[kRedThreads / 64];
+                                                             const CgScal *__restrict__ sc, bool back) {
   if (sc && sc->done) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t first = (int64_t)(blockIdx.x & 7) * chunk, last = min(nn, first + chunk);
@@ -455,7 +473,6 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
     v1 = v[i1];
     v2 = v[i2];
   };
-  double pq = 0.0;
   int64_t u = first + (int64_t)(blockIdx.x >> 3) * (kRedThreads / 64) + w;
   if (back && u < last) {  // the same nodes, last to first
     u += (last - 1 - u) / step * step;
@@ -468,8 +485,8 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
   }
   for (; u >= first && u < last; u += step) {
     const Node nxt = node(max(first, min(u + step, last - 1)));
-    const double pu = p[3 * u + min(lane, 2)];
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    const int l0 = cur.r1, l1 = cur.r2 - cur.r1, l2 = cur.r3 - cur.r2;  // the rows' lengths
+    double s = 0.0, s2 = 0.0;
     if (!cur.len && nxt.len) load(nxt, 0);
     for (int k0 = 0; k0 < cur.len; k0 += 64) {
       const int k = k0 + lane;
@@ -484,22 +501,51 @@ __global__ __launch_bounds__(kRedThreads, 8) void k_cg_spmv3(int64_t nn, int64_t
       const double a0 = v0, a1 = v1, a2 = v2;
       if (k0 + 64 < cur.len) load(cur, k0 + 64);
       else if (nxt.len) load(nxt, 0);
-      s0 += k < cur.r1 ? a0 * x0 : 0.0;
-      s1 += k < cur.r2 - cur.r1 ? a1 * x1 : 0.0;
-      s2 += k < cur.r3 - cur.r2 ? a2 * x2 : 0.0;
+      const int kg = k0 + lane % G;
+      if constexpr (G == 32) {  // s: row 0 in the lower lanes, row 1 in the upper; s2: row 2 in both
+        const Dbl2 a = swap32(a0, a1), x = swap32(x0, x1), b = swap32(a2, a2), y = swap32(x2, x2);
+        const int l01 = lane < 32 ? l0 : l1;
+        if (kg < l01) s = fma(a.a, x.a, s);
+        if (kg < l2) s2 = fma(b.a, y.a, s2);
+        if (kg + 32 < l01) s = fma(a.b, x.b, s);
+        if (kg + 32 < l2) s2 = fma(b.b, y.b, s2);
+      } else {  // s: rows 0, 1 and 2 in the first three 16 lanes
+        const Dbl2 a01 = swap16(a0, a1), a22 = swap16(a2, a2), x01 = swap16(x0, x1), x22 = swap16(x2, x2);
+        const Dbl2 a = swap32(a01.a, a22.a), x = swap32(x01.a, x22.a);
+        const Dbl2 b = swap32(a01.b, a22.b), y = swap32(x01.b, x22.b);
+        const int l = lane < 16 ? l0 : (lane < 32 ? l1 : l2);
+        if (kg < l) s = fma(a.a, x.a, s);
+        if (kg + 16 < l) s = fma(b.a, y.a, s);
+        if (kg + 32 < l) s = fma(a.b, x.b, s);
+        if (kg + 48 < l) s = fma(b.b, y.b, s);
+      }
     }
-    s0 = wave_sum(s0);
-    s1 = wave_sum(s1);
-    s2 = wave_sum(s2);
-    if (lane < 3) {
-      const double s = lane == 0 ? s0 : (lane == 1 ? s1 : s2);
-      q[3 * u + lane] = s;
-      pq += pu * s;
+    s = group_sum<G>(s);
+    if constexpr (G == 32) {
+      s2 = group_sum<G>(s2);
+      if (lane == 0 || lane == 32) q[3 * u + (lane >> 5)] = s;
+      if (lane == 1) q[3 * u + 2] = s2;
+    } else {
+      if (lane % 16 == 0 && lane < 48) q[3 * u + (lane >> 4)] = s;
     }
     cur = nxt;
   }
-  pq = block_sum(pq, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = pq;
+}
+
+// partials of p.q, apart from the product, whose blocks hold the rows in another
+// order than the one the sum is taken in: 4.8 us at 367,000 rows, q still in the
+// caches; in the product (another order of the sum) it came free
+__global__ __launch_bounds__(kRedThreads) void k_cg_dot(int64_t n, const double *__restrict__ p,
+                                                        const double *__restrict__ q,
+                                                        const CgScal *__restrict__ sc,
+                                                        double *__restrict__ part) {
+  __shared__ double sh[kRedThreads];
+  if (sc->done) return;
+  double s = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRedThreads)
+    s += p[i] * q[i];
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // alpha = r.z / p.q; x += alpha p, r -= alpha q, z = M^-1 r; partials of r.z and r.r
@@ -511,7 +557,7 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_update(int64_t nu, CgScal *_
                                                            const double *__restrict__ minv,
                                                            double *__restrict__ x, double *__restrict__ r,
                                                            double *__restrict__ z, double *__restrict__ part) {
-  __shared__ double sh[kRedThreads / 64];
+  __shared__ double sh[kRedThreads];
   if (sc->done) return;
   const double pq = partials_sum(ppart, np, sh), alpha = pq != 0.0 ? sc->rz / pq : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->pq = pq;  // for the next launch; none of this one reads it
@@ -539,7 +585,7 @@ __global__ __launch_bounds__(kRedThreads) void k_cg_direction(int64_t n, const C
                                                               const double *__restrict__ part, int np, double rtol,
                                                               const double *__restrict__ z, double *__restrict__ p,
                                                               CgScal *__restrict__ next) {
-  __shared__ double sh[kRedThreads / 64];
+  __shared__ double sh[kRedThreads];
   if (sc->done) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *next = *sc;
     return;
@@ -675,7 +721,7 @@ hipError_t csr_to_csc(hipStream_t s, int64_t n, int64_t nnz, int bits, const int
 // preconditioner storage (3 n: room for the 3x3 blocks) + r, z, p, q +
 // partials + scalars, then the full nodes' lists (an int per 9 entries)
 static size_t cg_vector_doubles(int64_t n) {
-  return 7 * (size_t)n + 3 * kRedBlocks + kMaxProdBlocks + 2 * sizeof(CgScal) / sizeof(double);
+  return 7 * (size_t)n + 4 * kRedBlocks + 2 * sizeof(CgScal) / sizeof(double);
 }
 size_t cg_workspace_doubles(int64_t n, int64_t nnz) { return cg_vector_doubles(n) + (size_t)nnz / 18 + 2; }
 
@@ -922,20 +968,22 @@ static int cg_prod_blocks(int64_t nu, int per, int64_t &chunk) {
 
 static hipError_t cg_product(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
                              const double *vals, const uint16_t *nslots, const int32_t *nodes, const double *p,
-                             double *q, const CgScal *sc, double *part, int *nblocks, bool back) {
+                             double *q, const CgScal *sc, bool back) {
   int64_t chunk;
-  if (nslots) {
-    *nblocks = cg_prod_blocks(n / 3, kRedThreads / 64, chunk);
-    k_cg_spmv3<<<(unsigned)*nblocks, kRedThreads, 0, s>>>(n / 3, chunk, indptr, indices, vals, nslots, nodes, p, q, sc,
-                                                          part, back);
+  const double mean = (double)nnz / (double)n;  // the bounds of launch_spmv
+  // a wavefront per node where a tile of its row has at least 24 of 64 columns
+  // (one cube of P1 elements has less); 16 or 32 lanes a sum, as launch_spmv
+  if (nslots && mean > 24) {
+    const int nblocks = cg_prod_blocks(n / 3, kRedThreads / 64, chunk);
+    auto k = mean > 64 ? k_cg_spmv3<32> : k_cg_spmv3<16>;
+    k<<<(unsigned)nblocks, kRedThreads, 0, s>>>(n / 3, chunk, indptr, indices, vals, nslots, nodes, p, q, sc, back);
     return hipGetLastError();
   }
   auto run = [&](auto g) {
     constexpr int G = decltype(g)::value;
-    *nblocks = cg_prod_blocks(n, kRedThreads / G, chunk);
-    k_cg_spmv<G><<<(unsigned)*nblocks, kRedThreads, 0, s>>>(n, chunk, indptr, indices, vals, p, q, sc, part);
+    const int nblocks = cg_prod_blocks(n, kRedThreads / G, chunk);
+    k_cg_spmv<G><<<(unsigned)nblocks, kRedThreads, 0, s>>>(n, chunk, indptr, indices, vals, p, q, sc);
   };
-  const double mean = (double)nnz / (double)n;  // as launch_spmv
   if (mean <= 12) run(std::integral_constant<int, 4>{});
   else if (mean <= 24) run(std::integral_constant<int, 8>{});
   else if (mean <= 64) run(std::integral_constant<int, 16>{});
@@ -950,7 +998,7 @@ static hipError_t cg_iterations(hipStream_t s, int64_t n, int64_t nnz, const int
                                 double *x, double rtol, int maxit, double *work, CgScal *h) {
   double *minv = work, *r = work + 3 * n, *z = work + 4 * n, *p = work + 5 * n, *q = work + 6 * n;
   double *part = work + 7 * n, *ppart = part + 3 * kRedBlocks;
-  CgScal *sc = reinterpret_cast<CgScal *>(ppart + kMaxProdBlocks);
+  CgScal *sc = reinterpret_cast<CgScal *>(ppart + kRedBlocks);
   const int64_t nu = n / QB;
   const int nb = (int)std::min<int64_t>(kRedBlocks, (nu + kRedThreads - 1) / kRedThreads);
   const int nd = (int)std::min<int64_t>(kRedBlocks, (n + kRedThreads - 1) / kRedThreads);
@@ -964,11 +1012,9 @@ static hipError_t cg_iterations(hipStream_t s, int64_t n, int64_t nnz, const int
     const int end = std::min(maxit, it + batch);
     for (; it < end; ++it) {
       CgScal *cur = sc + (it & 1), *next = sc + (~it & 1);
-      int np = 0;
-      if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, p, q, cur, ppart, &np, it & 1)) !=
-          hipSuccess)
-        return e;
-      k_cg_update<QB><<<nb, kRedThreads, 0, s>>>(nu, cur, ppart, np, p, q, minv, x, r, z, part);
+      if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, p, q, cur, it & 1)) != hipSuccess) return e;
+      k_cg_dot<<<nd, kRedThreads, 0, s>>>(n, p, q, cur, ppart);
+      k_cg_update<QB><<<nb, kRedThreads, 0, s>>>(nu, cur, ppart, nd, p, q, minv, x, r, z, part);
       k_cg_direction<<<nd, kRedThreads, 0, s>>>(n, cur, part, nb, rtol, z, p, next);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
@@ -994,10 +1040,7 @@ hipError_t cg_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr
   else k_inv_diag<<<nb256(n), 256, 0, s>>>(n, indptr, indices, vals, minv);
   if (qb != 3) nslots = nullptr;
   if (nslots) k_cg_nodes<<<nb256(8 * nu), 256, 0, s>>>(nu, nslots, indptr, indices, nodes);
-  int np = 0;
-  if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, x, r, nullptr, work + 7 * n, &np, false)) !=
-      hipSuccess)
-    return e;
+  if ((e = cg_product(s, n, nnz, indptr, indices, vals, nslots, nodes, x, r, nullptr, false)) != hipSuccess) return e;
   CgScal h{};
   e = qb == 3 ? cg_iterations<3>(s, n, nnz, indptr, indices, vals, nslots, nodes, b, x, rtol, maxit, work, &h)
               : cg_iterations<1>(s, n, nnz, indptr, indices, vals, nslots, nodes, b, x, rtol, maxit, work, &h);
