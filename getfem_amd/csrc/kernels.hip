@@ -318,7 +318,9 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
   const uint64_t *sg = sig + g * (NP * NV);
   // CHECK: the smallest of the entries whose stored bit is set, the largest of
   // the others (mn > thr and md <= thr: the bits are the stored ones), and
-  // whether every value is finite, where both say what the bits would
+  // whether every value is finite, where both say what the bits would; mn stays
+  // infinite where no bit is set (an all-zero element, whose threshold is
+  // infinite too)
   const uint64_t full = nblk == kWave ? ~0ull : (1ull << nblk) - 1ull;
   double mx = 0.0, mn = INFINITY, md = 0.0, fin = 0.0;
   for (int p = w; p < NP; p += kKeepWaves) {
@@ -353,7 +355,7 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
   bool pass2 = true;
   if constexpr (CHECK) {
     pass2 = __ballot(fin != 0.0) != 0;  // not a number: the bits themselves are compared
-    diff = __ballot(lane < nblk && !(mn > thr && md <= thr));
+    diff = __ballot(lane < nblk && !((mn > thr || mn == INFINITY) && md <= thr));
   }
   if (CHECK && pass2) diff = 0;
   for (int p = pass2 ? w : NP; p < NP; p += kKeepWaves) {

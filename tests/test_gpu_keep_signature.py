@@ -84,3 +84,34 @@ def test_new_coefficients(ctx, name, n):
     del views
     assemble(c1)
     equal(plan, at(case, c1))
+
+
+@pytest.mark.parametrize("name", ["p1_laplace", "p1_elast", "p2_elast", "p3_laplace"])
+@pytest.mark.parametrize("n", [1, 2, 3])  # 6, 48 and 162 elements: groups of 64 that are and are not full
+def test_void_elements_are_confirmed(ctx, name, n):
+    """New coefficients with the same void elements (all of them 0): the check
+    finds the stored bits again and nothing of the pattern is formed anew."""
+    from tests.launches import kernels
+    print("case: keep signature, void elements", name, n, flush=True)
+    k, q, term = CASES[name]
+    case = problems.Case(n, k, q, IM[k], term)
+    n_cv = case.cvx.shape[0]
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", case.pts, case.cvx)
+    c0, c1 = coefs(n_cv, q, 1), coefs(n_cv, q, 2)
+    for v in c0 + c1:
+        v[0] = v[-1] = 0.0
+        v[64:128] = 0.0  # (at 162 elements) a whole group
+    plan = ga.Plan(ga.MeshFem(mesh, case.fem, q), ga.MeshIm(mesh, IM[k]),
+                   ga.TERM_ISO_ELAST if q == 3 else ga.TERM_LAPLACE, c0)
+    plan.build_pattern()
+    plan.assemble()
+
+    def assemble():
+        for s, v in enumerate(c1):
+            plan.set_coef(s, v)
+        plan.assemble()
+
+    ran = kernels(assemble)
+    equal(plan, at(case, c1))
+    assert sum("k_keep<" in x for x in ran) == 1, ran
+    assert not any("k_keep_words" in x or "k_mask" in x for x in ran), ran
