@@ -1050,7 +1050,7 @@ static int plan_validate(gfx_plan *p, bool *fresh) {
   const gfx_mesh *m = p->mf->mesh;
   hipStream_t s = c->stream;
   *fresh = false;
-  if (p->nnz == 0) {  // no element: nothing to re-derive
+  if (m->n_cv == 0 || p->n_nodes == 0) {  // no element: nothing to re-derive
     p->pts_version = m->version;
     p->values_changed = false;
     return GFX_OK;

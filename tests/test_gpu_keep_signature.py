@@ -115,3 +115,24 @@ def test_void_elements_are_confirmed(ctx, name, n):
     equal(plan, at(case, c1))
     assert sum("k_keep<" in x for x in ran) == 1, ran
     assert not any("k_keep_words" in x or "k_mask" in x for x in ran), ran
+
+
+@pytest.mark.parametrize("name", ["p1_laplace", "p2_elast"])
+def test_a_body_without_material(ctx, name):
+    """A plan built where every coefficient is 0 has no entries; coefficients
+    given later bring them."""
+    print("case: keep signature, no material", name, flush=True)
+    k, q, term = CASES[name]
+    case = problems.Case(2, k, q, IM[k], term)
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", case.pts, case.cvx)
+    c = coefs(case.cvx.shape[0], q, 1)
+    plan = ga.Plan(ga.MeshFem(mesh, case.fem, q), ga.MeshIm(mesh, IM[k]),
+                   ga.TERM_ISO_ELAST if q == 3 else ga.TERM_LAPLACE, [0.0 * v for v in c])
+    plan.build_pattern()
+    plan.assemble()
+    assert plan.csr()[1].size == 0
+    for _ in range(2):
+        for s, v in enumerate(c):
+            plan.set_coef(s, v)
+        plan.assemble()
+        equal(plan, at(case, c))
