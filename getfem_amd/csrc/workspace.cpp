@@ -950,7 +950,10 @@ int sc_matrix(gfx_workspace *w) {
     WHIP(w, launch_poly_runs(s, sc->n_ent, sc->d_start, sc->d_src, sc->d_pelem, sc->d_place, sc->d_v, sc->d_err));
     WHIP(w, hipMemcpyAsync(&flag, sc->d_err, 4, hipMemcpyDeviceToHost, s));
     WHIP(w, hipStreamSynchronize(s));
-    if (flag & 1) return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
+    if (flag & 1) {
+      sc->nnz = -1;  // the sums so far, over the last matrix's values, are no matrix
+      return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
+    }
     if (sc->nnz >= 0 && !(flag & 4)) return GFX_OK;
     sc->nnz = -1;
     Scratch t;
@@ -1004,6 +1007,7 @@ int sc_sorted_matrix(gfx_workspace *w, int64_t total) {
     if (hipMalloc(&sc->d_sort, sb) != hipSuccess) return wfail(w, GFX_E_OOM, "order-2 route sort");
     sc->sort_cap = sb;
   }
+  sc->nnz = -1;  // the last matrix is written over
   WHIP(w, poly_to_csr(s, sc->d_sort, sc->sort_cap, sc->d_keys, sc->d_vals, sc->d_keys2, sc->d_vals2, total,
                       end_bit, n, n, sc->d_work, sc->d_ip, sc->d_ix, sc->d_v, sc->d_nnz));
   int flag = 0;
@@ -1118,6 +1122,7 @@ int sc_run(gfx_workspace *w, int order) {
     w->has_potential = true;
     return GFX_OK;
   }
+  w->V_out = nullptr;  // the last vector is written over
   WHIP(w, launch_fill_f64(s, sc->nvec, sc->d_V, 0.0));
   for (auto &v : sc->vars) {
     if (v.p.nm == 0) continue;

@@ -1,0 +1,57 @@
+"""Assemblies on the polynomial route that fail: the results of the last good
+one are not handed out under the failed one's name, the next good assembly
+gives what a new workspace gives, and nothing is left running."""
+import numpy as np
+import pytest
+
+import getfem_amd as ga
+from getfem_amd import meshes
+from getfem_amd.workspace import GaWorkspace
+
+pytestmark = pytest.mark.gpu
+
+MESH = {"tets": ("GT_PK(3,1)", "FEM_PK(3,2)", "FEM_PK(3,1)", "IM_TETRAHEDRON(5)"),
+        "hexes": ("GT_QK(3,1)", "FEM_QK(3,1)", "FEM_QK(3,1)", "IM_GAUSS_PARALLELEPIPED(3,3)")}
+EXPR = {"constant": "2*mu*Sym(Grad_u):Grad_Test_u - p*Div_Test_u - Test_p*Div_u - p*Test_p",
+        "field": "(1+p*p)*Grad_u:Grad_Test_u + mu*p*p*p*Test_p"}
+
+
+def model(ctx, kind, expr):
+    gt, fu, fp, im = MESH[kind]
+    pts, cvx = meshes.regular_unit_mesh(2, gt)
+    pts = meshes.jitter(pts, 2)
+    mesh = ga.Mesh(ctx, gt, pts, cvx)
+    mfu, mfp = ga.MeshFem(mesh, fu, 3), ga.MeshFem(mesh, fp, 1)
+    rng = np.random.default_rng(1)
+    ws = GaWorkspace(ctx)
+    ws.add_fem_variable("u", mfu, rng.standard_normal(mfu.nbdof()), first=0)
+    ws.add_fem_variable("p", mfp, rng.uniform(0.5, 1.5, mfp.nbdof()), first=mfu.nbdof())
+    ws.add_fixed_size_constant("mu", 0.8)
+    ws.add_expression(EXPR[expr], ga.MeshIm(mesh, im))
+    return ws, mesh, pts, cvx
+
+
+@pytest.mark.parametrize("kind", sorted(MESH))
+@pytest.mark.parametrize("expr", sorted(EXPR))
+def test_degenerate_element(ctx, kind, expr):
+    print("case: failed assembly", kind, expr, flush=True)
+    ws, mesh, pts, cvx = model(ctx, kind, expr)
+    ws.assembly(2)
+    ws.assembly(1)
+    good = ws.assembled_matrix_csr() + (ws.assembled_vector(),)
+    flat = pts.copy()
+    flat[cvx[3]] = flat[cvx[3][0]]
+    mesh.set_points(flat)
+    for _ in range(2):
+        for order in (2, 1):
+            with pytest.raises(ga.GfxError, match="degenerate"):
+                ws.assembly(order)
+        with pytest.raises(ga.GfxError, match="no matrix assembled"):
+            ws.assembled_matrix_csr()
+        with pytest.raises(ga.GfxError, match="no order-1 assembly"):
+            ws.assembled_vector()
+    mesh.set_points(pts)
+    ws.assembly(2)
+    ws.assembly(1)
+    for a, b in zip(ws.assembled_matrix_csr() + (ws.assembled_vector(),), good):
+        assert np.array_equal(a, b)
