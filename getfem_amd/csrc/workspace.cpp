@@ -290,8 +290,14 @@ int bind_coefs(gfx_workspace *w, const GwflKernelParams &params, int64_t n_cv, s
   return GFX_OK;
 }
 
+// the assembled vector goes with the buffer p that is about to be freed
+void drop_vector(gfx_workspace *w, const double *p) {
+  if (w->V_out == p) w->V_out = nullptr;
+}
+
 void drop_plans(gfx_workspace *w) {
   for (auto &t : w->trees) {
+    if (t.plan) drop_vector(w, t.plan->d_rhs);
     if (t.plan) gfx_plan_destroy(t.plan);
     if (t.plan1) gfx_plan_destroy(t.plan1);
     wfree(t.d_map);
@@ -474,6 +480,7 @@ int setup(gfx_workspace *w) {
   }
   if (w->ndof != u.mf->ndof || !w->d_u) {
     if (hipSetDevice(w->ctx->device) != hipSuccess) return wfail(w, GFX_E_HIP, "hipSetDevice");
+    drop_vector(w, w->d_V);
     wfree(w->d_u); wfree(w->d_V);
     const size_t bytes = 8 * (size_t)std::max<int64_t>(u.mf->ndof, 1);
     if (hipMalloc((void **)&w->d_u, bytes) != hipSuccess || hipMalloc((void **)&w->d_V, bytes) != hipSuccess)
@@ -540,6 +547,7 @@ int sc_build(gfx_workspace *w) {
   ScalarRoute *sc = w->sc;
   if (sc->version == w->version)
     return sc->err_code == GFX_OK ? GFX_OK : wfail(w, sc->err_code, sc->err);
+  drop_vector(w, sc->d_V);
   sc_release(sc);
   sc->version = w->version;
   sc->err_code = GFX_OK;

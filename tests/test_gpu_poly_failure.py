@@ -55,3 +55,17 @@ def test_degenerate_element(ctx, kind, expr):
     ws.assembly(1)
     for a, b in zip(ws.assembled_matrix_csr() + (ws.assembled_vector(),), good):
         assert np.array_equal(a, b)
+
+
+def test_vector_of_an_earlier_setup(ctx):
+    """A vector whose buffer was given back with the setup that it came from
+    is not handed out any more."""
+    print("case: vector of an earlier setup", flush=True)
+    ws, mesh, _, _ = model(ctx, "tets", "constant")
+    ws.assembly(1)
+    ws.assembled_vector()
+    ws.add_expression("p*Test_p", ga.MeshIm(mesh, "IM_TETRAHEDRON(5)"))
+    with pytest.raises(ga.GfxError):  # (two mesh_ims: refused after the setup was dropped)
+        ws.assembly(1)
+    with pytest.raises(ga.GfxError, match="no order-1 assembly"):
+        ws.assembled_vector()
