@@ -832,10 +832,17 @@ int sc_upload(gfx_workspace *w) {
     if (e != hipSuccess) sc->h_consts.clear();
     WHIP(w, e);
   }
-  // the host buffers above are read before they can change: every assembly
-  // ends with a synchronisation of the stream
+  // (the copies read the host buffers before these can change: sc_ended)
   WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
   return GFX_OK;
+}
+
+// What follows sc_upload ends with a wait for the stream: by itself where it
+// succeeds, here where it does not.  The copies from the variables' host
+// values, which the caller may write next, are over then.
+int sc_ended(gfx_workspace *w, int r) {
+  if (r != GFX_OK) (void)hipStreamSynchronize(w->ctx->stream);
+  return r;
 }
 
 int sc_grow(gfx_workspace *w, int64_t need) {
@@ -1028,20 +1035,13 @@ int sc_sorted_matrix(gfx_workspace *w, int64_t total) {
   return GFX_OK;
 }
 
-// assembly(2) on the polynomial route: every block's element matrices, then
-// the nvec x nvec matrix (tested dofs x trial dofs at the variables'
-// intervals) from their entries above the element threshold
-int sc_run2(gfx_workspace *w) {
-  if (!w->sc) w->sc = new (std::nothrow) ScalarRoute();
-  if (!w->sc) return wfail(w, GFX_E_OOM, "workspace");
-  int r;
-  if ((r = sc_build(w))) return r;
+// every block's element matrices, then the matrix from their entries above
+// the element threshold
+int sc_assemble2(gfx_workspace *w) {
   ScalarRoute *sc = w->sc;
-  if (!sc->err2.empty()) return wfail(w, GFX_E_UNSUPPORTED, sc->err2);
   gfx_mesh *m = sc->mim->mesh;
   hipStream_t s = w->ctx->stream;
-  for (auto &b : sc->blocks)
-    if (!sc_zero_ok(w, b.p.prog)) return GFX_E_UNSUPPORTED;
+  int r;
   if ((r = sc_upload(w))) return r;
   const int64_t n = sc->nvec;
   if (n > INT32_MAX) return wfail(w, GFX_E_UNSUPPORTED, "more than 2^31 dofs");
@@ -1085,20 +1085,25 @@ int sc_run2(gfx_workspace *w) {
   return GFX_OK;
 }
 
-// assembly(0): the potential; assembly(1): the vector of every fem variable's
-// derivative, at the variable's interval (first .. first + nb_dof)
-int sc_run(gfx_workspace *w, int order) {
+// assembly(2) on the polynomial route: the nvec x nvec matrix (tested dofs x
+// trial dofs at the variables' intervals)
+int sc_run2(gfx_workspace *w) {
   if (!w->sc) w->sc = new (std::nothrow) ScalarRoute();
   if (!w->sc) return wfail(w, GFX_E_OOM, "workspace");
   int r;
   if ((r = sc_build(w))) return r;
   ScalarRoute *sc = w->sc;
+  if (!sc->err2.empty()) return wfail(w, GFX_E_UNSUPPORTED, sc->err2);
+  for (auto &b : sc->blocks)
+    if (!sc_zero_ok(w, b.p.prog)) return GFX_E_UNSUPPORTED;
+  return sc_ended(w, sc_assemble2(w));
+}
+
+int sc_assemble(gfx_workspace *w, int order) {
+  ScalarRoute *sc = w->sc;
   gfx_mesh *m = sc->mim->mesh;
   hipStream_t s = w->ctx->stream;
-  if (order == 0 && !sc_zero_ok(w, sc->p0.prog)) return GFX_E_UNSUPPORTED;
-  if (order == 1)
-    for (auto &v : sc->vars)
-      if (!sc_zero_ok(w, v.p.prog)) return GFX_E_UNSUPPORTED;
+  int r;
   if ((r = sc_upload(w))) return r;
   ScalarArgs a{};
   a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx; a.nv = m->nv; a.gN = sc->d_gN;
@@ -1147,6 +1152,21 @@ int sc_run(gfx_workspace *w, int order) {
   w->V_out = sc->d_V;
   w->vec_n = sc->nvec;
   return GFX_OK;
+}
+
+// assembly(0): the potential; assembly(1): the vector of every fem variable's
+// derivative, at the variable's interval (first .. first + nb_dof)
+int sc_run(gfx_workspace *w, int order) {
+  if (!w->sc) w->sc = new (std::nothrow) ScalarRoute();
+  if (!w->sc) return wfail(w, GFX_E_OOM, "workspace");
+  int r;
+  if ((r = sc_build(w))) return r;
+  ScalarRoute *sc = w->sc;
+  if (order == 0 && !sc_zero_ok(w, sc->p0.prog)) return GFX_E_UNSUPPORTED;
+  if (order == 1)
+    for (auto &v : sc->vars)
+      if (!sc_zero_ok(w, v.p.prog)) return GFX_E_UNSUPPORTED;
+  return sc_ended(w, sc_assemble(w, order));
 }
 
 }  // namespace

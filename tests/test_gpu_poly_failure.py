@@ -69,3 +69,31 @@ def test_vector_of_an_earlier_setup(ctx):
         ws.assembly(1)
     with pytest.raises(ga.GfxError, match="no order-1 assembly"):
         ws.assembled_vector()
+
+
+def test_refusal_waits_for_its_uploads():
+    """An assembly that is refused after the variables' values went on their
+    way (here: more than 2^31 dofs) returns when the stream has ended."""
+    import torch
+    print("case: refusal behind a busy stream", flush=True)
+    c = ga.Context(0)
+    side = torch.cuda.Stream()
+    c.set_stream(side.cuda_stream)
+    pts, cvx = meshes.regular_unit_mesh(2)
+    mesh = ga.Mesh(c, "GT_PK(3,1)", pts, cvx)
+    mfu, mfp = ga.MeshFem(mesh, "FEM_PK(3,2)", 3), ga.MeshFem(mesh, "FEM_PK(3,1)", 1)
+    ws = GaWorkspace(c)
+    ws.add_fem_variable("u", mfu, np.ones(mfu.nbdof()), first=0)
+    ws.add_fem_variable("p", mfp, np.ones(mfp.nbdof()), first=2**31)
+    ws.add_expression("u.Test_u + p*Test_p", ga.MeshIm(mesh, "IM_TETRAHEDRON(5)"))
+    with pytest.raises(ga.GfxError, match="dofs"):  # (the setup's own waits are over)
+        ws.assembly(2)
+    x = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(200):
+            x = torch.clamp(x @ x, -1, 1)
+    busy = not side.query()
+    with pytest.raises(ga.GfxError, match="dofs"):
+        ws.assembly(2)
+    assert busy and side.query()
