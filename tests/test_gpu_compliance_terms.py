@@ -62,3 +62,37 @@ def test_against_autograd(ctx, n, penal):
             op.check()
             side.synchronize()
             assert torch.equal(out[1 + k], got[k]) and torch.equal(J1, J.detach())
+
+
+@pytest.mark.parametrize("penal", [2.0, 3.0, 5.0, 8.0])
+def test_whole_exponents_are_correctly_rounded(ctx, penal):
+    """dJ/drho of unit tetrahedra under a unit strain is p rho^(p-1) w: the
+    power (within half an ulp, 2^-53 relative, and terms of its square) and one
+    product with w may round, p = 2, 3, 5 and 8 by a third."""
+    from fractions import Fraction
+
+    import torch
+
+    from getfem_amd.torch_ops import Compliance
+    print("case: compliance exponent", penal, flush=True)
+    n = 1500
+    unit = np.array([[0.0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
+    pts = (unit[None] + 2.0 * np.arange(n)[:, None, None]).reshape(-1, 3)
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", pts, np.arange(4 * n, dtype=np.int32).reshape(n, 4))
+    mf = ga.MeshFem(mesh, "FEM_PK(3,1)", 3)
+    mim = ga.MeshIm(mesh, "IM_TETRAHEDRON(1)")
+    op = Compliance(mf, mim, 0.0, 0.5, 0.0, penal)  # 2 mu = 1: W = 1
+    u = np.zeros(mf.nbdof())
+    u[0::3] = mf.basic_dof_nodes()[:, 0] % 2.0  # the first coordinate in the element
+    rho = np.random.default_rng(int(penal)).uniform(0.05, 1.0, n)
+    out = [torch.empty((), dtype=torch.float64, device="cuda"), torch.empty(n, dtype=torch.float64, device="cuda"),
+           None, None]
+    dev = [torch.tensor(a, device="cuda") for a in (rho, pts, u)]
+    torch.cuda.synchronize()
+    op.eval(*dev, out=tuple(out))
+    op.check()
+    w = Fraction(float(mim.points()[1].sum()))
+    p = int(penal)
+    worst = max(abs(Fraction(float(g)) / (p * Fraction(float(r)) ** (p - 1) * w) - 1)
+                for g, r in zip(out[1].cpu().numpy(), rho))
+    assert float(worst) <= 3.1 * 2.0 ** -53
