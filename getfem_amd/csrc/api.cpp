@@ -431,9 +431,15 @@ static int plan_upload_coef(gfx_plan *p, int slot, const gfx_coef *cf) {
   p->coef[slot].h_values = nullptr;
   if (cf->kind == GFX_COEF_PER_ELEMENT) {
     // into the buffer that the slot has (an allocation and a free each time
-    // would wait for the device twice), after the assemblies that read it
+    // would wait for the device twice), after the assemblies that read it: by
+    // the stream's order, or by a wait where they ran on other streams
     const size_t n = (size_t)p->mf->mesh->n_cv;
     if (!p->d_coef[slot]) HIPCHK(c, dalloc(&p->d_coef[slot], n));
+    if (p->coef_streams || (p->coef_stream && p->coef_stream != c->stream)) {
+      HIPCHK(c, hipDeviceSynchronize());
+      p->coef_stream = nullptr;
+      p->coef_streams = false;
+    }
     HIPCHK(c, hipMemcpyAsync(p->d_coef[slot], cf->h_values, 8 * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
@@ -675,8 +681,16 @@ int gfx_plan_set_form(gfx_plan *p, int form, int precision) {
   return GFX_OK;
 }
 
+// the context's stream is about to read the coefficient buffers
+static void coefs_read(gfx_plan *p) {
+  hipStream_t s = p->ctx->stream;
+  p->coef_streams |= p->coef_stream && p->coef_stream != s;
+  p->coef_stream = s;
+}
+
 static RecordArgs record_args(gfx_plan *p) {
   const gfx_mesh *m = p->mf->mesh;
+  coefs_read(p);
   // coefficient c of the record: mu for elasticity (its Laplacian part), the
   // third coefficient of the isotropic term, none for the Laplacian
   const int sc = p->term == GFX_TERM_ISOTROPIC ? 2 : (p->term == GFX_TERM_ISO_ELAST ? 1 : -1);
@@ -723,6 +737,7 @@ static int plan_keep(gfx_plan *p, bool check) {
 
 static EbArgs eb_args(gfx_plan *p) {
   const gfx_mesh *m = p->mf->mesh;
+  coefs_read(p);
   EbArgs a{};
   a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx; a.dofs = p->mf->d_dofs; a.U = p->d_U;
   a.ca = p->coef[0].kind == GFX_COEF_PER_ELEMENT ? p->d_coef[0] : nullptr;

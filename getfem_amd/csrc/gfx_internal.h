@@ -490,6 +490,10 @@ struct gfx_plan {
   double coef_min[3] = {0.0, 0.0, 0.0};  // smallest value of each coefficient, where min_known
   bool min_known[3] = {false, false, false};
   double *d_coef[3] = {nullptr, nullptr, nullptr};
+  // the stream that last read them, and whether another one did before it
+  // (since they were last known to be idle)
+  hipStream_t coef_stream = nullptr;
+  bool coef_streams = false;
   // The stored pattern is GetFEM's for the values it was built from.  After
   // the coefficients, the node positions (mesh version) or the state change,
   // the next assembly re-derives the thresholds and keep bits and rebuilds

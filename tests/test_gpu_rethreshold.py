@@ -256,3 +256,37 @@ def test_compliance_degenerate_coordinates_reported(ctx):
     J = compliance(rho, None, u, op)  # the flag was cleared; the mesh's own points are fine
     J.backward()
     assert torch.isfinite(rho.grad).all()
+
+
+def test_new_coefficients_wait_for_assemblies_on_other_streams():
+    """An assembly queued on one stream reads the coefficients that were set
+    before it, also where the context has gone over to another stream by the
+    time that new ones are set."""
+    import torch
+    print("case: coefficients behind another stream's assembly", flush=True)
+    c = ga.Context(0)
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    pts, cvx = meshes.regular_unit_mesh(4)
+    mesh = ga.Mesh(c, "GT_PK(3,1)", pts, cvx)
+    lam, mu = meshes.lognormal_lame(cvx.shape[0])
+    mf, mim = ga.MeshFem(mesh, "FEM_PK(3,2)", 3), ga.MeshIm(mesh, "IM_TETRAHEDRON(5)")
+    c.set_stream(one.cuda_stream)
+    plan = ga.Plan(mf, mim, ga.TERM_ISO_ELAST, [lam, mu])
+    plan.build_pattern()
+    plan.assemble()
+    old = plan.csr()[2]
+    x = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(one):
+        for _ in range(200):
+            x = torch.clamp(x @ x, -1, 1)
+    plan.assemble()  # behind the products
+    busy = not one.query()
+    c.set_stream(two.cuda_stream)
+    plan.set_coef(0, 2.0 * lam)
+    plan.set_coef(1, 2.0 * mu)
+    torch.cuda.synchronize()
+    assert busy
+    assert np.array_equal(plan.csr()[2], old)
+    plan.assemble()
+    assert np.array_equal(plan.csr()[2], 2.0 * old)
