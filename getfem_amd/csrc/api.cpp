@@ -1144,7 +1144,8 @@ int gfx_plan_assemble(gfx_plan *p) {
     p->n_timed++;
     HIPCHK(c, hipEventRecord(ev[0], c->stream));
   }
-  const bool fused = !p->eb && !fresh && fused_records(p->nd, p->qdim, p->form, p->precision, p->mf->mesh->n_cv);
+  const bool fused = !p->eb && !fresh &&
+                     fused_records(p->term, p->nd, p->qdim, p->form, p->precision, p->mf->mesh->n_cv);
   if (!p->eb) {
     if (!fresh && !fused && (r = plan_records(p))) return r;
   } else if (!fresh || p->precision != GFX_PREC_FP64) {

@@ -336,7 +336,7 @@ hipError_t launch_mask_exact(hipStream_t s, const PatternArgs &a, int max_nslots
 hipError_t launch_fill_desc(hipStream_t s, int64_t n, int qdim, const int32_t *order, const int32_t *inc_ptr,
                             const uint16_t *nslots, const int64_t *indptr, PatchDesc *desc);
 // whether an assembly leaves the records to the patch kernel
-bool fused_records(int nd, int qdim, int form, int prec, int64_t n_cv);
+bool fused_records(int term, int nd, int qdim, int form, int prec, int64_t n_cv);
 hipError_t launch_assemble_patch(hipStream_t s, int term, int form, int prec, const PatchArgs &a);
 hipError_t scan_exclusive_i64(hipStream_t s, const int64_t *in, int64_t *out,
                               int64_t n, int64_t *tmp);

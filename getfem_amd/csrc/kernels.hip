@@ -1077,15 +1077,26 @@ hipError_t launch_fill_columns(hipStream_t s, const PatternArgs &a) {
 
 // P1 elements: a lane's record is a row of loads and some 250 instructions for
 // the one pair block it is used for, against a launch, the records' way through
-// memory and a round trip.  Vector fields gain at every size (FP64 elasticity:
-// 384 elements 9.3 -> 7.8 us, 48,000 21.5 -> 17.8, 3.07 M 692 -> 645), scalar
-// ones, with less to do per record, up to where the launch no longer counts
-// (FP64 Poisson: 384 elements 8.4 -> 6.9 us, 48,000 15.0 -> 13.7, 131,712 29.0
-// -> 28.5, 279,936 43.6 -> 50.0; FP32, whose records are half as long: 24,576
-// 10.0 -> 9.6, 48,000 12.1 -> 12.7).
-bool fused_records(int nd, int qdim, int form, int prec, int64_t n_cv) {
+// memory and a round trip.  It pays as long as the launch counts and, the more
+// the lane does with its record, the less long; FP32 records are half as long.
+// The lines lie at the last size that gained beyond the spread (1 %).
+// One plan, a pass after another, records kernel -> lanes, in us:
+//   elements            384     48,000    1.57 M    2.24 M    3.07 M    4.09 M
+//   scalar FP64      8.5-6.8  14.9-13.4
+//   Laplacian3 FP64 10.5-7.4  20.9-16.8   347-309   488-439   668-611   887-814
+//   Laplacian3 FP32 10.3-7.4  19.2-16.5   331-305   466-434   638-601   845-802
+//   elasticity FP64 10.6-7.9  21.6-18.7   361-348   508-492   693-687   920-925
+//   elasticity FP32 10.5-7.9  20.0-17.2   344-327   489-466   665-648   880-871
+//   isotropic FP64  10.7-7.9  21.7-18.0   361-357   510-503   695-715   921-960
+//   isotropic FP32  10.6-7.9  20.1-17.4   344-332   488-473   667-673   881-900
+// (scalar FP64 at 131,712 28.6-28.0 and FP32 at 29,478 10.9-9.8, at 48,000 12.4-12.3).
+bool fused_records(int term, int nd, int qdim, int form, int prec, int64_t n_cv) {
   if (nd != 4 || form != GFX_FORM_FACTORIZED || prec > GFX_PREC_FP32) return false;
-  return qdim > 1 || n_cv <= (prec == GFX_PREC_FP64 ? 131072 : 32768);
+  const bool d = prec == GFX_PREC_FP64;
+  if (qdim == 1) return n_cv <= (d ? 131072 : 32768);
+  if (term == GFX_TERM_LAPLACE) return true;
+  if (term == GFX_TERM_ISO_ELAST) return n_cv <= (d ? 2800000 : 3500000);
+  return n_cv <= (d ? 2000000 : 2400000);
 }
 
 template <int ND, int Q, int TERM>

@@ -36,3 +36,20 @@ def test_same_as_records(ctx, name, prec, n):
         plan.assemble()  # the same values again: from the lanes
         for a, b in zip(ref, plan.csr()):
             assert np.array_equal(a, b)
+
+
+def test_large_isotropic_plans_keep_the_records_kernel(ctx):
+    """Isotropic terms beyond some 2 M elements were faster with the records
+    kernel (three-component Laplacians are not)."""
+    from tests.launches import kernels
+    n = 71  # 2,147,466 elements
+    print("case: records of a large mesh", n, flush=True)
+    pts, cvx = meshes.regular_unit_mesh(n, "GT_PK(3,1)")
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", pts, cvx)
+    mf, mim = ga.MeshFem(mesh, "FEM_PK(3,1)", 3), ga.MeshIm(mesh, "IM_TETRAHEDRON(1)")
+    for term, coefs, records in ((ga.TERM_ISOTROPIC, [1.0, 0.5, 0.25], True), (ga.TERM_LAPLACE, [1.0], False)):
+        plan = ga.Plan(mf, mim, term, coefs)
+        plan.build_pattern()
+        plan.assemble()
+        assert any("k_records_tet" in k for k in kernels(plan.assemble)) == records
+        del plan
