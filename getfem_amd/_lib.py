@@ -105,6 +105,7 @@ SIGNATURES = {
     "gfx_ws_nb_trees": (_i32, [_P]),
     "gfx_ws_add_expression": (_i32, [_P, _cs, _P, _i32]),
     "gfx_ws_set_form": (_i32, [_P, _i32, _i32]),
+    "gfx_ws_set_structure_limit": (_i32, [_P, _i64]),
     "gfx_ws_compile": (_i32, [_P]),
     "gfx_ws_assembly": (_i32, [_P, _i32]),
     "gfx_ws_plan": (_i32, [_P, _pp]),

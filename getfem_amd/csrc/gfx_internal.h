@@ -292,7 +292,7 @@ hipError_t poly_pattern(hipStream_t s, int64_t n, const uint32_t *start, const u
                         const int32_t *row, const int32_t *col, int64_t nrows, int64_t *work, uint32_t *place,
                         int64_t *ip, int32_t *ix);
 hipError_t launch_poly_empty(hipStream_t s, int64_t nrows, int64_t *ip, int64_t *d_nnz);
-// beyond 2^31 candidates: entries above the threshold, counted and emitted
+// without the structure: entries above the threshold, counted and emitted
 hipError_t launch_poly_count(hipStream_t s, int64_t n_cv, int ne, const double *elem, int64_t *cnt);
 hipError_t launch_poly_emit(hipStream_t s, const PolyEmitArgs &a);
 // temporary storage of the stable key sort of n entries (bytes)

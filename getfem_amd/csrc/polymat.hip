@@ -24,8 +24,8 @@
 // assembly, and sees on the way whether the entries that have any candidate
 // are still the stored ones; only where they are not are the CSR's rows and
 // columns made anew (poly_pattern).
-// Beyond 2^31 candidates the kept entries are sorted at every assembly instead
-// (k_poly_emit, poly_to_csr).
+// Beyond 2^31 candidates, or the workspace's own limit, the kept entries are
+// sorted at every assembly instead (k_poly_emit, poly_to_csr).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(kPoly1d) void k_poly_places(int64_t n, const int64_
     for (int64_t rr = r + 1; rr <= nrows; ++rr) ip[rr] = pos[u] + stored[u];
 }
 
-// ------------------------------------------------- beyond 2^31 candidates
+// ------------------------------------------------- without the structure
 __global__ __launch_bounds__(kPm) void k_poly_count(int64_t n_cv, int ne, const double *__restrict__ elem,
                                                     int64_t *__restrict__ cnt) {
   const int64_t e = blockIdx.x;

@@ -122,16 +122,17 @@ struct ScalarRoute {
   // order 2 (polymat.hip): the blocks, or why they do not compile
   std::vector<ScBlock> blocks;
   std::string err2;
-  double *d_pelem = nullptr;    // element matrices: every block's, or one block's beyond 2^31 candidates
+  double *d_pelem = nullptr;    // element matrices: every block's, or one block's without the structure
   int64_t *d_nnz = nullptr;
   std::vector<double> h_consts;
   // The structure (polymat.hip): n_cand candidates of n_ent matrix entries;
-  // n_ent < 0: not built yet.
+  // n_ent < 0: not built yet.  Not kept beyond the workspace's limit.
   int64_t n_cand = 0, n_ent = -1;
+  bool structure = true;
   uint32_t *d_src = nullptr, *d_start = nullptr, *d_place = nullptr;
   int32_t *d_row = nullptr, *d_col = nullptr;
-  // beyond 2^31 candidates: kept entries (keys, values and their sorted
-  // copies), sort and run work
+  // without it: kept entries (keys, values and their sorted copies), sort and
+  // run work
   int64_t *d_cnt = nullptr, *d_off = nullptr, *d_scan = nullptr;
   int64_t cap = 0;
   uint64_t *d_keys = nullptr, *d_keys2 = nullptr;
@@ -170,6 +171,7 @@ struct gfx_workspace {
   // and tangents the matrix kernels do not cover (data fields, P0 or several
   // variables, blocks between mesh_fems, pulled-back coordinates, hexahedra)
   uint64_t version = 0;         // registrations and expressions; the route rebuilds on change
+  int64_t structure_limit = INT32_MAX;  // candidates up to which the polynomial route keeps its structure
   bool mat_fail = false;        // the order-2 compile failed at this version
   ScalarRoute *sc = nullptr;
   int64_t vec_n = 0;            // size of the last assembled vector
@@ -737,7 +739,7 @@ int sc_build(gfx_workspace *w) {
     if (upload(&b.p.d_mptr, mptr) != hipSuccess) return bail(GFX_E_OOM, "order-2 route programs");
     pelem = std::max(pelem, m->n_cv * b.ne);
   }
-  const bool structure = sc->n_cand <= INT32_MAX;
+  const bool structure = sc->structure = sc->n_cand <= w->structure_limit;
   if (structure) pelem = sc->n_cand;
   if (!sc->blocks.empty() &&
       (hipMalloc((void **)&sc->d_pelem, 8 * (size_t)std::max<int64_t>(pelem, 1)) != hipSuccess ||
@@ -987,7 +989,7 @@ int sc_matrix(gfx_workspace *w) {
   return GFX_OK;
 }
 
-// beyond 2^31 candidates: the kept entries of a block in element order
+// without the structure: the kept entries of a block in element order
 int sc_emit(gfx_workspace *w, const ScBlock &b, int64_t &total) {
   ScalarRoute *sc = w->sc;
   hipStream_t s = w->ctx->stream;
@@ -1050,7 +1052,7 @@ int sc_assemble2(gfx_workspace *w) {
         hipMalloc((void **)&sc->d_nnz, 8) != hipSuccess)
       return wfail(w, GFX_E_OOM, "order-2 route matrix");
   }
-  const bool structure = sc->n_cand <= INT32_MAX;
+  const bool structure = sc->structure;
   if (structure && sc->n_ent < 0 && (r = sc_structure(w))) return r;
   PolyMatArgs a{};
   a.n_cv = m->n_cv; a.pts = m->d_pts; a.cvx = m->d_cvx; a.nv = m->nv; a.gN = sc->d_gN;
@@ -1305,6 +1307,13 @@ int gfx_ws_set_form(gfx_workspace *w, int form, int precision) {
         int r = gfx_plan_set_form(p, form, precision);
         if (r) return r;
       }
+  return GFX_OK;
+}
+
+int gfx_ws_set_structure_limit(gfx_workspace *w, int64_t limit) {
+  if (!w || limit < 0 || limit > INT32_MAX) return GFX_E_INVALID;
+  w->structure_limit = limit;
+  ++w->version;  // the polynomial route is laid out anew
   return GFX_OK;
 }
 

@@ -76,6 +76,9 @@ class GaWorkspace:
     def set_form(self, form=FORM_FACTORIZED, precision=PREC_FP64):
         check(lib().gfx_ws_set_form(self.h, form, precision), self.ctx.h)
 
+    def set_structure_limit(self, limit):
+        check(lib().gfx_ws_set_structure_limit(self.h, limit), self.ctx.h)
+
     def compile(self):
         check(lib().gfx_ws_compile(self.h), self.ctx.h)
         return self.describe()

@@ -351,6 +351,12 @@ int gfx_ws_set_values_device(gfx_workspace *w, const char *name, const double *d
 /* ga_workspace::add_expression(expr, mim, region = all, der_order) (.h:425-428) */
 int gfx_ws_add_expression(gfx_workspace *w, const char *expr, gfx_mesh_im *mim, int der_order);
 int gfx_ws_set_form(gfx_workspace *w, int form, int precision);
+/* The polynomial route's order-2 assembly keeps, for every entry of every
+ * element matrix, its place in the matrix (some 12 bytes an entry), as long as
+ * there are no more of them than `limit` (at most, and unless set, 2^31 - 1).
+ * Beyond it the entries are sorted at every assembly, one block's element
+ * matrices at a time; the matrix is the same. */
+int gfx_ws_set_structure_limit(gfx_workspace *w, int64_t limit);
 /* the compile stage alone (GFX_E_UNSUPPORTED with a message outside the subset) */
 int gfx_ws_compile(gfx_workspace *w);
 /* ga_workspace::assembly(order) (.h:564).  order 0: the potential, the sum

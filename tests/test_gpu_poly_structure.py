@@ -66,3 +66,41 @@ def test_pattern_follows_values(ctx, name, n):
             assert np.array_equal(a, b)
         sizes.append(got[2].size)
     assert sizes[2] < sizes[0] == sizes[3]
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_same_matrix_without_the_structure(ctx, name):
+    """A limit below the number of candidates has the kept entries sorted at
+    every assembly: the same CSR bit for bit, also where values vanish and
+    return, where everything vanishes, and after the limit is lifted again."""
+    print("case: matrix without the structure", name, flush=True)
+    gt, femu, femp, expr = CASES[name]
+    pts, cvx = meshes.regular_unit_mesh(2, gt)
+    pts = meshes.jitter(pts, 2)
+    mesh = ga.Mesh(ctx, gt, pts, cvx)
+    mfs = (ga.MeshFem(mesh, femu, 1 if name == "q2_q1_hex" else 3), ga.MeshFem(mesh, femp, 1),
+           ga.MeshFem(mesh, "FEM_PK_DISCONTINUOUS(3,0)" if gt == "GT_PK(3,1)" else femp, 1))
+    mim = ga.MeshIm(mesh, IM[gt])
+    rng = np.random.default_rng(7)
+    vals = {"u": rng.standard_normal(mfs[0].nbdof()), "p": rng.uniform(0.5, 1.5, mfs[1].nbdof()),
+            "rho": rng.uniform(0.5, 2.0, mfs[2].nbdof())}
+    ws, ref = workspace(ctx, mfs, mim, vals, expr), workspace(ctx, mfs, mim, vals, expr)
+    ws.set_structure_limit(1000)
+    some = vals["rho"].copy()
+    some[:: 2] = 0.0
+
+    def same(rho):
+        for w in (ws, ref):
+            w.set_values("rho", rho)
+            w.assembly(2)
+        got, want = ws.assembled_matrix_csr(), ref.assembled_matrix_csr()
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
+        return want[2].size
+
+    sizes = [same(rho) for rho in (vals["rho"], some, 0.0 * some, -vals["rho"])]
+    assert sizes[2] < sizes[1] <= sizes[0] == sizes[3]
+    ws.set_structure_limit(2**31 - 1)
+    same(some)
+    with pytest.raises(ga.GfxError):
+        ws.set_structure_limit(-1)
