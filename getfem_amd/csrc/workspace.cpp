@@ -916,7 +916,10 @@ int sc_structure(gfx_workspace *w) {
   ScalarRoute *sc = w->sc;
   hipStream_t s = w->ctx->stream;
   const int64_t n = sc->n_cand;
-  if (n == 0) {
+  if (n == 0) {  // an empty matrix
+    wfree(sc->d_v); wfree(sc->d_ix);
+    if (hipMalloc((void **)&sc->d_v, 8) != hipSuccess || hipMalloc((void **)&sc->d_ix, 4) != hipSuccess)
+      return wfail(w, GFX_E_OOM, "order-2 route matrix");
     sc->n_ent = 0;
     return GFX_OK;
   }

@@ -104,3 +104,27 @@ def test_same_matrix_without_the_structure(ctx, name):
     same(some)
     with pytest.raises(ga.GfxError):
         ws.set_structure_limit(-1)
+
+
+def test_matrix_without_blocks(ctx):
+    """An expression whose second derivative vanishes: an empty matrix, whose
+    arrays are there all the same."""
+    import ctypes
+
+    from getfem_amd import _lib
+    print("case: matrix without blocks", flush=True)
+    pts, cvx = meshes.regular_unit_mesh(1)
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", pts, cvx)
+    mf = ga.MeshFem(mesh, "FEM_PK(3,2)", 1)
+    ws = GaWorkspace(ctx)
+    ws.add_fem_variable("u", mf)
+    ws.add_expression("3*u", ga.MeshIm(mesh, "IM_TETRAHEDRON(5)"))
+    ws.assembly(2)
+    ip, ix, v = ws.assembled_matrix_csr()
+    assert ip.size == mf.nbdof() + 1 and not ip.any() and ix.size == v.size == 0
+    p = [ctypes.c_void_p() for _ in range(3)]
+    n, nnz = ctypes.c_int64(), ctypes.c_int64()
+    _lib.check(_lib.lib().gfx_ws_device_csr(ws.h, ctypes.byref(n), ctypes.byref(nnz), *[ctypes.byref(x) for x in p]),
+               ctx.h)
+    assert nnz.value == 0 and all(x.value for x in p)
+    assert ws.assembled_matrix().nnz == 0
