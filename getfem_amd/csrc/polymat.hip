@@ -52,17 +52,22 @@ __device__ __forceinline__ int pm_wave_sum(int v) {
 // Bound by FP64 issue and the LDS.  A lane owns tiles of one column (j, b)
 // and the rows of kPmNodes test nodes, NP tiles in all, with their sums in
 // registers.  Per point the products of the outputs with the trial field's
-// base functions, U[(a, p)][(j, b)] = w_q |J| sum_r O[(a, p), (b, r)] psi_j[r],
-// are formed once in LDS and then serve every test node: 4 products an entry
-// and point instead of 20 with a load each.  Slots p, r that no output uses
-// are passed over.  Outputs without a fem field are the same at every point
-// and evaluated once.
-// Measured, u P2 vector + p P1 on 15^3 x 6 = 20,250 elements: the four blocks
-// 0.59 ms (the 30 x 30 one 0.27) against 6.15 ms with an LDS load a product and
-// the sums in LDS.
+// base functions, U[(a, p)][(j, b)] = sum_r O[(a, p), (b, r)] psi_j[r], are
+// formed once in LDS and then serve every test node: 5 products an entry and
+// point instead of 21 with a load each.  The test function's slots [P0, P1)
+// are those in use (its value, its gradient or both); so are r's.  Outputs
+// without a fem field are the same at every point and evaluated once.
+// A point's sum over p is formed before w_q |J| takes it into the entry, as
+// the reference does: adding the products one by one rounded the entry three
+// or four times a point, and its error against exact sums grew by 10 % (P2) to
+// 60 % (P3).
+// Measured, (1 + p^2) Grad_u:Grad_Test_u - p^2 Div_Test_u + p^3 Test_p with u P2
+// vector and p P1 on 15^3 x 6 = 20,250 elements: the three blocks 1.60 ms, a
+// whole assembly 1.73 ms against 6.26 ms with an LDS load a product and the
+// sums in LDS.
 constexpr int kPmNodes = 5;
 
-template <int QT, int NP>
+template <int QT, int NP, int P0, int P1>
 __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
   extern __shared__ double lds_pm[];
   const ScalarField &ft = a.f[a.vt], &fs = a.f[a.vs];
@@ -174,27 +179,34 @@ __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
     const double wJ = a.qw[q] * aJ;
     for (int x = t; x < 4 * QT * nc; x += kPm) {
       const int ap = x / nc, c = x - ap * nc, p = ap / QT, ca = ap - p * QT;  // U row p QT + ca
-      if (!(a.pmask >> p & 1)) continue;
+      if (p < P0 || p >= P1) continue;
       const int j = c / qs, cb = c - j * qs;
       const double *Or = O + (p == 0 ? ca : QT + 3 * ca + p - 1) * w4, *b = bs + 4 * j;
       double s = a.rmask & 1 ? Or[cb] * b[0] : 0.0;
-      if (a.rmask & 14) s += Or[qs + 3 * cb] * b[1] + Or[qs + 3 * cb + 1] * b[2] + Or[qs + 3 * cb + 2] * b[3];
-      U[x] = wJ * s;
+      if (a.rmask & 14) {
+        s += Or[qs + 3 * cb] * b[1];
+        s += Or[qs + 3 * cb + 1] * b[2];
+        s += Or[qs + 3 * cb + 2] * b[3];
+      }
+      U[x] = s;
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
+      double u[P1 - P0][QT];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        if (!(a.pmask >> p & 1)) continue;
-        double u[QT];
+      for (int p = P0; p < P1; ++p)
 #pragma unroll
-        for (int c = 0; c < QT; ++c) u[c] = U[(p * QT + c) * nc + col[k]];
+        for (int c = 0; c < QT; ++c) u[p - P0][c] = U[(p * QT + c) * nc + col[k]];
 #pragma unroll
-        for (int i = 0; i < kPmNodes; ++i) {
-          const double b = bt[4 * min(row0[k] + i, ndt - 1) + p];
+      for (int i = 0; i < kPmNodes; ++i) {
+        const double *b = bt + 4 * min(row0[k] + i, ndt - 1);
 #pragma unroll
-          for (int c = 0; c < QT; ++c) acc[k][i][c] += b * u[c];
+        for (int c = 0; c < QT; ++c) {
+          double s = b[P0] * u[0][c];
+#pragma unroll
+          for (int p = P0 + 1; p < P1; ++p) s += b[p] * u[p - P0][c];
+          acc[k][i][c] += wJ * s;
         }
       }
     }
@@ -551,16 +563,22 @@ unsigned pm_blocks(int64_t n) { return (unsigned)((n + kPoly1d - 1) / kPoly1d); 
 
 }  // namespace
 
-template <int QT>
-static hipError_t launch_poly_mat_q(hipStream_t s, const PolyMatArgs &a, size_t lds) {
+template <int QT, int P0, int P1>
+static hipError_t launch_poly_mat_p(hipStream_t s, const PolyMatArgs &a, size_t lds) {
   const int nc = a.f[a.vs].nd * a.f[a.vs].qdim, tiles = (a.f[a.vt].nd + kPmNodes - 1) / kPmNodes * nc;
   const unsigned grid = (unsigned)a.n_cv;
-  if (tiles <= kPm) k_poly_mat<QT, 1><<<grid, kPm, lds, s>>>(a);
-  else if (tiles <= 2 * kPm) k_poly_mat<QT, 2><<<grid, kPm, lds, s>>>(a);
-  else if (tiles <= 4 * kPm) k_poly_mat<QT, 4><<<grid, kPm, lds, s>>>(a);
-  else if (tiles <= 8 * kPm) k_poly_mat<QT, 8><<<grid, kPm, lds, s>>>(a);
+  if (tiles <= kPm) k_poly_mat<QT, 1, P0, P1><<<grid, kPm, lds, s>>>(a);
+  else if (tiles <= 2 * kPm) k_poly_mat<QT, 2, P0, P1><<<grid, kPm, lds, s>>>(a);
+  else if (tiles <= 4 * kPm) k_poly_mat<QT, 4, P0, P1><<<grid, kPm, lds, s>>>(a);
+  else if (tiles <= 8 * kPm) k_poly_mat<QT, 8, P0, P1><<<grid, kPm, lds, s>>>(a);
   else return hipErrorInvalidValue;
   return hipGetLastError();
+}
+
+template <int QT>
+static hipError_t launch_poly_mat_q(hipStream_t s, const PolyMatArgs &a, size_t lds) {
+  if (!(a.pmask & 14)) return launch_poly_mat_p<QT, 0, 1>(s, a, lds);
+  return a.pmask & 1 ? launch_poly_mat_p<QT, 0, 4>(s, a, lds) : launch_poly_mat_p<QT, 1, 4>(s, a, lds);
 }
 
 template <int QT, int QS>
