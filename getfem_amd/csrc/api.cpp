@@ -120,6 +120,26 @@ void close_or_mark(T *o) {
 
 }  // namespace
 
+// The smallest L of the denominators that integrals of base functions have,
+// with every v L a whole number; 0 if there is none.
+double gfx::common_denominator(const std::vector<double> &v) {
+  static const int kL[] = {1,    2,    3,    4,    5,    6,    8,    9,     10,    12,    15,
+                           16,   18,   20,   24,   30,   36,   40,   45,    48,    60,    72,
+                           80,   90,   96,   120,  144,  180,  240,  280,   315,   360,   420,
+                           480,  504,  560,  630,  720,  840,  1008, 1120,  1260,  1440,  1680,
+                           2016, 2240, 2520, 2880, 3360, 4032, 5040, 6720,  7560,  10080, 15120,
+                           20160, 30240, 40320, 60480, 80640, 120960, 181440, 362880};
+  for (int L : kL) {
+    bool ok = true;
+    for (double r : v) {
+      const double n = r * L;
+      if (std::fabs(n - std::nearbyint(n)) > 1e-9 * std::max(1.0, std::fabs(n))) { ok = false; break; }
+    }
+    if (ok) return L;
+  }
+  return 0.0;
+}
+
 void gfx::ref(gfx_ctx *c) { ++c->refs; }
 void gfx::unref(gfx_ctx *c) { if (--c->refs == 0 && c->closing) release(c); }
 void gfx::ref(gfx_mesh *m) { ++m->refs; }
@@ -489,39 +509,26 @@ int gfx_plan_destroy(gfx_plan *p) {
 // such form (a rule that does not integrate the products exactly).
 static void detect_int_reference(const std::vector<double> &R, int nblk, int &rk, double &L,
                                  std::vector<uint8_t> &out) {
-  static const int kL[] = {1,    2,    3,    4,    5,    6,    8,    9,     10,    12,    15,
-                           16,   18,   20,   24,   30,   36,   40,   45,    48,    60,    72,
-                           80,   90,   96,   120,  144,  180,  240,  280,   315,   360,   420,
-                           480,  504,  560,  630,  720,  840,  1008, 1120,  1260,  1440,  1680,
-                           2016, 2240, 2520, 2880, 3360, 4032, 5040, 6720,  7560,  10080, 15120,
-                           20160, 30240, 40320, 60480, 80640, 120960, 181440, 362880};
   rk = 0;
   L = 1.0;
-  for (int Lc : kL) {
-    double nmax = 0.0;
-    bool ok = true;
-    for (double r : R) {
-      const double n = r * Lc, rn = std::nearbyint(n);
-      if (std::fabs(n - rn) > 1e-9 * std::max(1.0, std::fabs(n))) { ok = false; break; }
-      nmax = std::max(nmax, std::fabs(rn));
-    }
-    if (!ok) continue;
-    if (nmax > 32767.0) return;
-    rk = nmax <= 127.0 ? 1 : 2;
-    L = Lc;
-    const int bs = rk == 1 ? 16 : 32;
-    out.assign((size_t)nblk * bs, 0);
-    for (int b = 0; b < nblk; ++b)
-      for (int t = 0; t < 9; ++t) {
-        const int n = (int)std::nearbyint(R[(size_t)b * 9 + t] * Lc);
-        if (rk == 1) out[(size_t)b * 16 + t] = (uint8_t)(int8_t)n;
-        else {
-          const uint16_t u = (uint16_t)(int16_t)n;
-          std::memcpy(&out[(size_t)b * 32 + 2 * t], &u, 2);
-        }
+  const double Lc = common_denominator(R);
+  if (Lc == 0.0) return;
+  double nmax = 0.0;
+  for (double r : R) nmax = std::max(nmax, std::fabs(std::nearbyint(r * Lc)));
+  if (nmax > 32767.0) return;
+  rk = nmax <= 127.0 ? 1 : 2;
+  L = Lc;
+  const int bs = rk == 1 ? 16 : 32;
+  out.assign((size_t)nblk * bs, 0);
+  for (int b = 0; b < nblk; ++b)
+    for (int t = 0; t < 9; ++t) {
+      const int n = (int)std::nearbyint(R[(size_t)b * 9 + t] * Lc);
+      if (rk == 1) out[(size_t)b * 16 + t] = (uint8_t)(int8_t)n;
+      else {
+        const uint16_t u = (uint16_t)(int16_t)n;
+        std::memcpy(&out[(size_t)b * 32 + 2 * t], &u, 2);
       }
-    return;
-  }
+    }
 }
 
 int gfx_plan_create(gfx_mesh_fem *mf, gfx_mesh_im *mim, int term, const gfx_coef *coefs,

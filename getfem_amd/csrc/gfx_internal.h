@@ -228,6 +228,7 @@ struct PolyMatArgs {
   int nsym;                  // symbols of the table
   bool varying;              // an output reads a fem field
   int pmask, rmask;          // slots (bit 0 value, 1 + b gradient) of the test and trial function in use
+  const double *R;           // the reference tensor, 16 x (pairs of base functions), or null
   double *elem;              // n_cv * nr * nc, row r = i qt + a, column c = j qs + b; entries at or
                              // below the element's threshold are 0
   int *err;
@@ -271,6 +272,7 @@ __device__ __forceinline__ bool poly_geometry(const double *pts, const int32_t *
   aJ = fabs(J);
   return true;
 }
+double common_denominator(const std::vector<double> &v);  // api.cpp
 hipError_t launch_poly_mat(hipStream_t s, const PolyMatArgs &a);
 // The structure: every block's candidates (position base + index in the
 // element matrices), sorted by key (temporary storage: poly_structure_bytes)

@@ -243,10 +243,12 @@ __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
 // A lane keeps its pair (i, j), and with it R_ij in registers, for all the
 // elements that its workgroup passes over, `epb` side by side; a chunk's
 // geometry is formed first, a lane an element.  Bound by FP64 issue and the
-// latency of the start (R is formed by every workgroup: the points' base
-// functions are read from the L2).
+// latency of the start.  R comes from the host, where it is summed in long
+// double: formed here, by every workgroup in FP64, its roundings were most of
+// the matrix's error.
 // Measured, u P2 vector + p P1 on 15^3 x 6 = 20,250 elements: the four blocks
-// 0.154 ms (67 us for the 30 x 30 one), through the points (k_poly_mat) 0.59 ms.
+// 0.107 ms (56 us for the 30 x 30 one), 0.154 ms with R formed by every
+// workgroup; through the points (k_poly_mat) 0.59 ms.
 constexpr int kPrIters = 8;      // passes of a workgroup where the elements are enough to fill the card
 constexpr int kPrMaxChunk = 512; // elements of a workgroup
 
@@ -283,17 +285,7 @@ __global__ __launch_bounds__(512) void k_poly_ref(PolyMatArgs a, int epb, int it
 #pragma unroll
   for (int p = 0; p < 4; ++p)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) R[p][r] = 0.0;
-  for (int q = 0; on && q < a.nq; ++q) {
-    const double *gt = ft.gref + ((int64_t)q * ndt + i) * 3, *gs = fs.gref + ((int64_t)q * nds + j) * 3;
-    const double w = a.qw[q];
-    const double f[4] = {ft.phi[q * ndt + i], gt[0], gt[1], gt[2]};
-    const double g[4] = {w * fs.phi[q * nds + j], w * gs[0], w * gs[1], w * gs[2]};
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) R[p][r] += f[p] * g[r];
-  }
+    for (int r = 0; r < 4; ++r) R[p][r] = on ? a.R[(4 * p + r) * pairs + pr] : 0.0;
   __syncthreads();
   for (int o = t; o < a.nout; o += blockDim.x) {  // its monomials in a fixed order
     double s = 0.0;
@@ -614,7 +606,7 @@ hipError_t launch_poly_mat(hipStream_t s, const PolyMatArgs &a) {
   // tetrahedra and a program without fem fields: one reference tensor a pair
   // serves every element (a field's values or a hexahedron's points make the
   // integrand another one in each)
-  if (!a.gN && !a.varying && a.f[a.vt].nd * a.f[a.vs].nd <= 512) {
+  if (a.R && a.f[a.vt].nd * a.f[a.vs].nd <= 512) {
     const int qs = a.f[a.vs].qdim;
 #define GFX_REF(QT, QS) \
   if (qt == QT && qs == QS) return launch_poly_ref<QT, QS>(s, a)

@@ -71,6 +71,7 @@ struct ScBlock {                // an order-2 block: test variable x trial varia
   int vt = 0, vs = 0;           // their fields
   bool varying = false;         // an output reads a fem field
   int pmask = 0, rmask = 0;     // slots of the test and trial function in use
+  double *d_R = nullptr;        // reference tensor (affine elements, outputs without fem fields)
   int ne = 0;                   // entries of an element matrix
   int64_t base = 0;             // its element matrices in d_pelem
 };
@@ -79,6 +80,7 @@ struct ScField {
   std::string name;
   gfx_mesh_fem *mf = nullptr;
   int off = 0;
+  std::vector<double> phi, gref;  // base functions and reference gradients at the points
   double *d_U = nullptr, *d_phi = nullptr, *d_gref = nullptr;
   const double *u = nullptr;    // the values that an assembly reads: d_U or the variable's device copy
 };
@@ -508,7 +510,7 @@ void sc_release(ScalarRoute *sc) {
   for (auto &v : sc->vars) { sc_free_prog(v.p); wfree(v.d_inc_ptr); wfree(v.d_inc); }
   wfree(sc->d_consts); wfree(sc->d_qw); wfree(sc->d_gN); wfree(sc->d_elem); wfree(sc->d_part); wfree(sc->d_sum);
   wfree(sc->d_V); wfree(sc->d_err);
-  for (auto &b : sc->blocks) sc_free_prog(b.p);
+  for (auto &b : sc->blocks) { sc_free_prog(b.p); wfree(b.d_R); }
   wfree(sc->d_pelem); wfree(sc->d_src); wfree(sc->d_start); wfree(sc->d_place); wfree(sc->d_row); wfree(sc->d_col);
   wfree(sc->d_cnt); wfree(sc->d_off); wfree(sc->d_scan);
   wfree(sc->d_nnz); wfree(sc->d_keys); wfree(sc->d_keys2); wfree(sc->d_vals); wfree(sc->d_vals2);
@@ -539,6 +541,36 @@ hipError_t upload(T **d, const std::vector<T> &h) {
   if (hipMalloc((void **)d, sizeof(T) * std::max<size_t>(h.size(), 1)) != hipSuccess) return hipErrorOutOfMemory;
   if (h.empty()) return hipSuccess;
   return hipMemcpy(*d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice);
+}
+
+// The reference tensor of a pair of fields, R[p][r][pair (i, j)] = sum_q w_q
+// phi_i^p psi_j^r (p, r: value, reference gradient).  It enters every entry of
+// every element, so it is summed in long double, and where a rule integrates
+// the products (they have a common denominator) the exact value is taken: its
+// error is a rounding, where fifteen rounded additions had doubled that of the
+// whole matrix.
+std::vector<double> sc_reference(const IntegrationRule &rule, const ScField &ft, const ScField &fs) {
+  const int nq = rule.n(), ndt = ft.mf->fem.nd, nds = fs.mf->fem.nd, pairs = ndt * nds;
+  std::vector<double> R((size_t)16 * pairs);
+  auto base = [](const ScField &f, int nd, int q, int i, int p) {
+    return p == 0 ? f.phi[(size_t)q * nd + i] : f.gref[((size_t)q * nd + i) * 3 + p - 1];
+  };
+  for (int g = 0; g < 4; ++g) {  // value or gradient of the test and of the trial function
+    std::vector<size_t> at;
+    std::vector<double> v;
+    for (int p = g & 1 ? 1 : 0; p < (g & 1 ? 4 : 1); ++p)
+      for (int r = g & 2 ? 1 : 0; r < (g & 2 ? 4 : 1); ++r)
+        for (int x = 0; x < pairs; ++x) {
+          long double s = 0.0L;
+          for (int q = 0; q < nq; ++q)
+            s += (long double)rule.w[q] * base(ft, ndt, q, x / nds, p) * base(fs, nds, q, x % nds, r);
+          at.push_back((size_t)(4 * p + r) * pairs + x);
+          v.push_back((double)s);
+        }
+    const double L = common_denominator(v);
+    for (size_t k = 0; k < v.size(); ++k) R[at[k]] = L != 0.0 ? std::nearbyint(v[k] * L) / L : v[k];
+  }
+  return R;
 }
 
 // Compile the potential and every fem variable's derivative into programs,
@@ -656,10 +688,11 @@ int sc_build(gfx_workspace *w) {
     f.off = off;
     off += 4 * v.mf->qdim;
     const int nd = v.mf->fem.nd;
-    std::vector<double> phi((size_t)nq * nd), gref((size_t)nq * nd * 3);
-    for (int q = 0; q < nq; ++q) fem_eval(v.mf->fem, &rule.pts[3 * (size_t)q], &phi[(size_t)q * nd],
-                                          &gref[(size_t)q * nd * 3]);
-    if (upload(&f.d_phi, phi) != hipSuccess || upload(&f.d_gref, gref) != hipSuccess ||
+    f.phi.resize((size_t)nq * nd);
+    f.gref.resize((size_t)nq * nd * 3);
+    for (int q = 0; q < nq; ++q) fem_eval(v.mf->fem, &rule.pts[3 * (size_t)q], &f.phi[(size_t)q * nd],
+                                          &f.gref[(size_t)q * nd * 3]);
+    if (upload(&f.d_phi, f.phi) != hipSuccess || upload(&f.d_gref, f.gref) != hipSuccess ||
         hipMalloc((void **)&f.d_U, 8 * (size_t)std::max<int64_t>(v.mf->ndof, 1)) != hipSuccess) {
       sc->fields.push_back(f);
       return bail(GFX_E_OOM, "polynomial route tables");
@@ -730,6 +763,9 @@ int sc_build(gfx_workspace *w) {
       b.rmask |= 1 << (os < qs ? 0 : 1 + (os - qs) % 3);
     }
     for (int x : b.p.slots) b.varying |= x < sc->const_off;
+    if (m->gt == GT_TET_P1 && !b.varying &&
+        upload(&b.d_R, sc_reference(rule, sc->fields[b.vt], sc->fields[b.vs])) != hipSuccess)
+      return bail(GFX_E_OOM, "order-2 route tables");
     b.ne = ft->fem.nd * qt * fs->fem.nd * qs;
     b.base = sc->n_cand;
     sc->n_cand += m->n_cv * b.ne;
@@ -1071,6 +1107,7 @@ int sc_assemble2(gfx_workspace *w) {
   for (auto &b : sc->blocks) {
     a.vt = b.vt; a.vs = b.vs;
     a.nout = b.p.prog.nout; a.varying = b.varying; a.pmask = b.pmask; a.rmask = b.rmask;
+    a.R = b.d_R;
     a.mcoef = b.p.d_coef; a.mptr = b.p.d_mptr; a.moff = b.p.d_off; a.msym = b.p.d_sym;
     a.elem = sc->d_pelem + (structure ? b.base : 0);
     WHIP(w, launch_poly_mat(s, a));

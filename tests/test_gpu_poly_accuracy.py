@@ -14,6 +14,8 @@ from getfem_amd.workspace import GaWorkspace
 pytestmark = pytest.mark.gpu
 
 CASES = {  # geometry, element of u, rule, whether the integrand reads a field
+    "p2_const": ("GT_PK(3,1)", "FEM_PK(3,2)", "IM_TETRAHEDRON(5)", False),
+    "p3_const": ("GT_PK(3,1)", "FEM_PK(3,3)", "IM_TETRAHEDRON(8)", False),
     "p2_field": ("GT_PK(3,1)", "FEM_PK(3,2)", "IM_TETRAHEDRON(5)", True),
     "p3_field": ("GT_PK(3,1)", "FEM_PK(3,3)", "IM_TETRAHEDRON(8)", True),
     "q1_const": ("GT_QK(3,1)", "FEM_QK(3,1)", "IM_GAUSS_PARALLELEPIPED(3,4)", False),
