@@ -14,7 +14,9 @@
 // potential's element value (one lane adds the points in order); order 1, the
 // element vector of the differentiated variable, a lane per dof,
 //   elem[i, a] = sum_q w_q |J| (c_a phi_i + sum_b c_(q + 3a + b) (B grad phi_i)_b),
-// with the B of a point taken to the coefficients' side.
+// with the B of a point taken to the coefficients' side and the sum over the
+// points compensated (the coefficients' own roundings cost up to 6 % of the
+// vector's error on hexahedra, which the sum's more than make good).
 // The program is the same for every thread (uniform loads).  Element vectors
 // go to a buffer and are summed per dof over the node's incidences (no
 // atomics); element values are summed by a fixed-order two-stage reduction,
@@ -137,13 +139,17 @@ __global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a, int ns
       for (int x = l; x < nl; x += G) {
         const int i = x / Q, c = x - i * Q;
         const double *w = lds_sc + (nsym + 4 * c) * kScThreads + g * G;  // point k: w[k]
-        double s = q0 && live ? el[x] : 0.0;
+        double s = q0 && live ? el[x] : 0.0, lost = 0.0;  // (what the sum's roundings take is added at the end)
         for (int k = 0; k < nq; ++k) {
           const int p = (q0 + k) * vf.nd + i;
           const double *h = vf.gref + (int64_t)p * 3;
-          s += w[k] * vf.phi[p] + w[kScThreads + k] * h[0] + w[2 * kScThreads + k] * h[1] + w[3 * kScThreads + k] * h[2];
+          const double v = w[k] * vf.phi[p] + w[kScThreads + k] * h[0] + w[2 * kScThreads + k] * h[1] +
+                           w[3 * kScThreads + k] * h[2];
+          const double y = s + v, r = y - s;
+          lost += (s - (y - r)) + (v - r);
+          s = y;
         }
-        if (live) el[x] = s;
+        if (live) el[x] = s + lost;
       }
     }
     __syncthreads();

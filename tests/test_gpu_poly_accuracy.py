@@ -1,4 +1,4 @@
-"""How far the polynomial route's matrices are from the exact ones, in long
+"""How far the polynomial route's matrices and vectors are from the exact ones, in long
 double: no further than the sum over the rule's points in plain float64, the
 order that the reference assembles in, but for a tenth (two ways of rounding
 one sum).  Exact: where the integrand is a polynomial that the rule integrates
@@ -126,3 +126,63 @@ def test_matrix(ctx, name, seed):
     far = [float(np.sqrt(((a - exact) ** 2).sum()) / norm) for a in (v, assembled(np.float64, args))]
     print("error %.3e, of the sum over the points in float64 %.3e" % tuple(far), flush=True)
     assert far[0] <= 1.1 * far[1]
+
+
+def point_vector(T, x, g1, W, phi, gref, psi, P, U):
+    """The same integrand's vector at the nodal values U, a point after another."""
+    x, U = x.astype(T), U.astype(T)
+    V = np.zeros(U.shape, dtype=T)
+    mu = T(MU)
+    for q in range(len(W)):
+        K = np.einsum("evr,vc->erc", x, g1[q].astype(T))
+        r, s = [1, 2, 0], [2, 0, 1]
+        cof = K[:, r][:, :, r] * K[:, s][:, :, s] - K[:, r][:, :, s] * K[:, s][:, :, r]
+        J = (K[:, 0] * cof[:, 0]).sum(axis=1)
+        h = np.einsum("erc,ic->eir", cof / J[:, None, None], gref[q].astype(T))
+        c = mu * (1 + (P.astype(T) @ psi[q].astype(T)) ** 2) if P is not None else mu + 0 * J
+        H = np.einsum("eia,eic->eac", U, h)
+        u = np.einsum("eia,i->ea", U, phi[q].astype(T))
+        S = c[:, None, None] * (H + H.transpose(0, 2, 1))
+        v = np.einsum("eac,eic->eia", S, h) + (c[:, None] * u)[:, None, :] * phi[q].astype(T)[None, :, None]
+        V += (T(W[q]) * np.abs(J))[:, None, None] * v
+    return V
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+@pytest.mark.parametrize("name", ["p2_const", "p3_const", "p3_field", "q1_const", "q1_field"])
+def test_vector(ctx, name, seed):
+    """(The element vectors' sums over the points are compensated: no tenth.)"""
+    print("case: accuracy of the polynomial route's vector", name, seed, flush=True)
+    gt, fem, im, field = CASES[name]
+    n = 4 if fem == "FEM_QK(3,1)" else 3
+    pts, cvx = meshes.regular_unit_mesh(n, gt)
+    pts = meshes.jitter(pts, n, seed=seed)
+    mesh = ga.Mesh(ctx, gt, pts, cvx)
+    mf, mfp = ga.MeshFem(mesh, fem, 3), ga.MeshFem(mesh, fem, 1)
+    rng = np.random.default_rng(seed)
+    p, u = rng.uniform(0.5, 1.5, mfp.nbdof()), rng.standard_normal(mf.nbdof())
+    ws = GaWorkspace(ctx)
+    ws.add_fem_variable("u", mf, u)
+    ws.add_fem_constant("p", mfp, p)
+    ws.add_fixed_size_constant("mu", MU)
+    ws.add_expression(("(1+p*p)*" if field else "") + "(mu*(Grad_u + Grad_u'):Grad_Test_u + mu*u.Test_u)",
+                      ga.MeshIm(mesh, im))
+    ws.assembly(1)
+    V = ws.assembled_vector()
+    P, W = core.integration_rule(im)
+    phi, gref = (np.stack(a) for a in zip(*(core.fem_eval(fem, x) for x in P)))
+    corner = np.array([[-1.0, -1, -1], [1, 0, 0], [0, 1, 0], [0, 0, 1]])
+    g1 = [core.fem_eval("FEM_QK(3,1)", x)[1] if gt == "GT_QK(3,1)" else corner for x in P]
+    dofs = mf.basic_dof_table().reshape(cvx.shape[0], -1)
+    dofs = dofs[:, :: dofs.shape[1] // phi.shape[1]][:, :, None] + np.arange(3)
+    args = (pts[cvx], g1, W, phi, gref, phi, p[mfp.basic_dof_table()] if field else None, u[dofs])
+
+    def assembled(T):
+        v = np.zeros(V.size, dtype=T)
+        np.add.at(v, dofs.ravel(), point_vector(T, *args).ravel())
+        return v
+
+    exact = assembled(np.longdouble)
+    far = [float(np.sqrt(((a - exact) ** 2).sum() / (exact ** 2).sum())) for a in (V, assembled(np.float64))]
+    print("error %.3e, of the sum over the points in float64 %.3e" % tuple(far), flush=True)
+    assert far[0] <= far[1]
