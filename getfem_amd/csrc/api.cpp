@@ -737,8 +737,8 @@ static int plan_keep(gfx_plan *p, bool check) {
   RecordArgs a = record_args(p);
   int r;
   if ((r = records32(p, a))) return r;
-  HIPCHK(c, launch_keep(c->stream, p->term, p->nd, p->qdim, a, p->d_Rp, p->d_sig, check, p->d_thr, p->d_keep,
-                        p->kwords));
+  HIPCHK(c, launch_keep(c->stream, p->term, p->nd, p->qdim, a, p->d_Rp, p->d_gref, p->d_qw, p->nq, p->d_sig, check,
+                        p->d_thr, p->d_keep, p->kwords));
   return GFX_OK;
 }
 
@@ -778,9 +778,8 @@ static int plan_eb_tangent(gfx_plan *p, int precision, int keep) {
   return GFX_OK;
 }
 
-static int check_err_flag(gfx_plan *p) {
+static int check_err_flag(gfx_plan *p, int &flag) {
   gfx_ctx *c = p->ctx;
-  int flag = 0;
   HIPCHK(c, hipMemcpyAsync(&flag, p->d_err, 4, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (flag & 1) return fail(c, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
@@ -1025,7 +1024,8 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   HIPCHK(c, scan_exclusive_i64(s, rowcnt, p->d_indptr, p->ndof, tmp64));
   int64_t nnz = 0;
   HIPCHK(c, hipMemcpyAsync(&nnz, p->d_indptr + p->ndof, 8, hipMemcpyDeviceToHost, s));
-  if ((r = check_err_flag(p))) return r;
+  int flag = 0;
+  if ((r = check_err_flag(p, flag))) return r;
   // nslots maximum for the assembly kernel's LDS
   std::vector<uint16_t> ns((size_t)nn);
   HIPCHK(c, hipMemcpy(ns.data(), p->d_nslots, 2 * (size_t)nn, hipMemcpyDeviceToHost));
@@ -1048,7 +1048,7 @@ int gfx_plan_build_pattern(gfx_plan *p, int64_t *nnz_out) {
   // the keep bits stay: re-validation after a change of values compares
   // the pattern they give with this one
   p->nnz = nnz;
-  p->keep_ok = true;
+  p->keep_ok = !(flag & 64);
   p->pts_version = m->version;
   p->values_changed = false;
   p->pattern_id++;
@@ -1123,7 +1123,7 @@ static int plan_validate(gfx_plan *p, bool *fresh) {
     *fresh = true;  // the rebuild ran at the current values
     return GFX_OK;
   }
-  p->keep_ok = true;
+  p->keep_ok = !(flag & 64);
   p->pts_version = m->version;
   p->values_changed = false;
   *fresh = true;

@@ -324,10 +324,14 @@ hipError_t launch_incidences(hipStream_t s, int64_t n_cv, int nd, int qdim,
 // Records with thresholds and the keep signature (keep_sig_words u64) of
 // every element; Rp: the upper pairs' reference blocks in the records' scale.
 // check: the signature is compared with sig (bit 32 of the error flag when it
-// differs), else it is written, and the keep words formed from it.
+// differs or an entry lies near its threshold), else it is written, and the
+// keep words formed from it; elements with an entry near the threshold get
+// theirs from the sum over the points (bit 64 of the error flag: the signature
+// does not hold them).
 int64_t keep_sig_words(int term, int nd, int qdim, int64_t n_cv);
 hipError_t launch_keep(hipStream_t s, int term, int nd, int qdim, const RecordArgs &a, const double *Rp,
-                       uint64_t *sig, bool check, double *thr, uint32_t *keep, int kwords);
+                       const double *gref, const double *qw, int nq, uint64_t *sig, bool check, double *thr,
+                       uint32_t *keep, int kwords);
 hipError_t launch_patch_build(hipStream_t s, const PatternArgs &a, int max_cand);
 hipError_t launch_fill_columns(hipStream_t s, const PatternArgs &a);
 // the pattern check against new keep bits: the thread-per-node pass (sets bit
@@ -523,7 +527,8 @@ struct gfx_plan {
   // Keep bits of every element: as words (what the presence bits are made
   // of) and, for the affine terms, as the signature that a check compares.
   // keep_ok: they are those that the stored pattern was built from or
-  // confirmed with (false while a refused change of pattern is pending).
+  // confirmed with (false while a refused change of pattern is pending, and
+  // where the signature does not hold them).
   uint32_t *d_keep = nullptr;
   uint64_t *d_sig = nullptr;
   double *d_Rp = nullptr;        // upper pairs' reference blocks, nd (nd + 1) / 2 x 9, in the records' scale

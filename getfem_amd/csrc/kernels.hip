@@ -244,6 +244,12 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 // compile_and_exec.cc:5441-5442), pass 2 forms the blocks again and compares
 // (a check of finite values needs no pass 2: it takes the smallest entry of
 // those that are stored as kept and the largest of the others in pass 1).
+// An element with an entry within a factor kKeepNear of its threshold is not
+// decided here: the factorized blocks round it otherwise than the sum over the
+// points that GetFEM compares, and k_keep_points decides it by that sum
+// (negative thr_out; a check counts such an element as changed).  Without that,
+// 55 of the 6.4 M stored entries of 72 P3 elasticity bodies of aspect ratio 1e6
+// to 3e6 were not GetFEM's, with it 14.
 // The blocks are those of the factorized form, G = B R_ij B^T: an integral
 // instead of a sum over the points (P2: 63 products a block instead of 600),
 // and the reference blocks are the same for every lane, so they come through
@@ -263,6 +269,7 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 // after them and 15 us of records before and after; an assembly with new
 // coefficients 4.91 -> 0.59 ms.
 constexpr int kKeepWaves = 4;
+constexpr double kKeepNear = 4.0;  // (the two forms differ by up to 13 % of the threshold, P1 to P3, aspect ratios to 1e6)
 
 template <int Q, int TERM>
 __device__ __forceinline__ void keep_block(const double *__restrict__ r, const double (&B)[9], double sa, double sb,
@@ -297,6 +304,7 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
   constexpr int NP = ND * (ND + 1) / 2, NV = TERM == GFX_TERM_LAPLACE ? 1 : Q * Q;
   __shared__ double2 stage[kWave * 9];  // records, rows padded as in k_records_tet
   __shared__ double red[kKeepWaves][kWave];
+  __shared__ uint64_t close[kKeepWaves];  // elements with an entry near the threshold
   const int lane = threadIdx.x % kWave, w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int64_t g = blockIdx.x, e0 = g * kWave;
   const int nblk = (int)min<int64_t>(kWave, a.n_cv - e0);
@@ -317,8 +325,8 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
   }
   const uint64_t *sg = sig + g * (NP * NV);
   // CHECK: the smallest of the entries whose stored bit is set, the largest of
-  // the others (mn > thr and md <= thr: the bits are the stored ones), and
-  // whether every value is finite, where both say what the bits would; mn stays
+  // the others (mn well above thr and md well below: the bits are the stored
+  // ones), and whether every value is finite, where both say what the bits would; mn stays
   // infinite where no bit is set (an all-zero element, whose threshold is
   // infinite too)
   const uint64_t full = nblk == kWave ? ~0ull : (1ull << nblk) - 1ull;
@@ -347,15 +355,14 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
 #pragma unroll
   for (int x = 0; x < kKeepWaves; ++x) mx = fmax(mx, red[x][lane]);
   const double thr = mx > 0.0 ? mx * 1e-14 : INFINITY;
-  if (w == 0 && lane < nblk) {
-    thr_out[e0 + lane] = thr;
-    reinterpret_cast<double *>(stage + 9 * lane)[11] = thr;
-  }
+  const double lo = thr / kKeepNear, hi = thr * kKeepNear;
+  if (w == 0 && lane < nblk) reinterpret_cast<double *>(stage + 9 * lane)[11] = thr;
   uint64_t diff = 0;
+  bool near = false;
   bool pass2 = true;
   if constexpr (CHECK) {
     pass2 = __ballot(fin != 0.0) != 0;  // not a number: the bits themselves are compared
-    diff = __ballot(lane < nblk && !((mn > thr || mn == INFINITY) && md <= thr));
+    diff = __ballot(lane < nblk && !((mn > hi || mn == INFINITY) && md <= lo));
   }
   if (CHECK && pass2) diff = 0;
   for (int p = pass2 ? w : NP; p < NP; p += kKeepWaves) {
@@ -364,12 +371,21 @@ __global__ __launch_bounds__(64 * kKeepWaves) void k_keep(RecordArgs a, const do
 #pragma unroll
     for (int x = 0; x < NV; ++x) {
       const uint64_t k = __ballot(fabs(v[x]) > thr);
+      near |= fabs(v[x]) > lo && fabs(v[x]) <= hi;
       if constexpr (CHECK) diff |= k ^ sg[p * NV + x];
       else if (lane == x) sig_out[(g * NP + p) * NV + x] = k;
     }
   }
-  if (CHECK && diff && lane == 0) atomicOr(a.err, 32);
+  const uint64_t cl = __ballot(near && lane < nblk);
+  if (CHECK && (diff | cl) && lane == 0) atomicOr(a.err, 32);
+  if (lane == 0) close[w] = cl;
   __syncthreads();
+  if (w == 0 && lane < nblk) {
+    uint64_t any = 0;
+#pragma unroll
+    for (int x = 0; x < kKeepWaves; ++x) any |= close[x];
+    thr_out[e0 + lane] = !CHECK && (any >> lane & 1) ? -thr : thr;
+  }
   // the records, 16-byte pieces of consecutive records from consecutive threads
   if (a.rec32) {
     float4 *dst = reinterpret_cast<float4 *>(a.rec32 + (int64_t)kRecStride * e0);
@@ -408,6 +424,61 @@ __global__ __launch_bounds__(256) void k_keep_words(int64_t n_cv, int kwords, co
       bits |= (uint32_t)((k >> lane) & 1u) << b;
     }
     if (e < n_cv) keep[e * kwords + wd] = bits;
+  }
+}
+
+// Threshold and keep words, by the sum over the points and every pair for
+// itself, of the elements that k_keep left open (negative thr); bit 64 of the
+// error flag when there are any.  A wavefront looks over 64 elements and takes
+// its open ones one after the other, a lane per pair.
+template <int Q, int TERM>
+__global__ __launch_bounds__(256) void k_keep_points(RecordArgs a, int nd, int nq, const double *__restrict__ gref,
+                                                     const double *__restrict__ qw, double *__restrict__ thr_out,
+                                                     uint32_t *__restrict__ keep, int kwords) {
+  extern __shared__ uint32_t kbits[];  // 4 waves x kwords
+  const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave, nl = nd * Q, npair = nd * nd;
+  const int64_t e0 = ((int64_t)blockIdx.x * 4 + w) * kWave;
+  uint32_t *my = kbits + w * kwords;
+  auto fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  uint64_t open = __ballot(e0 + lane < a.n_cv && thr_out[min(e0 + lane, a.n_cv - 1)] < 0.0);
+  if (open && lane == 0) atomicOr(a.err, 64);
+  for (; open; open &= open - 1) {
+    const int64_t e = e0 + __ffsll((unsigned long long)open) - 1;
+    const double *rec = a.rec + (int64_t)kRecStride * e;
+    for (int t = lane; t < kwords; t += kWave) my[t] = 0u;
+    double mx = 0.0;
+    for (int p = lane; p < npair; p += kWave) {
+      double v[Q][Q];
+      pair_block<Q, TERM, GFX_FORM_PERQP, double>(rec, p / nd, p % nd, nd, nq, gref, qw, nullptr, v);
+      for (int x = 0; x < Q; ++x)
+        for (int y = 0; y < Q; ++y) mx = fmax(mx, fabs(v[x][y]));
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, kWave));
+    const double thr = mx > 0.0 ? mx * 1e-14 : INFINITY;
+    fence();
+    for (int p = lane; p < npair; p += kWave) {
+      const int i = p / nd, j = p % nd;
+      double v[Q][Q];
+      pair_block<Q, TERM, GFX_FORM_PERQP, double>(rec, i, j, nd, nq, gref, qw, nullptr, v);
+      for (int x = 0; x < Q; ++x)
+        for (int y = 0; y < Q; ++y)
+          if (fabs(v[x][y]) > thr) {
+            const int bit = (i * Q + x) * nl + (j * Q + y);
+            atomicOr(&my[bit >> 5], 1u << (bit & 31));
+          }
+    }
+    fence();
+    for (int t = lane; t < kwords; t += kWave) keep[e * kwords + t] = my[t];
+    if (lane == 0) {
+      thr_out[e] = thr;
+      a.rec[kRecStride * e + 11] = thr;
+      if (a.rec32) a.rec32[kRecStride * e + 11] = (float)thr;
+    }
+    fence();
   }
 }
 
@@ -1006,24 +1077,29 @@ int64_t keep_sig_words(int term, int nd, int qdim, int64_t n_cv) {
 }
 
 template <int ND, int Q, int TERM>
-static hipError_t launch_keep3(hipStream_t s, const RecordArgs &a, const double *Rp, uint64_t *sig, bool check,
-                               double *thr, uint32_t *keep, int kwords) {
+static hipError_t launch_keep3(hipStream_t s, const RecordArgs &a, const double *Rp, const double *gref,
+                               const double *qw, int nq, uint64_t *sig, bool check, double *thr, uint32_t *keep,
+                               int kwords) {
   const unsigned grid = nblocks(a.n_cv, kWave);
   if (check) {
     k_keep<ND, Q, TERM, true><<<grid, kWave * kKeepWaves, 0, s>>>(a, Rp, sig, nullptr, thr);
   } else {
     k_keep<ND, Q, TERM, false><<<grid, kWave * kKeepWaves, 0, s>>>(a, Rp, sig, sig, thr);
     k_keep_words<ND, Q, TERM><<<grid, 256, 0, s>>>(a.n_cv, kwords, sig, keep);
+    k_keep_points<Q, TERM><<<nblocks(a.n_cv, 4 * kWave), 256, 16 * (size_t)kwords, s>>>(a, ND, nq, gref, qw, thr, keep,
+                                                                                        kwords);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_keep(hipStream_t s, int term, int nd, int qdim, const RecordArgs &a, const double *Rp,
-                       uint64_t *sig, bool check, double *thr, uint32_t *keep, int kwords) {
+                       const double *gref, const double *qw, int nq, uint64_t *sig, bool check, double *thr,
+                       uint32_t *keep, int kwords) {
   if (a.n_cv == 0) return hipSuccess;
   constexpr int L = GFX_TERM_LAPLACE, E = GFX_TERM_ISO_ELAST, I = GFX_TERM_ISOTROPIC;
 #define GFX_KEEP(ND, Q, T) \
-  if (nd == ND && qdim == Q && term == T) return launch_keep3<ND, Q, T>(s, a, Rp, sig, check, thr, keep, kwords)
+  if (nd == ND && qdim == Q && term == T) \
+  return launch_keep3<ND, Q, T>(s, a, Rp, gref, qw, nq, sig, check, thr, keep, kwords)
   GFX_KEEP(4, 1, L);
   GFX_KEEP(10, 1, L);
   GFX_KEEP(20, 1, L);
