@@ -228,7 +228,7 @@ struct PolyMatArgs {
   int nsym;                  // symbols of the table
   bool varying;              // an output reads a fem field
   int pmask, rmask;          // slots (bit 0 value, 1 + b gradient) of the test and trial function in use
-  const double *R;           // the reference tensor, 16 x (pairs of base functions), or null
+  const double *R;           // the reference tensor, 16 x (pairs of base functions), or null: by the points
   double *elem;              // n_cv * nr * nc, row r = i qt + a, column c = j qs + b; entries at or
                              // below the element's threshold are 0
   int *err;

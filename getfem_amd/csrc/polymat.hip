@@ -249,6 +249,10 @@ __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
 // Measured, u P2 vector + p P1 on 15^3 x 6 = 20,250 elements: the four blocks
 // 0.107 ms (56 us for the 30 x 30 one), 0.154 ms with R formed by every
 // workgroup; through the points (k_poly_mat) 0.59 ms.
+// An entry within a factor kPrNear of its element's threshold sets bit 16 of
+// the error flag: whether the reference stores it is decided by the roundings
+// of the sum over the points, and the caller has the matrices formed that way.
+constexpr double kPrNear = 4.0;
 constexpr int kPrIters = 8;      // passes of a workgroup where the elements are enough to fill the card
 constexpr int kPrMaxChunk = 512; // elements of a workgroup
 
@@ -356,12 +360,18 @@ __global__ __launch_bounds__(512) void k_poly_ref(PolyMatArgs a, int epb, int it
     __syncthreads();
     if (live) {
       const double m = __longlong_as_double((long long)smax[x]);
-      const double th = m > 0.0 ? 1e-14 * m : INFINITY;
+      const double th = m > 0.0 ? 1e-14 * m : INFINITY, lo = th / kPrNear, hi = th * kPrNear;
       double *dst = a.elem + e * ne + (int64_t)i * QT * nc + j * QS;
+      bool near = false;
 #pragma unroll
       for (int c = 0; c < QT; ++c)
 #pragma unroll
-        for (int b = 0; b < QS; ++b) dst[c * nc + b] = fabs(v[c][b]) > th ? v[c][b] : 0.0;
+        for (int b = 0; b < QS; ++b) {
+          const double x = fabs(v[c][b]);
+          near |= x > lo && x <= hi;
+          dst[c * nc + b] = x > th ? v[c][b] : 0.0;
+        }
+      if (near) atomicOr(a.err, 16);
     }
   }
 }

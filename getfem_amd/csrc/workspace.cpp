@@ -997,8 +997,10 @@ int sc_structure(gfx_workspace *w) {
 }
 
 // the matrix from the structure: sums into the stored entries, the pattern
-// anew where the element matrices give another
-int sc_matrix(gfx_workspace *w) {
+// anew where the element matrices give another; near: an entry is too near
+// its threshold for the form that the element matrices came in, and no matrix
+// is made
+int sc_matrix(gfx_workspace *w, bool &near) {
   ScalarRoute *sc = w->sc;
   hipStream_t s = w->ctx->stream;
   int flag = 0;
@@ -1010,7 +1012,9 @@ int sc_matrix(gfx_workspace *w) {
       sc->nnz = -1;  // the sums so far, over the last matrix's values, are no matrix
       return wfail(w, GFX_E_DEGENERATE_ELEMENT, "Non invertible matrix (degenerate element)");
     }
-    if (sc->nnz >= 0 && !(flag & 4)) return GFX_OK;
+    near = (flag & 16) != 0;
+    if (near) WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
+    if (near || (sc->nnz >= 0 && !(flag & 4))) return GFX_OK;
     sc->nnz = -1;
     Scratch t;
     int64_t *work = t.get<int64_t>((size_t)(2 * sc->n_ent + 1 + scan_tmp_elems(sc->n_ent)));
@@ -1029,15 +1033,21 @@ int sc_matrix(gfx_workspace *w) {
 }
 
 // without the structure: the kept entries of a block in element order
-int sc_emit(gfx_workspace *w, const ScBlock &b, int64_t &total) {
+// (near: as for sc_matrix)
+int sc_emit(gfx_workspace *w, const ScBlock &b, int64_t &total, bool &near) {
   ScalarRoute *sc = w->sc;
   hipStream_t s = w->ctx->stream;
   const int64_t n_cv = sc->mim->mesh->n_cv;
   WHIP(w, launch_poly_count(s, n_cv, b.ne, sc->d_pelem, sc->d_cnt));
   WHIP(w, scan_exclusive_i64(s, sc->d_cnt, sc->d_off, n_cv, sc->d_scan));
   int64_t nb = 0;
+  int flag = 0;
   WHIP(w, hipMemcpyAsync(&nb, sc->d_off + n_cv, 8, hipMemcpyDeviceToHost, s));
+  WHIP(w, hipMemcpyAsync(&flag, sc->d_err, 4, hipMemcpyDeviceToHost, s));
   WHIP(w, hipStreamSynchronize(s));
+  near = (flag & 16) != 0;
+  if (near) WHIP(w, hipMemsetAsync(sc->d_err, 0, 4, s));
+  if (near) return GFX_OK;
   if (total + nb > INT32_MAX) return wfail(w, GFX_E_UNSUPPORTED, "more than 2^31 kept entries");
   int r;
   if ((r = sc_grow(w, total + nb))) return r;
@@ -1103,17 +1113,27 @@ int sc_assemble2(gfx_workspace *w) {
   }
   a.nconst = (int)sc->consts.size(); a.const_off = sc->const_off; a.consts = sc->d_consts; a.nsym = sc->nsym;
   a.err = sc->d_err;
-  int64_t total = 0;
-  for (auto &b : sc->blocks) {
-    a.vt = b.vt; a.vs = b.vs;
-    a.nout = b.p.prog.nout; a.varying = b.varying; a.pmask = b.pmask; a.rmask = b.rmask;
-    a.R = b.d_R;
-    a.mcoef = b.p.d_coef; a.mptr = b.p.d_mptr; a.moff = b.p.d_off; a.msym = b.p.d_sym;
-    a.elem = sc->d_pelem + (structure ? b.base : 0);
-    WHIP(w, launch_poly_mat(s, a));
-    if (!structure && (r = sc_emit(w, b, total))) return r;
-  }
-  if ((r = structure ? sc_matrix(w) : sc_sorted_matrix(w, total))) return r;
+  // through the reference tensors where there are any and, where an entry is
+  // then too near its threshold, by the points
+  bool near = false;
+  do {
+    const bool points = near;
+    near = false;
+    int64_t total = 0;
+    for (auto &b : sc->blocks) {
+      a.vt = b.vt; a.vs = b.vs;
+      a.nout = b.p.prog.nout; a.varying = b.varying; a.pmask = b.pmask; a.rmask = b.rmask;
+      a.R = points ? nullptr : b.d_R;
+      a.mcoef = b.p.d_coef; a.mptr = b.p.d_mptr; a.moff = b.p.d_off; a.msym = b.p.d_sym;
+      a.elem = sc->d_pelem + (structure ? b.base : 0);
+      WHIP(w, launch_poly_mat(s, a));
+      if (!structure && (r = sc_emit(w, b, total, near))) return r;
+      if (near) break;
+    }
+    if (structure) r = sc_matrix(w, near);
+    else if (!near) r = sc_sorted_matrix(w, total);
+    if (r) return r;
+  } while (near);
   if (w->ext) {
     if (w->ext_n != n) return wfail(w, GFX_E_INVALID, "target matrix of another size");
     int flag = 0;

@@ -25,7 +25,7 @@ CASES = {
 }
 
 
-def matrix(ctx, mfu, mfp, mim, expr, scale, data):
+def matrix(ctx, mfu, mfp, mim, expr, scale, data, limit=None):
     ws = GaWorkspace(ctx)
     ws.add_fem_variable("u", mfu, np.zeros(mfu.nbdof()), first=0)
     ws.add_fem_variable("p", mfp, np.zeros(mfp.nbdof()), first=mfu.nbdof())
@@ -35,6 +35,8 @@ def matrix(ctx, mfu, mfp, mim, expr, scale, data):
         # terms without k: multiplied as well
         expr = " + ".join("one*(%s)" % t if "one" not in t else t for t in expr.replace(" - ", " + (-1)*").split(" + "))
     ws.add_expression(expr.replace("k*", "%r*" % scale), mim)
+    if limit is not None:
+        ws.set_structure_limit(limit)
     ws.assembly(2)
     return ws.assembled_matrix_csr()
 
@@ -58,3 +60,44 @@ def test_reference_and_points(ctx, name, n):
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
     # rounding of at most 15 (43 for degree 8) points and 16 slot pairs a value
     assert np.linalg.norm(a[2] - b[2]) <= 1e-13 * np.linalg.norm(b[2])
+
+
+@pytest.mark.parametrize("limit", [None, 0])
+@pytest.mark.parametrize("shape", ["flat", "needle"])
+@pytest.mark.parametrize("ku", [2, 3])
+def test_entries_at_the_threshold(ctx, shape, ku, limit):
+    """Stretched elements, whose entries spread across the threshold: the stored
+    entries are those of the sums over the points, one for one, whether the
+    structure is kept or not."""
+    print("case: polynomial reference tensor, entries at the threshold", shape, ku, limit, flush=True)
+    pts, cvx = meshes.regular_unit_mesh(2, "GT_PK(3,1)")
+    pts = meshes.jitter(pts, 2)
+    expr = "k*Div_u*Div_Test_u + k*Sym(Grad_u):Grad_Test_u + p*Test_p"
+    near = 0
+    for ratio in (1e6, 2e6, 3e6, 4e6, 5e6, 6e6, 7e6, 8e6):
+        mesh = ga.Mesh(ctx, "GT_PK(3,1)", pts * ([ratio, 1.3 * ratio, 1.0] if shape == "flat" else [ratio, 1.0, 1.0]), cvx)
+        mfu, mfp = ga.MeshFem(mesh, "FEM_PK(3,%d)" % ku, 3), ga.MeshFem(mesh, "FEM_PK(3,1)", 1)
+        one = ga.MeshFem(mesh, "FEM_PK_DISCONTINUOUS(3,0)", 1)
+        mim = ga.MeshIm(mesh, "IM_TETRAHEDRON(%d)" % (8 if ku == 3 else 5))
+        a = matrix(ctx, mfu, mfp, mim, expr, 1.5, None, limit)
+        b = matrix(ctx, mfu, mfp, mim, expr, 1.5, one)
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+        assert np.linalg.norm(a[2] - b[2]) <= 1e-13 * np.linalg.norm(b[2])
+        near += np.array_equal(a[2], b[2])
+    assert near  # (some of the bodies have entries near the threshold: the same sums)
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+@pytest.mark.parametrize("jittered", [False, True])
+def test_ordinary_meshes_stay_with_the_reference_tensor(ctx, name, jittered):
+    """The roundings left of entries that are 0 stay clear of the threshold."""
+    from tests.launches import kernels
+    qu, ku, qp, kp, expr = CASES[name]
+    print("case: polynomial reference tensor, ordinary mesh", name, jittered, flush=True)
+    pts, cvx = meshes.regular_unit_mesh(3, "GT_PK(3,1)")
+    mesh = ga.Mesh(ctx, "GT_PK(3,1)", meshes.jitter(pts, 3) if jittered else pts, cvx)
+    mfu = ga.MeshFem(mesh, "FEM_PK(3,%d)" % ku, qu)
+    mfp = ga.MeshFem(mesh, "FEM_PK(3,%d)" % kp, qp)
+    ran = kernels(lambda: matrix(ctx, mfu, mfp, ga.MeshIm(mesh, "IM_TETRAHEDRON(%d)" % (8 if ku == 3 else 5)), expr,
+                                 1.5, None))
+    assert any("k_poly_ref" in x for x in ran) and not any("k_poly_mat" in x for x in ran), ran
