@@ -32,15 +32,15 @@ __device__ __forceinline__ void two_sum_into(double &s, double &c, double b, dou
   c += err + bc;
 }
 
-// r^(n-1) and r^n for the SIMP exponents in use (whole, 1 to 8) by products
-// that carry their rounding errors along, so that both come out within half an
-// ulp (pow is within one; plain products would be off by n / 2): some twenty
-// instructions for both, where pow takes 150 for each.
+// r^(n-1) and r^n for the SIMP exponents in use (whole, 1 to 8) by products,
+// within an ulp as pow's: up to r^3 as they are, beyond it (plain products
+// would be off by n / 2 ulps) with their rounding errors carried along.  Some
+// twenty instructions at most for both, where pow takes 150 for each.
 __device__ __forceinline__ void int_powers(double r, int n, double &rn1, double &rn) {
   double h = 1.0, l = 0.0;  // the product so far and what rounding took from it
   auto step = [&]() {
     const double p = h * r;
-    l = fma(l, r, fma(h, r, -p));
+    if (n > 3) l = fma(l, r, fma(h, r, -p));
     h = p;
   };
   auto value = [&]() { return fabs(h) <= 1.7976931348623157e308 ? h + l : h; };
