@@ -835,7 +835,8 @@ static int plan_bins(gfx_plan *p, const std::vector<uint16_t> &ns, const std::ve
   }
   // a workgroup streams about eight incidences, all in flight at once (an
   // assembly at 48^3: 4.26 ms; with two 4.62, four 4.42, sixteen 4.32); its
-  // accumulators hold at most npw x 27 bmax slots, 216 by this rule
+  // accumulators hold at most 27 max(8, bmax) slots, and launch_gather_emat
+  // refuses what goes beyond 48 KB of them
   for (size_t b = 0; b < p->bins.size(); ++b)
     p->bins[b].npw = std::max(1, std::min({4, 8 / std::max(1, bmax[b]), 64 / std::max(1, p->max_inc)}));
   std::vector<int64_t> cur(p->bins.size());

@@ -390,7 +390,6 @@ hipError_t launch_dof_constraints(hipStream_t s, int64_t n, const int64_t *indpt
                                   double *vals, const uint8_t *fixed, const double *go, const double *pr,
                                   double *rhs, int flags, int *err);
 size_t cg_workspace_doubles(int64_t n, int64_t nnz);
-// nslots (may be null; qb = 3): the nodes' slot counts with the bit of the full nodes
 // Transposition of a CSR matrix with sorted columns (0 < nnz < 2^31) into CSC
 // with sorted rows: a stable sort by column (bits: of the largest column; tmp:
 // csc_sort_bytes).  row, pos, col, pos2: nnz each; vals may be null.
@@ -406,6 +405,7 @@ struct IluData;
 hipError_t gmres_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
                        const double *vals, const double *b, double *x, double rtol, int maxit, int m,
                        double *work, const IluData *ilu, int *iters, double *rel_res);
+// nslots (may be null; qb = 3): the nodes' slot counts with the bit of the full nodes
 hipError_t cg_solve(hipStream_t s, int64_t n, int64_t nnz, const int64_t *indptr, const int32_t *indices,
                     const double *vals, const uint16_t *nslots, const double *b, double *x, double rtol, int maxit,
                     int qb, double *work, int *iters, double *rel_res);
