@@ -342,8 +342,9 @@ __device__ __forceinline__ void nh_phase_b(int t, int64_t e, const double *pd, c
 // way instead of 243), so lane (x, y, z) is in turn a point or a node along
 // each direction and the partial sums pass through the element's own LDS
 // block; only the wavefront's own lanes read it, so no workgroup barrier is
-// needed.  Measured: 38 us at 31^3 elements (a residual alone took 720 us, with
-// the tangent kernel), 168 us with the points' values at 48^3 = 110,592.
+// needed.  Measured in kernel traces: 41 us at 31^3 elements (the tangent kernel,
+// which a residual took before, 835), 49 with the points' values, 172 with them
+// at 48^3 = 110,592.
 constexpr int kNhHalf = 32;
 
 __device__ __forceinline__ void wave_lds_fence() {
