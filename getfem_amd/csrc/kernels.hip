@@ -269,7 +269,9 @@ __global__ void k_inc_sort(int64_t n_nodes, const int32_t *__restrict__ inc_ptr,
 // after them and 15 us of records before and after; an assembly with new
 // coefficients 4.91 -> 0.59 ms.
 constexpr int kKeepWaves = 4;
-constexpr double kKeepNear = 4.0;  // (the two forms differ by up to 13 % of the threshold, P1 to P3, aspect ratios to 1e6)
+// the two forms differ by up to 13 % of the threshold (P1 to P3, aspect ratios
+// to 1e6)
+constexpr double kKeepNear = 4.0;
 
 template <int Q, int TERM>
 __device__ __forceinline__ void keep_block(const double *__restrict__ r, const double (&B)[9], double sa, double sb,

@@ -247,7 +247,7 @@ __global__ __launch_bounds__(kPm) void k_poly_mat(PolyMatArgs a) {
 // double: formed here, by every workgroup in FP64, its roundings were most of
 // the matrix's error.
 // Measured, u P2 vector + p P1 on 15^3 x 6 = 20,250 elements: the four blocks
-// 0.107 ms (56 us for the 30 x 30 one), 0.154 ms with R formed by every
+// 0.109 ms (58 us for the 30 x 30 one), 0.154 ms with R formed by every
 // workgroup; through the points (k_poly_mat) 0.59 ms.
 // An entry within a factor kPrNear of its element's threshold sets bit 16 of
 // the error flag: whether the reference stores it is decided by the roundings

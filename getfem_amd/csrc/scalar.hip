@@ -38,7 +38,7 @@ constexpr int kScRedBlocks = 256;
 // Bound by latency (dependent loads and FP64 chains), so the points go side by
 // side: with a lane per element, 20,250 elements were 317 wavefronts for the
 // whole chip, each with 15 points one after another.  Measured there (u P2
-// vector + p P1): 43 us a variable (58 us with a node's base function loaded
+// vector + p P1): 44 us a variable (58 us with a node's base function loaded
 // again for each component), 222 us with a lane per element.
 template <int G>
 __global__ __launch_bounds__(kScThreads) void k_scalar_elem(ScalarArgs a, int nsym, int nvals) {
